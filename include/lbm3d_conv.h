@@ -48,6 +48,19 @@ int lbm3d_conv3d_fwd(void *stream, const uint16_t *x, const uint16_t *w, const f
                      int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout, int32_t ks,
                      int32_t flags);
 
+/* Fragment order of 3x3x3 weights: BF16 elements of one packed set (cin x cout
+ * x 28 tap slots); lbm3d_conv3d_wpack rounds FP32 weights w[cout][kpad] into
+ * it for the forward convolution (wp) and, when wt is not NULL, for the data
+ * gradient (wt, the flipped weights of lbm3d_conv3d_wflip: a packed convolution
+ * from cout to cin channels). */
+int64_t lbm3d_conv3d_packed_elements(int32_t cin, int32_t cout);
+int lbm3d_conv3d_wpack(void *stream, const float *w, uint16_t *wp, uint16_t *wt, int32_t cin, int32_t cout);
+
+/* lbm3d_conv3d_fwd with ks = 3 and packed weights: the same results, with
+ * weight loads that are whole cache lines. */
+int lbm3d_conv3d_fwd_packed(void *stream, const uint16_t *x, const uint16_t *wp, const float *bias, uint16_t *y,
+                            int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout, int32_t flags);
+
 /* Weights of the data-gradient convolution: wt[ci][tap'*cout + co] =
  * w[co][tap*cin + ci] with tap' = ks^3 - 1 - tap (the kernel flipped and
  * its channel roles swapped), rows padded to lbm3d_conv_kpad(cout, ks). */

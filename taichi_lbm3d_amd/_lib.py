@@ -140,6 +140,9 @@ SIGNATURES = {
     "lbm3d_conv_last_error": (ctypes.c_char_p, []),
     "lbm3d_conv_kpad": (_i32, [_i32, _i32]),
     "lbm3d_conv3d_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
+    "lbm3d_conv3d_packed_elements": (_i64, [_i32, _i32]),
+    "lbm3d_conv3d_wpack": (_int, [_vp, _vp, _vp, _vp, _i32, _i32]),
+    "lbm3d_conv3d_fwd_packed": (_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_conv3d_wflip": (_int, [_vp, _vp, _vp, _i32, _i32, _i32]),
     "lbm3d_conv3d_dgrad": (_int, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_conv3d_wgrad_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32, _i32, _i32]),

@@ -3,11 +3,11 @@
 // ABI is declared in include/lbm3d_conv.h.
 //
 // Forward (and data gradient, which is a forward convolution of the output
-// gradient with flipped weights): GEMM with M = voxels, N = output channels,
+// gradient with flipped weights): GEMM with M = output channels, N = voxels,
 // K = taps x input channels.  Activations are channels-last, so the 8
 // consecutive K values a lane feeds to one MFMA are 8 consecutive channels of
-// one (shifted) voxel: a single 16-byte load.  A workgroup of 4 waves computes
-// 64 voxels x 16*NT channels; each wave owns 16 voxels.
+// one (shifted) voxel: a single 16-byte LDS read.  k_conv3z marches along z
+// (few input channels), k_conv3 walks bricks (many).
 //
 // Weight gradient: GEMM with M = output channels, N = input channels, K =
 // voxels.  Channels-last data must be transposed for that K, so each wave
@@ -26,14 +26,11 @@
 #include "lbm3d_conv.h"
 #include "xcd.h"
 
-#ifndef LBM3D_CONV_TILED
-#define LBM3D_CONV_TILED 1  // 3x3x3 forward convolutions stage the input brick in LDS
-#endif
 #ifndef LBM3D_CONV_XCD_CHUNK
 #define LBM3D_CONV_XCD_CHUNK 64  // tiled forward: runs of consecutive bricks per XCD (shared halos hit L2)
 #endif
-#ifndef LBM3D_CONV_WLDS
-#define LBM3D_CONV_WLDS 1  // tiled forward: the chunk's weights staged in LDS (0: loaded per K step)
+#ifndef LBM3D_CONVZ_XCD_CHUNK
+#define LBM3D_CONVZ_XCD_CHUNK 32  // marching forward: runs of consecutive columns per XCD
 #endif
 #ifndef LBM3D_CONV_WGRAD_TILED
 #define LBM3D_CONV_WGRAD_TILED 1  // weight gradients stage dy and x (with its halo) transposed in LDS
@@ -154,9 +151,9 @@ __device__ __forceinline__ uint16_t to_bf16(float f) {
 // MFMA 16x16x32 lane layout: A (16 x 32): lane l holds row l%16, k = 8*(l/16) .. +7;
 // B (32 x 16): column l%16, the same k; C (16 x 16): column l%16, rows 4*(l/16) .. +3.
 // ---------------------------------------------------------------------------
-// Each wave computes MW fragments of 16 voxels x NT fragments of 16 output
-// channels; the next K chunk's operands are loaded while the current chunk's
-// MFMAs run.
+// 1x1x1 convolutions: each wave computes MW fragments of 16 voxels x NT
+// fragments of 16 output channels; the next K chunk's operands are loaded while
+// the current chunk's MFMAs run.
 template <int NT, int MW>
 __global__ void __launch_bounds__(256)
     k_conv_fwd(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const float *__restrict__ bias,
@@ -247,77 +244,140 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---------------------------------------------------------------------------
-// Forward 3x3x3 convolution with the input tile in LDS.  A workgroup owns a
-// brick of 2 x 8 x 16 output voxels (z, y, x) of one volume and 16 output
-// channels (blockIdx.y).  For each chunk of 16 input channels it stages the
-// brick's halo (4 x 10 x 18 voxels) and the chunk's weight fragments of all 14
-// K steps in LDS in one round trip, so the K loop itself only reads LDS and
-// issues MFMAs.  One K step covers two taps x
-// 16 channels: lane group g takes tap 2s + g/2, channels 8*(g%2) .. +7.  Each
-// wave computes 64 of the brick's voxels (4 fragments of 16).
+// Forward 3x3x3 convolutions.  Both kernels below compute, per wave, fragments
+// of 16 voxels (one x row) x 16 output channels.  K runs over chunks of 16
+// input channels x 27 taps, 14 MFMA steps of two taps each (the 28th slot is
+// zero): lane group g holds tap 2s + g/2, channels 8 (g%2) .. +7.  The weights
+// are the MFMA's A operand (rows = output channels) and the voxels its B
+// operand, so a lane ends up with 4 consecutive channels of one voxel and
+// stores 8 bytes.  The order of the K steps is the same in both, so a result
+// does not depend on which kernel computes it.
 // ---------------------------------------------------------------------------
 constexpr int kBz = 2, kBy = 8, kBx = 16;                  // brick
 constexpr int kHz = kBz + 2, kHy = kBy + 2, kHx = kBx + 2;  // halo
 constexpr int kHalo = kHz * kHy * kHx;                     // 720 voxels
 constexpr int kSteps = 14;                                 // K steps per 16-channel chunk (28 tap slots)
+constexpr int kHaloLoads = 6;                              // 16-byte halo loads per thread (6 x 256 >= 2 x 720)
+constexpr int kHaloBuf = kHaloLoads * 256;                 // 16-byte entries of one LDS buffer
+constexpr int kWRing = 7;                                  // weight fragments in flight (divides kSteps)
 
-// halo-index offset of tap t (dz, dy, dx in -1..1)
+typedef const __attribute__((address_space(1))) void *gptr_t;
+typedef __attribute__((address_space(3))) void *lptr_t;
+
+__device__ const uint32_t conv_zero[4] = {0u, 0u, 0u, 0u};  // what a halo voxel outside the volume reads
+
+// halo-index offset of tap t from the halo voxel of its (-1, -1, -1) neighbour
 __host__ __device__ constexpr int tap_halo_offset(int t) {
-  return (t / 9 - 1) * kHy * kHx + ((t / 3) % 3 - 1) * kHx + (t % 3 - 1);
+  return (t / 9) * kHy * kHx + ((t / 3) % 3) * kHx + (t % 3);
 }
 
-__global__ void __launch_bounds__(256)
-    k_conv_fwd_tiled(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
-                     const float *__restrict__ bias, uint16_t *__restrict__ y, const Vol vol, int cin, int cout,
-                     int kpad, int relu, int nbz, int nby, int nbx, uint32_t nbricks) {
-  __shared__ u32x4 halo[kHalo * 2];  // [voxel][16 channels] as two 16-byte halves
-#if LBM3D_CONV_WLDS
-  __shared__ u32x4 wl[kSteps][64];    // [K step][lane]: the lane's B fragment
-#endif
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// A fragments of the weights: output channels 16 tile .. +15, a lane's row r16,
+// 8 K values.  Packed weights hold [chunk][step][tile][lane] fragments, plain
+// ones rows of kpad; both are a lane offset plus a uniform offset.  The 28th tap
+// slot is zero: stored so when packed, read past the resource's end when not.
+struct Weights {
+  __amdgpu_buffer_rsrc_t r;
+  int off, off_last, cin, cout, packed;
+  __device__ __forceinline__ Weights(const uint16_t *w, int packed_, int cin_, int cout_, int kpad, int tile, int lane)
+      : cin(cin_), cout(cout_), packed(packed_) {
+    const int g = lane >> 4, second = g >> 1;
+    r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(w), (short)0,
+                                          packed ? (cin / 16) * kSteps * cout * 64 : cout * kpad * 2, 0x00020000);
+    off = packed ? (tile * 64 + lane) * 16
+                 : 2 * ((16 * tile + (lane & 15)) * kpad + second * cin + 8 * (g & 1));
+    off_last = !packed && second ? 0x7fffffff : off;
+  }
+  __device__ __forceinline__ u32x4 operator()(int c, int s) const {  // chunk c, step s
+    const int so = packed ? (c * kSteps + s) * cout * 64 : 2 * (2 * s * cin + 16 * c);
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, s == kSteps - 1 ? off_last : off, so, 0);
+    return u32x4{v[0], v[1], v[2], v[3]};
+  }
+};
+
+// bias, ReLU and rounding of 4 channels of one voxel, packed for one 8-byte store
+__device__ __forceinline__ uint2 finish4(const f32x4 acc, const float b4[4], int relu) {
+  uint32_t o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float val = acc[e] + b4[e];
+    if (relu) val = val > 0.f ? val : 0.f;
+    o[e] = to_bf16(val);
+  }
+  return make_uint2(o[0] | (o[1] << 16), o[2] | (o[3] << 16));
+}
+
+// Bricks of one launch: n volumes of nbz x nby x nbx bricks, x fastest.
+struct Bricks {
+  uint32_t n;
+  Div dx, dy, dz;
+};
+
+Bricks make_bricks(int32_t n, int32_t d, int32_t h, int32_t w) {
+  const uint32_t nbz = (uint32_t)(d + kBz - 1) / kBz, nby = (uint32_t)(h + kBy - 1) / kBy,
+                 nbx = (uint32_t)(w + kBx - 1) / kBx;
+  Bricks b;
+  b.n = (uint32_t)n * nbz * nby * nbx;
+  b.dx = make_div(nbx);
+  b.dy = make_div(nby);
+  b.dz = make_div(nbz);
+  return b;
+}
+
+// brick -> volume and first voxel
+__device__ __forceinline__ void brick_origin(const Bricks &bk, uint32_t bi, int &bb, int &z0, int &y0, int &x0) {
+  const uint32_t t = qdiv(bi, bk.dx), u = qdiv(t, bk.dy), v = qdiv(u, bk.dz);
+  x0 = (int)(bi - t * bk.dx.d) * kBx;
+  y0 = (int)(t - u * bk.dy.d) * kBy;
+  z0 = (int)(u - v * bk.dz.d) * kBz;
+  bb = (int)v;
+}
+
+// Many input channels: workgroups loop over bricks of 2 x 8 x 16 output voxels
+// (z, y, x) and compute 16 CT output channels.  Wave w takes channel tile w % CT
+// and, of each brick, the rows y = YR (w / CT) .. +YR-1 (YR = 2 CT) of both
+// planes, MF = 2 YR fragments.  Per chunk of 16 input channels the brick's halo
+// (4 x 10 x 18 voxels) is staged in one of two LDS buffers, straight from
+// memory; the next chunk's (or brick's) halo is loaded while the MFMAs of the
+// current one run, so a chunk has one barrier and no exposed load.  Weight
+// fragments are streamed kWRing - 1 steps ahead.
+// Bound by the MFMAs and the LDS reads of the voxels (one 1 KB fragment per
+// MFMA): 192 -> 64 channels at 2 x 48^3 take 150 us (980 TFLOP/s) against 305
+// for one 16-channel tile per workgroup with its halo loaded behind a barrier.
+template <int CT>
+__global__ void __launch_bounds__(256, 2)
+    k_conv3(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, int packed,
+            const float *__restrict__ bias, uint16_t *__restrict__ y, const Vol vol, int cin, int cout, int kpad,
+            int relu, const Bricks bk) {
+  constexpr int YR = 2 * CT, MF = 2 * YR;
+  // [voxel][16 channels as two 16-byte halves]; two arrays, so that a read of
+  // one never waits for the loads into the other
+  __shared__ u32x4 haloA[kHaloBuf], haloB[kHaloBuf];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r16 = lane & 15;
   const int half = g & 1, second = g >> 1;  // channel half and tap parity of this lane's K values
-  // brick coordinates (bricks x fastest, then y, z, volume)
-  uint32_t bi = LBM3D_CONV_XCD_CHUNK > 0
-                    ? xcd_block(LBM3D_CONV_XCD_CHUNK, blockIdx.x & 7u, blockIdx.x >> 3, nbricks)
-                    : blockIdx.x;
-  if (bi >= nbricks) return;  // padding block of the grid
-  const int bx = (int)(bi % (uint32_t)nbx);
-  bi /= (uint32_t)nbx;
-  const int by = (int)(bi % (uint32_t)nby);
-  bi /= (uint32_t)nby;
-  const int bz = (int)(bi % (uint32_t)nbz);
-  const int bb = (int)(bi / (uint32_t)nbz);
-  const int z0 = bz * kBz, y0 = by * kBy, x0 = bx * kBx;
-  const int co = blockIdx.y * 16 + r16;  // this lane's output channel in the B and C fragments
+  const int tile = blockIdx.y * CT + wave % CT;
+  const int yr0 = (wave / CT) * YR;  // the wave's first brick row
+  const int nch = cin / 16;
   const int64_t vstride = (int64_t)vol.d * vol.h * vol.w;  // voxels per volume
-  const uint16_t *xv = x + (size_t)bb * vstride * cin;     // this brick's volume
-  // The A operand of voxel fragment f, tap t: halo entry 2 * (hc_f + T(t)) + half,
-  // hc_f = the halo index of this lane's voxel (brick-local 64*wave + 16*f + r16:
-  // x = r16, y = 4*(wave&1) + f, z = wave>>1) and T(t) the tap's halo offset.  As
-  // a byte address: ab_f + 32 T(t) with ab_f = 16 (2 hc_f + half).
-  uint32_t ab[4];
+
+  const Weights weight(w, packed, cin, cout, kpad, tile, lane);
+  u32x4 wr[kWRing];
 #pragma unroll
-  for (int f = 0; f < 4; ++f) {
-    const int hc = (((wave >> 1) + 1) * kHy + (4 * (wave & 1) + f + 1)) * kHx + (r16 + 1);
-    ab[f] = (uint32_t)(16 * (2 * hc + half));
-  }
-  f32x4 acc[4];
+  for (int s = 0; s < kWRing - 1; ++s) wr[s] = weight(0, s);
+
+  // halo loads of one brick: entry e = 256 q + thread is half e & 1 of halo
+  // voxel e / 2; its voxel index in the volume, or -1 outside it
+  int hvox[kHaloLoads];
+  const uint16_t *xv = x;
+  auto locate = [&](uint32_t bi) {
+    int bb, z0, y0, x0;
+    brick_origin(bk, bi, bb, z0, y0, x0);
+    xv = x + (size_t)bb * vstride * cin;
+    int t = (int)threadIdx.x;
+    asm volatile("" : "+v"(t));  // decompose the entries here, not once into registers held across the loop
 #pragma unroll
-  for (int f = 0; f < 4; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const char *hb = reinterpret_cast<const char *>(halo);
-  for (int c0 = 0; c0 < cin; c0 += 16) {
-    __syncthreads();  // the previous chunk's LDS reads are done
-#if LBM3D_CONV_WLDS
-    for (int e = threadIdx.x; e < kSteps * 64; e += 256) {
-      const int st = e >> 6, ln = e & 63, lg = ln >> 4;
-      const int tap = 2 * st + (lg >> 1);
-      wl[st][ln] = tap < 27 ? ld16(w + (size_t)(blockIdx.y * 16 + (ln & 15)) * kpad + tap * cin + c0 + 8 * (lg & 1))
-                            : u32x4{0u, 0u, 0u, 0u};
-    }
-#endif
-    // halo: one voxel (its 16 channels, two 16-byte loads) per thread and pass
-    for (int hv = threadIdx.x; hv < kHalo; hv += 256) {
+    for (int q = 0; q < kHaloLoads; ++q) {
+      const int hv = (t >> 1) + 128 * q;
       const int hz = hv / (kHy * kHx), r = hv - hz * (kHy * kHx);
       const int hy = r / kHx, hx = r - hy * kHx;
       int zz = z0 + hz - 1, yy = y0 + hy - 1, xx = x0 + hx - 1;
@@ -326,55 +386,282 @@ __global__ void __launch_bounds__(256)
         yy = wrap1(yy, vol.h);
         xx = wrap1(xx, vol.w);
       }
-      u32x4 lo = u32x4{0u, 0u, 0u, 0u}, hi = lo;
-      if ((unsigned)zz < (unsigned)vol.d && (unsigned)yy < (unsigned)vol.h && (unsigned)xx < (unsigned)vol.w) {
-        const uint16_t *src = xv + (((int64_t)zz * vol.h + yy) * vol.w + xx) * cin + c0;
-        lo = ld16(src);
-        hi = ld16(src + 8);
-      }
-      halo[2 * hv] = lo;
-      halo[2 * hv + 1] = hi;
+      const bool in = hv < kHalo && (unsigned)zz < (unsigned)vol.d && (unsigned)yy < (unsigned)vol.h &&
+                      (unsigned)xx < (unsigned)vol.w;
+      hvox[q] = in ? (zz * vol.h + yy) * vol.w + xx : -1;
     }
-    __syncthreads();
+  };
+  auto load_halo = [&](int c, u32x4 *buf) {
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-      // taps 2s and 2s+1 (this lane: 2s + second); the 28th slot (s = 13,
-      // second half) is zero padding
-      constexpr int kMin = -(kHy * kHx + kHx + 1);  // smallest tap offset
-      const int t1 = 2 * s + 1 < 27 ? 2 * s + 1 : 26;
-      const uint32_t dsec = second ? (uint32_t)(32 * (tap_halo_offset(t1) - tap_halo_offset(2 * s))) : 0u;
-      const uint32_t imm = (uint32_t)(32 * (tap_halo_offset(2 * s) - kMin));
-#if LBM3D_CONV_WLDS
-      const bf16x8 bv = __builtin_bit_cast(bf16x8, wl[s][lane]);
-#else
-      const bf16x8 bv = __builtin_bit_cast(
-          bf16x8, 2 * s + second < 27 ? ld16(w + (size_t)co * kpad + (2 * s + second) * cin + c0 + 8 * half)
-                                      : u32x4{0u, 0u, 0u, 0u});
-#endif
+    for (int q = 0; q < kHaloLoads; ++q) {
+      const uint16_t *src = xv + ((int64_t)hvox[q] * cin + 16 * c + 8 * ((int)threadIdx.x & 1));
+      if (hvox[q] < 0) src = reinterpret_cast<const uint16_t *>(conv_zero);
+      __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)(buf + 256 * q + 64 * wave), 16, 0, 0);
+    }
+  };
+
+  // B fragment f = (z, row), step s: halo byte address a0 + 32 (z kHy kHx + row
+  // kHx + T(2s)), plus for the second half of the lanes 32 (T(2s+1) - T(2s)),
+  // one of three values: the next voxel in x, the next row's or plane's first.
+  const uint32_t a0 = (uint32_t)(16 * (2 * (yr0 * kHx + r16) + half));
+  const uint32_t ax = a0 + (second ? 32u : 0u);
+  const uint32_t ay = a0 + (second ? (uint32_t)(32 * (kHx - 2)) : 0u);
+  const uint32_t az = a0 + (second ? (uint32_t)(32 * (kHy * kHx - 2 * kHx - 2)) : 0u);
+
+  // one chunk's 14 steps from buffer `buf`
+  auto multiply = [&](f32x4 *acc, const u32x4 *buf, int c) {
+    // fragments in groups of 4 (group k: step k / GS, fragments 4 (k % GS) ..
+    // +3), read one group ahead of their MFMAs; the scheduling barriers keep
+    // the compiler from reading further ahead and spilling
+    constexpr int GS = MF / 4, NG = kSteps * GS;
+    const char *const hb = reinterpret_cast<const char *>(buf);
+    u32x4 v[2][4];
+    auto read_group = [&](int k) {
+      const int s = k / GS, t0 = 2 * s, t1 = 2 * s + 1;
+      const uint32_t al = t1 >= 27 ? a0 : (t1 % 9 == 0 ? az : (t1 % 3 == 0 ? ay : ax));
 #pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        u32x4 a = *reinterpret_cast<const u32x4 *>(hb + (ab[f] + (uint32_t)(32 * kMin) + dsec) + imm);
-        if (s == kSteps - 1 && second) a = u32x4{0u, 0u, 0u, 0u};
-        acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), bv, acc[f], 0, 0, 0);
+      for (int j = 0; j < 4; ++j) {
+        const int f = 4 * (k % GS) + j;
+        const uint32_t imm = (uint32_t)(32 * ((f / YR) * kHy * kHx + (f % YR) * kHx + tap_halo_offset(t0)));
+        v[k & 1][j] = *reinterpret_cast<const u32x4 *>(hb + al + imm);
       }
+    };
+    read_group(0);
+#pragma unroll
+    for (int k = 0; k < NG; ++k) {
+      if (k + 1 < NG) read_group(k + 1);
+      const int s = k / GS;
+      if (k % GS == 0) {  // the fragment kWRing - 1 steps on, of this, the next or the next brick's first chunk
+        const int sn = s + kWRing - 1;
+        const int cn = sn < kSteps ? c : (c + 1 < nch ? c + 1 : 0);
+        wr[sn % kWRing] = weight(cn, sn % kSteps);
+      }
+      const bf16x8 av = __builtin_bit_cast(bf16x8, wr[s % kWRing]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int f = 4 * (k % GS) + j;
+        u32x4 vv = v[k & 1][j];
+        if (s == kSteps - 1 && second) vv = u32x4{0u, 0u, 0u, 0u};  // the 28th tap slot
+        acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf16x8, vv), acc[f], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  const uint32_t per_xcd = gridDim.x >> 3;
+  uint32_t it = blockIdx.x >> 3;
+  uint32_t bi = xcd_block(LBM3D_CONV_XCD_CHUNK, blockIdx.x & 7u, it, bk.n);
+  if (bi >= bk.n) return;  // uniform in the workgroup
+  locate(bi);
+  load_halo(0, haloA);
+  while (bi < bk.n) {
+    const uint32_t bcur = bi;
+    f32x4 acc[MF];
+#pragma unroll
+    for (int f = 0; f < MF; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto next_brick = [&](u32x4 *buf) {
+      it += per_xcd;
+      bi = xcd_block(LBM3D_CONV_XCD_CHUNK, blockIdx.x & 7u, it, bk.n);
+      if (bi < bk.n) {
+        locate(bi);
+        load_halo(0, buf);
+      }
+    };
+    // One chunk: wait for this thread's halo loads and (the barrier) everyone's;
+    // all waves are then past their reads of the other buffer, so the next
+    // chunk's (or brick's) loads into it can start.
+    auto chunk = [&](int c, u32x4 *cur, u32x4 *other) {
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+      __syncthreads();
+      if (c + 1 < nch)
+        load_halo(c + 1, other);
+      else if (!(nch & 1))
+        next_brick(other);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(acc, cur, c);
+    };
+    int c = 0;
+    for (; c + 1 < nch; c += 2) {
+      chunk(c, haloA, haloB);
+      chunk(c + 1, haloB, haloA);
+    }
+    if (c < nch) {  // an odd chunk count: the next brick starts in the same buffer, once it has been read
+      chunk(c, haloA, haloB);
+      __syncthreads();
+      next_brick(haloA);
+    }
+    // C layout: lane holds rows (channels) 4g .. 4g+3, column (voxel x) r16
+    int bb, z0, y0, x0;
+    brick_origin(bk, bcur, bb, z0, y0, x0);
+    const int co = 16 * tile + 4 * g;
+    float b4[4] = {0.f, 0.f, 0.f, 0.f};
+    if (bias) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) b4[e] = bias[co + e];
+    }
+    const int oy0 = y0 + yr0, ox = x0 + r16;
+    uint16_t *yv = y + ((size_t)bb * vstride + ((int64_t)z0 * vol.h + oy0) * vol.w + ox) * cout + co;
+#pragma unroll
+    for (int f = 0; f < MF; ++f) {
+      const int fz = f / YR, fy = f % YR;
+      if (z0 + fz < vol.d && oy0 + fy < vol.h && ox < vol.w)
+        *reinterpret_cast<uint2 *>(yv + ((int64_t)fz * vol.h + fy) * vol.w * cout) = finish4(acc[f], b4, relu);
     }
   }
-  // C layout: lane holds rows (voxels) 4g .. 4g+3 of each fragment, column
-  // (channel) r16: voxel x = 4g + e, y = 4*(wave&1) + f, z = wave>>1 of the brick
-  const float bsum = bias ? bias[co] : 0.f;
-  const int oz = z0 + (wave >> 1), oy0 = y0 + 4 * (wave & 1), ox0 = x0 + 4 * g;
-  if (oz >= vol.d) return;
-  uint16_t *yv = y + (size_t)bb * vstride * cout + (((int64_t)oz * vol.h + oy0) * vol.w + ox0) * cout + co;
+}
+
+// Few input channels (16 WCH, WCH <= 3): a march along z.  A workgroup owns a
+// column of TY x 16 output voxels (y, x), 16 CT output channels and a run of
+// planes.  The input planes it needs, with their one-voxel border and all
+// channels, go through a ring of 4 LDS slots: while output plane z is computed
+// from slots z-1, z, z+1, plane z+2 is loaded into the fourth, straight to LDS.
+// Every input plane is read once per column, in whole rows of all channels (the
+// bricks of k_conv3 read each plane twice, 32 bytes of a voxel at a time), and
+// the weights stay in registers.
+// Bound by HBM for 16 -> 16 channels (2 x 192^3: 250 us, 3.6 TB/s of
+// activations, against 480 us before and 360 us in bricks) and by the LDS reads
+// of the voxels for 48 -> 16 (624 us, 940 TFLOP/s, against 1,225 and 841).
+constexpr int kRing = 4;
+
+// Columns of one launch: n volumes of nby x nbx columns (x fastest), each cut
+// into segs runs of zl planes (the slowest index).
+struct Columns {
+  uint32_t n;  // workgroups
+  Div dx, dy, dn;
+  int32_t zl;
+};
+
+template <int WCH, int CT, int TY>
+__global__ void __launch_bounds__(256, 2)
+    k_conv3z(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, int packed,
+             const float *__restrict__ bias, uint16_t *__restrict__ y, const Vol vol, int cout, int kpad, int relu,
+             const Columns ck) {
+  constexpr int cin = 16 * WCH, P = 2 * WCH;          // 16-byte pieces of a voxel
+  constexpr int MF = TY * CT / 4;                     // rows (fragments) of a wave
+  constexpr int E = (TY + 2) * kHx * P;               // pieces of one slot
+  constexpr int NQ = (E + 255) / 256;                 // loads per thread and plane
+  constexpr int VB = 16 * P, RB = kHx * VB;           // bytes of a voxel and of a halo row
+  __shared__ u32x4 ring[kRing * E + P];               // one voxel of slack: the 28th tap slot reads past the end
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, r16 = lane & 15;
+  const int half = g & 1, second = g >> 1;
+  const int tile = blockIdx.y * CT + wave % CT;
+  const int row0 = (wave / CT) * MF;
+
+  const uint32_t b = xcd_block(LBM3D_CONVZ_XCD_CHUNK, blockIdx.x & 7u, blockIdx.x >> 3, ck.n);
+  if (b >= ck.n) return;  // padding block of the grid
+  const uint32_t t1_ = qdiv(b, ck.dx), t2_ = qdiv(t1_, ck.dy), seg = qdiv(t2_, ck.dn);
+  const int x0 = (int)(b - t1_ * ck.dx.d) * 16, y0 = (int)(t1_ - t2_ * ck.dy.d) * TY, bb = (int)(t2_ - seg * ck.dn.d);
+  const int z_begin = (int)seg * ck.zl, z_end = z_begin + ck.zl < vol.d ? z_begin + ck.zl : vol.d;
+  const int64_t vstride = (int64_t)vol.d * vol.h * vol.w, pstride = (int64_t)vol.h * vol.w;
+  const uint16_t *const xv = x + (size_t)bb * vstride * cin;
+
+  // this thread's pieces of a plane: entry e = 256 q + thread is piece e % P of
+  // halo voxel e / P; its byte offset in the plane, the same for every plane
+  uint32_t off[NQ];
+  uint32_t valid = 0;
 #pragma unroll
-  for (int f = 0; f < 4; ++f) {
-    if (oy0 + f >= vol.h) break;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (ox0 + e >= vol.w) break;
-      float val = acc[f][e] + bsum;
-      if (relu) val = val > 0.f ? val : 0.f;
-      yv[((int64_t)f * vol.w + e) * cout] = to_bf16(val);
+  for (int q = 0; q < NQ; ++q) {
+    const int e = 256 * q + (int)threadIdx.x;
+    const int hv = e / P, pc = e % P, hy = hv / kHx, hx = hv % kHx;
+    int yy = y0 + hy - 1, xx = x0 + hx - 1;
+    if (vol.periodic) {
+      yy = wrap1(yy, vol.h);
+      xx = wrap1(xx, vol.w);
     }
+    const bool in = e < E && (unsigned)yy < (unsigned)vol.h && (unsigned)xx < (unsigned)vol.w;
+    off[q] = in ? 2u * ((uint32_t)(yy * vol.w + xx) * (uint32_t)cin + 8u * (uint32_t)pc) : 0u;
+    valid |= (in ? 1u : 0u) << q;
+    if (e < E && !in)  // never loaded: zero in every slot
+      for (int sl = 0; sl < kRing; ++sl) ring[sl * E + e] = u32x4{0u, 0u, 0u, 0u};
+  }
+  auto load_plane = [&](int z, int slot) {
+    if (vol.periodic) z = wrap1(z, vol.d);
+    if ((unsigned)z < (unsigned)vol.d) {
+      const char *base = reinterpret_cast<const char *>(xv + z * pstride * cin);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        if ((valid >> q) & 1u)
+          __builtin_amdgcn_global_load_lds((gptr_t)(base + off[q]), (lptr_t)(ring + (slot * E + 256 * q + 64 * wave)),
+                                           16, 0, 0);
+    } else {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        if (256 * q + (int)threadIdx.x < E) ring[slot * E + 256 * q + threadIdx.x] = u32x4{0u, 0u, 0u, 0u};
+    }
+  };
+  load_plane(z_begin - 1, 0);
+  load_plane(z_begin, 1);
+  load_plane(z_begin + 1, 2);
+
+  const Weights weight(w, packed, cin, cout, kpad, tile, lane);
+  u32x4 wr[WCH * kSteps];
+#pragma unroll
+  for (int i = 0; i < WCH * kSteps; ++i) wr[i] = weight(i / kSteps, i % kSteps);
+  const int co = 16 * tile + 4 * g;
+  float b4[4] = {0.f, 0.f, 0.f, 0.f};
+  if (bias) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b4[e] = bias[co + e];
+  }
+
+  // B fragment f (row row0 + f), step s, chunk c: byte address l0 + slot of the
+  // tap's plane + RB (f + dy) + VB dx + 32 c; the second half of the lanes is one
+  // voxel on, or one row less two voxels on (steps whose second tap starts a
+  // row), or in the next plane (step 4)
+  const uint32_t l0 = (uint32_t)((row0 * kHx + r16) * VB + 16 * half);
+  const uint32_t dx1 = second ? (uint32_t)VB : 0u, dy1 = second ? (uint32_t)(RB - 2 * VB) : 0u;
+  const char *const lds = reinterpret_cast<const char *>(ring);
+  const int oy0 = y0 + row0, ox = x0 + r16;
+  uint16_t *yv = y + ((size_t)bb * vstride + ((int64_t)z_begin * vol.h + oy0) * vol.w + ox) * cout + co;
+  int slot = 0;  // of plane z - 1
+  for (int z = z_begin; z < z_end; ++z) {
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this thread's loads of plane z + 1
+    __syncthreads();                     // everyone's; and plane z - 2 has been read by all
+    if (z + 1 < z_end) load_plane(z + 2, (slot + 3) & 3);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t sA = (uint32_t)slot * (E * 16), sB = (uint32_t)((slot + 1) & 3) * (E * 16),
+                   sC = (uint32_t)((slot + 2) & 3) * (E * 16);
+    const uint32_t ax = l0 + sA + dx1, ay = l0 + sA + dy1, a4 = l0 + (second ? sB : sA + (uint32_t)(2 * RB + 2 * VB));
+    const uint32_t bx = l0 + sB + dx1, by = l0 + sB + dy1, cx = l0 + sC + dx1, cy = l0 + sC + dy1;
+    f32x4 acc[MF];
+#pragma unroll
+    for (int f = 0; f < MF; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int NI = WCH * kSteps * MF, NG = NI / 4;  // MFMAs, in groups of 4
+    static_assert(NI % 4 == 0, "whole groups");
+    u32x4 v[2][4];
+    auto read_group = [&](int k) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = 4 * k + j, f = i % MF, s = (i / MF) % kSteps, c = i / (MF * kSteps);
+        const int t = 2 * s, r = t % 9, dy = r / 3, dx = r % 3;  // first tap, in its plane
+        const bool row = (2 * s + 1) % 3 == 0;                    // the second tap starts a row
+        const uint32_t a = s == 4 ? a4 : (t < 9 ? (row ? ay : ax) : (t < 18 ? (row ? by : bx) : (row && s < 13 ? cy : cx)));
+        const uint32_t imm = (uint32_t)((s == 4 ? f * RB : (f + dy) * RB + dx * VB) + 32 * c);
+        v[k & 1][j] = *reinterpret_cast<const u32x4 *>(lds + a + imm);
+      }
+    };
+    read_group(0);
+#pragma unroll
+    for (int k = 0; k < NG; ++k) {
+      if (k + 1 < NG) read_group(k + 1);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = 4 * k + j, f = i % MF, s = (i / MF) % kSteps;
+        u32x4 vv = v[k & 1][j];
+        if (s == kSteps - 1 && second) vv = u32x4{0u, 0u, 0u, 0u};  // the 28th tap slot
+        acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wr[i / MF]),
+                                                         __builtin_bit_cast(bf16x8, vv), acc[f], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // C layout: lane holds rows (channels) 4g .. 4g+3, column (voxel x) r16
+#pragma unroll
+    for (int f = 0; f < MF; ++f)
+      if (oy0 + f < vol.h && ox < vol.w)
+        *reinterpret_cast<uint2 *>(yv + (int64_t)f * vol.w * cout) = finish4(acc[f], b4, relu);
+    yv += pstride * cout;
+    slot = (slot + 1) & 3;
   }
 }
 
@@ -392,6 +679,33 @@ __global__ void k_wflip(const uint16_t *__restrict__ w, uint16_t *__restrict__ w
     val = w[(size_t)co * kpad_in + tap * cin + ci];
   }
   wt[i] = val;
+}
+
+// FP32 weights w[cout][kpad] (3x3x3) to BF16 MFMA fragments: wp in k_conv3's
+// packed order, [chunk][step][tile][lane][8], and, when wt is not null, the
+// flipped weights of the data gradient (k_wflip's) in the same order.  One
+// thread per lane of a fragment; the 28th tap slot is zero.
+__global__ void __launch_bounds__(256) k_wpack(const float *__restrict__ w, uint16_t *__restrict__ wp,
+                                               uint16_t *__restrict__ wt, int cin, int cout, int kpad) {
+  const int frags = kSteps * (cin / 16) * (cout / 16);  // the same for both
+  int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  const bool flip = i >= frags * 64;
+  if (flip) i -= frags * 64;
+  if (i >= frags * 64 || (flip && !wt)) return;
+  const int ci_n = flip ? cout : cin, co_n = flip ? cin : cout;  // of the convolution the fragments are for
+  const int lane = i & 63, fr = i >> 6;
+  const int tile = fr % (co_n / 16), cs = fr / (co_n / 16);
+  const int s = cs % kSteps, c = cs / kSteps;
+  const int co = 16 * tile + (lane & 15), g = lane >> 4;
+  const int tap = 2 * s + (g >> 1), ci = 16 * c + 8 * (g & 1);
+  uint16_t *dst = (flip ? wt : wp) + (size_t)i * 8;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    uint16_t v = 0;
+    if (tap < 27)
+      v = to_bf16(flip ? w[(size_t)(ci + e) * kpad + (26 - tap) * cin + co] : w[(size_t)co * kpad + tap * cin + ci + e]);
+    dst[e] = v;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -839,6 +1153,85 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+template <int CT>
+void launch_conv3_bricks(hipStream_t s, const uint16_t *x, const uint16_t *w, int packed, const float *bias,
+                         uint16_t *y, const Vol &vol, int cin, int cout, int kpad, int relu, const Bricks &bk) {
+  const unsigned gy = (unsigned)(cout / (16 * CT));
+  // persistent workgroups: as many as are resident (3 per CU by LDS, 2 where the
+  // kernel takes more than 168 VGPRs), in whole groups of 8 XCDs
+  const int64_t resident = (CT <= 2 ? 768 : 512) / gy;
+  int64_t gx = xcd_grid(bk.n, LBM3D_CONV_XCD_CHUNK);
+  if (gx > resident) gx = resident & ~int64_t(7);
+  if (gx < 8) gx = 8;
+  k_conv3<CT><<<dim3((unsigned)gx, gy), 256, 0, s>>>(x, w, packed, bias, y, vol, cin, cout, kpad, relu, bk);
+}
+
+template <int WCH, int CT, int TY>
+void launch_conv3z(hipStream_t s, const uint16_t *x, const uint16_t *w, int packed, const float *bias, uint16_t *y,
+                   const Vol &vol, int cout, int kpad, int relu) {
+  const int64_t nbx = (vol.w + 15) / 16, nby = (vol.h + TY - 1) / TY, gy = cout / (16 * CT);
+  const int64_t cols = nbx * nby * vol.n;
+  // planes per workgroup: the cut that takes the fewest rounds of resident
+  // workgroups times planes (3 extra planes of border and start-up per run)
+  const int64_t slots = 256 * (WCH == 1 ? 3 : 2);
+  int64_t best = 1, best_cost = INT64_MAX;
+  for (int64_t segs = 1; segs <= vol.d; ++segs) {
+    const int64_t cost = ((cols * segs * gy + slots - 1) / slots) * ((vol.d + segs - 1) / segs + 3);
+    if (cost < best_cost) best = segs, best_cost = cost;
+    if (cols * segs * gy > 32 * slots) break;
+  }
+  Columns ck;
+  ck.zl = (int32_t)((vol.d + best - 1) / best);
+  const int64_t segs = (vol.d + ck.zl - 1) / ck.zl;
+  ck.n = (uint32_t)(cols * segs);
+  ck.dx = make_div((uint32_t)nbx);
+  ck.dy = make_div((uint32_t)nby);
+  ck.dn = make_div((uint32_t)vol.n);
+  const dim3 grid((unsigned)xcd_grid(ck.n, LBM3D_CONVZ_XCD_CHUNK), (unsigned)gy);
+  k_conv3z<WCH, CT, TY><<<grid, 256, 0, s>>>(x, w, packed, bias, y, vol, cout, kpad, relu, ck);
+}
+
+int launch_conv3(hipStream_t s, const uint16_t *x, const uint16_t *w, int packed, const float *bias, uint16_t *y,
+                 const Vol &vol, int cin, int cout, int kpad, int relu) {
+  const int tiles = cout / 16;
+  const Bricks bk = make_bricks(vol.n, vol.d, vol.h, vol.w);
+  if (xcd_grid(bk.n, LBM3D_CONV_XCD_CHUNK) > (int64_t)(UINT32_MAX / 256u))
+    return cfail(LBM3D_ESIZE, "too many bricks for one launch");
+  // March along z where the weights of all input channels fit the registers
+  // (16 channels, or up to 48 for at most two channel tiles per workgroup) and a
+  // plane's byte offsets fit 32 bits; bricks else.  Where both fit: 32 -> 32 at
+  // 2 x 96^3 119-123 us either way, 32 -> 64 at 2 x 48^3 35 us either way, 16 -> 32
+  // at 2 x 96^3 65 us marching and 79 in bricks.
+  if ((cin == 16 || (cin <= 48 && tiles % 4 != 0)) && (int64_t)vol.h * vol.w * cin < ((int64_t)1 << 31)) {
+#define LBM3D_CONV3Z(WCH, CT, TY) launch_conv3z<WCH, CT, TY>(s, x, w, packed, bias, y, vol, cout, kpad, relu)
+    if (tiles % 4 == 0) {
+      LBM3D_CONV3Z(1, 4, 8);
+    } else if (tiles % 2 == 0) {
+      if (cin == 16) LBM3D_CONV3Z(1, 2, 8);
+      else if (cin == 32) LBM3D_CONV3Z(2, 2, 8);
+      else LBM3D_CONV3Z(3, 2, 8);
+    } else {
+      if (cin == 16) LBM3D_CONV3Z(1, 1, 16);
+      else if (cin == 32) LBM3D_CONV3Z(2, 1, 8);
+      else LBM3D_CONV3Z(3, 1, 8);
+    }
+#undef LBM3D_CONV3Z
+    return ccheck("lbm3d_conv3d_fwd");
+  }
+  // as many channel tiles per workgroup (the halo is loaded once per workgroup)
+  // as leave 2 workgroups per CU: 128 -> 128 channels at 2 x 16^3 take 17 us with
+  // 256 workgroups of one tile, 32 us with 64 of four
+  int ct = tiles % 4 == 0 ? 4 : (tiles % 2 == 0 ? 2 : 1);
+  while (ct > 1 && (int64_t)bk.n * (tiles / ct) < 512) ct >>= 1;
+  if (ct == 4)
+    launch_conv3_bricks<4>(s, x, w, packed, bias, y, vol, cin, cout, kpad, relu, bk);
+  else if (ct == 2)
+    launch_conv3_bricks<2>(s, x, w, packed, bias, y, vol, cin, cout, kpad, relu, bk);
+  else
+    launch_conv3_bricks<1>(s, x, w, packed, bias, y, vol, cin, cout, kpad, relu, bk);
+  return ccheck("lbm3d_conv3d_fwd");
+}
+
 int relu_bias_plan(int64_t voxels, int C, int64_t &chunks, int64_t &per_block) {
   chunks = voxels * C / 8;
   int64_t blocks = (chunks + 256 * 8 - 1) / (256 * 8);  // about 8 chunks per thread
@@ -872,15 +1265,7 @@ int lbm3d_conv3d_fwd(void *stream, const uint16_t *x, const uint16_t *w, const f
   const Vol vol = make_vol(n, d, h, wd, (flags & LBM3D_CONV_PERIODIC) ? 1 : 0);
   const int kpad = lbm3d_conv_kpad(cin, ks);
   hipStream_t s = (hipStream_t)stream;
-  if (ks == 3 && LBM3D_CONV_TILED) {
-    const int nbz = (d + kBz - 1) / kBz, nby = (h + kBy - 1) / kBy, nbx = (wd + kBx - 1) / kBx;
-    const int64_t bricks = (int64_t)n * nbz * nby * nbx;
-    const int64_t grid = xcd_grid(bricks, LBM3D_CONV_XCD_CHUNK);
-    if (grid > (int64_t)(UINT32_MAX / 256u)) return cfail(LBM3D_ESIZE, "too many bricks for one launch");
-    k_conv_fwd_tiled<<<dim3((unsigned)grid, cout / 16), 256, 0, s>>>(x, w, bias, y, vol, cin, cout, kpad, relu, nbz,
-                                                                   nby, nbx, (uint32_t)bricks);
-    return ccheck("lbm3d_conv3d_fwd");
-  }
+  if (ks == 3) return launch_conv3(s, x, w, 0, bias, y, vol, cin, cout, kpad, relu);
   constexpr int MW = LBM3D_CONV_MW;
   const unsigned gx = (vol.vox + 64u * MW - 1u) / (64u * MW);
   if (cout % 64 == 0)
@@ -890,6 +1275,32 @@ int lbm3d_conv3d_fwd(void *stream, const uint16_t *x, const uint16_t *w, const f
   else
     k_conv_fwd<1, MW><<<dim3(gx, cout / 16), 256, 0, s>>>(x, w, bias, y, vol, cin, cout, ks, kpad, relu);
   return ccheck("lbm3d_conv3d_fwd");
+}
+
+int64_t lbm3d_conv3d_packed_elements(int32_t cin, int32_t cout) {
+  if (check_conv(1, 1, 1, 1, cin, cout, 3)) return 0;
+  return (int64_t)kSteps * 2 * cin * cout;
+}
+
+int lbm3d_conv3d_wpack(void *stream, const float *w, uint16_t *wp, uint16_t *wt, int32_t cin, int32_t cout) {
+  int rc = check_conv(1, 1, 1, 1, cin, cout, 3);
+  if (rc) return rc;
+  if (!w || !wp) return cfail(LBM3D_EINVAL, "NULL tensor");
+  const int lanes = kSteps * (cin / 16) * (cout / 16) * 64 * (wt ? 2 : 1);
+  k_wpack<<<(unsigned)((lanes + 255) / 256), 256, 0, (hipStream_t)stream>>>(w, wp, wt, cin, cout,
+                                                                          lbm3d_conv_kpad(cin, 3));
+  return ccheck("lbm3d_conv3d_wpack");
+}
+
+int lbm3d_conv3d_fwd_packed(void *stream, const uint16_t *x, const uint16_t *wp, const float *bias, uint16_t *y,
+                            int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout, int32_t flags) {
+  int rc = check_conv(n, d, h, wd, cin, cout, 3);
+  if (rc) return rc;
+  if (!x || !wp || !y) return cfail(LBM3D_EINVAL, "NULL tensor");
+  if (flags & ~(LBM3D_CONV_RELU | LBM3D_CONV_PERIODIC)) return cfail(LBM3D_EINVAL, "unknown flag bits");
+  return launch_conv3((hipStream_t)stream, x, wp, 1, bias, y,
+                      make_vol(n, d, h, wd, (flags & LBM3D_CONV_PERIODIC) ? 1 : 0), cin, cout,
+                      lbm3d_conv_kpad(cin, 3), (flags & LBM3D_CONV_RELU) ? 1 : 0);
 }
 
 int lbm3d_conv3d_wflip(void *stream, const uint16_t *w, uint16_t *wt, int32_t cin, int32_t cout, int32_t ks) {

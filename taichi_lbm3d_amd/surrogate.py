@@ -78,6 +78,31 @@ def conv_dgrad(dy, w_bf16, cin, ks):
     return dx
 
 
+def pack_weights(w, flip: bool):
+    """FP32 3x3x3 weights (cout, kpad) as BF16 MFMA fragments: (forward, data
+    gradient or None)."""
+    torch = _torch()
+    lib = _lib.lib()
+    cout, cin = w.shape[0], w.shape[1] // 27
+    cin -= cin % 16
+    n = lib.size("lbm3d_conv3d_packed_elements", cin, cout)
+    wp = torch.empty(n, dtype=torch.bfloat16, device=w.device)
+    wt = torch.empty(n, dtype=torch.bfloat16, device=w.device) if flip else None
+    lib.call("lbm3d_conv3d_wpack", _stream(w.device), _vp(w), _vp(wp), _vp(wt) if flip else None, cin, cout)
+    return wp, wt
+
+
+def conv_fwd_packed(x, wp, bias, cout, relu, periodic=False):
+    """conv_fwd with ks = 3 and the fragments of pack_weights."""
+    torch = _torch()
+    n, d, h, wd, cin = x.shape
+    y = torch.empty((n, d, h, wd, cout), dtype=torch.bfloat16, device=x.device)
+    flags = (CONV_RELU if relu else 0) | (CONV_PERIODIC if periodic else 0)
+    _lib.lib().call("lbm3d_conv3d_fwd_packed", _stream(x.device), _vp(x), _vp(wp),
+                    _vp(bias) if bias is not None else None, _vp(y), n, d, h, wd, cin, cout, flags)
+    return y
+
+
 def conv_wgrad(x, dy, ks):
     torch = _torch()
     n, d, h, wd, cin = x.shape
@@ -119,8 +144,13 @@ def _make_conv_function():
         @staticmethod
         def forward(ctx, x, w, b, ks, relu, need_dx, periodic):
             x = x.contiguous()
-            wb = w.to(torch.bfloat16).contiguous()
-            y = conv_fwd(x, wb, b, w.shape[0], ks, relu, periodic)
+            if ks == 3:
+                w = (w if w.dtype == torch.float32 else w.to(torch.bfloat16).float()).contiguous()
+                wp, wb = pack_weights(w, need_dx and ctx.needs_input_grad[0])
+                y = conv_fwd_packed(x, wp, b, w.shape[0], relu, periodic)
+            else:
+                wb = w.to(torch.bfloat16).contiguous()
+                y = conv_fwd(x, wb, b, w.shape[0], ks, relu, periodic)
             ctx.save_for_backward(x, wb, y if relu else None)
             ctx.ks, ctx.relu, ctx.need_dx, ctx.periodic = ks, relu, need_dx, periodic
             return y
@@ -132,7 +162,10 @@ def _make_conv_function():
             x, wb, y = ctx.saved_tensors
             g, db = relu_bias_grad(gy.contiguous().to(torch.bfloat16), y if ctx.relu else None)
             dw = conv_wgrad(x, g, ctx.ks)
-            dx = conv_dgrad(g, wb, x.shape[-1], ctx.ks) if ctx.need_dx else None
+            dx = None
+            if ctx.need_dx and ctx.needs_input_grad[0]:
+                dx = (conv_fwd_packed(g, wb, None, x.shape[-1], False) if ctx.ks == 3
+                      else conv_dgrad(g, wb, x.shape[-1], ctx.ks))
             return dx, dw, db, None, None, None, None
 
     return Conv3dMFMA
