@@ -99,6 +99,14 @@ int lbm3d_relu_bias_grad(void *stream, const uint16_t *g, const uint16_t *y, uin
 int lbm3d_distance_periodic(void *stream, const int8_t *solid, float *dist, float *work, int32_t n, int32_t d,
                             int32_t h, int32_t w, int32_t margin);
 
+/* The surrogate's inputs in one go: per voxel the mask (1 where solid != 0) and
+ * the periodic distance divided by `scale` (a power of two), as FP32 pairs
+ * out[v][2], or with network != 0 as the first two of 16 BF16 channels
+ * out[v][16] (rounded to nearest even, the others zero).  `work` holds
+ * 2 * n * d * h * w floats. */
+int lbm3d_surrogate_inputs(void *stream, const int8_t *solid, void *out, int network, float scale, float *work,
+                           int32_t n, int32_t d, int32_t h, int32_t w, int32_t margin);
+
 #ifdef __cplusplus
 }
 #endif

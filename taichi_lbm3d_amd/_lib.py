@@ -148,6 +148,7 @@ SIGNATURES = {
     "lbm3d_conv3d_wgrad_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_conv3d_wgrad": (_int, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _sz]),
     "lbm3d_distance_periodic": (_int, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32]),
+    "lbm3d_surrogate_inputs": (_int, [_vp, _vp, _vp, _int, ctypes.c_float, _vp, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_relu_bias_grad_workspace_bytes": (_sz, [_i64, _i32]),
     "lbm3d_relu_bias_grad": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _vp, _sz]),
     # include/lbm3d_io.h
@@ -187,7 +188,7 @@ class Lib:
     def call(self, name: str, *args):
         rc = getattr(self.cdll, name)(*args)
         if rc != 0:
-            conv = name.startswith("lbm3d_conv") or name == "lbm3d_distance_periodic"
+            conv = name.startswith("lbm3d_conv") or name in ("lbm3d_distance_periodic", "lbm3d_surrogate_inputs")
             msg = self.cdll.lbm3d_conv_last_error() if conv else None
             detail = msg.decode() if msg else self.last_error()
             raise LbmError(f"{name} failed ({rc}): {detail}")

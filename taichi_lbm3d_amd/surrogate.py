@@ -287,33 +287,52 @@ def periodic_distance(solid, margin: int = 24, device=None):
     `solid` is a (X, Y, Z) or (N, X, Y, Z) array or device tensor (nonzero =
     solid); returns a float32 tensor of that shape on the GPU."""
     torch = _torch()
+    s = _solid_bytes(solid, device, "periodic_distance")
+    dist = torch.empty(s.shape, dtype=torch.float32, device=s.device)
+    work = torch.empty_like(dist)
+    _lib.lib().call("lbm3d_distance_periodic", _stream(s.device), _vp(s), _vp(dist), _vp(work), *_volumes(s), margin)
+    return dist
+
+
+def _solid_bytes(solid, device, what):
+    """A geometry as contiguous int8 on the GPU (nonzero = solid); one-byte types are taken as they are."""
+    torch = _torch()
     if torch.is_tensor(solid):
-        s = (solid != 0).to(torch.int8)
-        if device is not None:
-            s = s.to(device)
+        s = solid if device is None else solid.to(device)
+        if s.dtype in (torch.bool, torch.uint8):
+            s = s.view(torch.int8)
+        elif s.dtype != torch.int8:
+            s = (s != 0).to(torch.int8)
     else:
         s = torch.as_tensor(np.asarray(solid) != 0, device=device).to(torch.int8)
     if s.device.type != "cuda":
-        raise RuntimeError("periodic_distance runs on the GPU (lbm3d_distance_periodic)")
-    s = s.contiguous()
-    shape = s.shape
-    vol = shape if s.dim() == 4 else (1,) + tuple(shape)
-    dist = torch.empty(shape, dtype=torch.float32, device=s.device)
-    work = torch.empty_like(dist)
-    _lib.lib().call("lbm3d_distance_periodic", _stream(s.device), _vp(s), _vp(dist), _vp(work), *vol, margin)
-    return dist
+        raise RuntimeError(f"{what} runs on the GPU (lbm3d_distance_periodic)")
+    return s.contiguous()
+
+
+def _volumes(s):
+    return tuple(s.shape) if s.dim() == 4 else (1,) + tuple(s.shape)
+
+
+def _inputs(s, network: bool, margin: int = 24):
+    torch = _torch()
+    out = torch.empty(tuple(s.shape) + ((CIN_PAD,) if network else (2,)),
+                      dtype=torch.bfloat16 if network else torch.float32, device=s.device)
+    work = torch.empty(2 * s.numel(), dtype=torch.float32, device=s.device)
+    _lib.lib().call("lbm3d_surrogate_inputs", _stream(s.device), _vp(s), _vp(out), int(network), DIST_SCALE,
+                    _vp(work), *_volumes(s), margin)
+    return out
 
 
 def make_inputs(solid, device=None):
     """(X, Y, Z, 2) float32 tensor on the device: solid mask and distance / DIST_SCALE.
     `solid` is a numpy array or a device tensor (nonzero = solid)."""
-    torch = _torch()
-    if torch.is_tensor(solid):
-        s = solid.to(device) if device is not None else solid
-        s = s != 0
-    else:
-        s = torch.as_tensor(np.asarray(solid) != 0, device=device)
-    return torch.stack([s.float(), periodic_distance(s) / DIST_SCALE], dim=-1)
+    return _inputs(_solid_bytes(solid, device, "make_inputs"), False)
+
+
+def network_inputs(solids):
+    """to_network_input(make_inputs(.)) of (N, X, Y, Z) geometries in one go."""
+    return _inputs(_solid_bytes(solids, None, "network_inputs"), True)
 
 
 def make_targets(rho, v, solid, fx, nu_eff):
@@ -410,11 +429,11 @@ def predict(net, solids, fx, nu_eff, batch: int = 2, wrap=None, density=False):
     with torch.no_grad():
         for b0 in range(0, len(solids), batch):
             sol = torch.stack([_device_solid(s, net.device) for s in solids[b0:b0 + batch]])
-            dist = periodic_distance(sol)
-            inp = torch.stack([sol.float(), dist / DIST_SCALE], dim=-1)
-            if not wrap:
-                inp = torch.stack([periodic_pad(t, pads) for t in inp])
-            pred = net(to_network_input(inp), periodic=wrap)
+            if wrap:
+                pred = net(network_inputs(sol), periodic=True)
+            else:
+                inp = torch.stack([periodic_pad(t, pads) for t in make_inputs(sol)])
+                pred = net(to_network_input(inp), periodic=False)
             (X, Y, Z), (px, py, pz) = shape, (p[0] for p in pads)
             for i in range(sol.shape[0]):
                 core = pred[i, px:px + X, py:py + Y, pz:pz + Z]
