@@ -61,6 +61,29 @@ int lbm3d_conv3d_wpack(void *stream, const float *w, uint16_t *wp, uint16_t *wt,
 int lbm3d_conv3d_fwd_packed(void *stream, const uint16_t *x, const uint16_t *wp, const float *bias, uint16_t *y,
                             int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout, int32_t flags);
 
+/* lbm3d_conv3d_fwd_packed with ReLU that also writes the 2 x 2 x 2 maximum of y
+ * to pool (n volumes of d/2 x h/2 x wd/2 voxels, cout channels; even extents). */
+int lbm3d_conv3d_fwd_pool(void *stream, const uint16_t *x, const uint16_t *wp, const float *bias, uint16_t *y,
+                          uint16_t *pool, int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout,
+                          int32_t flags);
+
+/* lbm3d_conv3d_fwd_packed of the concatenation of `low`, upsampled (nearest, by
+ * 2: n volumes of d/2 x h/2 x wd/2 voxels, c_low channels), and `skip` (c_skip
+ * channels at full extents, all even), which is never built. */
+int lbm3d_conv3d_fwd_up(void *stream, const uint16_t *low, const uint16_t *skip, const uint16_t *wp,
+                        const float *bias, uint16_t *y, int32_t n, int32_t d, int32_t h, int32_t wd, int32_t c_low,
+                        int32_t c_skip, int32_t cout, int32_t flags);
+/* Its gradients: the data gradient of the two parts from the flipped packed
+ * weights (d_low_full, c_low channels at full extents, is scratch; d_low its
+ * BF16 sums over 2 x 2 x 2 blocks), and the weight gradient (workspace of
+ * lbm3d_conv3d_wgrad_workspace_bytes for c_low + c_skip channels). */
+int lbm3d_conv3d_dgrad_up(void *stream, const uint16_t *dy, const uint16_t *wt, uint16_t *d_low_full, uint16_t *d_low,
+                          uint16_t *d_skip, int32_t n, int32_t d, int32_t h, int32_t wd, int32_t c_low,
+                          int32_t c_skip, int32_t cout);
+int lbm3d_conv3d_wgrad_up(void *stream, const uint16_t *low, const uint16_t *skip, const uint16_t *dy, float *dw,
+                          int32_t n, int32_t d, int32_t h, int32_t wd, int32_t c_low, int32_t c_skip, int32_t cout,
+                          void *workspace, size_t workspace_bytes);
+
 /* Weights of the data-gradient convolution: wt[ci][tap'*cout + co] =
  * w[co][tap*cin + ci] with tap' = ks^3 - 1 - tap (the kernel flipped and
  * its channel roles swapped), rows padded to lbm3d_conv_kpad(cout, ks). */
@@ -89,6 +112,14 @@ int lbm3d_conv3d_wgrad(void *stream, const uint16_t *x, const uint16_t *dy, floa
 size_t lbm3d_relu_bias_grad_workspace_bytes(int64_t voxels, int32_t c);
 int lbm3d_relu_bias_grad(void *stream, const uint16_t *g, const uint16_t *y, uint16_t *dz, float *db,
                          int64_t voxels, int32_t c, void *workspace, size_t workspace_bytes);
+
+/* lbm3d_relu_bias_grad of a ReLU output y that lbm3d_conv3d_fwd_pool also pooled:
+ * the gradient is g plus g_pool shared evenly, in BF16, among the voxels of each
+ * 2 x 2 x 2 block that attain its maximum, rounded to BF16.  `share` is scratch
+ * of pooled's size; workspace as lbm3d_relu_bias_grad's for n*d*h*w voxels. */
+int lbm3d_relu_pool_grad(void *stream, const uint16_t *g, const uint16_t *y, const uint16_t *pooled,
+                         const uint16_t *g_pool, uint16_t *dz, float *db, int32_t n, int32_t d, int32_t h, int32_t w,
+                         int32_t c, uint16_t *share, void *workspace, size_t workspace_bytes);
 
 /* The surrogate's distance input: dist[v] = Euclidean distance from voxel v to
  * the nearest solid voxel (solid[v] != 0) of its volume, with every volume

@@ -143,6 +143,11 @@ SIGNATURES = {
     "lbm3d_conv3d_packed_elements": (_i64, [_i32, _i32]),
     "lbm3d_conv3d_wpack": (_int, [_vp, _vp, _vp, _vp, _i32, _i32]),
     "lbm3d_conv3d_fwd_packed": (_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
+    "lbm3d_conv3d_fwd_pool": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
+    "lbm3d_conv3d_fwd_up": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
+    "lbm3d_conv3d_dgrad_up": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
+    "lbm3d_conv3d_wgrad_up": (_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _sz]),
+    "lbm3d_relu_pool_grad": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _sz]),
     "lbm3d_conv3d_wflip": (_int, [_vp, _vp, _vp, _i32, _i32, _i32]),
     "lbm3d_conv3d_dgrad": (_int, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_conv3d_wgrad_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32, _i32, _i32]),
@@ -188,7 +193,8 @@ class Lib:
     def call(self, name: str, *args):
         rc = getattr(self.cdll, name)(*args)
         if rc != 0:
-            conv = name.startswith("lbm3d_conv") or name in ("lbm3d_distance_periodic", "lbm3d_surrogate_inputs")
+            conv = name.startswith("lbm3d_conv") or name in ("lbm3d_distance_periodic", "lbm3d_surrogate_inputs",
+                                                             "lbm3d_relu_bias_grad", "lbm3d_relu_pool_grad")
             msg = self.cdll.lbm3d_conv_last_error() if conv else None
             detail = msg.decode() if msg else self.last_error()
             raise LbmError(f"{name} failed ({rc}): {detail}")

@@ -33,9 +33,6 @@
 #ifndef LBM3D_CONVZ_XCD_CHUNK
 #define LBM3D_CONVZ_XCD_CHUNK 32  // marching forward: runs of consecutive columns per XCD
 #endif
-#ifndef LBM3D_CONV_WGRAD_TILED
-#define LBM3D_CONV_WGRAD_TILED 1  // weight gradients stage dy and x (with its halo) transposed in LDS
-#endif
 #ifndef LBM3D_CONV_WGRAD_PREFETCH
 #define LBM3D_CONV_WGRAD_PREFETCH 0  // 1: load the next brick while the current one's MFMAs run (3 waves/SIMD)
 #endif
@@ -295,17 +292,68 @@ struct Weights {
   }
 };
 
-// bias, ReLU and rounding of 4 channels of one voxel, packed for one 8-byte store
-__device__ __forceinline__ uint2 finish4(const f32x4 acc, const float b4[4], int relu) {
-  uint32_t o[4];
+// What a forward kernel reads and writes besides a plain input and output.
+//   kUp    the input's first c_low channels are those of a volume of half the
+//          extents, upsampled (each voxel read for its 2 x 2 x 2 block), the
+//          others those of `x`: a concatenation that is never built
+//   kPool  the 2 x 2 x 2 maximum of the output is written too (half extents)
+// c_split > 0: output channels below it go to `y` (c_split per voxel), the
+// others to `y_hi`: the two parts of a concatenation's gradient.
+// The copies and reductions these replace took 2.9 of 6.2 ms of a 2 x 192^3
+// inference and 1.5 of 7.1 ms of a 2 x 128^3 training step; pooling in the
+// epilogue adds nothing to the 250 us of a 16 -> 16 layer, and reading the
+// upsampled part at half extents takes 96 -> 32 channels at 2 x 96^3 from 394 to
+// 328 us.
+enum ConvMode { kPlain = 0, kUp = 1, kPool = 2 };
+
+struct ConvExtra {
+  const uint16_t *low;  // kUp
+  int c_low;
+  uint16_t *pool;       // kPool
+  int c_split;
+  uint16_t *y_hi;
+};
+
+// bias and ReLU of 4 channels of one voxel
+__device__ __forceinline__ f32x4 finish4(f32x4 v, const f32x4 b4, int relu) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    float val = acc[e] + b4[e];
-    if (relu) val = val > 0.f ? val : 0.f;
-    o[e] = to_bf16(val);
+    v[e] += b4[e];
+    if (relu) v[e] = v[e] > 0.f ? v[e] : 0.f;
   }
-  return make_uint2(o[0] | (o[1] << 16), o[2] | (o[3] << 16));
+  return v;
 }
+
+// 4 channels rounded and packed for one 8-byte store
+__device__ __forceinline__ uint2 pack4(const f32x4 v) {
+  return make_uint2((uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16),
+                    (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16));
+}
+
+__device__ __forceinline__ f32x4 max4(const f32x4 a, const f32x4 b) {
+  return f32x4{fmaxf(a[0], b[0]), fmaxf(a[1], b[1]), fmaxf(a[2], b[2]), fmaxf(a[3], b[3])};
+}
+
+// the maximum over an x pair of voxels (lanes r16 and r16 ^ 1)
+__device__ __forceinline__ f32x4 max_xpair(f32x4 v) {
+  f32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)  // quad_perm [1, 0, 3, 2]
+    o[e] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v[e]), 0xB1, 0xF, 0xF, true));
+  return max4(v, o);
+}
+
+// where a tile's output goes: base pointer and channels per voxel
+struct OutPlace {
+  uint16_t *y;
+  int c, co;
+  __device__ __forceinline__ OutPlace(uint16_t *y_, int cout, int tile, int g, const ConvExtra &ex) {
+    const bool hi = ex.c_split > 0 && 16 * tile >= ex.c_split;
+    y = hi ? ex.y_hi : y_;
+    c = ex.c_split > 0 ? (hi ? cout - ex.c_split : ex.c_split) : cout;
+    co = 16 * tile + 4 * g - (hi ? ex.c_split : 0);
+  }
+};
 
 // Bricks of one launch: n volumes of nbz x nby x nbx bricks, x fastest.
 struct Bricks {
@@ -344,11 +392,11 @@ __device__ __forceinline__ void brick_origin(const Bricks &bk, uint32_t bi, int 
 // Bound by the MFMAs and the LDS reads of the voxels (one 1 KB fragment per
 // MFMA): 192 -> 64 channels at 2 x 48^3 take 150 us (980 TFLOP/s) against 305
 // for one 16-channel tile per workgroup with its halo loaded behind a barrier.
-template <int CT>
+template <int CT, int MODE>
 __global__ void __launch_bounds__(256, 2)
     k_conv3(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, int packed,
             const float *__restrict__ bias, uint16_t *__restrict__ y, const Vol vol, int cin, int cout, int kpad,
-            int relu, const Bricks bk) {
+            int relu, const Bricks bk, const ConvExtra ex) {
   constexpr int YR = 2 * CT, MF = 2 * YR;
   // [voxel][16 channels as two 16-byte halves]; two arrays, so that a read of
   // one never waits for the loads into the other
@@ -368,12 +416,14 @@ __global__ void __launch_bounds__(256, 2)
 
   // halo loads of one brick: entry e = 256 q + thread is half e & 1 of halo
   // voxel e / 2; its voxel index in the volume, or -1 outside it
-  int hvox[kHaloLoads];
-  const uint16_t *xv = x;
+  int hvox[kHaloLoads], lvox[MODE == kUp ? kHaloLoads : 1];  // lvox: in the half-extent volume
+  const uint16_t *xv = x, *lv = ex.low;
+  const int c_skip = MODE == kUp ? cin - ex.c_low : cin, nlow = MODE == kUp ? ex.c_low / 16 : 0;
   auto locate = [&](uint32_t bi) {
     int bb, z0, y0, x0;
     brick_origin(bk, bi, bb, z0, y0, x0);
-    xv = x + (size_t)bb * vstride * cin;
+    xv = x + (size_t)bb * vstride * c_skip;
+    if (MODE == kUp) lv = ex.low + (size_t)bb * (vstride >> 3) * ex.c_low;
     int t = (int)threadIdx.x;
     asm volatile("" : "+v"(t));  // decompose the entries here, not once into registers held across the loop
 #pragma unroll
@@ -390,12 +440,14 @@ __global__ void __launch_bounds__(256, 2)
       const bool in = hv < kHalo && (unsigned)zz < (unsigned)vol.d && (unsigned)yy < (unsigned)vol.h &&
                       (unsigned)xx < (unsigned)vol.w;
       hvox[q] = in ? (zz * vol.h + yy) * vol.w + xx : -1;
+      if (MODE == kUp) lvox[q] = in ? ((zz >> 1) * (vol.h >> 1) + (yy >> 1)) * (vol.w >> 1) + (xx >> 1) : -1;
     }
   };
   auto load_halo = [&](int c, u32x4 *buf) {
 #pragma unroll
     for (int q = 0; q < kHaloLoads; ++q) {
-      const uint16_t *src = xv + ((int64_t)hvox[q] * cin + 16 * c + 8 * ((int)threadIdx.x & 1));
+      const uint16_t *src = xv + ((int64_t)hvox[q] * c_skip + 16 * (c - nlow) + 8 * ((int)threadIdx.x & 1));
+      if (MODE == kUp && c < nlow) src = lv + ((int64_t)lvox[q] * ex.c_low + 16 * c + 8 * ((int)threadIdx.x & 1));
       if (hvox[q] < 0) src = reinterpret_cast<const uint16_t *>(conv_zero);
       __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)(buf + 256 * q + 64 * wave), 16, 0, 0);
     }
@@ -494,19 +546,31 @@ __global__ void __launch_bounds__(256, 2)
     // C layout: lane holds rows (channels) 4g .. 4g+3, column (voxel x) r16
     int bb, z0, y0, x0;
     brick_origin(bk, bcur, bb, z0, y0, x0);
-    const int co = 16 * tile + 4 * g;
-    float b4[4] = {0.f, 0.f, 0.f, 0.f};
+    const OutPlace op(y, cout, tile, g, ex);
+    f32x4 b4 = f32x4{0.f, 0.f, 0.f, 0.f};
     if (bias) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) b4[e] = bias[co + e];
+      for (int e = 0; e < 4; ++e) b4[e] = bias[16 * tile + 4 * g + e];
     }
     const int oy0 = y0 + yr0, ox = x0 + r16;
-    uint16_t *yv = y + ((size_t)bb * vstride + ((int64_t)z0 * vol.h + oy0) * vol.w + ox) * cout + co;
+    uint16_t *yv = op.y + ((size_t)bb * vstride + ((int64_t)z0 * vol.h + oy0) * vol.w + ox) * op.c + op.co;
 #pragma unroll
     for (int f = 0; f < MF; ++f) {
       const int fz = f / YR, fy = f % YR;
+      acc[f] = finish4(acc[f], b4, relu);
       if (z0 + fz < vol.d && oy0 + fy < vol.h && ox < vol.w)
-        *reinterpret_cast<uint2 *>(yv + ((int64_t)fz * vol.h + fy) * vol.w * cout) = finish4(acc[f], b4, relu);
+        *reinterpret_cast<uint2 *>(yv + ((int64_t)fz * vol.h + fy) * vol.w * op.c) = pack4(acc[f]);
+    }
+    if constexpr (MODE == kPool) {  // even extents: a block is inside whole or not at all
+#pragma unroll
+      for (int fy = 0; fy < YR; fy += 2) {
+        const f32x4 m = max_xpair(max4(max4(acc[fy], acc[fy + 1]), max4(acc[YR + fy], acc[YR + fy + 1])));
+        if (!(r16 & 1) && z0 < vol.d && oy0 + fy < vol.h && ox < vol.w)
+          *reinterpret_cast<uint2 *>(
+              ex.pool + ((size_t)bb * (vstride >> 3) +
+                         ((int64_t)(z0 >> 1) * (vol.h >> 1) + ((oy0 + fy) >> 1)) * (vol.w >> 1) + (ox >> 1)) * cout +
+              op.co) = pack4(m);
+      }
     }
   }
 }
@@ -532,11 +596,11 @@ struct Columns {
   int32_t zl;
 };
 
-template <int WCH, int CT, int TY>
+template <int WCH, int CT, int TY, int MODE>
 __global__ void __launch_bounds__(256, 2)
     k_conv3z(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, int packed,
              const float *__restrict__ bias, uint16_t *__restrict__ y, const Vol vol, int cout, int kpad, int relu,
-             const Columns ck) {
+             const Columns ck, const ConvExtra ex) {
   constexpr int cin = 16 * WCH, P = 2 * WCH;          // 16-byte pieces of a voxel
   constexpr int MF = TY * CT / 4;                     // rows (fragments) of a wave
   constexpr int E = (TY + 2) * kHx * P;               // pieces of one slot
@@ -555,12 +619,14 @@ __global__ void __launch_bounds__(256, 2)
   const int x0 = (int)(b - t1_ * ck.dx.d) * 16, y0 = (int)(t1_ - t2_ * ck.dy.d) * TY, bb = (int)(t2_ - seg * ck.dn.d);
   const int z_begin = (int)seg * ck.zl, z_end = z_begin + ck.zl < vol.d ? z_begin + ck.zl : vol.d;
   const int64_t vstride = (int64_t)vol.d * vol.h * vol.w, pstride = (int64_t)vol.h * vol.w;
-  const uint16_t *const xv = x + (size_t)bb * vstride * cin;
+  const int c_skip = MODE == kUp ? cin - ex.c_low : cin;
+  const uint16_t *const xv = x + (size_t)bb * vstride * c_skip;
+  const uint16_t *const lv = MODE == kUp ? ex.low + (size_t)bb * (vstride >> 3) * ex.c_low : nullptr;
 
   // this thread's pieces of a plane: entry e = 256 q + thread is piece e % P of
   // halo voxel e / P; its byte offset in the plane, the same for every plane
   uint32_t off[NQ];
-  uint32_t valid = 0;
+  uint32_t valid = 0, from_low = 0;
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
     const int e = 256 * q + (int)threadIdx.x;
@@ -571,7 +637,15 @@ __global__ void __launch_bounds__(256, 2)
       xx = wrap1(xx, vol.w);
     }
     const bool in = e < E && (unsigned)yy < (unsigned)vol.h && (unsigned)xx < (unsigned)vol.w;
-    off[q] = in ? 2u * ((uint32_t)(yy * vol.w + xx) * (uint32_t)cin + 8u * (uint32_t)pc) : 0u;
+    off[q] = in ? 2u * ((uint32_t)(yy * vol.w + xx) * (uint32_t)c_skip + 8u * (uint32_t)pc) : 0u;
+    if (MODE == kUp) {
+      if (8 * pc < ex.c_low) {
+        from_low |= 1u << q;
+        if (in) off[q] = 2u * ((uint32_t)((yy >> 1) * (vol.w >> 1) + (xx >> 1)) * (uint32_t)ex.c_low + 8u * (uint32_t)pc);
+      } else {
+        off[q] -= 2u * (uint32_t)ex.c_low;  // the skip volume's own channel
+      }
+    }
     valid |= (in ? 1u : 0u) << q;
     if (e < E && !in)  // never loaded: zero in every slot
       for (int sl = 0; sl < kRing; ++sl) ring[sl * E + e] = u32x4{0u, 0u, 0u, 0u};
@@ -579,12 +653,13 @@ __global__ void __launch_bounds__(256, 2)
   auto load_plane = [&](int z, int slot) {
     if (vol.periodic) z = wrap1(z, vol.d);
     if ((unsigned)z < (unsigned)vol.d) {
-      const char *base = reinterpret_cast<const char *>(xv + z * pstride * cin);
+      const char *base = reinterpret_cast<const char *>(xv + z * pstride * c_skip);
+      const char *low = MODE == kUp ? reinterpret_cast<const char *>(lv + (z >> 1) * (pstride >> 2) * ex.c_low) : base;
 #pragma unroll
       for (int q = 0; q < NQ; ++q)
         if ((valid >> q) & 1u)
-          __builtin_amdgcn_global_load_lds((gptr_t)(base + off[q]), (lptr_t)(ring + (slot * E + 256 * q + 64 * wave)),
-                                           16, 0, 0);
+          __builtin_amdgcn_global_load_lds((gptr_t)((MODE == kUp && ((from_low >> q) & 1u) ? low : base) + off[q]),
+                                           (lptr_t)(ring + (slot * E + 256 * q + 64 * wave)), 16, 0, 0);
     } else {
 #pragma unroll
       for (int q = 0; q < NQ; ++q)
@@ -599,11 +674,11 @@ __global__ void __launch_bounds__(256, 2)
   u32x4 wr[WCH * kSteps];
 #pragma unroll
   for (int i = 0; i < WCH * kSteps; ++i) wr[i] = weight(i / kSteps, i % kSteps);
-  const int co = 16 * tile + 4 * g;
-  float b4[4] = {0.f, 0.f, 0.f, 0.f};
+  const OutPlace op(y, cout, tile, g, ex);
+  f32x4 b4 = f32x4{0.f, 0.f, 0.f, 0.f};
   if (bias) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) b4[e] = bias[co + e];
+    for (int e = 0; e < 4; ++e) b4[e] = bias[16 * tile + 4 * g + e];
   }
 
   // B fragment f (row row0 + f), step s, chunk c: byte address l0 + slot of the
@@ -614,8 +689,9 @@ __global__ void __launch_bounds__(256, 2)
   const uint32_t dx1 = second ? (uint32_t)VB : 0u, dy1 = second ? (uint32_t)(RB - 2 * VB) : 0u;
   const char *const lds = reinterpret_cast<const char *>(ring);
   const int oy0 = y0 + row0, ox = x0 + r16;
-  uint16_t *yv = y + ((size_t)bb * vstride + ((int64_t)z_begin * vol.h + oy0) * vol.w + ox) * cout + co;
-  int slot = 0;  // of plane z - 1
+  uint16_t *yv = op.y + ((size_t)bb * vstride + ((int64_t)z_begin * vol.h + oy0) * vol.w + ox) * op.c + op.co;
+  f32x4 even[MODE == kPool ? MF / 2 : 1];  // the even plane's row-pair maxima (runs start on even planes)
+  int slot = 0;                            // of plane z - 1
   for (int z = z_begin; z < z_end; ++z) {
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this thread's loads of plane z + 1
     __syncthreads();                     // everyone's; and plane z - 2 has been read by all
@@ -658,10 +734,28 @@ __global__ void __launch_bounds__(256, 2)
     }
     // C layout: lane holds rows (channels) 4g .. 4g+3, column (voxel x) r16
 #pragma unroll
-    for (int f = 0; f < MF; ++f)
+    for (int f = 0; f < MF; ++f) {
+      acc[f] = finish4(acc[f], b4, relu);
       if (oy0 + f < vol.h && ox < vol.w)
-        *reinterpret_cast<uint2 *>(yv + (int64_t)f * vol.w * cout) = finish4(acc[f], b4, relu);
-    yv += pstride * cout;
+        *reinterpret_cast<uint2 *>(yv + (int64_t)f * vol.w * op.c) = pack4(acc[f]);
+    }
+    if constexpr (MODE == kPool) {
+#pragma unroll
+      for (int f = 0; f < MF; f += 2) {
+        const f32x4 m = max4(acc[f], acc[f + 1]);
+        if (!(z & 1)) {
+          even[f / 2] = m;
+        } else {
+          const f32x4 p = max_xpair(max4(even[f / 2], m));
+          if (!(r16 & 1) && oy0 + f < vol.h && ox < vol.w)
+            *reinterpret_cast<uint2 *>(
+                ex.pool + ((size_t)bb * (vstride >> 3) +
+                           ((int64_t)(z >> 1) * (vol.h >> 1) + ((oy0 + f) >> 1)) * (vol.w >> 1) + (ox >> 1)) * cout +
+                op.co) = pack4(p);
+        }
+      }
+    }
+    yv += pstride * op.c;
     slot = (slot + 1) & 3;
   }
 }
@@ -710,86 +804,6 @@ __global__ void __launch_bounds__(256) k_wpack(const float *__restrict__ w, uint
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient.  Workgroup (p, tap, cot): voxels [p*vblock, (p+1)*vblock),
-// one tap, output channels 16*cot .. +15; 2 waves, each taking 32 of every 64
-// voxels.  part[((p*2 + wave)*taps + tap)*cout + co][ci].
-// ---------------------------------------------------------------------------
-constexpr int kWgWaves = 2;
-constexpr int kLd = 40;        // LDS row stride (bf16): 80 bytes, conflict-free 16-byte reads
-constexpr int kMaxCinTiles = 16;  // cin <= 256
-
-template <int MAXT>
-__global__ void __launch_bounds__(64 * kWgWaves)
-    k_conv_wgrad(const uint16_t *__restrict__ x, const uint16_t *__restrict__ dy, float *__restrict__ part,
-                 const Vol vol, int cin, int cout, int ks, uint32_t vblock) {
-  extern __shared__ uint16_t lds[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane >> 4, r16 = lane & 15;
-  const int p = blockIdx.x, tap = blockIdx.y, co0 = blockIdx.z * 16;
-  const int taps = ks * ks * ks;
-  const int nt = cin / 16;
-  uint16_t *dyT = lds + (size_t)wave * (16 + cin) * kLd;  // [16][kLd]
-  uint16_t *xT = dyT + 16 * kLd;                           // [cin][kLd]
-  int dz, dyo, dx;
-  tap_offset(tap, ks, dz, dyo, dx);
-  const uint32_t v_begin = (uint32_t)p * vblock;
-  uint32_t v_end = v_begin + vblock;
-  if (v_end > vol.vox) v_end = vol.vox;
-  f32x4 acc[MAXT];
-#pragma unroll
-  for (int t = 0; t < MAXT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int groups = cin / 8;            // 8-channel groups per voxel row
-  const int pieces = 32 * groups;        // 16-byte pieces of x per 32 voxels
-  for (uint32_t base = v_begin; base < v_end; base += 32u * kWgWaves) {
-    const uint32_t c0 = base + 32u * (uint32_t)wave;  // this wave's 32 voxels
-    // dy^T: lane -> voxel c0 + lane/2, channels co0 + 8*(lane&1) .. +7
-    {
-      const uint32_t v = c0 + (uint32_t)(lane >> 1);
-      u32x4 val = u32x4{0u, 0u, 0u, 0u};
-      if (v < v_end) val = ld16(dy + (size_t)v * cout + co0 + 8 * (lane & 1));
-      const uint16_t *h = reinterpret_cast<const uint16_t *>(&val);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) dyT[(8 * (lane & 1) + e) * kLd + (lane >> 1)] = h[e];
-    }
-    // x^T of the tap-shifted voxels: piece -> voxel piece % 32, channel group piece / 32
-    for (int pc = lane; pc < pieces; pc += 64) {
-      const int vv = pc & 31, grp = pc >> 5;
-      const uint32_t v = c0 + (uint32_t)vv;
-      u32x4 val = u32x4{0u, 0u, 0u, 0u};
-      if (v < v_end) {
-        int b, z, yy, xx;
-        decode(vol, v, b, z, yy, xx);
-        const int64_t src = shifted(vol, b, z, yy, xx, dz, dyo, dx);
-        if (src >= 0) val = ld16(x + src * cin + 8 * grp);
-      }
-      const uint16_t *h = reinterpret_cast<const uint16_t *>(&val);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) xT[(8 * grp + e) * kLd + vv] = h[e];
-    }
-    __syncthreads();
-    const bf16x8 av = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(dyT + r16 * kLd + 8 * g));
-#pragma unroll
-    for (int t = 0; t < MAXT; ++t) {
-      if (t < nt) {
-        const bf16x8 bv =
-            __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(xT + (16 * t + r16) * kLd + 8 * g));
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[t], 0, 0, 0);
-      }
-    }
-    __syncthreads();
-  }
-  float *out = part + ((((size_t)p * kWgWaves + wave) * taps + tap) * cout + co0) * cin;
-#pragma unroll
-  for (int t = 0; t < MAXT; ++t) {
-    if (t < nt) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) out[(size_t)(4 * g + e) * cin + 16 * t + r16] = acc[t][e];
-    }
-  }
-}
-
-// dw[co][tap*cin + ci] = sum over the partial sets, in order; padding columns 0
-// ---------------------------------------------------------------------------
 // Weight gradient with the operands in LDS:
 //   dw[co][tap*cin + ci] = sum over voxels v of dy[v][co] * x[v + off(tap)][ci].
 // A workgroup owns 16 output channels co0.., 16 input channels c0.. and a run
@@ -817,7 +831,7 @@ template <int KS>
 __global__ void __launch_bounds__(256)
     k_conv_wgrad_tiled(const uint16_t *__restrict__ x, const uint16_t *__restrict__ dy, float *__restrict__ part,
                        const Vol vol, int cin, int cout, int nbz, int nby, int nbx, uint32_t nbricks,
-                       uint32_t per_block) {
+                       uint32_t per_block, const uint16_t *__restrict__ low, int c_low) {
   constexpr int taps = KS * KS * KS;
   constexpr int xchan = KS == 3 ? kXChan : kDyRow;
   constexpr int nacc = KS == 3 ? 7 : 1;
@@ -827,6 +841,10 @@ __global__ void __launch_bounds__(256)
   const int g = lane >> 4, r16 = lane & 15;
   const int nci = cin / 16;
   const int co0 = (blockIdx.y / nci) * 16, c0 = (blockIdx.y % nci) * 16;
+  // x's channels below c_low come from `low`, a volume of half the extents, upsampled
+  const bool up = c0 < c_low;
+  const uint16_t *const xs_src = up ? low : x;
+  const int xs_c = up ? c_low : cin - c_low, xs_c0 = up ? c0 : c0 - c_low, sh = up ? 1 : 0;
   const uint32_t b0 = blockIdx.x * per_block;
   const uint32_t b1 = b0 + per_block < nbricks ? b0 + per_block : nbricks;
   const int64_t vstride = (int64_t)vol.d * vol.h * vol.w;
@@ -870,7 +888,9 @@ __global__ void __launch_bounds__(256)
       const int zz = z0 + hz - 1, yy = y0 + hy - 1, xx = x0 + hx - 1;
       if (hv < kHalo && (unsigned)zz < (unsigned)vol.d && (unsigned)yy < (unsigned)vol.h &&
           (unsigned)xx < (unsigned)vol.w) {
-        const uint16_t *src = x + ((size_t)bb * vstride + ((int64_t)zz * vol.h + yy) * vol.w + xx) * cin + c0;
+        const uint16_t *src =
+            xs_src + ((size_t)bb * (vstride >> (3 * sh)) +
+                      ((int64_t)(zz >> sh) * (vol.h >> sh) + (yy >> sh)) * (vol.w >> sh) + (xx >> sh)) * xs_c + xs_c0;
         rh[q][0] = ld16(src);
         rh[q][1] = ld16(src + 8);
       }
@@ -1049,21 +1069,6 @@ int wgrad_tiled_plan(int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, i
   return (int)((nb + pb - 1) / pb);
 }
 
-void wgrad_plan(int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cout, int32_t ks, int &parts, uint32_t &vblock) {
-  const int64_t vox = (int64_t)n * d * h * wd;
-  const int taps = ks * ks * ks;
-  const int64_t per_part = (int64_t)taps * (cout / 16);
-  int64_t P = (kWgTargetBlocks + per_part - 1) / per_part;
-  const int64_t step = 32 * kWgWaves;
-  const int64_t max_parts = (vox + step - 1) / step;
-  if (P > max_parts) P = max_parts;
-  if (P < 1) P = 1;
-  int64_t vb = (vox + P - 1) / P;
-  vb = (vb + step - 1) / step * step;
-  parts = (int)((vox + vb - 1) / vb);
-  vblock = (uint32_t)vb;
-}
-
 // ---------------------------------------------------------------------------
 // Periodic distance to solid (the surrogate's second input channel): the
 // separable squared-distance transform as three min-plus passes,
@@ -1190,9 +1195,20 @@ __device__ __forceinline__ float bf16_to_f32(uint32_t h) { return __uint_as_floa
 // in FP32: part[block][c].  Data are [voxels][C] bf16, C dividing 2048, so a
 // thread's 8-element chunks (chunk q covers elements 8q .. 8q+7) always hold
 // the same 8 channels when the blocks' chunk ranges start on multiples of C/8.
+//
+// POOL: g has a second part, the gradient of y's 2 x 2 x 2 maximum: at the
+// voxels that attain it, `share` (its gradient over their number, k_pool_share);
+// the sum is rounded to BF16 first, as two accumulated gradients are.
+struct PoolGrad {
+  const uint16_t *pooled, *share;
+  Vol vol;
+  Div pieces;  // by C / 8
+};
+
+template <bool POOL>
 __global__ void __launch_bounds__(256)
     k_relu_bias_grad(const uint16_t *g, const uint16_t *__restrict__ y, uint16_t *dz,  // dz may be g
-                     float *__restrict__ part, int64_t chunks, int C, int64_t per_block) {
+                     float *__restrict__ part, int64_t chunks, int C, int64_t per_block, const PoolGrad pg) {
   __shared__ float red[256][9];
   const int t = (int)threadIdx.x;
   const int64_t q0 = (int64_t)blockIdx.x * per_block;
@@ -1204,6 +1220,26 @@ __global__ void __launch_bounds__(256)
     u32x4 a = ld16(g + q * 8);
     if (y) {
       const u32x4 m = ld16(y + q * 8);
+      if constexpr (POOL) {
+        int b, z, yy, x;
+        const uint32_t v = chunks < ((int64_t)1 << 31) ? qdiv((uint32_t)q, pg.pieces) : (uint32_t)(q / pg.pieces.d);
+        decode(pg.vol, v, b, z, yy, x);
+        const int64_t o = ((((int64_t)b * (pg.vol.d >> 1) + (z >> 1)) * (pg.vol.h >> 1) + (yy >> 1)) * (pg.vol.w >> 1) +
+                           (x >> 1)) * C + 8 * (q - (int64_t)v * pg.pieces.d);
+        const u32x4 top = ld16(pg.pooled + o), share = ld16(pg.share + o);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          uint32_t r[2];
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            const uint32_t yk = (m[w] >> (16 * k)) & 0xFFFFu, tk = (top[w] >> (16 * k)) & 0xFFFFu;
+            const float sk = bf16_to_f32((share[w] >> (16 * k)) & 0xFFFFu);
+            const float gk = bf16_to_f32((a[w] >> (16 * k)) & 0xFFFFu);
+            r[k] = to_bf16(gk + (yk == tk ? sk : sk * 0.0f));
+          }
+          a[w] = r[0] | (r[1] << 16);
+        }
+      }
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
         uint32_t lo = a[w] & 0xFFFFu, hi = a[w] >> 16;
@@ -1232,47 +1268,99 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-template <int CT>
-void launch_conv3_bricks(hipStream_t s, const uint16_t *x, const uint16_t *w, int packed, const float *bias,
-                         uint16_t *y, const Vol &vol, int cin, int cout, int kpad, int relu, const Bricks &bk) {
-  const unsigned gy = (unsigned)(cout / (16 * CT));
+// The gradient of a 2 x 2 x 2 maximum, shared among the voxels that attain it:
+// share = BF16(gp / count), one 16-byte piece (8 channels) per thread.  y >= 0
+// (a ReLU output), so equal values have equal bits.
+__global__ void __launch_bounds__(256)
+    k_pool_share(const uint16_t *__restrict__ y, const uint16_t *__restrict__ pooled, const uint16_t *__restrict__ gp,
+                 uint16_t *__restrict__ share, const Vol low, Div pieces, int64_t total) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const uint32_t v = total < ((int64_t)1 << 31) ? qdiv((uint32_t)i, pieces) : (uint32_t)(i / pieces.d);
+  const int pc = (int)(i - (int64_t)v * pieces.d), c = 8 * (int)pieces.d;
+  int b, z, yy, x;
+  decode(low, v, b, z, yy, x);
+  const int64_t h2 = 2 * low.h, w2 = 2 * low.w;
+  const uint16_t *src = y + ((((int64_t)b * low.d + z) * 2 * h2 + 2 * yy) * w2 + 2 * x) * c + 8 * pc;
+  const u32x4 top = ld16(pooled + i * 8), g = ld16(gp + i * 8);
+  int cnt[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) cnt[e] = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const u32x4 a = ld16(src + (((k >> 2) * h2 + ((k >> 1) & 1)) * w2 + (k & 1)) * c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      cnt[2 * e] += (a[e] & 0xFFFFu) == (top[e] & 0xFFFFu);
+      cnt[2 * e + 1] += (a[e] >> 16) == (top[e] >> 16);
+    }
+  }
+  u32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    o[e] = (uint32_t)to_bf16(bf16_to_f32(g[e] & 0xFFFFu) / (float)cnt[2 * e]) |
+           ((uint32_t)to_bf16(bf16_to_f32(g[e] >> 16) / (float)cnt[2 * e + 1]) << 16);
+  *reinterpret_cast<u32x4 *>(share + i * 8) = o;
+}
+
+// One forward convolution, as the launchers pass it on.
+struct ConvCall {
+  const uint16_t *x, *w;
+  int packed;
+  const float *bias;
+  uint16_t *y;
+  Vol vol;
+  int cin, cout, kpad, relu;
+  ConvExtra ex;
+};
+
+template <int CT, int MODE>
+void launch_conv3_bricks(hipStream_t s, const ConvCall &a, const Bricks &bk) {
+  const unsigned gy = (unsigned)(a.cout / (16 * CT));
   // persistent workgroups: as many as are resident (3 per CU by LDS, 2 where the
   // kernel takes more than 168 VGPRs), in whole groups of 8 XCDs
-  const int64_t resident = (CT <= 2 ? 768 : 512) / gy;
+  const int64_t resident = (CT == 1 || (CT == 2 && MODE != kUp) ? 768 : 512) / gy;
   int64_t gx = xcd_grid(bk.n, LBM3D_CONV_XCD_CHUNK);
   if (gx > resident) gx = resident & ~int64_t(7);
   if (gx < 8) gx = 8;
-  k_conv3<CT><<<dim3((unsigned)gx, gy), 256, 0, s>>>(x, w, packed, bias, y, vol, cin, cout, kpad, relu, bk);
+  k_conv3<CT, MODE><<<dim3((unsigned)gx, gy), 256, 0, s>>>(a.x, a.w, a.packed, a.bias, a.y, a.vol, a.cin, a.cout,
+                                                           a.kpad, a.relu, bk, a.ex);
 }
 
-template <int WCH, int CT, int TY>
-void launch_conv3z(hipStream_t s, const uint16_t *x, const uint16_t *w, int packed, const float *bias, uint16_t *y,
-                   const Vol &vol, int cout, int kpad, int relu) {
-  const int64_t nbx = (vol.w + 15) / 16, nby = (vol.h + TY - 1) / TY, gy = cout / (16 * CT);
+template <int WCH, int CT, int TY, int MODE>
+void launch_conv3z(hipStream_t s, const ConvCall &a) {
+  const Vol &vol = a.vol;
+  const int64_t nbx = (vol.w + 15) / 16, nby = (vol.h + TY - 1) / TY, gy = a.cout / (16 * CT);
   const int64_t cols = nbx * nby * vol.n;
   // planes per workgroup: the cut that takes the fewest rounds of resident
-  // workgroups times planes (3 extra planes of border and start-up per run)
+  // workgroups times planes (3 extra planes of border and start-up per run);
+  // an even number with pooling
   const int64_t slots = 256 * (WCH == 1 ? 3 : 2);
-  int64_t best = 1, best_cost = INT64_MAX;
+  int64_t best = vol.d, best_cost = INT64_MAX;
   for (int64_t segs = 1; segs <= vol.d; ++segs) {
-    const int64_t cost = ((cols * segs * gy + slots - 1) / slots) * ((vol.d + segs - 1) / segs + 3);
-    if (cost < best_cost) best = segs, best_cost = cost;
+    int64_t zl = (vol.d + segs - 1) / segs;
+    if (MODE == kPool) zl = (zl + 1) & ~int64_t(1);
+    const int64_t runs = (vol.d + zl - 1) / zl;
+    const int64_t cost = ((cols * runs * gy + slots - 1) / slots) * (zl + 3);
+    if (cost < best_cost) best = zl, best_cost = cost;
     if (cols * segs * gy > 32 * slots) break;
   }
   Columns ck;
-  ck.zl = (int32_t)((vol.d + best - 1) / best);
+  ck.zl = (int32_t)best;
   const int64_t segs = (vol.d + ck.zl - 1) / ck.zl;
   ck.n = (uint32_t)(cols * segs);
   ck.dx = make_div((uint32_t)nbx);
   ck.dy = make_div((uint32_t)nby);
   ck.dn = make_div((uint32_t)vol.n);
   const dim3 grid((unsigned)xcd_grid(ck.n, LBM3D_CONVZ_XCD_CHUNK), (unsigned)gy);
-  k_conv3z<WCH, CT, TY><<<grid, 256, 0, s>>>(x, w, packed, bias, y, vol, cout, kpad, relu, ck);
+  k_conv3z<WCH, CT, TY, MODE><<<grid, 256, 0, s>>>(a.x, a.w, a.packed, a.bias, a.y, vol, a.cout, a.kpad, a.relu, ck,
+                                                   a.ex);
 }
 
-int launch_conv3(hipStream_t s, const uint16_t *x, const uint16_t *w, int packed, const float *bias, uint16_t *y,
-                 const Vol &vol, int cin, int cout, int kpad, int relu) {
-  const int tiles = cout / 16;
+template <int MODE>
+int launch_conv3(hipStream_t s, const ConvCall &a) {
+  const Vol &vol = a.vol;
+  const int tiles = a.cout / 16, cin = a.cin;
   const Bricks bk = make_bricks(vol.n, vol.d, vol.h, vol.w);
   if (xcd_grid(bk.n, LBM3D_CONV_XCD_CHUNK) > (int64_t)(UINT32_MAX / 256u))
     return cfail(LBM3D_ESIZE, "too many bricks for one launch");
@@ -1282,19 +1370,21 @@ int launch_conv3(hipStream_t s, const uint16_t *x, const uint16_t *w, int packed
   // 2 x 96^3 119-123 us either way, 32 -> 64 at 2 x 48^3 35 us either way, 16 -> 32
   // at 2 x 96^3 65 us marching and 79 in bricks.
   if ((cin == 16 || (cin <= 48 && tiles % 4 != 0)) && (int64_t)vol.h * vol.w * cin < ((int64_t)1 << 31)) {
-#define LBM3D_CONV3Z(WCH, CT, TY) launch_conv3z<WCH, CT, TY>(s, x, w, packed, bias, y, vol, cout, kpad, relu)
-    if (tiles % 4 == 0) {
-      LBM3D_CONV3Z(1, 4, 8);
-    } else if (tiles % 2 == 0) {
-      if (cin == 16) LBM3D_CONV3Z(1, 2, 8);
-      else if (cin == 32) LBM3D_CONV3Z(2, 2, 8);
-      else LBM3D_CONV3Z(3, 2, 8);
+    if (cin == 16) {
+      if constexpr (MODE != kUp) {  // an upsampled and a skip part take 32 channels at least
+        if (tiles % 4 == 0) launch_conv3z<1, 4, 8, MODE>(s, a);
+        else if (tiles % 2 == 0) launch_conv3z<1, 2, 8, MODE>(s, a);
+        else launch_conv3z<1, 1, 16, MODE>(s, a);
+      }
+    } else if (cin == 32) {
+      if (tiles % 2 == 0) launch_conv3z<2, 2, 8, MODE>(s, a);
+      else launch_conv3z<2, 1, 8, MODE>(s, a);
     } else {
-      if (cin == 16) LBM3D_CONV3Z(1, 1, 16);
-      else if (cin == 32) LBM3D_CONV3Z(2, 1, 8);
-      else LBM3D_CONV3Z(3, 1, 8);
+      if (MODE != kPool && tiles % 2 == 0)  // pooling's row maxima would spill
+        launch_conv3z<3, 2, 8, MODE == kPool ? kPlain : MODE>(s, a);
+      else
+        launch_conv3z<3, 1, 8, MODE>(s, a);
     }
-#undef LBM3D_CONV3Z
     return ccheck("lbm3d_conv3d_fwd");
   }
   // as many channel tiles per workgroup (the halo is loaded once per workgroup)
@@ -1302,13 +1392,40 @@ int launch_conv3(hipStream_t s, const uint16_t *x, const uint16_t *w, int packed
   // 256 workgroups of one tile, 32 us with 64 of four
   int ct = tiles % 4 == 0 ? 4 : (tiles % 2 == 0 ? 2 : 1);
   while (ct > 1 && (int64_t)bk.n * (tiles / ct) < 512) ct >>= 1;
-  if (ct == 4)
-    launch_conv3_bricks<4>(s, x, w, packed, bias, y, vol, cin, cout, kpad, relu, bk);
-  else if (ct == 2)
-    launch_conv3_bricks<2>(s, x, w, packed, bias, y, vol, cin, cout, kpad, relu, bk);
-  else
-    launch_conv3_bricks<1>(s, x, w, packed, bias, y, vol, cin, cout, kpad, relu, bk);
+  if (ct == 4) launch_conv3_bricks<4, MODE>(s, a, bk);
+  else if (ct == 2) launch_conv3_bricks<2, MODE>(s, a, bk);
+  else launch_conv3_bricks<1, MODE>(s, a, bk);
   return ccheck("lbm3d_conv3d_fwd");
+}
+
+// Gradient of nearest upsampling by 2: out[v] = sum of the 2 x 2 x 2 block of g
+// (BF16, FP32 sum), one 16-byte piece (8 channels) per thread.
+__global__ void __launch_bounds__(256)
+    k_up_grad(const uint16_t *__restrict__ g, uint16_t *__restrict__ out, const Vol low, Div pieces, int64_t total) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const int64_t v = total < ((int64_t)1 << 31) ? (int64_t)qdiv((uint32_t)i, pieces) : i / pieces.d;
+  const int pc = (int)(i - v * pieces.d), c = 8 * (int)pieces.d;
+  int b, z, yy, x;
+  decode(low, (uint32_t)v, b, z, yy, x);
+  const int64_t h2 = 2 * low.h, w2 = 2 * low.w;
+  const uint16_t *src = g + ((((int64_t)b * low.d + z) * 2 * h2 + 2 * yy) * w2 + 2 * x) * c + 8 * pc;
+  float sum[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const u32x4 a = ld16(src + (((k >> 2) * h2 + ((k >> 1) & 1)) * w2 + (k & 1)) * c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      sum[2 * e] += __uint_as_float(a[e] << 16);
+      sum[2 * e + 1] += __uint_as_float(a[e] & 0xFFFF0000u);
+    }
+  }
+  u32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = (uint32_t)to_bf16(sum[2 * e]) | ((uint32_t)to_bf16(sum[2 * e + 1]) << 16);
+  *reinterpret_cast<u32x4 *>(out + v * c + 8 * pc) = o;
 }
 
 int relu_bias_plan(int64_t voxels, int C, int64_t &chunks, int64_t &per_block) {
@@ -1344,7 +1461,7 @@ int lbm3d_conv3d_fwd(void *stream, const uint16_t *x, const uint16_t *w, const f
   const Vol vol = make_vol(n, d, h, wd, (flags & LBM3D_CONV_PERIODIC) ? 1 : 0);
   const int kpad = lbm3d_conv_kpad(cin, ks);
   hipStream_t s = (hipStream_t)stream;
-  if (ks == 3) return launch_conv3(s, x, w, 0, bias, y, vol, cin, cout, kpad, relu);
+  if (ks == 3) return launch_conv3<kPlain>(s, ConvCall{x, w, 0, bias, y, vol, cin, cout, kpad, relu, ConvExtra{}});
   constexpr int MW = LBM3D_CONV_MW;
   const unsigned gx = (vol.vox + 64u * MW - 1u) / (64u * MW);
   if (cout % 64 == 0)
@@ -1371,15 +1488,68 @@ int lbm3d_conv3d_wpack(void *stream, const float *w, uint16_t *wp, uint16_t *wt,
   return ccheck("lbm3d_conv3d_wpack");
 }
 
-int lbm3d_conv3d_fwd_packed(void *stream, const uint16_t *x, const uint16_t *wp, const float *bias, uint16_t *y,
-                            int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout, int32_t flags) {
+static int packed_call(const uint16_t *x, const uint16_t *wp, const float *bias, uint16_t *y, int32_t n, int32_t d,
+                       int32_t h, int32_t wd, int32_t cin, int32_t cout, int32_t flags, ConvCall &a) {
   int rc = check_conv(n, d, h, wd, cin, cout, 3);
   if (rc) return rc;
   if (!x || !wp || !y) return cfail(LBM3D_EINVAL, "NULL tensor");
   if (flags & ~(LBM3D_CONV_RELU | LBM3D_CONV_PERIODIC)) return cfail(LBM3D_EINVAL, "unknown flag bits");
-  return launch_conv3((hipStream_t)stream, x, wp, 1, bias, y,
-                      make_vol(n, d, h, wd, (flags & LBM3D_CONV_PERIODIC) ? 1 : 0), cin, cout,
-                      lbm3d_conv_kpad(cin, 3), (flags & LBM3D_CONV_RELU) ? 1 : 0);
+  a = ConvCall{x,   wp,   1, bias, y, make_vol(n, d, h, wd, (flags & LBM3D_CONV_PERIODIC) ? 1 : 0), cin, cout,
+               lbm3d_conv_kpad(cin, 3), (flags & LBM3D_CONV_RELU) ? 1 : 0, ConvExtra{}};
+  return LBM3D_OK;
+}
+
+int lbm3d_conv3d_fwd_packed(void *stream, const uint16_t *x, const uint16_t *wp, const float *bias, uint16_t *y,
+                            int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout, int32_t flags) {
+  ConvCall a;
+  if (int rc = packed_call(x, wp, bias, y, n, d, h, wd, cin, cout, flags, a)) return rc;
+  return launch_conv3<kPlain>((hipStream_t)stream, a);
+}
+
+int lbm3d_conv3d_fwd_pool(void *stream, const uint16_t *x, const uint16_t *wp, const float *bias, uint16_t *y,
+                          uint16_t *pool, int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout,
+                          int32_t flags) {
+  ConvCall a;
+  if (int rc = packed_call(x, wp, bias, y, n, d, h, wd, cin, cout, flags, a)) return rc;
+  if (!pool) return cfail(LBM3D_EINVAL, "NULL tensor");
+  if (!a.relu) return cfail(LBM3D_EINVAL, "pooling goes with LBM3D_CONV_RELU");
+  if ((d | h | wd) & 1) return cfail(LBM3D_EINVAL, "pooling needs even extents");
+  a.ex.pool = pool;
+  return launch_conv3<kPool>((hipStream_t)stream, a);
+}
+
+int lbm3d_conv3d_fwd_up(void *stream, const uint16_t *low, const uint16_t *skip, const uint16_t *wp,
+                        const float *bias, uint16_t *y, int32_t n, int32_t d, int32_t h, int32_t wd, int32_t c_low,
+                        int32_t c_skip, int32_t cout, int32_t flags) {
+  if (c_low < 16 || c_low % 16 || c_skip < 16 || c_skip % 16 || c_low > 240 || c_skip > 240)
+    return cfail(LBM3D_EINVAL, "channel counts must be multiples of 16, together at most 256");
+  ConvCall a;
+  if (int rc = packed_call(skip, wp, bias, y, n, d, h, wd, c_low + c_skip, cout, flags, a)) return rc;
+  if (!low) return cfail(LBM3D_EINVAL, "NULL tensor");
+  if ((d | h | wd) & 1) return cfail(LBM3D_EINVAL, "upsampling needs even extents");
+  a.ex.low = low;
+  a.ex.c_low = c_low;
+  return launch_conv3<kUp>((hipStream_t)stream, a);
+}
+
+int lbm3d_conv3d_dgrad_up(void *stream, const uint16_t *dy, const uint16_t *wt, uint16_t *d_low_full, uint16_t *d_low,
+                          uint16_t *d_skip, int32_t n, int32_t d, int32_t h, int32_t wd, int32_t c_low,
+                          int32_t c_skip, int32_t cout) {
+  if (c_low < 16 || c_low % 16 || c_skip < 16 || c_skip % 16 || c_low > 240 || c_skip > 240)
+    return cfail(LBM3D_EINVAL, "channel counts must be multiples of 16, together at most 256");
+  ConvCall a;
+  if (int rc = packed_call(dy, wt, nullptr, d_low_full, n, d, h, wd, cout, c_low + c_skip, 0, a)) return rc;
+  if (!d_low || !d_skip) return cfail(LBM3D_EINVAL, "NULL tensor");
+  if ((d | h | wd) & 1) return cfail(LBM3D_EINVAL, "upsampling needs even extents");
+  a.ex.c_split = c_low;
+  a.ex.y_hi = d_skip;
+  hipStream_t s = (hipStream_t)stream;
+  if (int rc = launch_conv3<kPlain>(s, a)) return rc;
+  const int64_t total = (int64_t)n * (d / 2) * (h / 2) * (wd / 2) * (c_low / 8);
+  if ((total + 255) / 256 > (int64_t)(UINT32_MAX / 256u)) return cfail(LBM3D_ESIZE, "volume too large for one launch");
+  k_up_grad<<<(unsigned)((total + 255) / 256), 256, 0, s>>>(d_low_full, d_low, make_vol(n, d / 2, h / 2, wd / 2),
+                                                           make_div((uint32_t)c_low / 8), total);
+  return ccheck("lbm3d_conv3d_dgrad_up");
 }
 
 int lbm3d_conv3d_wflip(void *stream, const uint16_t *w, uint16_t *wt, int32_t cin, int32_t cout, int32_t ks) {
@@ -1402,59 +1572,49 @@ int lbm3d_conv3d_dgrad(void *stream, const uint16_t *dy, const uint16_t *wt, uin
 size_t lbm3d_conv3d_wgrad_workspace_bytes(int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout,
                                           int32_t ks) {
   if (check_conv(n, d, h, wd, cin, cout, ks)) return 0;
-  if (LBM3D_CONV_WGRAD_TILED) {
-    uint32_t nbricks, per;
-    const int parts = wgrad_tiled_plan(n, d, h, wd, cin, cout, nbricks, per);
-    return (size_t)parts * wgrad_sets(ks) * ks * ks * ks * cout * cin * sizeof(float);
-  }
-  int parts;
-  uint32_t vb;
-  wgrad_plan(n, d, h, wd, cout, ks, parts, vb);
-  return (size_t)parts * kWgWaves * ks * ks * ks * cout * cin * sizeof(float);
+  uint32_t nbricks, per;
+  const int parts = wgrad_tiled_plan(n, d, h, wd, cin, cout, nbricks, per);
+  return (size_t)parts * wgrad_sets(ks) * ks * ks * ks * cout * cin * sizeof(float);
 }
 
-int lbm3d_conv3d_wgrad(void *stream, const uint16_t *x, const uint16_t *dy, float *dw, int32_t n, int32_t d, int32_t h,
-                       int32_t wd, int32_t cin, int32_t cout, int32_t ks, void *workspace, size_t workspace_bytes) {
+// the tiled weight gradient and its fold; low / c_low: the upsampled part of x, if any
+static int wgrad_run(void *stream, const uint16_t *x, const uint16_t *dy, float *dw, int32_t n, int32_t d, int32_t h,
+                     int32_t wd, int32_t cin, int32_t cout, int32_t ks, void *workspace, size_t workspace_bytes,
+                     const uint16_t *low, int c_low) {
   int rc = check_conv(n, d, h, wd, cin, cout, ks);
   if (rc) return rc;
-  if (!x || !dy || !dw || !workspace) return cfail(LBM3D_EINVAL, "NULL tensor or workspace");
+  if (!x || !dy || !dw || !workspace || (c_low > 0 && !low)) return cfail(LBM3D_EINVAL, "NULL tensor or workspace");
   if (workspace_bytes < lbm3d_conv3d_wgrad_workspace_bytes(n, d, h, wd, cin, cout, ks))
     return cfail(LBM3D_EINVAL, "wgrad workspace too small");
   const Vol vol = make_vol(n, d, h, wd);
   hipStream_t s = (hipStream_t)stream;
-  if (LBM3D_CONV_WGRAD_TILED) {
-    uint32_t nbricks, per;
-    const int parts = wgrad_tiled_plan(n, d, h, wd, cin, cout, nbricks, per);
-    const int nbz = (d + kBz - 1) / kBz, nby = (h + kBy - 1) / kBy, nbx = (wd + kBx - 1) / kBx;
-    const dim3 grid((unsigned)parts, (unsigned)((cout / 16) * (cin / 16)));
-    if (ks == 3)
-      k_conv_wgrad_tiled<3>
-          <<<grid, 256, 0, s>>>(x, dy, (float *)workspace, vol, cin, cout, nbz, nby, nbx, nbricks, per);
-    else
-      k_conv_wgrad_tiled<1>
-          <<<grid, 256, 0, s>>>(x, dy, (float *)workspace, vol, cin, cout, nbz, nby, nbx, nbricks, per);
-    if ((rc = ccheck("lbm3d_conv3d_wgrad"))) return rc;
-    const int kpad = lbm3d_conv_kpad(cin, ks);
-    return wgrad_fold(s, (float *)workspace, dw, parts * wgrad_sets(ks), ks * ks * ks, cin, cout, kpad);
-  }
-  int parts;
-  uint32_t vb;
-  wgrad_plan(n, d, h, wd, cout, ks, parts, vb);
-  const int taps = ks * ks * ks;
-  const size_t lds = (size_t)kWgWaves * (16 + cin) * kLd * sizeof(uint16_t);
-  const dim3 grid((unsigned)parts, (unsigned)taps, (unsigned)(cout / 16));
-  float *part = (float *)workspace;
-  if (cin <= 64)
-    k_conv_wgrad<4><<<grid, 64 * kWgWaves, lds, s>>>(x, dy, part, vol, cin, cout, ks, vb);
-  else if (cin <= 128)
-    k_conv_wgrad<8><<<grid, 64 * kWgWaves, lds, s>>>(x, dy, part, vol, cin, cout, ks, vb);
+  uint32_t nbricks, per;
+  const int parts = wgrad_tiled_plan(n, d, h, wd, cin, cout, nbricks, per);
+  const int nbz = (d + kBz - 1) / kBz, nby = (h + kBy - 1) / kBy, nbx = (wd + kBx - 1) / kBx;
+  const dim3 grid((unsigned)parts, (unsigned)((cout / 16) * (cin / 16)));
+  if (ks == 3)
+    k_conv_wgrad_tiled<3><<<grid, 256, 0, s>>>(x, dy, (float *)workspace, vol, cin, cout, nbz, nby, nbx, nbricks, per,
+                                               low, c_low);
   else
-    k_conv_wgrad<kMaxCinTiles><<<grid, 64 * kWgWaves, lds, s>>>(x, dy, part, vol, cin, cout, ks, vb);
+    k_conv_wgrad_tiled<1><<<grid, 256, 0, s>>>(x, dy, (float *)workspace, vol, cin, cout, nbz, nby, nbx, nbricks, per,
+                                               nullptr, 0);
   if ((rc = ccheck("lbm3d_conv3d_wgrad"))) return rc;
   const int kpad = lbm3d_conv_kpad(cin, ks);
-  const int64_t total = (int64_t)cout * kpad;
-  k_wgrad_fold<<<(unsigned)((total + 255) / 256), 256, 0, s>>>(part, dw, parts * kWgWaves, 1, taps, cin, cout, kpad);
-  return ccheck("lbm3d_conv3d_wgrad/fold");
+  return wgrad_fold(s, (float *)workspace, dw, parts * wgrad_sets(ks), ks * ks * ks, cin, cout, kpad);
+}
+
+int lbm3d_conv3d_wgrad(void *stream, const uint16_t *x, const uint16_t *dy, float *dw, int32_t n, int32_t d, int32_t h,
+                       int32_t wd, int32_t cin, int32_t cout, int32_t ks, void *workspace, size_t workspace_bytes) {
+  return wgrad_run(stream, x, dy, dw, n, d, h, wd, cin, cout, ks, workspace, workspace_bytes, nullptr, 0);
+}
+
+int lbm3d_conv3d_wgrad_up(void *stream, const uint16_t *low, const uint16_t *skip, const uint16_t *dy, float *dw,
+                          int32_t n, int32_t d, int32_t h, int32_t wd, int32_t c_low, int32_t c_skip, int32_t cout,
+                          void *workspace, size_t workspace_bytes) {
+  if (c_low < 16 || c_low % 16 || c_skip < 16 || c_skip % 16 || c_low > 240 || c_skip > 240)
+    return cfail(LBM3D_EINVAL, "channel counts must be multiples of 16, together at most 256");
+  if ((d | h | wd) & 1) return cfail(LBM3D_EINVAL, "upsampling needs even extents");
+  return wgrad_run(stream, skip, dy, dw, n, d, h, wd, c_low + c_skip, cout, 3, workspace, workspace_bytes, low, c_low);
 }
 
 size_t lbm3d_relu_bias_grad_workspace_bytes(int64_t voxels, int32_t c) {
@@ -1473,9 +1633,34 @@ int lbm3d_relu_bias_grad(void *stream, const uint16_t *g, const uint16_t *y, uin
   int64_t chunks, per;
   const int blocks = relu_bias_plan(voxels, c, chunks, per);
   hipStream_t s = (hipStream_t)stream;
-  k_relu_bias_grad<<<(unsigned)blocks, 256, 0, s>>>(g, y, dz, (float *)workspace, chunks, c, per);
+  k_relu_bias_grad<false><<<(unsigned)blocks, 256, 0, s>>>(g, y, dz, (float *)workspace, chunks, c, per, PoolGrad{});
   if (int rc = ccheck("lbm3d_relu_bias_grad")) return rc;
   // the wgrad fold with one tap and one output row: db[k] = sum over blocks of part[block][k]
+  return wgrad_fold(s, (float *)workspace, db, blocks, 1, c, 1, c);
+}
+
+int lbm3d_relu_pool_grad(void *stream, const uint16_t *g, const uint16_t *y, const uint16_t *pooled,
+                         const uint16_t *g_pool, uint16_t *dz, float *db, int32_t n, int32_t d, int32_t h, int32_t w,
+                         int32_t c, uint16_t *share, void *workspace, size_t workspace_bytes) {
+  if (n < 1 || d < 1 || h < 1 || w < 1 || ((d | h | w) & 1)) return cfail(LBM3D_EINVAL, "extents must be even");
+  if (c < 8 || c > 256 || 2048 % c) return cfail(LBM3D_EINVAL, "channels must divide 2048, 8..256");
+  if (!g || !y || !pooled || !g_pool || !dz || !db || !share || !workspace)
+    return cfail(LBM3D_EINVAL, "NULL tensor or workspace");
+  const int64_t voxels = (int64_t)n * d * h * w;
+  if (voxels >= ((int64_t)1 << 31)) return cfail(LBM3D_ESIZE, "more than 2^31-1 voxels");
+  if (workspace_bytes < lbm3d_relu_bias_grad_workspace_bytes(voxels, c))
+    return cfail(LBM3D_EINVAL, "relu/bias workspace too small");
+  hipStream_t s = (hipStream_t)stream;
+  const Div pieces = make_div((uint32_t)c / 8);
+  const int64_t low = voxels / 8 * (c / 8);
+  k_pool_share<<<(unsigned)((low + 255) / 256), 256, 0, s>>>(y, pooled, g_pool, share,
+                                                            make_vol(n, d / 2, h / 2, w / 2), pieces, low);
+  if (int rc = ccheck("lbm3d_relu_pool_grad")) return rc;
+  int64_t chunks, per;
+  const int blocks = relu_bias_plan(voxels, c, chunks, per);
+  k_relu_bias_grad<true><<<(unsigned)blocks, 256, 0, s>>>(g, y, dz, (float *)workspace, chunks, c, per,
+                                                         PoolGrad{pooled, share, make_vol(n, d, h, w), pieces});
+  if (int rc = ccheck("lbm3d_relu_pool_grad")) return rc;
   return wgrad_fold(s, (float *)workspace, db, blocks, 1, c, 1, c);
 }
 

@@ -135,8 +135,33 @@ def relu_bias_grad(g, y=None):
     return dz, db
 
 
-def _make_conv_function():
+def relu_pool_grad(g, g_pool, y, pooled):
+    """(dz, db) of relu_bias_grad for a layer whose output y was also pooled:
+    g_pool is the gradient of its 2x2x2 maximum `pooled`, shared evenly among
+    the voxels that attain it and added to g in BF16 (lbm3d_relu_pool_grad)."""
     torch = _torch()
+    n, d, h, wd, c = y.shape
+    lib = _lib.lib()
+    ws_bytes = lib.size("lbm3d_relu_bias_grad_workspace_bytes", n * d * h * wd, c)
+    ws = torch.empty(max(ws_bytes, 4), dtype=torch.uint8, device=g.device)
+    share = torch.empty_like(pooled)
+    dz = torch.empty_like(y)
+    db = torch.empty(c, dtype=torch.float32, device=g.device)
+    lib.call("lbm3d_relu_pool_grad", _stream(g.device), _vp(g), _vp(y), _vp(pooled), _vp(g_pool), _vp(dz), _vp(db),
+             n, d, h, wd, c, _vp(share), _vp(ws), ws_bytes)
+    return dz, db
+
+
+def _bf16(t):
+    return t.contiguous().to(_torch().bfloat16)
+
+
+def _make_conv_functions():
+    torch = _torch()
+
+    def packed(w, flip):
+        w = w if w.dtype == torch.float32 else w.to(torch.bfloat16).float()
+        return pack_weights(w.contiguous(), flip)
 
     class Conv3dMFMA(torch.autograd.Function):
         """y = act(conv3d(x, w) + b) with the MFMA kernels in both directions."""
@@ -145,8 +170,7 @@ def _make_conv_function():
         def forward(ctx, x, w, b, ks, relu, need_dx, periodic):
             x = x.contiguous()
             if ks == 3:
-                w = (w if w.dtype == torch.float32 else w.to(torch.bfloat16).float()).contiguous()
-                wp, wb = pack_weights(w, need_dx and ctx.needs_input_grad[0])
+                wp, wb = packed(w, need_dx and ctx.needs_input_grad[0])
                 y = conv_fwd_packed(x, wp, b, w.shape[0], relu, periodic)
             else:
                 wb = w.to(torch.bfloat16).contiguous()
@@ -160,7 +184,7 @@ def _make_conv_function():
             if ctx.periodic:
                 raise NotImplementedError("periodic convolutions are forward-only (inference)")
             x, wb, y = ctx.saved_tensors
-            g, db = relu_bias_grad(gy.contiguous().to(torch.bfloat16), y if ctx.relu else None)
+            g, db = relu_bias_grad(_bf16(gy), y if ctx.relu else None)
             dw = conv_wgrad(x, g, ctx.ks)
             dx = None
             if ctx.need_dx and ctx.needs_input_grad[0]:
@@ -168,30 +192,100 @@ def _make_conv_function():
                       else conv_dgrad(g, wb, x.shape[-1], ctx.ks))
             return dx, dw, db, None, None, None, None
 
-    return Conv3dMFMA
+    class ConvPool(torch.autograd.Function):
+        """(y, 2x2x2 max of y) for y = relu(conv3d(x, w) + b), 3x3x3."""
+
+        @staticmethod
+        def forward(ctx, x, w, b, periodic):
+            x = x.contiguous()
+            n, d, h, wd, cin = x.shape
+            cout = w.shape[0]
+            wp, wt = packed(w, ctx.needs_input_grad[0])
+            y = torch.empty((n, d, h, wd, cout), dtype=torch.bfloat16, device=x.device)
+            pooled = torch.empty((n, d // 2, h // 2, wd // 2, cout), dtype=torch.bfloat16, device=x.device)
+            _lib.lib().call("lbm3d_conv3d_fwd_pool", _stream(x.device), _vp(x), _vp(wp), _vp(b), _vp(y), _vp(pooled),
+                            n, d, h, wd, cin, cout, CONV_RELU | (CONV_PERIODIC if periodic else 0))
+            ctx.save_for_backward(x, wt, y, pooled)
+            ctx.periodic = periodic
+            return y, pooled
+
+        @staticmethod
+        def backward(ctx, gy, g_pool):
+            if ctx.periodic:
+                raise NotImplementedError("periodic convolutions are forward-only (inference)")
+            x, wt, y, pooled = ctx.saved_tensors
+            g, db = relu_pool_grad(_bf16(gy), _bf16(g_pool), y, pooled)
+            dw = conv_wgrad(x, g, 3)
+            dx = conv_fwd_packed(g, wt, None, x.shape[-1], False) if ctx.needs_input_grad[0] else None
+            return dx, dw, db, None
+
+    class ConvUp(torch.autograd.Function):
+        """relu(conv3d(cat(upsampled low, skip), w) + b), 3x3x3, without the concatenation."""
+
+        @staticmethod
+        def forward(ctx, low, skip, w, b, periodic):
+            low, skip = low.contiguous(), skip.contiguous()
+            n, d, h, wd, c_skip = skip.shape
+            cout = w.shape[0]
+            wp, wt = packed(w, ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
+            y = torch.empty((n, d, h, wd, cout), dtype=torch.bfloat16, device=skip.device)
+            _lib.lib().call("lbm3d_conv3d_fwd_up", _stream(skip.device), _vp(low), _vp(skip), _vp(wp), _vp(b), _vp(y),
+                            n, d, h, wd, low.shape[-1], c_skip, cout, CONV_RELU | (CONV_PERIODIC if periodic else 0))
+            ctx.save_for_backward(low, skip, wt, y)
+            ctx.periodic = periodic
+            return y
+
+        @staticmethod
+        def backward(ctx, gy):
+            if ctx.periodic:
+                raise NotImplementedError("periodic convolutions are forward-only (inference)")
+            low, skip, wt, y = ctx.saved_tensors
+            g, db = relu_bias_grad(_bf16(gy), y)
+            n, d, h, wd, c_skip = skip.shape
+            c_low, cout = low.shape[-1], g.shape[-1]
+            lib, s = _lib.lib(), _stream(g.device)
+            kpad = lib.cdll.lbm3d_conv_kpad(c_low + c_skip, 3)
+            ws_bytes = lib.size("lbm3d_conv3d_wgrad_workspace_bytes", n, d, h, wd, c_low + c_skip, cout, 3)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=g.device)
+            dw = torch.empty((cout, kpad), dtype=torch.float32, device=g.device)
+            lib.call("lbm3d_conv3d_wgrad_up", s, _vp(low), _vp(skip), _vp(g), _vp(dw), n, d, h, wd, c_low, c_skip,
+                     cout, _vp(ws), ws_bytes)
+            d_low = d_skip = None
+            if wt is not None:
+                full = torch.empty((n, d, h, wd, c_low), dtype=torch.bfloat16, device=g.device)
+                d_low, d_skip = torch.empty_like(low), torch.empty_like(skip)
+                lib.call("lbm3d_conv3d_dgrad_up", s, _vp(g), _vp(wt), _vp(full), _vp(d_low), _vp(d_skip), n, d, h, wd,
+                         c_low, c_skip, cout)
+            return d_low, d_skip, dw, db, None
+
+    return Conv3dMFMA, ConvPool, ConvUp
 
 
 _CONV = None
 
 
-def conv3d(x, w, b, ks: int = 3, relu: bool = True, need_dx: bool = True, periodic: bool = False):
+def _conv_functions():
     global _CONV
     if _CONV is None:
-        _CONV = _make_conv_function()
-    return _CONV.apply(x, w, b, ks, relu, need_dx, periodic)
+        _CONV = _make_conv_functions()
+    return _CONV
+
+
+def conv3d(x, w, b, ks: int = 3, relu: bool = True, need_dx: bool = True, periodic: bool = False):
+    return _conv_functions()[0].apply(x, w, b, ks, relu, need_dx, periodic)
+
+
+def conv3d_pool(x, w, b, periodic: bool = False):
+    """(y, its 2x2x2 maximum) of a 3x3x3 layer with ReLU; even extents."""
+    return _conv_functions()[1].apply(x, w, b, periodic)
+
+
+def conv3d_up(low, skip, w, b, periodic: bool = False):
+    """A 3x3x3 layer with ReLU on the concatenation of `low`, upsampled by 2 (nearest), and `skip`."""
+    return _conv_functions()[2].apply(low, skip, w, b, periodic)
 
 
 # ---- the network ------------------------------------------------------------------------------
-
-def _pool(x):
-    n, d, h, w, c = x.shape
-    return x.view(n, d // 2, 2, h // 2, 2, w // 2, 2, c).amax(dim=(2, 4, 6))
-
-
-def _up(x):
-    n, d, h, w, c = x.shape
-    return x[:, :, None, :, None, :, None, :].expand(n, d, 2, h, 2, w, 2, c).reshape(n, 2 * d, 2 * h, 2 * w, c)
-
 
 class UNet3D:
     """Parameters as FP32 master tensors; forward through the MFMA convolutions."""
@@ -246,15 +340,18 @@ class UNet3D:
         X, Y, Z must be multiples of 8.  periodic: every volume is one period of a
         periodic geometry, and the convolutions wrap around its faces instead of
         zero padding (forward only)."""
-        torch = _torch()
         p = periodic
-        e1 = self._c("e1b", self._c("e1a", x, need_dx=False, periodic=p), periodic=p)
-        e2 = self._c("e2b", self._c("e2a", _pool(e1), periodic=p), periodic=p)
-        e3 = self._c("e3b", self._c("e3a", _pool(e2), periodic=p), periodic=p)
-        e4 = self._c("e4b", self._c("e4a", _pool(e3), periodic=p), periodic=p)
-        d3 = self._c("d3b", self._c("d3a", torch.cat([_up(e4), e3], dim=-1), periodic=p), periodic=p)
-        d2 = self._c("d2b", self._c("d2a", torch.cat([_up(d3), e2], dim=-1), periodic=p), periodic=p)
-        d1 = self._c("d1b", self._c("d1a", torch.cat([_up(d2), e1], dim=-1), periodic=p), periodic=p)
+
+        def layer(name):
+            return self.params[name + ".w"], self.params[name + ".b"]
+
+        e1, low = conv3d_pool(self._c("e1a", x, need_dx=False, periodic=p), *layer("e1b"), p)
+        e2, low = conv3d_pool(self._c("e2a", low, periodic=p), *layer("e2b"), p)
+        e3, low = conv3d_pool(self._c("e3a", low, periodic=p), *layer("e3b"), p)
+        e4 = self._c("e4b", self._c("e4a", low, periodic=p), periodic=p)
+        d3 = self._c("d3b", conv3d_up(e4, e3, *layer("d3a"), p), periodic=p)
+        d2 = self._c("d2b", conv3d_up(d3, e2, *layer("d2a"), p), periodic=p)
+        d1 = self._c("d1b", conv3d_up(d2, e1, *layer("d1a"), p), periodic=p)
         out = self._c("head", d1, relu=False, periodic=p)
         return out[..., :4].float()
 
