@@ -10,14 +10,12 @@
 // (few input channels), k_conv3 walks bricks (many).
 //
 // Weight gradient: GEMM with M = output channels, N = input channels, K =
-// voxels.  Channels-last data must be transposed for that K, so each wave
-// stages 32 voxels of dy and of the tap-shifted x in LDS as [channel][voxel]
-// rows and reads its MFMA operands from there.  Workgroups own (voxel block,
-// tap, 16 output channels) and write partial sums; a second kernel folds them
-// in a fixed order.
+// voxels, the operands transposed by the LDS reads.  Workgroups write partial
+// sums; k_fold_sets adds them in a fixed order.
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -33,8 +31,8 @@
 #ifndef LBM3D_CONVZ_XCD_CHUNK
 #define LBM3D_CONVZ_XCD_CHUNK 32  // marching forward: runs of consecutive columns per XCD
 #endif
-#ifndef LBM3D_CONV_WGRAD_PREFETCH
-#define LBM3D_CONV_WGRAD_PREFETCH 0  // 1: load the next brick while the current one's MFMAs run (3 waves/SIMD)
+#ifndef LBM3D_CONV_WGRAD_XCD_CHUNK
+#define LBM3D_CONV_WGRAD_XCD_CHUNK 64  // weight gradient: runs of consecutive jobs per XCD (16 or 256: the same to 1 %)
 #endif
 #ifndef LBM3D_CONV_MW
 #define LBM3D_CONV_MW 2  // 16-voxel fragments per wave in the forward kernel
@@ -804,242 +802,307 @@ __global__ void __launch_bounds__(256) k_wpack(const float *__restrict__ w, uint
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient with the operands in LDS:
-//   dw[co][tap*cin + ci] = sum over voxels v of dy[v][co] * x[v + off(tap)][ci].
-// A workgroup owns 16 output channels co0.., 16 input channels c0.. and a run
-// of bricks (2 x 8 x 16 voxels, as the forward kernel's).  Per brick it stages
-// dy transposed, dyT[co][voxel], and x transposed, xs[ci][...]: for 3x3x3
-// kernels x's halo as [ci][halo row][x], for 1x1x1 kernels the brick itself as
-// [ci][voxel].  For each K chunk of 32 brick voxels (two brick rows) a wave
-// reads one A fragment from dyT and, for each of its taps, one B fragment from
-// xs: the 8 halo voxels the chunk's voxels see through that tap, consecutive
-// in an xs row but offset by dx + 1 elements, so assembled from one or two
-// aligned LDS reads.  3x3x3: wave w accumulates taps w, w+4, ... over all
-// chunks.  1x1x1: wave w accumulates chunks 2w and 2w+1.  Each wave writes one
-// partial 16 x 16 block per tap; k_wgrad_fold sums the partials in a fixed
-// order.
+// Weight gradients,
+//   dw[co][tap*cin + ci] = sum over voxels v of dy[v][co] * x[v + off(tap)][ci]:
+// MFMAs with M = 16 output channels (A = dy), N = 16 input channels (B = x) and
+// K = 32 voxels.  Both operands need 8 consecutive voxels of one channel per
+// lane from channels-last data: ds_read_b64_tr_b16 transposes a block of 4
+// voxels x 16 channels on the way out of LDS, so dy and x are staged as they
+// are, straight from memory.
+//
+// 3x3x3: a workgroup takes 16 input and 16 WCO output channels and a run of
+// bricks (2 x 8 x 16 voxels, as the forward kernel's), which it stages one at a time.  A K chunk
+// is two rows of the brick.  A wave owns one channel tile and one dx, that is 9
+// taps: it keeps the brick's 8 A fragments in registers and reads each of the 36
+// B fragments that its taps share (halo plane, first halo row) once, for 72
+// MFMAs.  Every tap sees the chunks of a brick in order, and the bricks in
+// order, so a set's sums do not depend on how the fragments are shared.
+// Bound by HBM and the L2 misses of the halos at 16 -> 16 channels (2 x 128^3: 118
+// us with the fold, 190 us with the operands transposed by 2-byte LDS writes and
+// each B fragment read for one MFMA), by the LDS reads (0.6 fragments per MFMA)
+// at more (96 -> 32 at 2 x 64^3: 130 us, 388 before), and by writing and folding
+// the sets where voxels are few (128 -> 128 at 2 x 16^3: 31 us, 43 before).
 // ---------------------------------------------------------------------------
-constexpr int kXRow = 24;  // halo row in xs, bf16 (18 used; 48 bytes keep rows 16-byte aligned)
-constexpr int kXRows = kHz * kHy;  // 40 halo rows
-// channel strides of the LDS tiles, in bf16: 4 dwords modulo 32 banks, so the
-// 16 lanes reading 16 channels at one position hit distinct banks
-constexpr int kXChan = kXRows * kXRow + 8;  // 968
-constexpr int kDyRow = 256 + 8;             // 264
-constexpr int wgrad_sets(int ks) { return ks == 3 ? 1 : 4; }  // partial sets a workgroup writes
+typedef short bf16x4 __attribute__((ext_vector_type(4)));
+typedef short bf16x8s __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) bf16x4 *ltr_t;
 
-template <int KS>
-__global__ void __launch_bounds__(256)
-    k_conv_wgrad_tiled(const uint16_t *__restrict__ x, const uint16_t *__restrict__ dy, float *__restrict__ part,
-                       const Vol vol, int cin, int cout, int nbz, int nby, int nbx, uint32_t nbricks,
-                       uint32_t per_block, const uint16_t *__restrict__ low, int c_low) {
-  constexpr int taps = KS * KS * KS;
-  constexpr int xchan = KS == 3 ? kXChan : kDyRow;
-  constexpr int nacc = KS == 3 ? 7 : 1;
-  __shared__ __align__(16) uint16_t dyT[16 * kDyRow];
-  __shared__ __align__(16) uint16_t xs[16 * xchan];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane >> 4, r16 = lane & 15;
-  const int nci = cin / 16;
-  const int co0 = (blockIdx.y / nci) * 16, c0 = (blockIdx.y % nci) * 16;
-  // x's channels below c_low come from `low`, a volume of half the extents, upsampled
-  const bool up = c0 < c_low;
-  const uint16_t *const xs_src = up ? low : x;
-  const int xs_c = up ? c_low : cin - c_low, xs_c0 = up ? c0 : c0 - c_low, sh = up ? 1 : 0;
-  const uint32_t b0 = blockIdx.x * per_block;
-  const uint32_t b1 = b0 + per_block < nbricks ? b0 + per_block : nbricks;
-  const int64_t vstride = (int64_t)vol.d * vol.h * vol.w;
-  f32x4 acc[nacc];
-#pragma unroll
-  for (int i = 0; i < nacc; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // Global loads of one brick into registers: dy (and x for 1x1x1) of this
-  // thread's brick voxel, and for 3x3x3 up to three of x's halo voxels.
-  constexpr int nh = KS == 3 ? (kHalo + 255) / 256 : 0;
-  u32x4 rdy[2], rx[2], rh[nh > 0 ? nh : 1][2];
-  auto load_brick = [&](uint32_t br) {
-    uint32_t bi = br;
-    const int bx = (int)(bi % (uint32_t)nbx);
-    bi /= (uint32_t)nbx;
-    const int by = (int)(bi % (uint32_t)nby);
-    bi /= (uint32_t)nby;
-    const int bz = (int)(bi % (uint32_t)nbz);
-    const int bb = (int)(bi / (uint32_t)nbz);
-    const int z0 = bz * kBz, y0 = by * kBy, x0 = bx * kBx;
-    const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
-    {
-      const int t = threadIdx.x;
-      const int z = z0 + (t >> 7), y = y0 + ((t >> 4) & 7), xx = x0 + (t & 15);
-      rdy[0] = rdy[1] = rx[0] = rx[1] = zero;
-      if (z < vol.d && y < vol.h && xx < vol.w) {
-        const size_t v = (size_t)bb * vstride + ((int64_t)z * vol.h + y) * vol.w + xx;
-        rdy[0] = ld16(dy + v * cout + co0);
-        rdy[1] = ld16(dy + v * cout + co0 + 8);
-        if (KS == 1) {
-          rx[0] = ld16(x + v * cin + c0);
-          rx[1] = ld16(x + v * cin + c0 + 8);
-        }
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < nh; ++q) {
-      const int hv = threadIdx.x + 256 * q;
-      rh[q][0] = rh[q][1] = zero;
-      const int hz = hv / (kHy * kHx), r = hv - hz * (kHy * kHx);
-      const int hy = r / kHx, hx = r - hy * kHx;
-      const int zz = z0 + hz - 1, yy = y0 + hy - 1, xx = x0 + hx - 1;
-      if (hv < kHalo && (unsigned)zz < (unsigned)vol.d && (unsigned)yy < (unsigned)vol.h &&
-          (unsigned)xx < (unsigned)vol.w) {
-        const uint16_t *src =
-            xs_src + ((size_t)bb * (vstride >> (3 * sh)) +
-                      ((int64_t)(zz >> sh) * (vol.h >> sh) + (yy >> sh)) * (vol.w >> sh) + (xx >> sh)) * xs_c + xs_c0;
-        rh[q][0] = ld16(src);
-        rh[q][1] = ld16(src + 8);
-      }
-    }
-  };
-  // registers -> LDS, transposed
-  auto store_brick = [&]() {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      dyT[c * kDyRow + t] = (uint16_t)(rdy[0][c >> 1] >> (16 * (c & 1)));
-      dyT[(8 + c) * kDyRow + t] = (uint16_t)(rdy[1][c >> 1] >> (16 * (c & 1)));
-      if (KS == 1) {
-        xs[c * xchan + t] = (uint16_t)(rx[0][c >> 1] >> (16 * (c & 1)));
-        xs[(8 + c) * xchan + t] = (uint16_t)(rx[1][c >> 1] >> (16 * (c & 1)));
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < nh; ++q) {
-      const int hv = threadIdx.x + 256 * q;
-      if (hv < kHalo) {
-        const int hz = hv / (kHy * kHx), r = hv - hz * (kHy * kHx);
-        const int hy = r / kHx, hx = r - hy * kHx;
-        const int e = (hz * kHy + hy) * kXRow + hx;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          xs[c * xchan + e] = (uint16_t)(rh[q][0][c >> 1] >> (16 * (c & 1)));
-          xs[(8 + c) * xchan + e] = (uint16_t)(rh[q][1][c >> 1] >> (16 * (c & 1)));
-        }
-      }
-    }
-  };
-  if (LBM3D_CONV_WGRAD_PREFETCH) load_brick(b0);
-  for (uint32_t br = b0; br < b1; ++br) {
-    if (!LBM3D_CONV_WGRAD_PREFETCH) load_brick(br);
-    __syncthreads();  // the previous brick's LDS reads are done
-    store_brick();
-    __syncthreads();
-    // the next brick's loads are in flight while this one's MFMAs run
-    if (LBM3D_CONV_WGRAD_PREFETCH && br + 1 < b1) load_brick(br + 1);
-    if (KS == 1) {
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int k0 = 32 * (2 * wave + q) + 8 * g;
-        const u32x4 a = *reinterpret_cast<const u32x4 *>(&dyT[r16 * kDyRow + k0]);
-        const u32x4 b = *reinterpret_cast<const u32x4 *>(&xs[r16 * xchan + k0]);
-        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
-                                                         acc[0], 0, 0, 0);
-      }
-    } else {
-#pragma unroll 2
-      for (int kc = 0; kc < 8; ++kc) {
-        // K values 8g .. 8g+7 of this chunk: brick voxels x = 8(g&1) .. +7 of
-        // row y = (2kc + g/2) % 8, z = kc / 4
-        const u32x4 a = *reinterpret_cast<const u32x4 *>(&dyT[r16 * kDyRow + 32 * kc + 8 * g]);
-        const int lz = kc >> 2, ly = (2 * kc + (g >> 1)) & 7, jx = 8 * (g & 1);
-#pragma unroll
-        for (int i = 0; i < nacc; ++i) {
-          const int t = wave + 4 * i;  // wave-uniform
-          if (t < taps) {
-            const int dz = t / 9 - 1, dyo = (t / 3) % 3 - 1, dx = t % 3 - 1;
-            const uint16_t *rowp = &xs[r16 * xchan + ((lz + dz + 1) * kHy + (ly + dyo + 1)) * kXRow + jx];
-            // halo x = jx + dx + 1 .. +7, shifted by dx + 1 elements from an aligned read
-            const u32x4 w0 = *reinterpret_cast<const u32x4 *>(rowp);
-            u32x4 b = w0;
-            if (dx >= 0) {
-              const uint32_t w4 = *reinterpret_cast<const uint32_t *>(rowp + 8);
-              if (dx == 0)
-                b = u32x4{__builtin_amdgcn_alignbyte(w0[1], w0[0], 2u), __builtin_amdgcn_alignbyte(w0[2], w0[1], 2u),
-                          __builtin_amdgcn_alignbyte(w0[3], w0[2], 2u), __builtin_amdgcn_alignbyte(w4, w0[3], 2u)};
-              else
-                b = u32x4{w0[1], w0[2], w0[3], w4};
-            }
-            acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                             __builtin_bit_cast(bf16x8, b), acc[i], 0, 0, 0);
-          }
-        }
-      }
-    }
-  }
-  // C layout: lane holds rows (co) 4g .. 4g+3, column (ci) r16; part[set][tap][co][ci]
-  // with set = block (3x3x3) or 4 * block + wave (1x1x1)
-#pragma unroll
-  for (int i = 0; i < nacc; ++i) {
-    const int t = KS == 3 ? wave + 4 * i : 0;
-    const size_t set = KS == 3 ? blockIdx.x : (size_t)blockIdx.x * 4 + wave;
-    if (t >= taps) break;
-    float *dst = part + (set * taps + t) * cout * cin + (size_t)(co0 + 4 * g) * cin + c0 + r16;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) dst[(size_t)e * cin] = acc[i][e];
-  }
+// 8 voxels of one channel: a 4-voxel transposed read and the next
+__device__ __forceinline__ bf16x8 read_tr(const char *p, int next) {
+  const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ltr_t)p);
+  const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ltr_t)(p + next));
+  return __builtin_bit_cast(bf16x8, (bf16x8s)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// One pass of the tree fold of partial weight-gradient sets, in place: the
-// thread for (group q, element e) sums sets q*16*stride + j*stride, j < 16, at
-// element e into the group's first set.  Passes with stride 1, 16, 256, ...
-// leave the total in set 0, summed in an order fixed by the set count alone.
-__global__ void k_wgrad_fold_pass(float *__restrict__ part, int64_t set_size, int nsets, int stride) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t groups = (nsets + 16ll * stride - 1) / (16ll * stride);
-  if (i >= groups * set_size) return;
-  const int64_t q = i / set_size, e = i - q * set_size;
-  const int64_t first = q * 16 * stride;
-  float v[16];
+template <int WCO, bool UP>
+__global__ void __launch_bounds__(192 * WCO)
+    k_wgrad3(const uint16_t *__restrict__ x, const uint16_t *__restrict__ dy, float *__restrict__ part, const Vol vol,
+             int cin, int cout, int kpad, const Bricks bk, uint32_t per_block, uint32_t n, Div tiles,
+             const uint16_t *__restrict__ low, int c_low) {
+  constexpr int T = 192 * WCO;                                // threads
+  constexpr int PX = 2, PD = 2 * WCO;                         // 16-byte pieces of a voxel of x and of dy
+  constexpr int VX = 16 * PX, VD = 16 * PD;                   // bytes
+  constexpr int EX = kHalo * PX, ED = 256 * PD;               // pieces of x's halo and of dy
+  constexpr int NX = (EX + T - 1) / T, ND = (ED + T - 1) / T;  // loads per thread
+  __shared__ u32x4 tile[EX + ED];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, r16 = lane & 15;
+  const int dx = wave % 3, wco = wave / 3;
+  // (set, channel tiles) with the tiles fastest, in runs per XCD: the workgroups
+  // that read the same bricks, and their halos, run together on one L2 (48 -> 16
+  // channels at 2 x 128^3: 295 us, 552 in plain order)
+  const uint32_t job = xcd_block(LBM3D_CONV_WGRAD_XCD_CHUNK, blockIdx.x & 7u, blockIdx.x >> 3, n);
+  if (job >= n) return;  // padding block of the grid
+  const uint32_t set = qdiv(job, tiles), ct = job - set * tiles.d;
+  const uint32_t nci = (uint32_t)cin / 16u;
+  const int co0 = (int)(ct / nci) * 16 * WCO, c0 = (int)(ct % nci) * 16;
+  // UP: x's channels below c_low come from `low`, a volume of half the extents, upsampled
+  const bool from_low = UP && c0 < c_low;
+  const int sh = from_low ? 1 : 0, xd = vol.d >> sh, xh = vol.h >> sh, xw = vol.w >> sh;
+  const int xc = from_low ? c_low : (UP ? cin - c_low : cin), xc0 = UP && !from_low ? c0 - c_low : c0;
+  const uint16_t *const xsrc = from_low ? low : x;
+  const int64_t vstride = (int64_t)vol.d * vol.h * vol.w;
+
+  int hpos[NX];  // halo coordinates of this thread's pieces of x: hz << 10 | hy << 5 | hx
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int64_t set = first + (int64_t)j * stride;
-    v[j] = set < nsets ? part[set * set_size + e] : 0.f;
+  for (int q = 0; q < NX; ++q) {
+    const int hv = (T * q + (int)threadIdx.x) / PX;
+    hpos[q] = hv / (kHy * kHx) << 10 | hv / kHx % kHy << 5 | hv % kHx;
   }
+  auto load = [&](uint32_t brick) {
+    const uint16_t *const zero = reinterpret_cast<const uint16_t *>(conv_zero);
+    int bb, z0, y0, x0;
+    brick_origin(bk, brick, bb, z0, y0, x0);
+    const uint16_t *const xv = xsrc + (size_t)bb * xd * xh * xw * xc + xc0;
+    const uint16_t *const dv = dy + (size_t)bb * vstride * cout + co0;
+#pragma unroll
+    for (int q = 0; q < NX; ++q) {
+      const int e = T * q + (int)threadIdx.x;
+      const int zz = z0 - 1 + (hpos[q] >> 10), yy = y0 - 1 + (hpos[q] >> 5 & 31), xx = x0 - 1 + (hpos[q] & 31);
+      const bool in = (unsigned)zz < (unsigned)vol.d && (unsigned)yy < (unsigned)vol.h && (unsigned)xx < (unsigned)vol.w;
+      const uint16_t *src = xv + ((int64_t)(((zz >> sh) * xh + (yy >> sh)) * xw + (xx >> sh)) * xc + 8 * (e % PX));
+      if (NX * T == EX || e < EX)
+        __builtin_amdgcn_global_load_lds((gptr_t)(in ? src : zero), (lptr_t)(tile + T * q + 64 * wave), 16, 0, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < ND; ++q) {
+      const int e = T * q + (int)threadIdx.x, v = e / PD;
+      const int zz = z0 + (v >> 7), yy = y0 + (v >> 4 & 7), xx = x0 + (v & 15);
+      const bool in = zz < vol.d && yy < vol.h && xx < vol.w;
+      const uint16_t *src = dv + ((int64_t)((zz * vol.h + yy) * vol.w + xx) * cout + 8 * (e % PD));
+      if (ND * T == ED || e < ED)
+        __builtin_amdgcn_global_load_lds((gptr_t)(in ? src : zero), (lptr_t)(tile + EX + T * q + 64 * wave), 16, 0, 0);
+    }
+  };
+
+  // transposed reads: lane 16 g + i takes 4 channels of voxel i / 4 of the 4
+  // (then the next 4) of row g / 2 of the pair, x half g % 2
+  const char *const xb = reinterpret_cast<const char *>(tile) +
+                         (((g >> 1) * kHx + dx + 8 * (g & 1) + (r16 >> 2)) * VX + 8 * (r16 & 3));
+  const char *const db =
+      reinterpret_cast<const char *>(tile) + EX * 16 + ((8 * g + (r16 >> 2)) * VD + 32 * wco + 8 * (r16 & 3));
+  f32x4 acc[9];  // taps (tz, ty) of this dx
+#pragma unroll
+  for (int t = 0; t < 9; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const uint32_t b0 = set * per_block, b1 = b0 + per_block < bk.n ? b0 + per_block : bk.n;
+  for (uint32_t br = b0; br < b1; ++br) {
+    if (br != b0) __syncthreads();  // the previous brick's reads are done
+    load(br);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    __syncthreads();
+    bf16x8 a[8];
+#pragma unroll
+    for (int kc = 0; kc < 8; ++kc) a[kc] = read_tr(db + 32 * kc * VD, 4 * VD);
+    // B fragment n = (halo plane hz, first halo row hy), two read ahead; the
+    // scheduling barriers keep the compiler from reading further ahead
+    bf16x8 b[3];
+    auto read_b = [&](int n) { b[n % 3] = read_tr(xb + ((n / 9) * kHy + n % 9) * kHx * VX, 4 * VX); };
+    read_b(0);
+    read_b(1);
+#pragma unroll
+    for (int n = 0; n < 36; ++n) {
+      const int hz = n / 9, hy = n % 9;
+      if (n + 2 < 36) read_b(n + 2);
+#pragma unroll
+      for (int tz = 0; tz < 3; ++tz)
+#pragma unroll
+        for (int ty = 0; ty < 3; ++ty) {
+          const int z = hz - tz, y2 = hy - ty;  // the chunk's plane and first row
+          if (z >= 0 && z < 2 && y2 >= 0 && y2 < 8 && !(y2 & 1))
+            acc[3 * tz + ty] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[4 * z + y2 / 2], b[n % 3], acc[3 * tz + ty],
+                                                                     0, 0, 0);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // C layout: lane holds rows (co) 4g .. 4g+3, column (ci) r16; part[set][co][kpad]
+  float *dst = part + (size_t)set * cout * kpad + (size_t)(co0 + 16 * wco + 4 * g) * kpad + c0 + r16;
+#pragma unroll
+  for (int t = 0; t < 9; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dst[(size_t)e * kpad + (3 * t + dx) * cin] = acc[t][e];
+}
+
+// 1x1x1: workgroup (p, channel tiles): a run of bricks, staged one at a time in
+// 16 KB, so that eight workgroups' loads are in flight on a CU; wave w takes K
+// chunks 2w and 2w + 1 of each.  Partial sets: one per wave, part[4 p +
+// wave][co][kpad].  Bound by HBM.
+__global__ void __launch_bounds__(256)
+    k_wgrad1(const uint16_t *__restrict__ x, const uint16_t *__restrict__ dy, float *__restrict__ part, const Vol vol,
+             int cin, int cout, int kpad, const Bricks bk, uint32_t per_block) {
+  __shared__ u32x4 tile[1024];  // 256 voxels x 16 channels of x, then of dy
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, r16 = lane & 15;
+  const int nci = cin / 16;
+  const int co0 = (int)(blockIdx.y / (unsigned)nci) * 16, c0 = (int)(blockIdx.y % (unsigned)nci) * 16;
+  auto load = [&](uint32_t brick) {
+    const uint16_t *const zero = reinterpret_cast<const uint16_t *>(conv_zero);
+    int bb, z0, y0, x0;
+    brick_origin(bk, brick, bb, z0, y0, x0);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int e = 256 * q + (int)threadIdx.x, v = e >> 1;
+      const int zz = z0 + (v >> 7), yy = y0 + (v >> 4 & 7), xx = x0 + (v & 15);
+      const bool in = zz < vol.d && yy < vol.h && xx < vol.w;
+      const int64_t vx = (((int64_t)bb * vol.d + zz) * vol.h + yy) * vol.w + xx;
+      const uint16_t *const xs = x + (vx * cin + c0 + 8 * (e & 1)), *const ds = dy + (vx * cout + co0 + 8 * (e & 1));
+      __builtin_amdgcn_global_load_lds((gptr_t)(in ? xs : zero), (lptr_t)(tile + 256 * q + 64 * wave), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((gptr_t)(in ? ds : zero), (lptr_t)(tile + 512 + 256 * q + 64 * wave), 16, 0, 0);
+    }
+  };
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int off = (64 * wave + 8 * g + (r16 >> 2)) * 32 + 8 * (r16 & 3);
+  const uint32_t b0 = blockIdx.x * per_block, b1 = b0 + per_block < bk.n ? b0 + per_block : bk.n;
+  const char *const p = reinterpret_cast<const char *>(tile) + off;
+  for (uint32_t br = b0; br < b1; ++br) {
+    if (br != b0) __syncthreads();  // the previous brick's reads are done
+    load(br);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(read_tr(p + 8192 + 1024 * c, 128), read_tr(p + 1024 * c, 128), acc,
+                                                    0, 0, 0);
+  }
+  float *dst = part + ((size_t)blockIdx.x * 4 + wave) * cout * kpad + (size_t)(co0 + 4 * g) * kpad + c0 + r16;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) dst[(size_t)e * kpad] = acc[e];
+}
+
+// v[0] = ((v0 + v8) + (v4 + v12)) + ...: the sum of 16 terms, halves first
+__device__ __forceinline__ float tree16(float v[16]) {
 #pragma unroll
   for (int w = 8; w >= 1; w >>= 1)
 #pragma unroll
     for (int j = 0; j < w; ++j) v[j] += v[j + w];
-  part[first * set_size + e] = v[0];
+  return v[0];
 }
 
-// Sums nsets partial sets into dw: tree passes of k_wgrad_fold_pass while more
-// than 16 sets remain, then k_wgrad_fold over the survivors.
-int wgrad_fold(hipStream_t s, float *part, float *dw, int nsets, int taps, int cin, int cout, int kpad);
-
-__global__ void k_wgrad_fold(const float *__restrict__ part, float *__restrict__ dw, int nsets, int set_step, int taps,
-                             int cin, int cout, int kpad) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)cout * kpad) return;
-  const int co = (int)(i / kpad), k = (int)(i % kpad);
+// dst[e] = sum of the terms part[q step + e] of nsets <= 4096 sets (step: the size
+// of a set, or of 16 after a first level), in an order fixed by nsets alone:
+// groups of 16 consecutive sets by tree16 while more than 16 terms remain, the
+// last (at most 16) terms one after another.  A block takes 64 elements; its wave
+// w sums the groups w, w + 16, ..., so that 16 waves hold one group of groups at
+// a time: one launch for what took a pass per level.  Elements whose column (e %
+// kpad) is past `used` are padding: 0.
+__global__ void __launch_bounds__(1024)
+    k_fold_sets(const float *__restrict__ part, float *__restrict__ dst, int64_t size, int64_t step, int nsets,
+                int kpad, int used) {
+  __shared__ float red[16][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t e = (int64_t)blockIdx.x * 64 + lane;
+  const bool live = e < size && (int)(e % kpad) < used;
+  const float *const p = part + e;
+  if (nsets <= 16) {  // one term a set
+    red[wave][lane] = live && wave < nsets ? p[wave * step] : 0.f;
+    __syncthreads();
+    if (wave == 0 && e < size) {
+      float s = 0.f;
+      for (int q = 0; q < nsets; ++q) s += red[q][lane];
+      dst[e] = s;
+    }
+    return;
+  }
+  const int groups = (nsets + 15) / 16;
   float s = 0.f;
-  if (k < taps * cin) {
-    const int tap = k / cin, ci = k % cin;
-    const size_t stride = (size_t)taps * cout * cin;
-    const size_t off = ((size_t)tap * cout + co) * cin + ci;
-    for (int q = 0; q < nsets; ++q) s += part[(size_t)q * set_step * stride + off];
+  for (int q0 = 0; q0 < groups; q0 += 16) {  // uniform in the block
+    const int first = (q0 + wave) * 16;
+    float v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = live && first + j < nsets ? p[(first + j) * step] : 0.f;
+    if (q0) __syncthreads();  // the previous group of groups has been read
+    red[wave][lane] = tree16(v);
+    __syncthreads();
+    if (wave == 0) {
+      if (groups <= 16) {  // at most 16 terms: one after another
+        for (int q = 0; q < groups; ++q) s += red[q][lane];
+      } else {
+        float u[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) u[j] = red[j][lane];
+        s += tree16(u);
+      }
+    }
   }
-  dw[i] = s;
+  if (wave == 0 && e < size) dst[e] = s;
 }
 
-int wgrad_fold(hipStream_t s, float *part, float *dw, int nsets, int taps, int cin, int cout, int kpad) {
-  const int64_t set_size = (int64_t)taps * cout * cin;
-  int stride = 1;
-  while (nsets > 16 * stride) {  // sets 0, stride, 2*stride, ... hold the partial sums
-    const int64_t groups = (nsets + 16ll * stride - 1) / (16ll * stride);
-    const int64_t threads = groups * set_size;
-    k_wgrad_fold_pass<<<(unsigned)((threads + 255) / 256), 256, 0, s>>>(part, set_size, nsets, stride);
-    if (int rc = ccheck("lbm3d_conv3d_wgrad/fold pass")) return rc;
-    stride *= 16;
+// The same for at most 256 sets of many elements: one thread an element.
+__global__ void __launch_bounds__(256)
+    k_fold_few(const float *__restrict__ part, float *__restrict__ dst, int64_t size, int nsets, int kpad, int used) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= size) return;
+  float s = 0.f;
+  if ((int)(e % kpad) < used) {
+    const float *const p = part + e;
+    if (nsets <= 16) {
+      float v[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v[j] = j < nsets ? p[(int64_t)j * size] : 0.f;
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (j < nsets) s += v[j];
+    } else {
+      for (int first = 0; first < nsets; first += 16) {
+        float v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = first + j < nsets ? p[(int64_t)(first + j) * size] : 0.f;
+        s += tree16(v);
+      }
+    }
   }
-  const int64_t total = (int64_t)cout * kpad;
-  k_wgrad_fold<<<(unsigned)((total + 255) / 256), 256, 0, s>>>(part, dw, (nsets + stride - 1) / stride, stride, taps,
-                                                                cin, cout, kpad);
-  return ccheck("lbm3d_conv3d_wgrad/fold");
+  dst[e] = s;
+}
+
+// One level of the fold for more sets: part[16 q] = tree16 of sets 16 q .. +15, in place.
+__global__ void __launch_bounds__(256)
+    k_fold_level(float *__restrict__ part, int64_t size, int nsets) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (int64_t)((nsets + 15) / 16) * size) return;
+  const int64_t q = i / size, e = i - q * size;
+  float v[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) v[j] = 16 * q + j < nsets ? part[(16 * q + j) * size + e] : 0.f;
+  part[16 * q * size + e] = tree16(v);
+}
+
+int fold_sets(hipStream_t s, float *part, float *dst, int64_t size, int nsets, int kpad, int used) {
+  // a thread an element where there are enough elements to fill the GPU: 32 sets of
+  // 442 k (the gradient of 128 -> 128 channels, 2 x 16^3, takes 30 us in all; 60
+  // with a block of 16 waves for 64 elements), but 128 sets of 57 k 29 us with
+  // the block and 35 with the thread
+  if (nsets <= 256 && size >= 100000) {
+    k_fold_few<<<(unsigned)((size + 255) / 256), 256, 0, s>>>(part, dst, size, nsets, kpad, used);
+  } else if (nsets <= 4096) {
+    k_fold_sets<<<(unsigned)((size + 63) / 64), 1024, 0, s>>>(part, dst, size, size, nsets, kpad, used);
+  } else {
+    const int64_t n = (int64_t)((nsets + 15) / 16) * size;
+    k_fold_level<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(part, size, nsets);
+    if (int rc = ccheck("fold of partial sums")) return rc;
+    k_fold_sets<<<(unsigned)((size + 63) / 64), 1024, 0, s>>>(part, dst, size, 16 * size, (nsets + 15) / 16, kpad, used);
+  }
+  return ccheck("fold of partial sums");
 }
 
 int check_conv(int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout, int32_t ks) {
@@ -1054,20 +1117,21 @@ int check_conv(int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t
 
 constexpr int kWgTargetBlocks = 2048;
 
-// Tiled weight gradient: bricks per workgroup and workgroups along the brick
-// range, about kWgTargetBlocks workgroups in all.
-int wgrad_tiled_plan(int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout, uint32_t &nbricks,
-                     uint32_t &per) {
-  const int64_t nb = (int64_t)n * ((d + kBz - 1) / kBz) * ((h + kBy - 1) / kBy) * ((wd + kBx - 1) / kBx);
+// Weight gradient: bricks per set of partial sums and sets, about kWgTargetBlocks
+// (set, channel tile) pairs in all.  A set's bricks and the number of sets fix
+// the order of the sums.
+int wgrad_plan(const Bricks &bk, int32_t cin, int32_t cout, uint32_t &per) {
+  const int64_t nb = bk.n;
   const int64_t tiles = (int64_t)(cout / 16) * (cin / 16);
   int64_t P = (kWgTargetBlocks + tiles - 1) / tiles;
   if (P > nb) P = nb;
   if (P < 1) P = 1;
   const int64_t pb = (nb + P - 1) / P;
-  nbricks = (uint32_t)nb;
   per = (uint32_t)pb;
   return (int)((nb + pb - 1) / pb);
 }
+
+constexpr int wgrad_sets(int ks) { return ks == 3 ? 1 : 4; }  // partial sets of a workgroup
 
 // ---------------------------------------------------------------------------
 // Periodic distance to solid (the surrogate's second input channel): the
@@ -1410,16 +1474,18 @@ __global__ void __launch_bounds__(256)
   decode(low, (uint32_t)v, b, z, yy, x);
   const int64_t h2 = 2 * low.h, w2 = 2 * low.w;
   const uint16_t *src = g + ((((int64_t)b * low.d + z) * 2 * h2 + 2 * yy) * w2 + 2 * x) * c + 8 * pc;
+  // the order of torch's sum over the block: z pairs, then the four in turn
   float sum[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+  for (int k = 0; k < 4; ++k) {
+    const uint16_t *q = src + ((int64_t)(k >> 1) * w2 + (k & 1)) * c;
+    const u32x4 a0 = ld16(q), a1 = ld16(q + h2 * w2 * c);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const u32x4 a = ld16(src + (((k >> 2) * h2 + ((k >> 1) & 1)) * w2 + (k & 1)) * c);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      sum[2 * e] += __uint_as_float(a[e] << 16);
-      sum[2 * e + 1] += __uint_as_float(a[e] & 0xFFFF0000u);
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t u0 = e & 1 ? a0[e >> 1] & 0xFFFF0000u : a0[e >> 1] << 16;
+      const uint32_t u1 = e & 1 ? a1[e >> 1] & 0xFFFF0000u : a1[e >> 1] << 16;
+      const float pair = __uint_as_float(u0) + __uint_as_float(u1);
+      sum[e] = k == 0 ? pair : sum[e] + pair;
     }
   }
   u32x4 o;
@@ -1572,12 +1638,12 @@ int lbm3d_conv3d_dgrad(void *stream, const uint16_t *dy, const uint16_t *wt, uin
 size_t lbm3d_conv3d_wgrad_workspace_bytes(int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t cout,
                                           int32_t ks) {
   if (check_conv(n, d, h, wd, cin, cout, ks)) return 0;
-  uint32_t nbricks, per;
-  const int parts = wgrad_tiled_plan(n, d, h, wd, cin, cout, nbricks, per);
-  return (size_t)parts * wgrad_sets(ks) * ks * ks * ks * cout * cin * sizeof(float);
+  uint32_t per;
+  return (size_t)wgrad_plan(make_bricks(n, d, h, wd), cin, cout, per) * wgrad_sets(ks) * cout *
+         lbm3d_conv_kpad(cin, ks) * sizeof(float);
 }
 
-// the tiled weight gradient and its fold; low / c_low: the upsampled part of x, if any
+// a weight gradient and its fold; low / c_low: the upsampled part of x, if any
 static int wgrad_run(void *stream, const uint16_t *x, const uint16_t *dy, float *dw, int32_t n, int32_t d, int32_t h,
                      int32_t wd, int32_t cin, int32_t cout, int32_t ks, void *workspace, size_t workspace_bytes,
                      const uint16_t *low, int c_low) {
@@ -1588,19 +1654,32 @@ static int wgrad_run(void *stream, const uint16_t *x, const uint16_t *dy, float 
     return cfail(LBM3D_EINVAL, "wgrad workspace too small");
   const Vol vol = make_vol(n, d, h, wd);
   hipStream_t s = (hipStream_t)stream;
-  uint32_t nbricks, per;
-  const int parts = wgrad_tiled_plan(n, d, h, wd, cin, cout, nbricks, per);
-  const int nbz = (d + kBz - 1) / kBz, nby = (h + kBy - 1) / kBy, nbx = (wd + kBx - 1) / kBx;
-  const dim3 grid((unsigned)parts, (unsigned)((cout / 16) * (cin / 16)));
-  if (ks == 3)
-    k_conv_wgrad_tiled<3><<<grid, 256, 0, s>>>(x, dy, (float *)workspace, vol, cin, cout, nbz, nby, nbx, nbricks, per,
-                                               low, c_low);
-  else
-    k_conv_wgrad_tiled<1><<<grid, 256, 0, s>>>(x, dy, (float *)workspace, vol, cin, cout, nbz, nby, nbx, nbricks, per,
-                                               nullptr, 0);
+  const Bricks bk = make_bricks(n, d, h, wd);
+  uint32_t per;
+  const int sets = wgrad_plan(bk, cin, cout, per), kpad = lbm3d_conv_kpad(cin, ks);
+  float *part = (float *)workspace;
+  if (ks == 1) {
+    k_wgrad1<<<dim3((unsigned)sets, (unsigned)((cout / 16) * (cin / 16))), 256, 0, s>>>(x, dy, part, vol, cin, cout,
+                                                                                      kpad, bk, per);
+  } else {
+    // two output channel tiles a workgroup where there are, which share the staged x
+    const int wco = cout % 32 == 0 ? 2 : 1;
+    const uint32_t tiles = (uint32_t)((cout / (16 * wco)) * (cin / 16)), jobs = (uint32_t)sets * tiles;
+    const unsigned grid = (unsigned)xcd_grid(jobs, LBM3D_CONV_WGRAD_XCD_CHUNK);
+    const Div td = make_div(tiles);
+#define LBM3D_WGRAD3(O, U) \
+  k_wgrad3<O, U><<<grid, 192 * (O), 0, s>>>(x, dy, part, vol, cin, cout, kpad, bk, per, jobs, td, low, c_low)
+    if (wco == 2) {
+      if (c_low > 0) LBM3D_WGRAD3(2, true);
+      else LBM3D_WGRAD3(2, false);
+    } else {
+      if (c_low > 0) LBM3D_WGRAD3(1, true);
+      else LBM3D_WGRAD3(1, false);
+    }
+#undef LBM3D_WGRAD3
+  }
   if ((rc = ccheck("lbm3d_conv3d_wgrad"))) return rc;
-  const int kpad = lbm3d_conv_kpad(cin, ks);
-  return wgrad_fold(s, (float *)workspace, dw, parts * wgrad_sets(ks), ks * ks * ks, cin, cout, kpad);
+  return fold_sets(s, part, dw, (int64_t)cout * kpad, sets * wgrad_sets(ks), kpad, ks * ks * ks * cin);
 }
 
 int lbm3d_conv3d_wgrad(void *stream, const uint16_t *x, const uint16_t *dy, float *dw, int32_t n, int32_t d, int32_t h,
@@ -1635,8 +1714,7 @@ int lbm3d_relu_bias_grad(void *stream, const uint16_t *g, const uint16_t *y, uin
   hipStream_t s = (hipStream_t)stream;
   k_relu_bias_grad<false><<<(unsigned)blocks, 256, 0, s>>>(g, y, dz, (float *)workspace, chunks, c, per, PoolGrad{});
   if (int rc = ccheck("lbm3d_relu_bias_grad")) return rc;
-  // the wgrad fold with one tap and one output row: db[k] = sum over blocks of part[block][k]
-  return wgrad_fold(s, (float *)workspace, db, blocks, 1, c, 1, c);
+  return fold_sets(s, (float *)workspace, db, c, blocks, c, c);
 }
 
 int lbm3d_relu_pool_grad(void *stream, const uint16_t *g, const uint16_t *y, const uint16_t *pooled,
@@ -1661,7 +1739,7 @@ int lbm3d_relu_pool_grad(void *stream, const uint16_t *g, const uint16_t *y, con
   k_relu_bias_grad<true><<<(unsigned)blocks, 256, 0, s>>>(g, y, dz, (float *)workspace, chunks, c, per,
                                                          PoolGrad{pooled, share, make_vol(n, d, h, w), pieces});
   if (int rc = ccheck("lbm3d_relu_pool_grad")) return rc;
-  return wgrad_fold(s, (float *)workspace, db, blocks, 1, c, 1, c);
+  return fold_sets(s, (float *)workspace, db, c, blocks, c, c);
 }
 
 static int distance_passes(void *stream, const int8_t *solid, void *out, int mode, float *work, int32_t n, int32_t d,
