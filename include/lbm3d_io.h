@@ -33,6 +33,15 @@ int64_t lbm3d_read_geo_ascii(const char *path, int32_t nx, int32_t ny, int32_t n
 int lbm3d_voxelize(void *stream, const float *tris, int32_t n_tris, double x0, double y0, double z0, double dx,
                    int32_t nx, int32_t ny, int32_t nz, int8_t *solid);
 
+/* The same flags, faster: blocks of nodes away from the surface are decided by
+ * one bounded sum at their centre, and only nodes that a bounded FP32 sum leaves
+ * open take lbm3d_voxelize's FP64 sum.  `workspace`: DEVICE,
+ * lbm3d_voxelize_workspace_bytes(nx, ny, nz) bytes. */
+size_t lbm3d_voxelize_workspace_bytes(int32_t nx, int32_t ny, int32_t nz);
+int lbm3d_voxelize_blocks(void *stream, const float *tris, int32_t n_tris, double x0, double y0, double z0, double dx,
+                          int32_t nx, int32_t ny, int32_t nz, int8_t *solid, void *workspace,
+                          size_t workspace_bytes);
+
 #ifdef __cplusplus
 }
 #endif

@@ -161,6 +161,9 @@ SIGNATURES = {
     "lbm3d_read_geo_ascii": (_i64, [ctypes.c_char_p, _i32, _i32, _i32, _vp]),
     "lbm3d_voxelize": (_int, [_vp, _vp, _i32, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double,
                               _i32, _i32, _i32, _vp]),
+    "lbm3d_voxelize_workspace_bytes": (_sz, [_i32, _i32, _i32]),
+    "lbm3d_voxelize_blocks": (_int, [_vp, _vp, _i32, ctypes.c_double, ctypes.c_double, ctypes.c_double,
+                                     ctypes.c_double, _i32, _i32, _i32, _vp, _vp, _sz]),
 }
 
 

@@ -12,9 +12,13 @@
 // solid angle of Van Oosterom and Strackee,
 //   tan(Omega/2) = a.(b x c) / (|a||b||c| + (a.b)|c| + (b.c)|a| + (c.a)|b|),
 // a, b, c the triangle's corners relative to p, in FP64; the node is solid when
-// w >= 1/2.  One thread per node; triangles are staged through LDS in tiles.
+// w >= 1/2.  k_winding does that for every node, one thread each, triangles
+// staged through LDS in tiles.  lbm3d_voxelize_blocks gives the same flags from
+// far fewer sums: away from the surface whole blocks of nodes share a flag, and a
+// bounded FP32 sum settles nearly every node of the others.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cerrno>
 #include <cmath>
 #include <cstdint>
@@ -37,6 +41,25 @@ int iofail(int code, const char *msg, const char *what = "") {
 
 constexpr int kTriTile = 256;
 
+// twice the FP64 angle of one triangle's solid angle at (px, py, pz)
+__device__ __forceinline__ double triangle_angle(const float *v, double px, double py, double pz) {
+  const double ax = v[0] - px, ay = v[1] - py, az = v[2] - pz;
+  const double bx = v[3] - px, by = v[4] - py, bz = v[5] - pz;
+  const double cx = v[6] - px, cy = v[7] - py, cz = v[8] - pz;
+  const double la = sqrt(ax * ax + ay * ay + az * az);
+  const double lb = sqrt(bx * bx + by * by + bz * bz);
+  const double lc = sqrt(cx * cx + cy * cy + cz * cz);
+  const double det = ax * (by * cz - bz * cy) - ay * (bx * cz - bz * cx) + az * (bx * cy - by * cx);
+  const double den = la * lb * lc + (ax * bx + ay * by + az * bz) * lc + (bx * cx + by * cy + bz * cz) * la +
+                     (cx * ax + cy * ay + cz * az) * lb;
+  return 2.0 * atan2(det, den);
+}
+
+__device__ __forceinline__ int8_t winding_flag(double omega) {
+  const double w = omega / (4.0 * M_PI);
+  return w >= 0.5 ? 1 : 0;
+}
+
 __global__ void __launch_bounds__(256)
     k_winding(const float *__restrict__ tris, int32_t n_tris, double x0, double y0, double z0, double dx, int32_t nx,
               int32_t ny, int32_t nz, int8_t *__restrict__ solid) {
@@ -58,25 +81,180 @@ __global__ void __launch_bounds__(256)
     for (int e = threadIdx.x; e < cnt * 9; e += blockDim.x) s_tri[e] = tris[(int64_t)base * 9 + e];
     __syncthreads();
     if (id < n) {
-      for (int t = 0; t < cnt; ++t) {
-        const float *v = s_tri + 9 * t;
-        const double ax = v[0] - px, ay = v[1] - py, az = v[2] - pz;
-        const double bx = v[3] - px, by = v[4] - py, bz = v[5] - pz;
-        const double cx = v[6] - px, cy = v[7] - py, cz = v[8] - pz;
-        const double la = sqrt(ax * ax + ay * ay + az * az);
-        const double lb = sqrt(bx * bx + by * by + bz * bz);
-        const double lc = sqrt(cx * cx + cy * cy + cz * cz);
-        const double det = ax * (by * cz - bz * cy) - ay * (bx * cz - bz * cx) + az * (bx * cy - by * cx);
-        const double den = la * lb * lc + (ax * bx + ay * by + az * bz) * lc + (bx * cx + by * cy + bz * cz) * la +
-                           (cx * ax + cy * ay + cz * az) * lb;
-        omega += 2.0 * atan2(det, den);
+      for (int t = 0; t < cnt; ++t) omega += triangle_angle(s_tri + 9 * t, px, py, pz);
+    }
+  }
+  if (id < n) solid[id] = winding_flag(omega);
+}
+
+// ---------------------------------------------------------------------------
+// The same flags block by block.  The solid angle Omega of the mesh changes by at
+// most rho * sum_t 2 A_t / (d_t - rho)^3 within rho of a point (A_t a triangle's
+// area, d_t its distance; the field of a surface element falls off as 1/r^2), so
+// if Omega at a block's centre is further from the threshold 2 pi than that and
+// than the error of the sum, all of the block's nodes have one flag.  Blocks of 4
+// nodes a side are tried first, 2 a side where those are undecided, then single
+// nodes, whose sum needs no such bound; a node that the error bound leaves open
+// (on the surface, in the plane of a triangle next to it) gets the FP64 sum in
+// triangle order, bit for bit k_winding's.
+//
+// Omega / 2 is the argument of prod_t (den_t + i det_t): a wave takes a parent
+// block, its lanes the triangles in turn, and each lane keeps 8 running products
+// (the parent's 8 children), normalised, with the turns they have made.  Lengths
+// are in cells, relative to the parent's centre (FP64 difference, rounded once).
+// 7,680 triangles on 96 x 104 x 88 nodes: 2.57 ms against 33.2 ms for all nodes
+// in FP64; bound by FP32 arithmetic.
+// ---------------------------------------------------------------------------
+struct VoxGrid {
+  double x0, y0, z0, dx;
+  int32_t nx, ny, nz;
+  int32_t n_tris;
+  float eta;  // FP64 rounding of a node's coordinates, in cells
+};
+
+// how many blocks of side s cover n nodes
+__host__ __device__ __forceinline__ int32_t blocks_of(int32_t n, int32_t s) { return (n + s - 1) / s; }
+
+// The children of side S of the parents (side 2S) in `list` (all parents if it is
+// null): flags of the decided ones, the others' block indices to `next`.
+template <int S>
+__global__ void __launch_bounds__(256)
+    k_winding_blocks(const float *__restrict__ tris, const VoxGrid gr, const int32_t *__restrict__ list,
+                     const int32_t *__restrict__ count, int32_t all, int32_t *__restrict__ next,
+                     int32_t *__restrict__ next_count, int8_t *__restrict__ solid) {
+  const int lane = threadIdx.x & 63;
+  const int32_t waves = (int32_t)(gridDim.x * 4);
+  const int32_t n = list ? *count : all;
+  const int32_t pny = blocks_of(gr.ny, 2 * S), pnz = blocks_of(gr.nz, 2 * S);
+  const int32_t cnx = blocks_of(gr.nx, S), cny = blocks_of(gr.ny, S), cnz = blocks_of(gr.nz, S);
+  const double inv = 1.0 / gr.dx;
+  for (int32_t it = (int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6)); it < n; it += waves) {
+    const int32_t id = __builtin_amdgcn_readfirstlane(list ? list[it] : it);
+    const int32_t bk = id % pnz, bt = id / pnz, bj = bt % pny, bi = bt / pny;
+    // the parent's reference point, and its children's centres relative to it, in cells
+    const double pi = 2 * S * bi + S - 0.5, pj = 2 * S * bj + S - 0.5, pk = 2 * S * bk + S - 0.5;
+    const double px = gr.x0 + gr.dx * pi, py = gr.y0 + gr.dx * pj, pz = gr.z0 + gr.dx * pk;
+    float zr[8], zi[8], err[8];
+    int turns[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      zr[c] = 1.f;
+      zi[c] = err[c] = 0.f;
+      turns[c] = 0;
+    }
+    constexpr float off = 0.5f * S;                    // a child's centre, per axis
+    constexpr float rho = 0.866026f * (S - 1);         // its half diagonal
+    constexpr float reach = 2.f * 1.7320508f * off;    // twice the offset's length
+    for (int32_t t = lane; t < gr.n_tris; t += 64) {
+      const float *v = tris + (int64_t)t * 9;
+      const float ax = (float)(((double)v[0] - px) * inv), ay = (float)(((double)v[1] - py) * inv),
+                  az = (float)(((double)v[2] - pz) * inv);
+      const float bx = (float)(((double)v[3] - px) * inv), by = (float)(((double)v[4] - py) * inv),
+                  bz = (float)(((double)v[5] - pz) * inv);
+      const float cx = (float)(((double)v[6] - px) * inv), cy = (float)(((double)v[7] - py) * inv),
+                  cz = (float)(((double)v[8] - pz) * inv);
+      float area2 = 0.f, edge = 0.f;  // 2 A and a bound on how far the triangle reaches from its nearest corner
+      if constexpr (S > 1) {
+        const float ux = bx - ax, uy = by - ay, uz = bz - az, wx = cx - ax, wy = cy - ay, wz = cz - az;
+        const float nx = uy * wz - uz * wy, ny = uz * wx - ux * wz, nz = ux * wy - uy * wx;
+        area2 = 1.02f * sqrtf(nx * nx + ny * ny + nz * nz) + 1e-5f * (ux * ux + uy * uy + uz * uz + wx * wx + wy * wy + wz * wz);
+        const float vx = cx - bx, vy = cy - by, vz = cz - bz;
+        edge = 0.58f * sqrtf(fmaxf(fmaxf(ux * ux + uy * uy + uz * uz, wx * wx + wy * wy + wz * wz), vx * vx + vy * vy + vz * vz));
+      }
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const float ox = c & 4 ? off : -off, oy = c & 2 ? off : -off, oz = c & 1 ? off : -off;
+        const float Ax = ax - ox, Ay = ay - oy, Az = az - oz, Bx = bx - ox, By = by - oy, Bz = bz - oz, Cx = cx - ox,
+                    Cy = cy - oy, Cz = cz - oz;
+        const float la = __builtin_amdgcn_sqrtf(Ax * Ax + Ay * Ay + Az * Az);
+        const float lb = __builtin_amdgcn_sqrtf(Bx * Bx + By * By + Bz * Bz);
+        const float lc = __builtin_amdgcn_sqrtf(Cx * Cx + Cy * Cy + Cz * Cz);
+        const float det = Ax * (By * Cz - Bz * Cy) - Ay * (Bx * Cz - Bz * Cx) + Az * (Bx * Cy - By * Cx);
+        const float L = la * lb * lc;
+        const float den = L + (Ax * Bx + Ay * By + Az * Bz) * lc + (Bx * Cx + By * Cy + Bz * Cz) * la +
+                          (Cx * Ax + Cy * Ay + Cz * Az) * lb;
+        const float lmin = fminf(fminf(la, lb), lc);
+        const float rz = __builtin_amdgcn_rsqf(det * det + den * den);
+        // Rounding.  A corner is off by at most 2^-24 kappa of its length, kappa = 1 +
+        // (reach + eta 2^24) / lmin; det and den then by (15 kappa + 74) 2^-24 L
+        // together, and the angle by that over |den + i det| (1.5 times for the arc).
+        const float kappa = 1.f + (reach + 1.7e7f * gr.eta) * __builtin_amdgcn_rcpf(lmin);
+        const float q = L * rz;  // at least 17^-1/2, unless something under- or overflowed
+        float e = (1.6e-6f * kappa + 7e-6f) * q;
+        // near the branch cut the sign of det, and with it a full turn, is open
+        if (!(q > 0.2f && e < 0.2f) || (den < 0.f && fabsf(det) * rz <= e)) e = 1e30f;
+        e += 1e-6f;  // the product's own rounding
+        if constexpr (S > 1) {
+          const float gap = lmin * 0.999f - edge - rho;
+          const float r = __builtin_amdgcn_rcpf(gap);
+          e += gap > 0.05f ? 0.51f * rho * area2 * (r * r * r) : 1e30f;  // of Omega / 2
+        }
+        err[c] += e;
+        const float ur = den * rz, ui = det * rz;
+        const float nr = zr[c] * ur - zi[c] * ui, ni = zr[c] * ui + zi[c] * ur;
+        // past +-pi: both angles on one side of the real axis, their sum on the other
+        turns[c] += (zi[c] >= 0.f && ui >= 0.f && ni < 0.f ? 1 : 0) - (zi[c] < 0.f && ui < 0.f && ni >= 0.f ? 1 : 0);
+        zr[c] = nr;
+        zi[c] = ni;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      float half = atan2f(zi[c], zr[c]) + 6.2831853f * (float)turns[c], e = err[c] + 5e-6f * (1.f + fabsf((float)turns[c]));
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1) {
+        half += __shfl_xor(half, d);
+        e += __shfl_xor(e, d);
+      }
+      const int32_t ci = 2 * bi + (c >> 2 & 1), cj = 2 * bj + (c >> 1 & 1), ck = 2 * bk + (c & 1);
+      if (ci >= cnx || cj >= cny || ck >= cnz) continue;  // uniform in the wave
+      // Omega >= 2 pi, Omega / 2 >= pi; rounding of the wave's sum included
+      const bool in = half >= 3.14159265f;
+      if (fabsf(half - 3.14159265f) > 1.01f * e + 1e-4f) {  // false for NaN
+        for (int q = lane; q < S * S * S; q += 64) {
+          const int i = S * ci + q / (S * S), j = S * cj + q / S % S, k = S * ck + q % S;
+          if (i < gr.nx && j < gr.ny && k < gr.nz) solid[((int64_t)i * gr.ny + j) * gr.nz + k] = in ? 1 : 0;
+        }
+      } else if (lane == 0) {
+        next[atomicAdd(next_count, 1)] = (ci * cny + cj) * cnz + ck;
       }
     }
   }
-  if (id < n) {
-    const double w = omega / (4.0 * M_PI);
-    solid[id] = w >= 0.5 ? 1 : 0;
+}
+
+// Nodes left open: one wave per node, the lanes' angles added in triangle order.
+__global__ void __launch_bounds__(256)
+    k_winding_nodes(const float *__restrict__ tris, const VoxGrid gr, const int32_t *__restrict__ list,
+                    const int32_t *__restrict__ count, int8_t *__restrict__ solid) {
+  const int lane = threadIdx.x & 63;
+  const int32_t n = *count, waves = (int32_t)(gridDim.x * 4);
+  for (int32_t it = (int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6)); it < n; it += waves) {
+    const int32_t id = __builtin_amdgcn_readfirstlane(list[it]);
+    const int32_t k = id % gr.nz, t0 = id / gr.nz, j = t0 % gr.ny, i = t0 / gr.ny;
+    const double px = gr.x0 + gr.dx * (double)i, py = gr.y0 + gr.dx * (double)j, pz = gr.z0 + gr.dx * (double)k;
+    double omega = 0.0;
+    for (int32_t base = 0; base < gr.n_tris; base += 64) {
+      const int32_t t = base + lane;
+      const double term = t < gr.n_tris ? triangle_angle(tris + (int64_t)t * 9, px, py, pz) : 0.0;
+      const int cnt = gr.n_tris - base < 64 ? gr.n_tris - base : 64;
+      for (int q = 0; q < cnt; ++q) omega += __shfl(term, q);
+    }
+    if (lane == 0) solid[id] = winding_flag(omega);
   }
+}
+
+__global__ void k_clear_counts(int32_t *counts) {
+  if (threadIdx.x < 4) counts[threadIdx.x] = 0;
+}
+
+// list places of a workspace, in int32: 4 counts, then the undecided blocks of 4,
+// of 2 and the open nodes
+int64_t vox_list(int32_t nx, int32_t ny, int32_t nz, int level) {
+  int64_t at = 64;
+  if (level > 0) at += (int64_t)blocks_of(nx, 4) * blocks_of(ny, 4) * blocks_of(nz, 4);
+  if (level > 1) at += (int64_t)blocks_of(nx, 2) * blocks_of(ny, 2) * blocks_of(nz, 2);
+  if (level > 2) at += (int64_t)nx * ny * nz;
+  return at;
 }
 
 }  // namespace
@@ -87,6 +265,43 @@ const char *lbm3d_io_last_error(void) { return io_err; }
 
 int64_t lbm3d_read_geo_ascii(const char *path, int32_t nx, int32_t ny, int32_t nz, int8_t *solid) {
   return lbm3d_ascii::read_geo(path, nx, ny, nz, solid, io_err, sizeof(io_err));
+}
+
+size_t lbm3d_voxelize_workspace_bytes(int32_t nx, int32_t ny, int32_t nz) {
+  if (nx < 1 || ny < 1 || nz < 1) return 0;
+  return (size_t)vox_list(nx, ny, nz, 3) * sizeof(int32_t);
+}
+
+int lbm3d_voxelize_blocks(void *stream, const float *tris, int32_t n_tris, double x0, double y0, double z0, double dx,
+                          int32_t nx, int32_t ny, int32_t nz, int8_t *solid, void *workspace,
+                          size_t workspace_bytes) {
+  if (nx < 1 || ny < 1 || nz < 1 || n_tris < 0 || !(dx > 0)) return iofail(LBM3D_EINVAL, "bad grid or mesh size");
+  if ((n_tris > 0 && !tris) || !solid || !workspace) return iofail(LBM3D_EINVAL, "NULL mesh, output or workspace");
+  if ((int64_t)nx * ny * nz > INT32_MAX) return iofail(LBM3D_ESIZE, "grid has more than 2^31-1 nodes");
+  if (workspace_bytes < lbm3d_voxelize_workspace_bytes(nx, ny, nz)) return iofail(LBM3D_EINVAL, "workspace too small");
+  // the error bound of the FP32 sums grows by about 4e-6 a triangle: past 400,000
+  // it would leave most nodes open
+  if (n_tris > 400000) return lbm3d_voxelize(stream, tris, n_tris, x0, y0, z0, dx, nx, ny, nz, solid);
+  VoxGrid gr{x0, y0, z0, dx, nx, ny, nz, n_tris, 0.f};
+  const double far = std::fmax(std::fmax(std::fmax(std::fabs(x0), std::fabs(x0 + dx * nx)),
+                                         std::fmax(std::fabs(y0), std::fabs(y0 + dx * ny))),
+                               std::fmax(std::fabs(z0), std::fabs(z0 + dx * nz)));
+  gr.eta = (float)(1e-15 * far / dx);
+  int32_t *const ws = (int32_t *)workspace;
+  int32_t *const list4 = ws + vox_list(nx, ny, nz, 0), *const list2 = ws + vox_list(nx, ny, nz, 1),
+                 *const list1 = ws + vox_list(nx, ny, nz, 2);
+  hipStream_t s = (hipStream_t)stream;
+  const int32_t all = blocks_of(nx, 8) * blocks_of(ny, 8) * blocks_of(nz, 8);
+  constexpr unsigned kMost = 2048;  // workgroups of 4 waves: 8 per CU
+  k_clear_counts<<<1, 64, 0, s>>>(ws);
+  k_winding_blocks<4><<<std::min<unsigned>(kMost, (unsigned)(all + 3) / 4), 256, 0, s>>>(tris, gr, nullptr, nullptr,
+                                                                                       all, list4, ws, solid);
+  k_winding_blocks<2><<<kMost, 256, 0, s>>>(tris, gr, list4, ws, 0, list2, ws + 1, solid);
+  k_winding_blocks<1><<<kMost, 256, 0, s>>>(tris, gr, list2, ws + 1, 0, list1, ws + 2, solid);
+  k_winding_nodes<<<kMost, 256, 0, s>>>(tris, gr, list1, ws + 2, solid);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return iofail(LBM3D_EHIP, "lbm3d_voxelize_blocks: ", hipGetErrorString(e));
+  return LBM3D_OK;
 }
 
 int lbm3d_voxelize(void *stream, const float *tris, int32_t n_tris, double x0, double y0, double z0, double dx,

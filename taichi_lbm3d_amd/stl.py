@@ -66,9 +66,11 @@ def voxelize(tris, lower, upper, dx: float, device=None) -> np.ndarray:
     with torch.cuda.device(dev):
         stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
         lib = _lib.lib()
-        rc = lib.cdll.lbm3d_voxelize(stream, ctypes.c_void_p(t.data_ptr()), len(tris), float(lower[0]),
-                                     float(lower[1]), float(lower[2]), float(dx), nx, ny, nz,
-                                     ctypes.c_void_p(out.data_ptr()))
+        ws_bytes = lib.size("lbm3d_voxelize_workspace_bytes", nx, ny, nz)
+        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
+        rc = lib.cdll.lbm3d_voxelize_blocks(stream, ctypes.c_void_p(t.data_ptr()), len(tris), float(lower[0]),
+                                            float(lower[1]), float(lower[2]), float(dx), nx, ny, nz,
+                                            ctypes.c_void_p(out.data_ptr()), ctypes.c_void_p(ws.data_ptr()), ws_bytes)
         if rc != 0:
             raise _lib.LbmError(f"lbm3d_voxelize failed ({rc}): {lib.cdll.lbm3d_io_last_error().decode()}")
     return out.cpu().numpy()
