@@ -207,6 +207,25 @@ class Lib:
         return int(getattr(self.cdll, name)(*args))
 
 
+def raw_stream(index: int) -> int:
+    """torch's current HIP stream of device `index`, as the pointer the C ABI takes."""
+    import torch
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
+def call_on(device, name: str, *args):
+    """lib().call(name, current stream of `device`, *args) with `device` current.
+    Pointers are plain integers (no ctypes object to build for each).  A device context
+    costs as much as the call itself, so it is entered only when another device is current."""
+    import torch
+    current = torch.cuda.current_device()
+    index = current if device.index is None else device.index
+    if index == current:
+        return lib().call(name, raw_stream(index), *args)
+    with torch.cuda.device(index):
+        return lib().call(name, raw_stream(index), *args)
+
+
 _LIB: Lib | None = None
 
 

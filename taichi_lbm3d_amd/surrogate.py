@@ -18,7 +18,6 @@ network serves any small force.
 """
 from __future__ import annotations
 
-import ctypes
 import math
 
 import numpy as np
@@ -39,12 +38,11 @@ def _torch():
 
 
 def _vp(t):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _stream(dev):
-    torch = _torch()
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    return _lib.raw_stream(_torch().cuda.current_device() if dev.index is None else dev.index)
 
 
 # ---- the convolution as an autograd function ----------------------------------------------
