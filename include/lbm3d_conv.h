@@ -121,6 +121,24 @@ int lbm3d_relu_pool_grad(void *stream, const uint16_t *g, const uint16_t *y, con
                          const uint16_t *g_pool, uint16_t *dz, float *db, int32_t n, int32_t d, int32_t h, int32_t w,
                          int32_t c, uint16_t *share, void *workspace, size_t workspace_bytes);
 
+/* The network's head: a 1x1x1 convolution from cin to 16 channels, of which the
+ * first 4 are used, rounded to BF16 and returned in FP32.  w: the convolution's
+ * weights (BF16 w[16][kpad]; rows 0-3 are read), bias its 16 biases (or NULL).
+ * out[voxels][4]; or, for the box `core` at `origin` of one volume x of
+ * `extents` (3 each, D x H x W), a warm start at once: v[3] = channels 0-2 *
+ * scale_v * fluid, rho = 1 + channel 3 * scale_rho * fluid (1 with rho_one), with
+ * fluid = solid[voxel of the box] ? 0 : 1. */
+int lbm3d_conv_head_fwd(void *stream, const uint16_t *x, const uint16_t *w, const float *bias, float *out,
+                        int64_t voxels, int32_t cin);
+int lbm3d_conv_head_fields(void *stream, const uint16_t *x, const uint16_t *w, const float *bias, const int8_t *solid,
+                           float *rho, float *v, const int32_t extents[3], const int32_t origin[3],
+                           const int32_t core[3], int32_t cin, float scale_v, float scale_rho, int rho_one);
+/* From the FP32 gradient g[voxels][4] of lbm3d_conv_head_fwd's output: dz[voxels][16],
+ * the BF16 gradient of the 16 channels, and db[16], the sums of dz as
+ * lbm3d_relu_bias_grad forms them (its workspace, for 16 channels). */
+int lbm3d_conv_head_grad(void *stream, const float *g, uint16_t *dz, float *db, int64_t voxels, void *workspace,
+                         size_t workspace_bytes);
+
 /* The surrogate's distance input: dist[v] = Euclidean distance from voxel v to
  * the nearest solid voxel (solid[v] != 0) of its volume, with every volume
  * periodic, exact up to `margin` voxels and capped there (also when a volume

@@ -148,6 +148,10 @@ SIGNATURES = {
     "lbm3d_conv3d_dgrad_up": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_conv3d_wgrad_up": (_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _sz]),
     "lbm3d_relu_pool_grad": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _sz]),
+    "lbm3d_conv_head_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i32]),
+    "lbm3d_conv_head_fields": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, ctypes.c_float,
+                                      ctypes.c_float, _int]),
+    "lbm3d_conv_head_grad": (_int, [_vp, _vp, _vp, _vp, _i64, _vp, _sz]),
     "lbm3d_conv3d_wflip": (_int, [_vp, _vp, _vp, _i32, _i32, _i32]),
     "lbm3d_conv3d_dgrad": (_int, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_conv3d_wgrad_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32, _i32, _i32]),

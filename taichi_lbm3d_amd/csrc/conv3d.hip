@@ -34,9 +34,6 @@
 #ifndef LBM3D_CONV_WGRAD_XCD_CHUNK
 #define LBM3D_CONV_WGRAD_XCD_CHUNK 64  // weight gradient: runs of consecutive jobs per XCD (16 or 256: the same to 1 %)
 #endif
-#ifndef LBM3D_CONV_MW
-#define LBM3D_CONV_MW 2  // 16-voxel fragments per wave in the forward kernel
-#endif
 
 namespace {
 
@@ -107,33 +104,8 @@ __device__ __forceinline__ void decode(const Vol &v, uint32_t m, int &b, int &z,
   b = (int)bb;
 }
 
-// tap -> offset (dz, dy, dx); ks = 1 has the single tap 0 at offset 0
-__device__ __forceinline__ void tap_offset(int tap, int ks, int &dz, int &dy, int &dx) {
-  if (ks == 3) {
-    dz = tap / 9 - 1;
-    dy = (tap / 3) % 3 - 1;
-    dx = tap % 3 - 1;
-  } else {
-    dz = dy = dx = 0;
-  }
-}
-
 // a coordinate one step outside [0, n) wrapped back in
 __device__ __forceinline__ int wrap1(int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); }
-
-// neighbour voxel of (b,z,y,x) at tap offset (|offset| <= 1), wrapped when the
-// volume is periodic, else -1 outside the volume (zero padding)
-__device__ __forceinline__ int64_t shifted(const Vol &v, int b, int z, int y, int x, int dz, int dy, int dx) {
-  int z2 = z + dz, y2 = y + dy, x2 = x + dx;
-  if (v.periodic) {
-    z2 = wrap1(z2, v.d);
-    y2 = wrap1(y2, v.h);
-    x2 = wrap1(x2, v.w);
-  } else if (z2 < 0 || z2 >= v.d || y2 < 0 || y2 >= v.h || x2 < 0 || x2 >= v.w) {
-    return -1;
-  }
-  return (((int64_t)b * v.d + z2) * v.h + y2) * v.w + x2;
-}
 
 __device__ __forceinline__ u32x4 ld16(const uint16_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
 
@@ -147,98 +119,6 @@ __device__ __forceinline__ uint16_t to_bf16(float f) {
 // MFMA 16x16x32 lane layout: A (16 x 32): lane l holds row l%16, k = 8*(l/16) .. +7;
 // B (32 x 16): column l%16, the same k; C (16 x 16): column l%16, rows 4*(l/16) .. +3.
 // ---------------------------------------------------------------------------
-// 1x1x1 convolutions: each wave computes MW fragments of 16 voxels x NT
-// fragments of 16 output channels; the next K chunk's operands are loaded while
-// the current chunk's MFMAs run.
-template <int NT, int MW>
-__global__ void __launch_bounds__(256)
-    k_conv_fwd(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const float *__restrict__ bias,
-               uint16_t *__restrict__ y, const Vol vol, int cin, int cout, int ks, int kpad, int relu) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane >> 4, r16 = lane & 15;
-  const uint32_t mb = blockIdx.x * (64u * MW) + (uint32_t)wave * (16u * MW);
-  const int co0 = blockIdx.y * 16 * NT;
-  bool mvalid[MW];
-  int vb[MW], vz[MW], vy[MW], vx[MW];
-#pragma unroll
-  for (int f = 0; f < MW; ++f) {
-    const uint32_t m = mb + 16u * f + (uint32_t)r16;
-    mvalid[f] = m < vol.vox;
-    vb[f] = vz[f] = vy[f] = vx[f] = 0;
-    if (mvalid[f]) decode(vol, m, vb[f], vz[f], vy[f], vx[f]);
-  }
-  const int K = ks * ks * ks * cin;
-  const uint16_t *wrow[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) wrow[t] = w + (size_t)(co0 + 16 * t + r16) * kpad + 8 * g;
-  f32x4 acc[MW][NT];
-#pragma unroll
-  for (int f = 0; f < MW; ++f)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // this lane's 8 K values of a chunk: k = kc + 8g .. +7, i.e. channels ci .. ci+7 of tap
-  int kk = 8 * g;
-  int tap = kk / cin, ci = kk - tap * cin;
-  auto load_a = [&](int f, int tp, int c, int k) -> u32x4 {
-    u32x4 a = u32x4{0u, 0u, 0u, 0u};
-    if (mvalid[f] && k < K) {
-      int dz, dy, dx;
-      tap_offset(tp, ks, dz, dy, dx);
-      const int64_t src = shifted(vol, vb[f], vz[f], vy[f], vx[f], dz, dy, dx);
-      if (src >= 0) a = ld16(x + src * cin + c);
-    }
-    return a;
-  };
-  u32x4 a[MW], b[NT];
-#pragma unroll
-  for (int f = 0; f < MW; ++f) a[f] = load_a(f, tap, ci, kk);
-#pragma unroll
-  for (int t = 0; t < NT; ++t) b[t] = ld16(wrow[t]);
-  for (int kc = 0; kc < kpad; kc += 32) {
-    int kk2 = kk + 32, ci2 = ci + 32, tap2 = tap;
-    while (ci2 >= cin) {
-      ci2 -= cin;
-      ++tap2;
-    }
-    u32x4 an[MW], bn[NT];
-    const bool more = kc + 32 < kpad;
-#pragma unroll
-    for (int f = 0; f < MW; ++f) an[f] = more ? load_a(f, tap2, ci2, kk2) : u32x4{0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int t = 0; t < NT; ++t) bn[t] = more ? ld16(wrow[t] + kc + 32) : u32x4{0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const bf16x8 bv = __builtin_bit_cast(bf16x8, b[t]);
-#pragma unroll
-      for (int f = 0; f < MW; ++f)
-        acc[f][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[f]), bv, acc[f][t], 0, 0, 0);
-    }
-#pragma unroll
-    for (int f = 0; f < MW; ++f) a[f] = an[f];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) b[t] = bn[t];
-    kk = kk2;
-    ci = ci2;
-    tap = tap2;
-  }
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int co = co0 + 16 * t + r16;
-    const float bb = bias ? bias[co] : 0.f;
-#pragma unroll
-    for (int f = 0; f < MW; ++f)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t mo = mb + 16u * f + (uint32_t)(4 * g + e);
-        if (mo >= vol.vox) continue;
-        float val = acc[f][t][e] + bb;
-        if (relu) val = val > 0.f ? val : 0.f;
-        y[(size_t)mo * cout + co] = to_bf16(val);
-      }
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Forward 3x3x3 convolutions.  Both kernels below compute, per wave, fragments
 // of 16 voxels (one x row) x 16 output channels.  K runs over chunks of 16
@@ -326,6 +206,135 @@ __device__ __forceinline__ f32x4 finish4(f32x4 v, const f32x4 b4, int relu) {
 __device__ __forceinline__ uint2 pack4(const f32x4 v) {
   return make_uint2((uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16),
                     (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16));
+}
+
+// 1x1x1 convolutions: a matrix product of the voxels' channels, bound by its
+// bytes.  A wave computes 4 fragments of 16 voxels x NT of 16 output channels with
+// the weights as the A operand, so a lane has 4 channels of a voxel (8-byte
+// stores, whole lines per fragment) and all of a chunk's loads are in flight
+// together.  16 -> 16 channels at 2 x 128^3 (268 MB): 75 us with 2-byte stores and
+// an address from coordinates per load -> 48 us (5.6 TB/s).
+template <int NT>
+__global__ void __launch_bounds__(256)
+    k_conv1(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const float *__restrict__ bias,
+            uint16_t *__restrict__ y, uint32_t vox, int cin, int cout, int kpad, int relu) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, r16 = lane & 15;
+  const uint32_t m0 = blockIdx.x * 256u + (threadIdx.x & ~63u) + (uint32_t)r16;
+  const int co0 = blockIdx.y * 16 * NT;
+  f32x4 acc[4][NT];
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int kc = 0; kc < cin; kc += 32) {
+    const int k = kc + 8 * g;
+    u32x4 b[4], a[NT];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      const uint32_t m = m0 + 16u * f;
+      b[f] = m < vox && k < cin ? ld16(x + (size_t)m * cin + k) : u32x4{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) a[t] = ld16(w + (size_t)(co0 + 16 * t + r16) * kpad + k);  // kpad: 32-multiple
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+        acc[f][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[t]),
+                                                            __builtin_bit_cast(bf16x8, b[f]), acc[f][t], 0, 0, 0);
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int co = co0 + 16 * t + 4 * g;
+    f32x4 b4 = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (bias) b4 = f32x4{bias[co], bias[co + 1], bias[co + 2], bias[co + 3]};
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      const uint32_t m = m0 + 16u * f;
+      if (m < vox) *reinterpret_cast<uint2 *>(y + (size_t)m * cout + co) = pack4(finish4(acc[f][t], b4, relu));
+    }
+  }
+}
+
+// The network's head: a 1x1x1 convolution whose first 4 of 16 output channels are
+// used, rounded to BF16 and returned in FP32.  A wave takes 64 voxels: fragment f's
+// weights stand in rows 4f .. 4f+3 of its A operand, so that lane group f ends
+// with the 4 channels of fragment f's voxels, lane l with those of voxel l.
+//
+// kHeadOut writes the channels.  kHeadFields turns them into a warm start at once:
+// v = channels 0-2 times scale_v, rho = 1 + channel 3 times scale_rho (or 1 with
+// rho_one), both as a product with 1 on fluid voxels and 0 on solid ones, for the
+// voxels of a box (core) of the volume, each step rounded on its own.  Per voxel
+// of 16 channels 32 + 16 and 33 + 16 bytes, against 64 for the padded output and
+// 56 more for the passes that read it: at 2 x 192^3 a convolution of 276 us and
+// 400 us of passes -> 128 us (5.4 TB/s).
+enum HeadMode { kHeadOut = 0, kHeadFields = 1 };
+
+struct HeadFields {
+  Vol core;             // one volume: the box
+  int32_t h, w;         // extents of the volume it lies in
+  int64_t first;        // the box's first voxel there
+  const int8_t *solid;  // of the box
+  float scale_v, scale_rho;
+  int rho_one;
+  float *rho, *v;
+};
+
+template <int MODE>
+__global__ void __launch_bounds__(256)
+    k_head(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const float *__restrict__ bias,
+           float *__restrict__ out, uint32_t vox, int cin, int kpad, const HeadFields hf) {
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x & 63, g = lane >> 4, r16 = lane & 15;
+  const uint32_t mw = blockIdx.x * 256u + (threadIdx.x & ~63u);
+  if (mw >= vox) return;
+  const uint16_t *src[4];
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    uint32_t m = mw + 16u * f + (uint32_t)r16;
+    if (m >= vox) m = vox - 1;
+    int64_t at = m;
+    if constexpr (MODE == kHeadFields) {
+      int b, z, yy, xx;
+      decode(hf.core, m, b, z, yy, xx);
+      at = hf.first + ((int64_t)z * hf.h + yy) * hf.w + xx;
+    }
+    src[f] = x + at * cin;
+  }
+  f32x4 acc[4];
+#pragma unroll
+  for (int f = 0; f < 4; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int kc = 0; kc < cin; kc += 32) {
+    const int k = kc + 8 * g;
+    const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
+    u32x4 b[4];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) b[f] = k < cin ? ld16(src[f] + k) : zero;
+    const u32x4 row = ld16(w + (size_t)(r16 & 3) * kpad + k);  // the row of one of the 4 channels
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      const u32x4 a = (r16 >> 2) == f ? row : zero;
+      acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b[f]),
+                                                       acc[f], 0, 0, 0);
+    }
+  }
+  const uint32_t m = mw + (uint32_t)lane;
+  if (m >= vox) return;
+  float p[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float lo = (g & 1) ? acc[1][e] : acc[0][e], hi = (g & 1) ? acc[3][e] : acc[2][e];
+    p[e] = __uint_as_float((uint32_t)to_bf16(((g & 2) ? hi : lo) + (bias ? bias[e] : 0.f)) << 16);
+  }
+  if constexpr (MODE == kHeadOut) {
+    *reinterpret_cast<float4 *>(out + (size_t)m * 4) = make_float4(p[0], p[1], p[2], p[3]);
+  } else {
+    const float fluid = hf.solid[m] ? 0.f : 1.f;
+    float *const vm = hf.v + (size_t)m * 3;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) vm[e] = p[e] * hf.scale_v * fluid;
+    hf.rho[m] = hf.rho_one ? 1.f : 1.f + p[3] * hf.scale_rho * fluid;
+  }
 }
 
 __device__ __forceinline__ f32x4 max4(const f32x4 a, const f32x4 b) {
@@ -1260,7 +1269,7 @@ __device__ __forceinline__ float bf16_to_f32(uint32_t h) { return __uint_as_floa
 // thread's 8-element chunks (chunk q covers elements 8q .. 8q+7) always hold
 // the same 8 channels when the blocks' chunk ranges start on multiples of C/8.
 //
-// POOL: g has a second part, the gradient of y's 2 x 2 x 2 maximum: at the
+// kGradPool: g has a second part, the gradient of y's 2 x 2 x 2 maximum: at the
 // voxels that attain it, `share` (its gradient over their number, k_pool_share);
 // the sum is rounded to BF16 first, as two accumulated gradients are.
 struct PoolGrad {
@@ -1269,7 +1278,12 @@ struct PoolGrad {
   Div pieces;  // by C / 8
 };
 
-template <bool POOL>
+//
+// kGradHead: g is the FP32 gradient of k_head's 4 channels; dz is it in BF16 as the
+// first 4 of 16 channels (the others zero), and there is no ReLU.
+enum GradMode { kGradPlain = 0, kGradPool = 1, kGradHead = 2 };
+
+template <int MODE>
 __global__ void __launch_bounds__(256)
     k_relu_bias_grad(const uint16_t *g, const uint16_t *__restrict__ y, uint16_t *dz,  // dz may be g
                      float *__restrict__ part, int64_t chunks, int C, int64_t per_block, const PoolGrad pg) {
@@ -1281,10 +1295,17 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
   for (int64_t q = q0 + t; q < q1; q += 256) {
-    u32x4 a = ld16(g + q * 8);
-    if (y) {
+    u32x4 a = u32x4{0u, 0u, 0u, 0u};
+    if constexpr (MODE != kGradHead) {
+      a = ld16(g + q * 8);
+    } else if (!(q & 1)) {
+      const float4 p = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(g) + q * 2);
+      const uint2 r = pack4(f32x4{p.x, p.y, p.z, p.w});
+      a = u32x4{r.x, r.y, 0u, 0u};
+    }
+    if (MODE != kGradHead && y) {
       const u32x4 m = ld16(y + q * 8);
-      if constexpr (POOL) {
+      if constexpr (MODE == kGradPool) {
         int b, z, yy, x;
         const uint32_t v = chunks < ((int64_t)1 << 31) ? qdiv((uint32_t)q, pg.pieces) : (uint32_t)(q / pg.pieces.d);
         decode(pg.vol, v, b, z, yy, x);
@@ -1528,14 +1549,13 @@ int lbm3d_conv3d_fwd(void *stream, const uint16_t *x, const uint16_t *w, const f
   const int kpad = lbm3d_conv_kpad(cin, ks);
   hipStream_t s = (hipStream_t)stream;
   if (ks == 3) return launch_conv3<kPlain>(s, ConvCall{x, w, 0, bias, y, vol, cin, cout, kpad, relu, ConvExtra{}});
-  constexpr int MW = LBM3D_CONV_MW;
-  const unsigned gx = (vol.vox + 64u * MW - 1u) / (64u * MW);
+  const unsigned gx = (vol.vox + 255u) / 256u;
   if (cout % 64 == 0)
-    k_conv_fwd<4, MW><<<dim3(gx, cout / 64), 256, 0, s>>>(x, w, bias, y, vol, cin, cout, ks, kpad, relu);
+    k_conv1<4><<<dim3(gx, cout / 64), 256, 0, s>>>(x, w, bias, y, vol.vox, cin, cout, kpad, relu);
   else if (cout % 32 == 0)
-    k_conv_fwd<2, MW><<<dim3(gx, cout / 32), 256, 0, s>>>(x, w, bias, y, vol, cin, cout, ks, kpad, relu);
+    k_conv1<2><<<dim3(gx, cout / 32), 256, 0, s>>>(x, w, bias, y, vol.vox, cin, cout, kpad, relu);
   else
-    k_conv_fwd<1, MW><<<dim3(gx, cout / 16), 256, 0, s>>>(x, w, bias, y, vol, cin, cout, ks, kpad, relu);
+    k_conv1<1><<<dim3(gx, cout / 16), 256, 0, s>>>(x, w, bias, y, vol.vox, cin, cout, kpad, relu);
   return ccheck("lbm3d_conv3d_fwd");
 }
 
@@ -1712,9 +1732,52 @@ int lbm3d_relu_bias_grad(void *stream, const uint16_t *g, const uint16_t *y, uin
   int64_t chunks, per;
   const int blocks = relu_bias_plan(voxels, c, chunks, per);
   hipStream_t s = (hipStream_t)stream;
-  k_relu_bias_grad<false><<<(unsigned)blocks, 256, 0, s>>>(g, y, dz, (float *)workspace, chunks, c, per, PoolGrad{});
+  k_relu_bias_grad<kGradPlain><<<(unsigned)blocks, 256, 0, s>>>(g, y, dz, (float *)workspace, chunks, c, per, PoolGrad{});
   if (int rc = ccheck("lbm3d_relu_bias_grad")) return rc;
   return fold_sets(s, (float *)workspace, db, c, blocks, c, c);
+}
+
+int lbm3d_conv_head_fwd(void *stream, const uint16_t *x, const uint16_t *w, const float *bias, float *out,
+                        int64_t voxels, int32_t cin) {
+  if (voxels < 1 || cin < 16 || cin > 256 || cin % 16) return cfail(LBM3D_EINVAL, "bad head shape");
+  if (voxels >= ((int64_t)1 << 31)) return cfail(LBM3D_ESIZE, "more than 2^31-1 voxels");
+  if (!x || !w || !out) return cfail(LBM3D_EINVAL, "NULL tensor");
+  k_head<kHeadOut><<<(unsigned)((voxels + 255) / 256), 256, 0, (hipStream_t)stream>>>(
+      x, w, bias, out, (uint32_t)voxels, cin, lbm3d_conv_kpad(cin, 1), HeadFields{});
+  return ccheck("lbm3d_conv_head_fwd");
+}
+
+int lbm3d_conv_head_fields(void *stream, const uint16_t *x, const uint16_t *w, const float *bias, const int8_t *solid,
+                           float *rho, float *v, const int32_t extents[3], const int32_t origin[3],
+                           const int32_t core[3], int32_t cin, float scale_v, float scale_rho, int rho_one) {
+  if (!x || !w || !solid || !rho || !v || !extents || !origin || !core) return cfail(LBM3D_EINVAL, "NULL tensor");
+  if (cin < 16 || cin > 256 || cin % 16) return cfail(LBM3D_EINVAL, "bad head shape");
+  for (int a = 0; a < 3; ++a)
+    if (core[a] < 1 || origin[a] < 0 || extents[a] < 1 || origin[a] > extents[a] - core[a])
+      return cfail(LBM3D_EINVAL, "the box does not lie in the volume");
+  const int64_t vox = (int64_t)core[0] * core[1] * core[2];
+  if (vox >= ((int64_t)1 << 31)) return cfail(LBM3D_ESIZE, "more than 2^31-1 voxels");
+  const int64_t first = ((int64_t)origin[0] * extents[1] + origin[1]) * extents[2] + origin[2];
+  const HeadFields hf{make_vol(1, core[0], core[1], core[2]), extents[1], extents[2], first, solid, scale_v, scale_rho,
+                      rho_one, rho, v};
+  k_head<kHeadFields><<<(unsigned)((vox + 255) / 256), 256, 0, (hipStream_t)stream>>>(
+      x, w, bias, nullptr, (uint32_t)vox, cin, lbm3d_conv_kpad(cin, 1), hf);
+  return ccheck("lbm3d_conv_head_fields");
+}
+
+int lbm3d_conv_head_grad(void *stream, const float *g, uint16_t *dz, float *db, int64_t voxels, void *workspace,
+                         size_t workspace_bytes) {
+  if (voxels < 1) return cfail(LBM3D_EINVAL, "no voxels");
+  if (!g || !dz || !db || !workspace) return cfail(LBM3D_EINVAL, "NULL tensor or workspace");
+  if (workspace_bytes < lbm3d_relu_bias_grad_workspace_bytes(voxels, 16))
+    return cfail(LBM3D_EINVAL, "head gradient workspace too small");
+  int64_t chunks, per;
+  const int blocks = relu_bias_plan(voxels, 16, chunks, per);
+  hipStream_t s = (hipStream_t)stream;
+  k_relu_bias_grad<kGradHead><<<(unsigned)blocks, 256, 0, s>>>(reinterpret_cast<const uint16_t *>(g), nullptr, dz,
+                                                               (float *)workspace, chunks, 16, per, PoolGrad{});
+  if (int rc = ccheck("lbm3d_conv_head_grad")) return rc;
+  return fold_sets(s, (float *)workspace, db, 16, blocks, 16, 16);
 }
 
 int lbm3d_relu_pool_grad(void *stream, const uint16_t *g, const uint16_t *y, const uint16_t *pooled,
@@ -1736,7 +1799,7 @@ int lbm3d_relu_pool_grad(void *stream, const uint16_t *g, const uint16_t *y, con
   if (int rc = ccheck("lbm3d_relu_pool_grad")) return rc;
   int64_t chunks, per;
   const int blocks = relu_bias_plan(voxels, c, chunks, per);
-  k_relu_bias_grad<true><<<(unsigned)blocks, 256, 0, s>>>(g, y, dz, (float *)workspace, chunks, c, per,
+  k_relu_bias_grad<kGradPool><<<(unsigned)blocks, 256, 0, s>>>(g, y, dz, (float *)workspace, chunks, c, per,
                                                          PoolGrad{pooled, share, make_vol(n, d, h, w), pieces});
   if (int rc = ccheck("lbm3d_relu_pool_grad")) return rc;
   return fold_sets(s, (float *)workspace, db, c, blocks, c, c);

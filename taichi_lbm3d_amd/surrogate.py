@@ -150,6 +150,41 @@ def relu_pool_grad(g, g_pool, y, pooled):
     return dz, db
 
 
+def head_fwd(x, w_bf16, bias):
+    """The head's 4 channels, rounded to BF16, in FP32 (lbm3d_conv_head_fwd)."""
+    torch = _torch()
+    cin = x.shape[-1]
+    y = torch.empty(x.shape[:-1] + (4,), dtype=torch.float32, device=x.device)
+    _lib.lib().call("lbm3d_conv_head_fwd", _stream(x.device), _vp(x), _vp(w_bf16), _vp(bias), _vp(y), x.numel() // cin,
+                    cin)
+    return y
+
+
+def head_fields(x, w_bf16, bias, solid, origin, scale_v, scale_rho, rho_one):
+    """(rho, v) of the box at `origin`, of `solid`'s shape, from one volume x
+    (X, Y, Z, C) of the last layer's output (lbm3d_conv_head_fields)."""
+    torch = _torch()
+    rho = torch.empty(solid.shape, dtype=torch.float32, device=x.device)
+    v = torch.empty(tuple(solid.shape) + (3,), dtype=torch.float32, device=x.device)
+    box = [(_lib.ctypes.c_int32 * 3)(*t) for t in (x.shape[:3], origin, solid.shape)]
+    _lib.lib().call("lbm3d_conv_head_fields", _stream(x.device), _vp(x), _vp(w_bf16), _vp(bias), _vp(solid), _vp(rho),
+                    _vp(v), *box, x.shape[-1], scale_v, scale_rho, int(rho_one))
+    return rho, v
+
+
+def head_grad(g):
+    """(dz, db) of the head's 16 channels from the gradient of its 4 outputs (lbm3d_conv_head_grad)."""
+    torch = _torch()
+    vox = g.numel() // 4
+    lib = _lib.lib()
+    ws_bytes = lib.size("lbm3d_relu_bias_grad_workspace_bytes", vox, HEAD_PAD)
+    ws = torch.empty(max(ws_bytes, 4), dtype=torch.uint8, device=g.device)
+    dz = torch.empty(g.shape[:-1] + (HEAD_PAD,), dtype=torch.bfloat16, device=g.device)
+    db = torch.empty(HEAD_PAD, dtype=torch.float32, device=g.device)
+    lib.call("lbm3d_conv_head_grad", _stream(g.device), _vp(g), _vp(dz), _vp(db), vox, _vp(ws), ws_bytes)
+    return dz, db
+
+
 def _bf16(t):
     return t.contiguous().to(_torch().bfloat16)
 
@@ -256,7 +291,25 @@ def _make_conv_functions():
                          c_low, c_skip, cout)
             return d_low, d_skip, dw, db, None
 
-    return Conv3dMFMA, ConvPool, ConvUp
+    class Head(torch.autograd.Function):
+        """The first 4 channels of a 1x1x1 layer without ReLU, rounded to BF16, as FP32."""
+
+        @staticmethod
+        def forward(ctx, x, w, b):
+            x = x.contiguous()
+            wb = w.to(torch.bfloat16).contiguous()
+            ctx.save_for_backward(x, wb)
+            return head_fwd(x, wb, b)
+
+        @staticmethod
+        def backward(ctx, gy):
+            x, wb = ctx.saved_tensors
+            g, db = head_grad(gy.contiguous())
+            dw = conv_wgrad(x, g, 1)
+            dx = conv_dgrad(g, wb, x.shape[-1], 1) if ctx.needs_input_grad[0] else None
+            return dx, dw, db
+
+    return Conv3dMFMA, ConvPool, ConvUp, Head
 
 
 _CONV = None
@@ -281,6 +334,11 @@ def conv3d_pool(x, w, b, periodic: bool = False):
 def conv3d_up(low, skip, w, b, periodic: bool = False):
     """A 3x3x3 layer with ReLU on the concatenation of `low`, upsampled by 2 (nearest), and `skip`."""
     return _conv_functions()[2].apply(low, skip, w, b, periodic)
+
+
+def conv_head(x, w, b):
+    """The network's head: (..., C) bf16 -> (..., 4) float32."""
+    return _conv_functions()[3].apply(x, w, b)
 
 
 # ---- the network ------------------------------------------------------------------------------
@@ -338,7 +396,10 @@ class UNet3D:
         X, Y, Z must be multiples of 8.  periodic: every volume is one period of a
         periodic geometry, and the convolutions wrap around its faces instead of
         zero padding (forward only)."""
-        p = periodic
+        return conv_head(self._features(x, periodic), self.params["head.w"], self.params["head.b"])
+
+    def _features(self, x, p):
+        """The last layer's output before the head, (N,X,Y,Z,C) bf16; p: periodic."""
 
         def layer(name):
             return self.params[name + ".w"], self.params[name + ".b"]
@@ -349,9 +410,7 @@ class UNet3D:
         e4 = self._c("e4b", self._c("e4a", low, periodic=p), periodic=p)
         d3 = self._c("d3b", conv3d_up(e4, e3, *layer("d3a"), p), periodic=p)
         d2 = self._c("d2b", conv3d_up(d3, e2, *layer("d2a"), p), periodic=p)
-        d1 = self._c("d1b", conv3d_up(d2, e1, *layer("d1a"), p), periodic=p)
-        out = self._c("head", d1, relu=False, periodic=p)
-        return out[..., :4].float()
+        return self._c("d1b", conv3d_up(d2, e1, *layer("d1a"), p), periodic=p)
 
     __call__ = forward
 
@@ -457,10 +516,15 @@ def fields_from_prediction(pred, fluid, fx, nu_eff, density=False):
     rho_pred = 1.0 + p[..., 3] * (fx * RHO_SCALE) * fl
     if not density:
         return torch.ones_like(rho_pred), v, rho_pred
+    return _mean_one(rho_pred, fluid), v, rho_pred
+
+
+def _mean_one(rho_pred, fluid):
+    """The density shifted to mean 1 over the fluid, 1 elsewhere."""
+    fl = fluid.to(rho_pred.dtype)
     n = fl.sum().clamp_min(1.0)
     dev = (rho_pred - 1.0) * fl
-    rho = 1.0 + (dev - dev.sum() / n) * fl
-    return rho, v, rho_pred
+    return 1.0 + (dev - dev.sum() / n) * fl
 
 
 def to_network_input(inp):
@@ -521,15 +585,24 @@ def predict(net, solids, fx, nu_eff, batch: int = 2, wrap=None, density=False):
     if wrap and any(n % 8 for n in shape):
         raise ValueError(f"periodic inference needs extents that are multiples of 8, got {shape}")
     pads = inference_pads(shape, wrap)
+    # a network with a forward of its own, or a force per component, goes through its output
+    fused = type(net) is UNet3D and isinstance(fx, float) and isinstance(nu_eff, float)
     with torch.no_grad():
         for b0 in range(0, len(solids), batch):
             sol = torch.stack([_device_solid(s, net.device) for s in solids[b0:b0 + batch]])
             if wrap:
-                pred = net(network_inputs(sol), periodic=True)
+                inp = network_inputs(sol)
             else:
-                inp = torch.stack([periodic_pad(t, pads) for t in make_inputs(sol)])
-                pred = net(to_network_input(inp), periodic=False)
+                inp = to_network_input(torch.stack([periodic_pad(t, pads) for t in make_inputs(sol)]))
             (X, Y, Z), (px, py, pz) = shape, (p[0] for p in pads)
+            if fused:  # the head gives the fields of fields_from_prediction itself
+                feat, (w, b) = net._features(inp, wrap), (net.params["head.w"], net.params["head.b"])
+                w = w.to(torch.bfloat16).contiguous()
+                for i in range(sol.shape[0]):
+                    rho, v = head_fields(feat[i], w, b, sol[i], (px, py, pz), fx / nu_eff, fx * RHO_SCALE, not density)
+                    out.append((_mean_one(rho, ~sol[i]) if density else rho, v))
+                continue
+            pred = net(inp, periodic=wrap)
             for i in range(sol.shape[0]):
                 core = pred[i, px:px + X, py:py + Y, pz:pz + Z]
                 out.append(fields_from_prediction(core, ~sol[i], fx, nu_eff, density)[:2])
