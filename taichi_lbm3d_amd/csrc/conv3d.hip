@@ -1011,50 +1011,55 @@ __device__ __forceinline__ float tree16(float v[16]) {
 // dst[e] = sum of the terms part[q step + e] of nsets <= 4096 sets (step: the size
 // of a set, or of 16 after a first level), in an order fixed by nsets alone:
 // groups of 16 consecutive sets by tree16 while more than 16 terms remain, the
-// last (at most 16) terms one after another.  A block takes 64 elements; its wave
-// w sums the groups w, w + 16, ..., so that 16 waves hold one group of groups at
-// a time: one launch for what took a pass per level.  Elements whose column (e %
-// kpad) is past `used` are padding: 0.
+// last (at most 16) terms one after another.  A block takes E elements and sums
+// G = 1024 / E groups at a time, a group a thread, in one launch.  Elements whose
+// column (e % kpad) is past `used` are padding: 0.
+template <int E>
 __global__ void __launch_bounds__(1024)
-    k_fold_sets(const float *__restrict__ part, float *__restrict__ dst, int64_t size, int64_t step, int nsets,
+    k_fold_sets(const float *__restrict__ part, float *__restrict__ dst, uint32_t size, uint32_t step, int nsets,
                 int kpad, int used) {
-  __shared__ float red[16][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t e = (int64_t)blockIdx.x * 64 + lane;
-  const bool live = e < size && (int)(e % kpad) < used;
-  const float *const p = part + e;
+  constexpr int G = 1024 / E, T = G / 16;  // groups, and groups of groups, of a round
+  __shared__ float red[G][E], top[T][E];
+  const int col = threadIdx.x % E, row = threadIdx.x / E;
+  const uint32_t e = blockIdx.x * E + col;
+  const bool live = e < size && e % (uint32_t)kpad < (uint32_t)used, last = row == 0 && e < size;
+  const float *const p = part + (e < size ? e : size - 1);  // terms past the end: clamped loads, then 0
+  float s = 0.f;
   if (nsets <= 16) {  // one term a set
-    red[wave][lane] = live && wave < nsets ? p[wave * step] : 0.f;
+    red[row][col] = live && row < nsets ? p[row * (int64_t)step] : 0.f;
     __syncthreads();
-    if (wave == 0 && e < size) {
-      float s = 0.f;
-      for (int q = 0; q < nsets; ++q) s += red[q][lane];
+    if (last) {
+      for (int q = 0; q < nsets; ++q) s += red[q][col];
       dst[e] = s;
     }
     return;
   }
   const int groups = (nsets + 15) / 16;
-  float s = 0.f;
-  for (int q0 = 0; q0 < groups; q0 += 16) {  // uniform in the block
-    const int first = (q0 + wave) * 16;
+  for (int q0 = 0; q0 < groups; q0 += G) {  // uniform in the block
+    const int first = (q0 + row) * 16;
     float v[16];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) v[j] = live && first + j < nsets ? p[(first + j) * step] : 0.f;
-    if (q0) __syncthreads();  // the previous group of groups has been read
-    red[wave][lane] = tree16(v);
-    __syncthreads();
-    if (wave == 0) {
-      if (groups <= 16) {  // at most 16 terms: one after another
-        for (int q = 0; q < groups; ++q) s += red[q][lane];
-      } else {
-        float u[16];
+    for (int j = 0; j < 16; ++j) v[j] = p[(int64_t)(first + j < nsets ? first + j : nsets - 1) * step];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) u[j] = red[j][lane];
-        s += tree16(u);
-      }
+    for (int j = 0; j < 16; ++j) v[j] = live && first + j < nsets ? v[j] : 0.f;
+    red[row][col] = tree16(v);  // the round before has read its rows: see the barrier below
+    __syncthreads();
+    if (groups <= 16) {  // at most 16 terms: one after another
+      if (last)
+        for (int q = 0; q < groups; ++q) s += red[q][col];
+      break;
     }
+    if (row < T) {
+      float u[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) u[j] = red[16 * row + j][col];
+      top[row][col] = tree16(u);
+    }
+    __syncthreads();
+    if (last)
+      for (int t = 0; t < T && q0 + 16 * t < groups; ++t) s += top[t][col];
   }
-  if (wave == 0 && e < size) dst[e] = s;
+  if (last) dst[e] = s;
 }
 
 // The same for at most 256 sets of many elements: one thread an element.
@@ -1096,6 +1101,22 @@ __global__ void __launch_bounds__(256)
   part[16 * q * size + e] = tree16(v);
 }
 
+// Elements a block of k_fold_sets takes: whole lines of 64 elements where there are
+// blocks for every CU, 32 for the two smallest weight gradients (13,824 of 2048
+// sets: 38 us with the gradient, 47 with 16, 64 with 8; 7,168: 102-111 with any of
+// 16, 32, 64), and 4 for a layer's bias gradient (16 of 2048 sets: 88 us with the
+// pass over 2 x 128^3 voxels before it, 97 with 64, where one block walks them in
+// eight rounds).
+void fold_block(hipStream_t s, const float *part, float *dst, uint32_t size, uint32_t step, int nsets, int kpad,
+                int used) {
+  if (size >= 16384)
+    k_fold_sets<64><<<(size + 63) / 64, 1024, 0, s>>>(part, dst, size, step, nsets, kpad, used);
+  else if (size >= 1024)
+    k_fold_sets<32><<<(size + 31) / 32, 1024, 0, s>>>(part, dst, size, step, nsets, kpad, used);
+  else
+    k_fold_sets<4><<<(size + 3) / 4, 1024, 0, s>>>(part, dst, size, step, nsets, kpad, used);
+}
+
 int fold_sets(hipStream_t s, float *part, float *dst, int64_t size, int nsets, int kpad, int used) {
   // a thread an element where there are enough elements to fill the GPU: 32 sets of
   // 442 k (the gradient of 128 -> 128 channels, 2 x 16^3, takes 30 us in all; 60
@@ -1104,12 +1125,12 @@ int fold_sets(hipStream_t s, float *part, float *dst, int64_t size, int nsets, i
   if (nsets <= 256 && size >= 100000) {
     k_fold_few<<<(unsigned)((size + 255) / 256), 256, 0, s>>>(part, dst, size, nsets, kpad, used);
   } else if (nsets <= 4096) {
-    k_fold_sets<<<(unsigned)((size + 63) / 64), 1024, 0, s>>>(part, dst, size, size, nsets, kpad, used);
+    fold_block(s, part, dst, (uint32_t)size, (uint32_t)size, nsets, kpad, used);
   } else {
     const int64_t n = (int64_t)((nsets + 15) / 16) * size;
     k_fold_level<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(part, size, nsets);
     if (int rc = ccheck("fold of partial sums")) return rc;
-    k_fold_sets<<<(unsigned)((size + 63) / 64), 1024, 0, s>>>(part, dst, size, 16 * size, (nsets + 15) / 16, kpad, used);
+    fold_block(s, part, dst, (uint32_t)size, (uint32_t)(16 * size), (nsets + 15) / 16, kpad, used);
   }
   return ccheck("fold of partial sums");
 }
