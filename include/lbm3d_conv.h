@@ -74,10 +74,10 @@ int lbm3d_conv3d_fwd_up(void *stream, const uint16_t *low, const uint16_t *skip,
                         const float *bias, uint16_t *y, int32_t n, int32_t d, int32_t h, int32_t wd, int32_t c_low,
                         int32_t c_skip, int32_t cout, int32_t flags);
 /* Its gradients: the data gradient of the two parts from the flipped packed
- * weights (d_low_full, c_low channels at full extents, is scratch; d_low its
- * BF16 sums over 2 x 2 x 2 blocks), and the weight gradient (workspace of
+ * weights (d_low: BF16 sums over 2 x 2 x 2 blocks of the BF16 gradient at full
+ * extents, which is not written), and the weight gradient (workspace of
  * lbm3d_conv3d_wgrad_workspace_bytes for c_low + c_skip channels). */
-int lbm3d_conv3d_dgrad_up(void *stream, const uint16_t *dy, const uint16_t *wt, uint16_t *d_low_full, uint16_t *d_low,
+int lbm3d_conv3d_dgrad_up(void *stream, const uint16_t *dy, const uint16_t *wt, uint16_t *d_low,
                           uint16_t *d_skip, int32_t n, int32_t d, int32_t h, int32_t wd, int32_t c_low,
                           int32_t c_skip, int32_t cout);
 int lbm3d_conv3d_wgrad_up(void *stream, const uint16_t *low, const uint16_t *skip, const uint16_t *dy, float *dw,

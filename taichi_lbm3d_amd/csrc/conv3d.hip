@@ -175,6 +175,11 @@ struct Weights {
 //          extents, upsampled (each voxel read for its 2 x 2 x 2 block), the
 //          others those of `x`: a concatenation that is never built
 //   kPool  the 2 x 2 x 2 maximum of the output is written too (half extents)
+//   kDown  of the output channels below c_split only the sum over 2 x 2 x 2 blocks
+//          is written (half extents): the gradient of kUp's low part.  A
+//          separate pass over the full extents took 84 us of a 2 x 128^3 training
+//          step, and the 16 -> 48 convolution there takes 150 us where it took
+//          193 with the store.
 // c_split > 0: output channels below it go to `y` (c_split per voxel), the
 // others to `y_hi`: the two parts of a concatenation's gradient.
 // The copies and reductions these replace took 2.9 of 6.2 ms of a 2 x 192^3
@@ -182,12 +187,12 @@ struct Weights {
 // epilogue adds nothing to the 250 us of a 16 -> 16 layer, and reading the
 // upsampled part at half extents takes 96 -> 32 channels at 2 x 96^3 from 394 to
 // 328 us.
-enum ConvMode { kPlain = 0, kUp = 1, kPool = 2 };
+enum ConvMode { kPlain = 0, kUp = 1, kPool = 2, kDown = 3 };
 
 struct ConvExtra {
   const uint16_t *low;  // kUp
   int c_low;
-  uint16_t *pool;       // kPool
+  uint16_t *pool;       // kPool, kDown (c_split channels)
   int c_split;
   uint16_t *y_hi;
 };
@@ -342,12 +347,25 @@ __device__ __forceinline__ f32x4 max4(const f32x4 a, const f32x4 b) {
 }
 
 // the maximum over an x pair of voxels (lanes r16 and r16 ^ 1)
-__device__ __forceinline__ f32x4 max_xpair(f32x4 v) {
+__device__ __forceinline__ f32x4 other_x(f32x4 v) {  // the value of the other voxel of the x pair
   f32x4 o;
 #pragma unroll
   for (int e = 0; e < 4; ++e)  // quad_perm [1, 0, 3, 2]
     o[e] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v[e]), 0xB1, 0xF, 0xF, true));
-  return max4(v, o);
+  return o;
+}
+__device__ __forceinline__ f32x4 max_xpair(f32x4 v) { return max4(v, other_x(v)); }
+
+// The sum over a 2 x 2 x 2 block of voxels rounded to BF16, at its even x, in the
+// order of torch's sum: z pairs, then the four (y, x) in turn.  a0, a1: this x, the
+// even row, both planes; b0, b1: the odd row.
+__device__ __forceinline__ f32x4 unpack4(uint2 v) {
+  return f32x4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xFFFF0000u), __uint_as_float(v.y << 16),
+               __uint_as_float(v.y & 0xFFFF0000u)};
+}
+__device__ __forceinline__ f32x4 sum_block(uint2 a0, uint2 a1, uint2 b0, uint2 b1) {
+  const f32x4 a = unpack4(a0) + unpack4(a1), b = unpack4(b0) + unpack4(b1);
+  return ((a + other_x(a)) + b) + other_x(b);
 }
 
 // where a tile's output goes: base pointer and channels per voxel
@@ -560,12 +578,13 @@ __global__ void __launch_bounds__(256, 2)
       for (int e = 0; e < 4; ++e) b4[e] = bias[16 * tile + 4 * g + e];
     }
     const int oy0 = y0 + yr0, ox = x0 + r16;
+    const bool down = MODE == kDown && 16 * tile < ex.c_split;  // uniform in the wave
     uint16_t *yv = op.y + ((size_t)bb * vstride + ((int64_t)z0 * vol.h + oy0) * vol.w + ox) * op.c + op.co;
 #pragma unroll
     for (int f = 0; f < MF; ++f) {
       const int fz = f / YR, fy = f % YR;
       acc[f] = finish4(acc[f], b4, relu);
-      if (z0 + fz < vol.d && oy0 + fy < vol.h && ox < vol.w)
+      if (!down && z0 + fz < vol.d && oy0 + fy < vol.h && ox < vol.w)
         *reinterpret_cast<uint2 *>(yv + ((int64_t)fz * vol.h + fy) * vol.w * op.c) = pack4(acc[f]);
     }
     if constexpr (MODE == kPool) {  // even extents: a block is inside whole or not at all
@@ -577,6 +596,17 @@ __global__ void __launch_bounds__(256, 2)
               ex.pool + ((size_t)bb * (vstride >> 3) +
                          ((int64_t)(z0 >> 1) * (vol.h >> 1) + ((oy0 + fy) >> 1)) * (vol.w >> 1) + (ox >> 1)) * cout +
               op.co) = pack4(m);
+      }
+    }
+    if (MODE == kDown && down) {
+#pragma unroll
+      for (int fy = 0; fy < YR; fy += 2) {
+        const f32x4 m = sum_block(pack4(acc[fy]), pack4(acc[YR + fy]), pack4(acc[fy + 1]), pack4(acc[YR + fy + 1]));
+        if (!(r16 & 1) && z0 < vol.d && oy0 + fy < vol.h && ox < vol.w)
+          *reinterpret_cast<uint2 *>(
+              ex.pool + ((size_t)bb * (vstride >> 3) +
+                         ((int64_t)(z0 >> 1) * (vol.h >> 1) + ((oy0 + fy) >> 1)) * (vol.w >> 1) + (ox >> 1)) *
+                            ex.c_split + op.co) = pack4(m);
       }
     }
   }
@@ -698,6 +728,8 @@ __global__ void __launch_bounds__(256, 2)
   const int oy0 = y0 + row0, ox = x0 + r16;
   uint16_t *yv = op.y + ((size_t)bb * vstride + ((int64_t)z_begin * vol.h + oy0) * vol.w + ox) * op.c + op.co;
   f32x4 even[MODE == kPool ? MF / 2 : 1];  // the even plane's row-pair maxima (runs start on even planes)
+  uint2 evenb[MODE == kDown ? MF : 1];     // the even plane's rounded values
+  const bool down = MODE == kDown && 16 * tile < ex.c_split;  // uniform in the wave
   int slot = 0;                            // of plane z - 1
   for (int z = z_begin; z < z_end; ++z) {
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this thread's loads of plane z + 1
@@ -743,7 +775,7 @@ __global__ void __launch_bounds__(256, 2)
 #pragma unroll
     for (int f = 0; f < MF; ++f) {
       acc[f] = finish4(acc[f], b4, relu);
-      if (oy0 + f < vol.h && ox < vol.w)
+      if (!down && oy0 + f < vol.h && ox < vol.w)
         *reinterpret_cast<uint2 *>(yv + (int64_t)f * vol.w * op.c) = pack4(acc[f]);
     }
     if constexpr (MODE == kPool) {
@@ -759,6 +791,23 @@ __global__ void __launch_bounds__(256, 2)
                 ex.pool + ((size_t)bb * (vstride >> 3) +
                            ((int64_t)(z >> 1) * (vol.h >> 1) + ((oy0 + f) >> 1)) * (vol.w >> 1) + (ox >> 1)) * cout +
                 op.co) = pack4(p);
+        }
+      }
+    }
+    if (MODE == kDown && down) {
+#pragma unroll
+      for (int f = 0; f < MF; f += 2) {
+        const uint2 lo = pack4(acc[f]), hi = pack4(acc[f + 1]);
+        if (!(z & 1)) {
+          evenb[f] = lo;
+          evenb[f + 1] = hi;
+        } else {
+          const f32x4 p = sum_block(evenb[f], lo, evenb[f + 1], hi);
+          if (!(r16 & 1) && oy0 + f < vol.h && ox < vol.w)
+            *reinterpret_cast<uint2 *>(
+                ex.pool + ((size_t)bb * (vstride >> 3) +
+                           ((int64_t)(z >> 1) * (vol.h >> 1) + ((oy0 + f) >> 1)) * (vol.w >> 1) + (ox >> 1)) *
+                              ex.c_split + op.co) = pack4(p);
         }
       }
     }
@@ -1440,12 +1489,12 @@ void launch_conv3z(hipStream_t s, const ConvCall &a) {
   const int64_t cols = nbx * nby * vol.n;
   // planes per workgroup: the cut that takes the fewest rounds of resident
   // workgroups times planes (3 extra planes of border and start-up per run);
-  // an even number with pooling
+  // an even number with pooling and block sums
   const int64_t slots = 256 * (WCH == 1 ? 3 : 2);
   int64_t best = vol.d, best_cost = INT64_MAX;
   for (int64_t segs = 1; segs <= vol.d; ++segs) {
     int64_t zl = (vol.d + segs - 1) / segs;
-    if (MODE == kPool) zl = (zl + 1) & ~int64_t(1);
+    if (MODE == kPool || MODE == kDown) zl = (zl + 1) & ~int64_t(1);
     const int64_t runs = (vol.d + zl - 1) / zl;
     const int64_t cost = ((cols * runs * gy + slots - 1) / slots) * (zl + 3);
     if (cost < best_cost) best = zl, best_cost = cost;
@@ -1486,8 +1535,9 @@ int launch_conv3(hipStream_t s, const ConvCall &a) {
       if (tiles % 2 == 0) launch_conv3z<2, 2, 8, MODE>(s, a);
       else launch_conv3z<2, 1, 8, MODE>(s, a);
     } else {
-      if (MODE != kPool && tiles % 2 == 0)  // pooling's row maxima would spill
-        launch_conv3z<3, 2, 8, MODE == kPool ? kPlain : MODE>(s, a);
+      constexpr bool kTwo = MODE == kPlain || MODE == kUp;  // the even plane's values would spill
+      if (kTwo && tiles % 2 == 0)
+        launch_conv3z<3, 2, 8, kTwo ? MODE : kPlain>(s, a);
       else
         launch_conv3z<3, 1, 8, MODE>(s, a);
     }
@@ -1502,38 +1552,6 @@ int launch_conv3(hipStream_t s, const ConvCall &a) {
   else if (ct == 2) launch_conv3_bricks<2, MODE>(s, a, bk);
   else launch_conv3_bricks<1, MODE>(s, a, bk);
   return ccheck("lbm3d_conv3d_fwd");
-}
-
-// Gradient of nearest upsampling by 2: out[v] = sum of the 2 x 2 x 2 block of g
-// (BF16, FP32 sum), one 16-byte piece (8 channels) per thread.
-__global__ void __launch_bounds__(256)
-    k_up_grad(const uint16_t *__restrict__ g, uint16_t *__restrict__ out, const Vol low, Div pieces, int64_t total) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= total) return;
-  const int64_t v = total < ((int64_t)1 << 31) ? (int64_t)qdiv((uint32_t)i, pieces) : i / pieces.d;
-  const int pc = (int)(i - v * pieces.d), c = 8 * (int)pieces.d;
-  int b, z, yy, x;
-  decode(low, (uint32_t)v, b, z, yy, x);
-  const int64_t h2 = 2 * low.h, w2 = 2 * low.w;
-  const uint16_t *src = g + ((((int64_t)b * low.d + z) * 2 * h2 + 2 * yy) * w2 + 2 * x) * c + 8 * pc;
-  // the order of torch's sum over the block: z pairs, then the four in turn
-  float sum[8];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const uint16_t *q = src + ((int64_t)(k >> 1) * w2 + (k & 1)) * c;
-    const u32x4 a0 = ld16(q), a1 = ld16(q + h2 * w2 * c);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t u0 = e & 1 ? a0[e >> 1] & 0xFFFF0000u : a0[e >> 1] << 16;
-      const uint32_t u1 = e & 1 ? a1[e >> 1] & 0xFFFF0000u : a1[e >> 1] << 16;
-      const float pair = __uint_as_float(u0) + __uint_as_float(u1);
-      sum[e] = k == 0 ? pair : sum[e] + pair;
-    }
-  }
-  u32x4 o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) o[e] = (uint32_t)to_bf16(sum[2 * e]) | ((uint32_t)to_bf16(sum[2 * e + 1]) << 16);
-  *reinterpret_cast<u32x4 *>(out + v * c + 8 * pc) = o;
 }
 
 int relu_bias_plan(int64_t voxels, int C, int64_t &chunks, int64_t &per_block) {
@@ -1639,24 +1657,18 @@ int lbm3d_conv3d_fwd_up(void *stream, const uint16_t *low, const uint16_t *skip,
   return launch_conv3<kUp>((hipStream_t)stream, a);
 }
 
-int lbm3d_conv3d_dgrad_up(void *stream, const uint16_t *dy, const uint16_t *wt, uint16_t *d_low_full, uint16_t *d_low,
-                          uint16_t *d_skip, int32_t n, int32_t d, int32_t h, int32_t wd, int32_t c_low,
-                          int32_t c_skip, int32_t cout) {
+int lbm3d_conv3d_dgrad_up(void *stream, const uint16_t *dy, const uint16_t *wt, uint16_t *d_low, uint16_t *d_skip,
+                          int32_t n, int32_t d, int32_t h, int32_t wd, int32_t c_low, int32_t c_skip, int32_t cout) {
   if (c_low < 16 || c_low % 16 || c_skip < 16 || c_skip % 16 || c_low > 240 || c_skip > 240)
     return cfail(LBM3D_EINVAL, "channel counts must be multiples of 16, together at most 256");
   ConvCall a;
-  if (int rc = packed_call(dy, wt, nullptr, d_low_full, n, d, h, wd, cout, c_low + c_skip, 0, a)) return rc;
-  if (!d_low || !d_skip) return cfail(LBM3D_EINVAL, "NULL tensor");
+  if (int rc = packed_call(dy, wt, nullptr, d_skip, n, d, h, wd, cout, c_low + c_skip, 0, a)) return rc;
+  if (!d_low) return cfail(LBM3D_EINVAL, "NULL tensor");
   if ((d | h | wd) & 1) return cfail(LBM3D_EINVAL, "upsampling needs even extents");
   a.ex.c_split = c_low;
   a.ex.y_hi = d_skip;
-  hipStream_t s = (hipStream_t)stream;
-  if (int rc = launch_conv3<kPlain>(s, a)) return rc;
-  const int64_t total = (int64_t)n * (d / 2) * (h / 2) * (wd / 2) * (c_low / 8);
-  if ((total + 255) / 256 > (int64_t)(UINT32_MAX / 256u)) return cfail(LBM3D_ESIZE, "volume too large for one launch");
-  k_up_grad<<<(unsigned)((total + 255) / 256), 256, 0, s>>>(d_low_full, d_low, make_vol(n, d / 2, h / 2, wd / 2),
-                                                           make_div((uint32_t)c_low / 8), total);
-  return ccheck("lbm3d_conv3d_dgrad_up");
+  a.ex.pool = d_low;
+  return launch_conv3<kDown>((hipStream_t)stream, a);
 }
 
 int lbm3d_conv3d_wflip(void *stream, const uint16_t *w, uint16_t *wt, int32_t cin, int32_t cout, int32_t ks) {

@@ -285,10 +285,9 @@ def _make_conv_functions():
                      cout, _vp(ws), ws_bytes)
             d_low = d_skip = None
             if wt is not None:
-                full = torch.empty((n, d, h, wd, c_low), dtype=torch.bfloat16, device=g.device)
                 d_low, d_skip = torch.empty_like(low), torch.empty_like(skip)
-                lib.call("lbm3d_conv3d_dgrad_up", s, _vp(g), _vp(wt), _vp(full), _vp(d_low), _vp(d_skip), n, d, h, wd,
-                         c_low, c_skip, cout)
+                lib.call("lbm3d_conv3d_dgrad_up", s, _vp(g), _vp(wt), _vp(d_low), _vp(d_skip), n, d, h, wd, c_low,
+                         c_skip, cout)
             return d_low, d_skip, dw, db, None
 
     class Head(torch.autograd.Function):

@@ -74,7 +74,7 @@ def test_pooled_convolution_gradients(gpu, form):
 # n, d, h, w (full extents), c_low, c_skip, cout
 UP = [(1, 2, 2, 2, 16, 16, 16), (2, 6, 18, 34, 32, 16, 16), (1, 4, 10, 18, 16, 16, 32), (1, 8, 8, 16, 16, 32, 32),
       (1, 4, 10, 18, 64, 32, 32), (2, 4, 6, 10, 128, 64, 64), (1, 34, 40, 36, 128, 64, 64), (1, 2, 4, 6, 64, 16, 16),
-      (1, 70, 16, 16, 32, 16, 16)]
+      (1, 70, 16, 16, 32, 16, 16), (1, 6, 10, 18, 16, 32, 48), (1, 12, 20, 34, 32, 32, 96)]
 
 
 @pytest.mark.parametrize("form", UP)
