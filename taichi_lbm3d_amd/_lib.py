@@ -84,6 +84,12 @@ class BatchSizes(ctypes.Structure):
                 ("desc_bytes", ctypes.c_int64)]
 
 
+class ConvPack(ctypes.Structure):
+    """lbm3d_conv_pack (include/lbm3d_conv.h)."""
+    _fields_ = [("w", ctypes.c_void_p), ("wp", ctypes.c_void_p), ("wt", ctypes.c_void_p),
+                ("cin", ctypes.c_int32), ("cout", ctypes.c_int32)]
+
+
 class Launch(ctypes.Structure):
     """Mirror of struct lbm3d_launch."""
     _fields_ = [("block", ctypes.c_int32), ("grid_per_cu", ctypes.c_int32), ("reverse", ctypes.c_int32),
@@ -142,6 +148,7 @@ SIGNATURES = {
     "lbm3d_conv3d_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_conv3d_packed_elements": (_i64, [_i32, _i32]),
     "lbm3d_conv3d_wpack": (_int, [_vp, _vp, _vp, _vp, _i32, _i32]),
+    "lbm3d_conv3d_wpack_many": (_int, [_vp, _i32, ctypes.POINTER(ConvPack)]),
     "lbm3d_conv3d_fwd_packed": (_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_conv3d_fwd_pool": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_conv3d_fwd_up": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),

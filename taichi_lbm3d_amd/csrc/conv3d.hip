@@ -835,28 +835,49 @@ __global__ void k_wflip(const uint16_t *__restrict__ w, uint16_t *__restrict__ w
 // FP32 weights w[cout][kpad] (3x3x3) to BF16 MFMA fragments: wp in k_conv3's
 // packed order, [chunk][step][tile][lane][8], and, when wt is not null, the
 // flipped weights of the data gradient (k_wflip's) in the same order.  One
-// thread per lane of a fragment; the 28th tap slot is zero.
-__global__ void __launch_bounds__(256) k_wpack(const float *__restrict__ w, uint16_t *__restrict__ wp,
-                                               uint16_t *__restrict__ wt, int cin, int cout, int kpad) {
+// thread per lane of a fragment; the 28th tap slot is zero.  A launch takes up to
+// kPackItems layers: one is 4 to 6 us of latency, so the network's 14 layers take
+// 9 us together and 66 one by one.
+constexpr int kPackItems = 16;
+
+struct PackItem {
+  const float *w;
+  uint16_t *wp, *wt;
+  int32_t cin, cout, kpad;
+  uint32_t first;  // block
+};
+struct PackList {
+  int n;
+  PackItem item[kPackItems];
+};
+
+__global__ void __launch_bounds__(256) k_wpack(const PackList list) {
+  int k = 0;
+  while (k + 1 < list.n && blockIdx.x >= list.item[k + 1].first) ++k;  // uniform
+  const PackItem &it = list.item[k];
+  const float *const w = it.w;
+  const int cin = it.cin, cout = it.cout, kpad = it.kpad;
   const int frags = kSteps * (cin / 16) * (cout / 16);  // the same for both
-  int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  int i = (int)((blockIdx.x - it.first) * 256 + threadIdx.x);
   const bool flip = i >= frags * 64;
   if (flip) i -= frags * 64;
-  if (i >= frags * 64 || (flip && !wt)) return;
+  if (i >= frags * 64 || (flip && !it.wt)) return;
   const int ci_n = flip ? cout : cin, co_n = flip ? cin : cout;  // of the convolution the fragments are for
   const int lane = i & 63, fr = i >> 6;
   const int tile = fr % (co_n / 16), cs = fr / (co_n / 16);
   const int s = cs % kSteps, c = cs / kSteps;
   const int co = 16 * tile + (lane & 15), g = lane >> 4;
   const int tap = 2 * s + (g >> 1), ci = 16 * c + 8 * (g & 1);
-  uint16_t *dst = (flip ? wt : wp) + (size_t)i * 8;
+  u32x4 v = u32x4{0u, 0u, 0u, 0u};
+  if (tap < 27) {
+    float f[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    uint16_t v = 0;
-    if (tap < 27)
-      v = to_bf16(flip ? w[(size_t)(ci + e) * kpad + (26 - tap) * cin + co] : w[(size_t)co * kpad + tap * cin + ci + e]);
-    dst[e] = v;
+    for (int e = 0; e < 8; ++e)
+      f[e] = flip ? w[(size_t)(ci + e) * kpad + (26 - tap) * cin + co] : w[(size_t)co * kpad + tap * cin + ci + e];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (uint32_t)to_bf16(f[2 * e]) | ((uint32_t)to_bf16(f[2 * e + 1]) << 16);
   }
+  *reinterpret_cast<u32x4 *>((flip ? it.wt : it.wp) + (size_t)i * 8) = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -1603,14 +1624,29 @@ int64_t lbm3d_conv3d_packed_elements(int32_t cin, int32_t cout) {
   return (int64_t)kSteps * 2 * cin * cout;
 }
 
+int lbm3d_conv3d_wpack_many(void *stream, int32_t count, const lbm3d_conv_pack *layers) {
+  if (count < 0 || (count > 0 && !layers)) return cfail(LBM3D_EINVAL, "no layers");
+  for (int32_t k = 0; k < count; ++k) {
+    if (int rc = check_conv(1, 1, 1, 1, layers[k].cin, layers[k].cout, 3)) return rc;
+    if (!layers[k].w || !layers[k].wp) return cfail(LBM3D_EINVAL, "NULL tensor");
+  }
+  for (int32_t k0 = 0; k0 < count; k0 += kPackItems) {
+    PackList list{};
+    uint32_t blocks = 0;
+    for (int32_t k = k0; k < count && k < k0 + kPackItems; ++k) {
+      const lbm3d_conv_pack &l = layers[k];
+      list.item[list.n++] = PackItem{l.w, l.wp, l.wt, l.cin, l.cout, lbm3d_conv_kpad(l.cin, 3), blocks};
+      blocks += (uint32_t)(kSteps * (l.cin / 16) * (l.cout / 16) * 64 * (l.wt ? 2 : 1) + 255) / 256;
+    }
+    k_wpack<<<blocks, 256, 0, (hipStream_t)stream>>>(list);
+    if (int rc = ccheck("lbm3d_conv3d_wpack")) return rc;
+  }
+  return LBM3D_OK;
+}
+
 int lbm3d_conv3d_wpack(void *stream, const float *w, uint16_t *wp, uint16_t *wt, int32_t cin, int32_t cout) {
-  int rc = check_conv(1, 1, 1, 1, cin, cout, 3);
-  if (rc) return rc;
-  if (!w || !wp) return cfail(LBM3D_EINVAL, "NULL tensor");
-  const int lanes = kSteps * (cin / 16) * (cout / 16) * 64 * (wt ? 2 : 1);
-  k_wpack<<<(unsigned)((lanes + 255) / 256), 256, 0, (hipStream_t)stream>>>(w, wp, wt, cin, cout,
-                                                                          lbm3d_conv_kpad(cin, 3));
-  return ccheck("lbm3d_conv3d_wpack");
+  const lbm3d_conv_pack one{w, wp, wt, cin, cout};
+  return lbm3d_conv3d_wpack_many(stream, 1, &one);
 }
 
 static int packed_call(const uint16_t *x, const uint16_t *wp, const float *bias, uint16_t *y, int32_t n, int32_t d,

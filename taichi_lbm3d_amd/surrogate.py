@@ -79,15 +79,28 @@ def conv_dgrad(dy, w_bf16, cin, ks):
 def pack_weights(w, flip: bool):
     """FP32 3x3x3 weights (cout, kpad) as BF16 MFMA fragments: (forward, data
     gradient or None)."""
+    return pack_layers([(w, flip)])[0]
+
+
+def pack_layers(layers):
+    """pack_weights of several (w, flip), in one launch."""
     torch = _torch()
     lib = _lib.lib()
-    cout, cin = w.shape[0], w.shape[1] // 27
-    cin -= cin % 16
-    n = lib.size("lbm3d_conv3d_packed_elements", cin, cout)
-    wp = torch.empty(n, dtype=torch.bfloat16, device=w.device)
-    wt = torch.empty(n, dtype=torch.bfloat16, device=w.device) if flip else None
-    lib.call("lbm3d_conv3d_wpack", _stream(w.device), _vp(w), _vp(wp), _vp(wt) if flip else None, cin, cout)
-    return wp, wt
+    if not layers:
+        return []
+    items, spans, total = (_lib.ConvPack * len(layers))(), [], 0
+    for it, (w, flip) in zip(items, layers):
+        it.cout, it.cin = w.shape[0], w.shape[1] // 27 // 16 * 16
+        n = lib.size("lbm3d_conv3d_packed_elements", it.cin, it.cout)
+        spans.append((total, n, flip))
+        total += n * (2 if flip else 1)
+    dev = layers[0][0].device
+    buf = torch.empty(total, dtype=torch.bfloat16, device=dev)
+    for it, (w, _), (at, n, flip) in zip(items, layers, spans):
+        it.w, it.wp = w.data_ptr(), buf.data_ptr() + 2 * at
+        it.wt = it.wp + 2 * n if flip else None
+    lib.call("lbm3d_conv3d_wpack_many", _stream(dev), len(layers), items)
+    return [(buf[at:at + n], buf[at + n:at + 2 * n] if flip else None) for at, n, flip in spans]
 
 
 def conv_fwd_packed(x, wp, bias, cout, relu, periodic=False):
@@ -192,7 +205,9 @@ def _bf16(t):
 def _make_conv_functions():
     torch = _torch()
 
-    def packed(w, flip):
+    def packed(w, flip, given):  # given: the layer's fragments from pack_layers, or None
+        if given is not None:
+            return given[0], given[1] if flip else None
         w = w if w.dtype == torch.float32 else w.to(torch.bfloat16).float()
         return pack_weights(w.contiguous(), flip)
 
@@ -200,10 +215,10 @@ def _make_conv_functions():
         """y = act(conv3d(x, w) + b) with the MFMA kernels in both directions."""
 
         @staticmethod
-        def forward(ctx, x, w, b, ks, relu, need_dx, periodic):
+        def forward(ctx, x, w, b, ks, relu, need_dx, periodic, given):
             x = x.contiguous()
             if ks == 3:
-                wp, wb = packed(w, need_dx and ctx.needs_input_grad[0])
+                wp, wb = packed(w, need_dx and ctx.needs_input_grad[0], given)
                 y = conv_fwd_packed(x, wp, b, w.shape[0], relu, periodic)
             else:
                 wb = w.to(torch.bfloat16).contiguous()
@@ -223,17 +238,17 @@ def _make_conv_functions():
             if ctx.need_dx and ctx.needs_input_grad[0]:
                 dx = (conv_fwd_packed(g, wb, None, x.shape[-1], False) if ctx.ks == 3
                       else conv_dgrad(g, wb, x.shape[-1], ctx.ks))
-            return dx, dw, db, None, None, None, None
+            return dx, dw, db, None, None, None, None, None
 
     class ConvPool(torch.autograd.Function):
         """(y, 2x2x2 max of y) for y = relu(conv3d(x, w) + b), 3x3x3."""
 
         @staticmethod
-        def forward(ctx, x, w, b, periodic):
+        def forward(ctx, x, w, b, periodic, given):
             x = x.contiguous()
             n, d, h, wd, cin = x.shape
             cout = w.shape[0]
-            wp, wt = packed(w, ctx.needs_input_grad[0])
+            wp, wt = packed(w, ctx.needs_input_grad[0], given)
             y = torch.empty((n, d, h, wd, cout), dtype=torch.bfloat16, device=x.device)
             pooled = torch.empty((n, d // 2, h // 2, wd // 2, cout), dtype=torch.bfloat16, device=x.device)
             _lib.lib().call("lbm3d_conv3d_fwd_pool", _stream(x.device), _vp(x), _vp(wp), _vp(b), _vp(y), _vp(pooled),
@@ -250,17 +265,17 @@ def _make_conv_functions():
             g, db = relu_pool_grad(_bf16(gy), _bf16(g_pool), y, pooled)
             dw = conv_wgrad(x, g, 3)
             dx = conv_fwd_packed(g, wt, None, x.shape[-1], False) if ctx.needs_input_grad[0] else None
-            return dx, dw, db, None
+            return dx, dw, db, None, None
 
     class ConvUp(torch.autograd.Function):
         """relu(conv3d(cat(upsampled low, skip), w) + b), 3x3x3, without the concatenation."""
 
         @staticmethod
-        def forward(ctx, low, skip, w, b, periodic):
+        def forward(ctx, low, skip, w, b, periodic, given):
             low, skip = low.contiguous(), skip.contiguous()
             n, d, h, wd, c_skip = skip.shape
             cout = w.shape[0]
-            wp, wt = packed(w, ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
+            wp, wt = packed(w, ctx.needs_input_grad[0] or ctx.needs_input_grad[1], given)
             y = torch.empty((n, d, h, wd, cout), dtype=torch.bfloat16, device=skip.device)
             _lib.lib().call("lbm3d_conv3d_fwd_up", _stream(skip.device), _vp(low), _vp(skip), _vp(wp), _vp(b), _vp(y),
                             n, d, h, wd, low.shape[-1], c_skip, cout, CONV_RELU | (CONV_PERIODIC if periodic else 0))
@@ -288,7 +303,7 @@ def _make_conv_functions():
                 d_low, d_skip = torch.empty_like(low), torch.empty_like(skip)
                 lib.call("lbm3d_conv3d_dgrad_up", s, _vp(g), _vp(wt), _vp(d_low), _vp(d_skip), n, d, h, wd, c_low,
                          c_skip, cout)
-            return d_low, d_skip, dw, db, None
+            return d_low, d_skip, dw, db, None, None
 
     class Head(torch.autograd.Function):
         """The first 4 channels of a 1x1x1 layer without ReLU, rounded to BF16, as FP32."""
@@ -321,18 +336,19 @@ def _conv_functions():
     return _CONV
 
 
-def conv3d(x, w, b, ks: int = 3, relu: bool = True, need_dx: bool = True, periodic: bool = False):
-    return _conv_functions()[0].apply(x, w, b, ks, relu, need_dx, periodic)
+def conv3d(x, w, b, ks: int = 3, relu: bool = True, need_dx: bool = True, periodic: bool = False, packed=None):
+    """act(conv(x, w) + b); packed: the weights' pack_layers entry, if there is one."""
+    return _conv_functions()[0].apply(x, w, b, ks, relu, need_dx, periodic, packed)
 
 
-def conv3d_pool(x, w, b, periodic: bool = False):
+def conv3d_pool(x, w, b, periodic: bool = False, packed=None):
     """(y, its 2x2x2 maximum) of a 3x3x3 layer with ReLU; even extents."""
-    return _conv_functions()[1].apply(x, w, b, periodic)
+    return _conv_functions()[1].apply(x, w, b, periodic, packed)
 
 
-def conv3d_up(low, skip, w, b, periodic: bool = False):
+def conv3d_up(low, skip, w, b, periodic: bool = False, packed=None):
     """A 3x3x3 layer with ReLU on the concatenation of `low`, upsampled by 2 (nearest), and `skip`."""
-    return _conv_functions()[2].apply(low, skip, w, b, periodic)
+    return _conv_functions()[2].apply(low, skip, w, b, periodic, packed)
 
 
 def conv_head(x, w, b):
@@ -386,9 +402,14 @@ class UNet3D:
     def parameters(self):
         return list(self.params.values())
 
-    def _c(self, name, x, relu=True, need_dx=True, periodic=False):
-        cin, cout, ks = self.specs[name]
-        return conv3d(x, self.params[name + ".w"], self.params[name + ".b"], ks, relu, need_dx, periodic)
+    def _packed(self):
+        """Every 3x3x3 layer's weight fragments by name: the data gradient's too where one will be taken."""
+        torch = _torch()
+        ws = {n: self.params[n + ".w"] for n, (_, _, ks) in self.specs.items() if ks == 3}
+        if not all(w.dtype == torch.float32 and w.is_contiguous() for w in ws.values()):
+            return {}  # a layer at a time
+        grad = torch.is_grad_enabled()
+        return dict(zip(ws, pack_layers([(w.detach(), grad and n != "e1a") for n, w in ws.items()])))
 
     def forward(self, x, periodic: bool = False):
         """x (N,X,Y,Z,16) bf16 with channels 0-1 the inputs -> (N,X,Y,Z,4) float32.
@@ -399,17 +420,25 @@ class UNet3D:
 
     def _features(self, x, p):
         """The last layer's output before the head, (N,X,Y,Z,C) bf16; p: periodic."""
+        packs = self._packed()
+
+        def conv(name, x, need_dx=True):
+            return conv3d(x, *layer(name), 3, True, need_dx, p, packs.get(name))
 
         def layer(name):
             return self.params[name + ".w"], self.params[name + ".b"]
 
-        e1, low = conv3d_pool(self._c("e1a", x, need_dx=False, periodic=p), *layer("e1b"), p)
-        e2, low = conv3d_pool(self._c("e2a", low, periodic=p), *layer("e2b"), p)
-        e3, low = conv3d_pool(self._c("e3a", low, periodic=p), *layer("e3b"), p)
-        e4 = self._c("e4b", self._c("e4a", low, periodic=p), periodic=p)
-        d3 = self._c("d3b", conv3d_up(e4, e3, *layer("d3a"), p), periodic=p)
-        d2 = self._c("d2b", conv3d_up(d3, e2, *layer("d2a"), p), periodic=p)
-        return self._c("d1b", conv3d_up(d2, e1, *layer("d1a"), p), periodic=p)
+        def level(a, b, x, need_dx=True):  # of the encoder: its output, and pooled
+            return conv3d_pool(conv(a, x, need_dx), *layer(b), p, packs.get(b))
+
+        def up(a, b, low, skip):  # of the decoder
+            return conv(b, conv3d_up(low, skip, *layer(a), p, packs.get(a)))
+
+        e1, low = level("e1a", "e1b", x, False)
+        e2, low = level("e2a", "e2b", low)
+        e3, low = level("e3a", "e3b", low)
+        d3 = up("d3a", "d3b", conv("e4b", conv("e4a", low)), e3)
+        return up("d1a", "d1b", up("d2a", "d2b", d3, e2), e1)
 
     __call__ = forward
 

@@ -84,3 +84,17 @@ def test_packed_weights_round_to_nearest_and_place_every_tap(gpu):
 
     np.testing.assert_array_equal(wp, fragments(wb, cin, cout))
     np.testing.assert_array_equal(wt, fragments(wb.transpose(2, 1, 0)[:, ::-1], cout, cin))
+
+
+def test_layers_packed_together_equal_layers_packed_alone(gpu):
+    """18 layers (more than one launch takes), with and without the flipped weights."""
+    import torch
+    from taichi_lbm3d_amd import surrogate as sg
+    shapes = [(16, 16), (48, 16), (16, 64), (96, 32), (112, 48), (256, 16)] * 3
+    ws = [make_case((1, 1, 1, 1, cin, cout, 3), 60 + i)[1].float().to(gpu) for i, (cin, cout) in enumerate(shapes)]
+    many = sg.pack_layers([(w, i % 2 == 0) for i, w in enumerate(ws)])
+    for i, (w, (wp, wt)) in enumerate(zip(ws, many)):
+        one, flipped = sg.pack_weights(w, True)
+        assert torch.equal(wp, one)
+        assert torch.equal(wt, flipped) if i % 2 == 0 else wt is None
+    assert sg.pack_layers([]) == []
