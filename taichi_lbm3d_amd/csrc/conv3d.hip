@@ -20,6 +20,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <type_traits>
 
 #include "lbm3d.h"
 #include "lbm3d_conv.h"
@@ -1241,12 +1242,19 @@ constexpr int wgrad_sets(int ks) { return ks == 3 ? 1 : 4; }  // partial sets of
 // dist = min(sqrt(f), M).  Exact for distances up to M; larger ones are capped.
 // f >= 0, so an offset with o^2 >= the best value so far cannot improve it: a
 // thread searches outwards, two offsets a round, and stops there: in a porous
-// medium after a few offsets instead of 2M + 1.  The innermost pass takes its
-// distances from ballots where M < 64 (k_dist_rows).  Threads run along the
-// innermost axis, so every pass reads coalesced rows.  2 x 192^3 voxels, M = 24:
-// 40 us (117 with the search) + 89 us + 146 us, the last bound by the 453 MB of
-// network input it writes, against 528 us a pass for all 49 offsets with a
-// modulo each and about 300 us of conversions after them.
+// medium after a few offsets instead of 2M + 1.  Threads run along the innermost
+// axis, so every pass reads coalesced rows.
+//
+// k_dist_lines keeps the lines of 64 neighbouring voxels along the searched axis in
+// LDS (256 bytes a coordinate), so a line is read from memory once instead of once
+// per offset tried, and the innermost pass is part of the middle one (ballots,
+// dist_row).  Longer lines than 256 and margins from 64 take k_dist_rows and
+// k_dist_axis, one pass an axis.  Bound by the rounds of LDS reads where a wave's 128
+// voxels have one far from any solid.  M = 24:
+//   157 x 149 x 160                         26 + 26 + 16 us -> 24 + 20 us
+//   2 x 192^3, 16 BF16 channels written     40 + 90 + 148 us -> 55 + 96 us
+//   100 x 110 x 66, whole call 25 -> 22 us; 192 x 192 x 20 the same (lanes past
+//   the row's end idle); 8 waves a block and one voxel at a time 52 us for the first
 // ---------------------------------------------------------------------------
 // what the last pass writes: the distance; {mask, distance / scale} in FP32; or
 // 16 BF16 channels of which those are the first two and the others zero
@@ -1259,6 +1267,147 @@ struct DistGeo {
   int32_t margin;
   float inv_scale;       // a power of two
 };
+
+// The outward search along a line of n values, from coordinates c and d at a time.
+// An offset of m + 1 (the last round of an odd m) gives more than m^2, which the
+// last pass caps.
+template <class At>
+__device__ __forceinline__ float2 dist_search2(const At &at, int c, int d, int n, int m) {
+  float best_c = at(c), best_d = at(d);
+  int lo_c = c, hi_c = c, lo_d = d, hi_d = d;
+  float near = 1.f, far = 4.f;  // o^2, (o + 1)^2
+  const auto below = [&](int i) { return i == 0 ? n - 1 : i - 1; };
+  const auto above = [&](int i) { return i == n - 1 ? 0 : i + 1; };
+  for (int o = 1; o <= m && near < fmaxf(best_c, best_d); o += 2) {
+    const int lo_c1 = below(lo_c), hi_c1 = above(hi_c), lo_d1 = below(lo_d), hi_d1 = above(hi_d);
+    lo_c = below(lo_c1), hi_c = above(hi_c1), lo_d = below(lo_d1), hi_d = above(hi_d1);
+    best_c = fminf(best_c, fminf(fminf(at(lo_c1), at(hi_c1)) + near, fminf(at(lo_c), at(hi_c)) + far));
+    best_d = fminf(best_d, fminf(fminf(at(lo_d1), at(hi_d1)) + near, fminf(at(lo_d), at(hi_d)) + far));
+    near = far + (float)(2 * o + 3);
+    far = near + (float)(2 * o + 5);
+  }
+  return make_float2(best_c, best_d);
+}
+
+// The innermost pass for margins below 64, without a search, for the 64 voxels of a
+// wave: the solid bits of the row's coordinates z0 - 64 .. z0 + 127 (wrapped); each
+// lane finds its nearest set bit on either side.
+__device__ __forceinline__ float dist_row(uint64_t before, uint64_t here, uint64_t after, int lane, int m) {
+  // bit i of up: solid at distance i above (0 .. 63); bit 63 - i of down: below
+  const uint64_t up = lane ? (here >> lane) | (after << (64 - lane)) : here;
+  const uint64_t down = lane < 63 ? (here << (63 - lane)) | (before >> (lane + 1)) : here;
+  const int du = up ? __ffsll((unsigned long long)up) - 1 : 64, dd = down ? __clzll((long long)down) : 64;
+  const int dmin = du < dd ? du : dd;
+  return (float)(dmin <= m ? dmin * dmin : 3 * m * m + 1);
+}
+
+// mask and scaled distance as the first two of 16 BF16 channels, in one word
+__device__ __forceinline__ uint32_t net_word(float mask, float scaled) {
+  return (uint32_t)to_bf16(mask) | ((uint32_t)to_bf16(scaled) << 16);
+}
+
+// The middle (AXIS 1: with the innermost pass before it) or the outer axis (AXIS 0)
+// of the lines through 64 voxels z0 .. z0 + 63 of a row; 16 waves.  LDS is filled
+// first, 8 values per lane in flight; a row's three bytes give its distances.  Then
+// every wave searches two of the line's rows at a time.  A voxel is solid where the
+// squared distance is 0, so the last pass needs no mask.
+constexpr int kDistWaves = 16, kDistAhead = 8;
+constexpr int kDistLine = 256;  // longest line: 64 KB of LDS
+
+template <int AXIS, int OUT>
+__global__ void __launch_bounds__(64 * kDistWaves)
+    k_dist_lines(const int8_t *__restrict__ solid, const float *__restrict__ f, void *__restrict__ out,
+                 const DistGeo gm, const Div segs) {
+  extern __shared__ float lines[];  // [coordinate][64]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = AXIS == 1 ? gm.d1 : gm.d0, m = gm.margin;
+  const uint32_t t = qdiv(blockIdx.x, segs);
+  const int z0 = (int)(blockIdx.x - t * segs.d) * 64;
+  const int64_t plane = (int64_t)gm.d1 * gm.d2, stride = AXIS == 1 ? gm.d2 : plane;
+  int64_t first = t * plane;  // of coordinate 0
+  if (AXIS == 0) {
+    const uint32_t vol = qdiv(t, gm.div1);
+    first = (int64_t)vol * gm.d0 * plane + (int64_t)(t - vol * (uint32_t)gm.d1) * gm.d2;
+  }
+  const bool in = z0 + lane < gm.d2;
+  const int z = in ? z0 + lane : gm.d2 - 1;
+  const auto last = [&](int c) { return c < n ? c : n - 1; };
+  if constexpr (AXIS == 1) {
+    // coordinates z0 + lane - 64, + 0, + 64, each wrapped into the row
+    const int zw = (z0 + lane) % gm.d2, step = 64 % gm.d2;
+    const int zm = zw < step ? zw - step + gm.d2 : zw - step, zp = zw + step >= gm.d2 ? zw + step - gm.d2 : zw + step;
+    for (int c0 = wave; c0 < n; c0 += kDistWaves * kDistAhead) {
+      int8_t a[kDistAhead], b[kDistAhead], c[kDistAhead];
+#pragma unroll
+      for (int i = 0; i < kDistAhead; ++i) {
+        const int8_t *const row = solid + first + (int64_t)last(c0 + kDistWaves * i) * stride;
+        a[i] = row[zm];
+        b[i] = row[zw];
+        c[i] = row[zp];
+      }
+#pragma unroll
+      for (int i = 0; i < kDistAhead; ++i) {
+        const float v = dist_row(__ballot(a[i] != 0), __ballot(b[i] != 0), __ballot(c[i] != 0), lane, m);
+        if (c0 + kDistWaves * i < n) lines[(c0 + kDistWaves * i) * 64 + lane] = v;
+      }
+    }
+  } else {
+    for (int c0 = wave; c0 < n; c0 += kDistWaves * kDistAhead) {
+      float v[kDistAhead];
+#pragma unroll
+      for (int i = 0; i < kDistAhead; ++i) v[i] = f[first + last(c0 + kDistWaves * i) * stride + z];
+#pragma unroll
+      for (int i = 0; i < kDistAhead; ++i)
+        if (c0 + kDistWaves * i < n) lines[(c0 + kDistWaves * i) * 64 + lane] = v[i];
+    }
+  }
+  __syncthreads();
+  auto put = [&](int c, float best) {
+    const int64_t v = first + c * stride + z;
+    if constexpr (AXIS == 1) {
+      if (in) static_cast<float *>(out)[v] = best;
+    } else {
+      // correctly rounded: the distance an exact EDT (FP64) reports, cast to FP32
+      const float dist = fminf(sqrtf(best), (float)m), mask = best == 0.f ? 1.f : 0.f, scaled = dist * gm.inv_scale;
+      if constexpr (OUT == kDistPlain) {
+        if (in) static_cast<float *>(out)[v] = dist;
+      } else if constexpr (OUT == kDistPair) {
+        if (in) static_cast<float2 *>(out)[v] = make_float2(mask, scaled);
+      } else {
+        // 32 bytes a voxel: a store takes 32 voxels, whole lines
+        const uint32_t word = net_word(mask, scaled);
+        u32x4 *const o4 = static_cast<u32x4 *>(out) + 2 * (first + c * stride + z0);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint32_t other = (uint32_t)__shfl((int)word, 32 * h + (lane >> 1));
+          if (z0 + 32 * h + (lane >> 1) < gm.d2) o4[64 * h + lane] = u32x4{lane & 1 ? 0u : other, 0u, 0u, 0u};
+        }
+      }
+    }
+  };
+  const auto at = [&](int c) { return lines[c * 64 + lane]; };
+  for (int c = wave; c < n; c += 2 * kDistWaves) {
+    const int d = c + kDistWaves < n ? c + kDistWaves : c;
+    const float2 best = dist_search2(at, c, d, n, m);
+    put(c, best.x);
+    if (d != c) put(d, best.y);
+  }
+}
+
+// the innermost pass by itself, one wave per 64 voxels of a row
+__global__ void __launch_bounds__(256)
+    k_dist_rows(const int8_t *__restrict__ solid, float *__restrict__ out, const DistGeo gm, Div segs, int64_t waves) {
+  const int64_t wv = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (wv >= waves) return;  // whole waves
+  const int lane = threadIdx.x & 63, n = gm.d2;
+  const int64_t row = waves < ((int64_t)1 << 31) ? (int64_t)qdiv((uint32_t)wv, segs) : wv / segs.d;
+  const int z0 = (int)(wv - row * segs.d) * 64;
+  const int8_t *line = solid + row * n;
+  const int z = (z0 + lane) % n, step = 64 % n;
+  const int zm = z < step ? z - step + n : z - step, zp = z + step >= n ? z + step - n : z + step;
+  const float v = dist_row(__ballot(line[zm] != 0), __ballot(line[z] != 0), __ballot(line[zp] != 0), lane, gm.margin);
+  if (z0 + lane < n) out[row * n + z0 + lane] = v;
+}
 
 template <int AXIS, int OUT>
 __global__ void __launch_bounds__(256)
@@ -1314,36 +1463,11 @@ __global__ void __launch_bounds__(256)
         static_cast<float2 *>(out)[v] = make_float2(mask, scaled);
       } else {
         u32x4 *o4 = static_cast<u32x4 *>(out) + 2 * v;
-        o4[0] = u32x4{(uint32_t)to_bf16(mask) | ((uint32_t)to_bf16(scaled) << 16), 0u, 0u, 0u};
+        o4[0] = u32x4{net_word(mask, scaled), 0u, 0u, 0u};
         o4[1] = u32x4{0u, 0u, 0u, 0u};
       }
     }
   }
-}
-
-// The innermost pass for margins below 64, without a search: one wave per 64
-// voxels of a row.  Three loads and ballots give the solid bits of the row's
-// coordinates z0 - 64 .. z0 + 127 (wrapped), and each lane finds its nearest set
-// bit on either side.
-__global__ void __launch_bounds__(256)
-    k_dist_rows(const int8_t *__restrict__ solid, float *__restrict__ out, const DistGeo gm, Div segs, int64_t waves) {
-  const int64_t wv = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (wv >= waves) return;  // whole waves
-  const int lane = threadIdx.x & 63, n = gm.d2, m = gm.margin;
-  const int64_t row = waves < ((int64_t)1 << 31) ? (int64_t)qdiv((uint32_t)wv, segs) : wv / segs.d;
-  const int z0 = (int)(wv - row * segs.d) * 64;
-  const int8_t *line = solid + row * n;
-  // z0 + lane - 64, + 0, + 64, each wrapped into [0, n)
-  int z = (z0 + lane) % n;
-  const int step = 64 % n;
-  const int zm = z < step ? z - step + n : z - step, zp = z + step >= n ? z + step - n : z + step;
-  const uint64_t before = __ballot(line[zm] != 0), here = __ballot(line[z] != 0), after = __ballot(line[zp] != 0);
-  // bit i of up: solid at distance i above (0 .. 63); bit 63 - i of down: below
-  const uint64_t up = lane ? (here >> lane) | (after << (64 - lane)) : here;
-  const uint64_t down = lane < 63 ? (here << (63 - lane)) | (before >> (lane + 1)) : here;
-  const int du = up ? __ffsll((unsigned long long)up) - 1 : 64, dd = down ? __clzll((long long)down) : 64;
-  const int dmin = du < dd ? du : dd;
-  if (z0 + lane < n) out[row * n + z0 + lane] = (float)(dmin <= m ? dmin * dmin : 3 * m * m + 1);
 }
 
 // bf16 y > 0 (false for -0, negatives and NaN)
@@ -1891,21 +2015,31 @@ static int distance_passes(void *stream, const int8_t *solid, void *out, int mod
   gm.inv_scale = inv_scale;
   hipStream_t s = (hipStream_t)stream;
   const unsigned grid = (unsigned)((gm.total + 255) / 256);
-  // innermost axis from the solid mask into `second`, then the middle axis into
-  // work and the outer axis into out (a pass cannot run in place: it reads
-  // values other threads overwrite)
-  const int64_t rows = (int64_t)n * d * h, segs = ((int64_t)w + 63) / 64, blocks = (rows * segs + 3) / 4;
-  if (margin < 64 && blocks <= (int64_t)(UINT32_MAX / 256u))
-    k_dist_rows<<<(unsigned)blocks, 256, 0, s>>>(solid, second, gm, make_div((uint32_t)segs), rows * segs);
-  else
-    k_dist_axis<2, 0><<<grid, 256, 0, s>>>(solid, nullptr, second, gm);
-  k_dist_axis<1, 0><<<grid, 256, 0, s>>>(solid, second, work, gm);
-  if (mode == kDistNet)
-    k_dist_axis<0, kDistNet><<<grid, 256, 0, s>>>(solid, work, out, gm);
-  else if (mode == kDistPair)
-    k_dist_axis<0, kDistPair><<<grid, 256, 0, s>>>(solid, work, out, gm);
-  else
-    k_dist_axis<0, kDistPlain><<<grid, 256, 0, s>>>(solid, work, out, gm);
+  const int64_t segs = ((int64_t)w + 63) / 64, most = (int64_t)(UINT32_MAX / (64u * kDistWaves));
+  const Div dsegs = make_div((uint32_t)segs);
+  // a pass cannot run in place: it reads values that other threads overwrite
+  if (margin < 64 && h <= kDistLine && (int64_t)n * d * segs <= most) {
+    k_dist_lines<1, 0><<<(unsigned)(n * d * segs), 64 * kDistWaves, 256 * h, s>>>(solid, nullptr, work, gm, dsegs);
+  } else {
+    const int64_t rows = (int64_t)n * d * h, blocks = (rows * segs + 3) / 4;
+    if (margin < 64 && blocks <= (int64_t)(UINT32_MAX / 256u))
+      k_dist_rows<<<(unsigned)blocks, 256, 0, s>>>(solid, second, gm, dsegs, rows * segs);
+    else
+      k_dist_axis<2, 0><<<grid, 256, 0, s>>>(solid, nullptr, second, gm);
+    k_dist_axis<1, 0><<<grid, 256, 0, s>>>(solid, second, work, gm);
+  }
+  if (int rc = ccheck("lbm3d_distance_periodic")) return rc;
+  const bool lines = d <= kDistLine && (int64_t)n * h * segs <= most;
+  auto outer = [&](auto m) {
+    constexpr int kOut = decltype(m)::value;
+    if (lines)
+      k_dist_lines<0, kOut><<<(unsigned)(n * h * segs), 64 * kDistWaves, 256 * d, s>>>(solid, work, out, gm, dsegs);
+    else
+      k_dist_axis<0, kOut><<<grid, 256, 0, s>>>(solid, work, out, gm);
+  };
+  if (mode == kDistNet) outer(std::integral_constant<int, kDistNet>{});
+  else if (mode == kDistPair) outer(std::integral_constant<int, kDistPair>{});
+  else outer(std::integral_constant<int, kDistPlain>{});
   return ccheck("lbm3d_distance_periodic");
 }
 

@@ -48,3 +48,19 @@ def test_inputs_are_mask_and_scaled_distance(gpu, dtype):
     assert torch.equal(pair, want)
     assert torch.equal(sg.network_inputs(t), sg.to_network_input(want))
     assert torch.equal(sg.make_inputs(t.transpose(1, 3)), sg.make_inputs(t.transpose(1, 3).contiguous()))
+
+
+@pytest.mark.parametrize("shape", [(257, 3, 5), (3, 257, 5), (256, 2, 70), (2, 256, 64), (33, 16, 129)])
+@pytest.mark.parametrize("margin", [3, 24, 63])
+def test_lines_at_the_limit_of_the_lds(gpu, shape, margin):
+    """Lines of 256 and 257 voxels along the outer and the middle axis, batched; whole and partial waves."""
+    import torch
+    from taichi_lbm3d_amd import surrogate as sg
+    rng = np.random.default_rng(margin)
+    solids = [(rng.random(shape) < f).astype(np.uint8) for f in (0.004, 0.03)]
+    batch = torch.from_numpy(np.stack(solids)).to(gpu)
+    want = np.stack([nearest_solid(s, margin) for s in solids])
+    np.testing.assert_array_equal(sg.periodic_distance(batch, margin=margin).cpu().numpy(), want)
+    if margin == 24:
+        pair = torch.stack([batch.float(), torch.from_numpy(want).to(gpu) / sg.DIST_SCALE], dim=-1)
+        assert torch.equal(sg.network_inputs(batch), sg.to_network_input(pair))
