@@ -99,21 +99,97 @@ __global__ void __launch_bounds__(256)
 // triangle order, bit for bit k_winding's.
 //
 // Omega / 2 is the argument of prod_t (den_t + i det_t): a wave takes a parent
-// block, its lanes the triangles in turn, and each lane keeps 8 running products
-// (the parent's 8 children), normalised, with the turns they have made.  Lengths
-// are in cells, relative to the parent's centre (FP64 difference, rounded once).
-// 7,680 triangles on 96 x 104 x 88 nodes: 2.57 ms against 33.2 ms for all nodes
-// in FP64; bound by FP32 arithmetic.
+// block, its lanes the triangles in turn, and each lane keeps running products,
+// normalised, with the turns they have made.  A triangle further than kFar times the
+// parent's reach R (centre to outermost node) is taken once, at the parent's centre,
+// for all 8 children, which adds R * 2 A / (d - R)^3 to the bound; the others once per
+// child, as soon as there are 64 of them.  Over a plane the far ones add about
+// 2 pi / (kFar - 1), of the distance pi that Omega / 2 has from the threshold on either
+// side of a closed surface; a smaller kFar leaves more nodes open where surfaces meet.
+// Lengths are in cells, relative to the parent's centre.
+// Bound by FP32 arithmetic.  7,680 triangles on 96 x 104 x 88 nodes: every node in FP64
+// 33.2 ms; every triangle for every child 3.2 ms; kFar 10.5 to 12 1.65 ms, 9 1.87 ms
+// and 16 1.74 ms.  With corners from FP64 differences and near triangles as they come
+// kFar 12 took 2.02 ms, 6 8.3 ms.  Loading the next triangle ahead changed nothing.
 // ---------------------------------------------------------------------------
+constexpr float kFar = 11.f;
+
 struct VoxGrid {
   double x0, y0, z0, dx;
   int32_t nx, ny, nz;
   int32_t n_tris;
-  float eta;  // FP64 rounding of a node's coordinates, in cells
+  float eta;  // rounding of a node's coordinates in FP64 and of a centre's in two FP32, in cells
 };
 
 // how many blocks of side s cover n nodes
 __host__ __device__ __forceinline__ int32_t blocks_of(int32_t n, int32_t s) { return (n + s - 1) / s; }
+
+// A triangle from a point, in cells: its corners, twice its area, a bound on how far it
+// reaches from its nearest corner, that corner's squared distance.
+struct Seen {
+  float ax, ay, az, bx, by, bz, cx, cy, cz, area2, edge, near2;
+  // from the point hi + lo: v - hi is exact where it is not much larger than lo, so
+  // a coordinate is off by 3 roundings of its own size and by the point's 2^-48 (and
+  // by inv's, which scales all alike)
+  __device__ __forceinline__ Seen(const float *tris, int32_t t, const float3 hi, const float3 lo, float inv) {
+    const float *v = tris + (int64_t)t * 9;
+    ax = ((v[0] - hi.x) - lo.x) * inv, ay = ((v[1] - hi.y) - lo.y) * inv, az = ((v[2] - hi.z) - lo.z) * inv;
+    bx = ((v[3] - hi.x) - lo.x) * inv, by = ((v[4] - hi.y) - lo.y) * inv, bz = ((v[5] - hi.z) - lo.z) * inv;
+    cx = ((v[6] - hi.x) - lo.x) * inv, cy = ((v[7] - hi.y) - lo.y) * inv, cz = ((v[8] - hi.z) - lo.z) * inv;
+    const float ux = bx - ax, uy = by - ay, uz = bz - az, wx = cx - ax, wy = cy - ay, wz = cz - az;
+    const float vx = cx - bx, vy = cy - by, vz = cz - bz;
+    const float nx = uy * wz - uz * wy, ny = uz * wx - ux * wz, nz = ux * wy - uy * wx;
+    const float u2 = ux * ux + uy * uy + uz * uz, w2 = wx * wx + wy * wy + wz * wz, v2 = vx * vx + vy * vy + vz * vz;
+    area2 = 1.02f * __builtin_amdgcn_sqrtf(nx * nx + ny * ny + nz * nz) + 1e-5f * (u2 + w2);
+    edge = 0.58f * __builtin_amdgcn_sqrtf(fmaxf(fmaxf(u2, w2), v2));
+    near2 = fminf(fminf(ax * ax + ay * ay + az * az, bx * bx + by * by + bz * bz), cx * cx + cy * cy + cz * cz);
+  }
+};
+
+// a running product of den + i det with its turns, and the bound on its argument's error
+struct Product {
+  float zr = 1.f, zi = 0.f, err = 0.f;
+  int turns = 0;
+
+  // The factor of a triangle seen from the origin.  slack: how far its corners may be
+  // off, in units of 2^-24, besides their own rounding; rho > 0: it stands for all
+  // points within rho.
+  __device__ __forceinline__ void take(float Ax, float Ay, float Az, float Bx, float By, float Bz, float Cx, float Cy,
+                                       float Cz, float slack, float area2, float edge, float rho) {
+    const float la = __builtin_amdgcn_sqrtf(Ax * Ax + Ay * Ay + Az * Az);
+    const float lb = __builtin_amdgcn_sqrtf(Bx * Bx + By * By + Bz * Bz);
+    const float lc = __builtin_amdgcn_sqrtf(Cx * Cx + Cy * Cy + Cz * Cz);
+    const float det = Ax * (By * Cz - Bz * Cy) - Ay * (Bx * Cz - Bz * Cx) + Az * (Bx * Cy - By * Cx);
+    const float L = la * lb * lc;
+    const float den = L + (Ax * Bx + Ay * By + Az * Bz) * lc + (Bx * Cx + By * Cy + Bz * Cz) * la +
+                      (Cx * Ax + Cy * Ay + Cz * Az) * lb;
+    const float lmin = fminf(fminf(la, lb), lc);
+    const float rz = __builtin_amdgcn_rsqf(det * det + den * den);
+    // Rounding.  A corner is off by at most 2^-24 kappa of its length, kappa = 3 +
+    // slack / lmin; det and den then by (15 kappa + 74) 2^-24 L together, and the
+    // angle by that over |den + i det| (1.5 times for the arc).
+    const float kappa = 3.f + slack * __builtin_amdgcn_rcpf(lmin);
+    const float q = L * rz;  // at least 17^-1/2, unless something under- or overflowed
+    float e = (1.6e-6f * kappa + 7e-6f) * q;
+    // near the branch cut the sign of det, and with it a full turn, is open
+    if (!(q > 0.2f && e < 0.2f) || (den < 0.f && fabsf(det) * rz <= e)) e = 1e30f;
+    e += 1e-6f;  // the product's own rounding
+    if (rho > 0.f) {
+      const float gap = lmin * 0.999f - edge - rho;
+      const float r = __builtin_amdgcn_rcpf(gap);
+      e += gap > 0.05f ? 0.51f * rho * area2 * (r * r * r) : 1e30f;  // of Omega / 2
+    }
+    err += e;
+    const float ur = den * rz, ui = det * rz;
+    const float nr = zr * ur - zi * ui, ni = zr * ui + zi * ur;
+    // past +-pi: both angles on one side of the real axis, their sum on the other
+    turns += (zi >= 0.f && ui >= 0.f && ni < 0.f ? 1 : 0) - (zi < 0.f && ui < 0.f && ni >= 0.f ? 1 : 0);
+    zr = nr;
+    zi = ni;
+  }
+  __device__ __forceinline__ float angle() const { return atan2f(zi, zr) + 6.2831853f * (float)turns; }
+  __device__ __forceinline__ float bound() const { return err + 5e-6f * (1.f + fabsf((float)turns)); }
+};
 
 // The children of side S of the parents (side 2S) in `list` (all parents if it is
 // null): flags of the decided ones, the others' block indices to `next`.
@@ -122,85 +198,65 @@ __global__ void __launch_bounds__(256)
     k_winding_blocks(const float *__restrict__ tris, const VoxGrid gr, const int32_t *__restrict__ list,
                      const int32_t *__restrict__ count, int32_t all, int32_t *__restrict__ next,
                      int32_t *__restrict__ next_count, int8_t *__restrict__ solid) {
-  const int lane = threadIdx.x & 63;
+  // near triangles wait here until there is one for every lane (up to 63 + 64 of them)
+  __shared__ int32_t queue[4][128];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int32_t waves = (int32_t)(gridDim.x * 4);
   const int32_t n = list ? *count : all;
   const int32_t pny = blocks_of(gr.ny, 2 * S), pnz = blocks_of(gr.nz, 2 * S);
   const int32_t cnx = blocks_of(gr.nx, S), cny = blocks_of(gr.ny, S), cnz = blocks_of(gr.nz, S);
-  const double inv = 1.0 / gr.dx;
+  const float inv = (float)(1.0 / gr.dx);
   for (int32_t it = (int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6)); it < n; it += waves) {
     const int32_t id = __builtin_amdgcn_readfirstlane(list ? list[it] : it);
     const int32_t bk = id % pnz, bt = id / pnz, bj = bt % pny, bi = bt / pny;
     // the parent's reference point, and its children's centres relative to it, in cells
     const double pi = 2 * S * bi + S - 0.5, pj = 2 * S * bj + S - 0.5, pk = 2 * S * bk + S - 0.5;
     const double px = gr.x0 + gr.dx * pi, py = gr.y0 + gr.dx * pj, pz = gr.z0 + gr.dx * pk;
-    float zr[8], zi[8], err[8];
-    int turns[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      zr[c] = 1.f;
-      zi[c] = err[c] = 0.f;
-      turns[c] = 0;
-    }
+    const float3 hi = make_float3((float)px, (float)py, (float)pz);
+    const float3 lo = make_float3((float)(px - (double)hi.x), (float)(py - (double)hi.y), (float)(pz - (double)hi.z));
+    Product child[8], all8;
     constexpr float off = 0.5f * S;                    // a child's centre, per axis
     constexpr float rho = 0.866026f * (S - 1);         // its half diagonal
     constexpr float reach = 2.f * 1.7320508f * off;    // twice the offset's length
-    for (int32_t t = lane; t < gr.n_tris; t += 64) {
-      const float *v = tris + (int64_t)t * 9;
-      const float ax = (float)(((double)v[0] - px) * inv), ay = (float)(((double)v[1] - py) * inv),
-                  az = (float)(((double)v[2] - pz) * inv);
-      const float bx = (float)(((double)v[3] - px) * inv), by = (float)(((double)v[4] - py) * inv),
-                  bz = (float)(((double)v[5] - pz) * inv);
-      const float cx = (float)(((double)v[6] - px) * inv), cy = (float)(((double)v[7] - py) * inv),
-                  cz = (float)(((double)v[8] - pz) * inv);
-      float area2 = 0.f, edge = 0.f;  // 2 A and a bound on how far the triangle reaches from its nearest corner
-      if constexpr (S > 1) {
-        const float ux = bx - ax, uy = by - ay, uz = bz - az, wx = cx - ax, wy = cy - ay, wz = cz - az;
-        const float nx = uy * wz - uz * wy, ny = uz * wx - ux * wz, nz = ux * wy - uy * wx;
-        area2 = 1.02f * sqrtf(nx * nx + ny * ny + nz * nz) + 1e-5f * (ux * ux + uy * uy + uz * uz + wx * wx + wy * wy + wz * wz);
-        const float vx = cx - bx, vy = cy - by, vz = cz - bz;
-        edge = 0.58f * sqrtf(fmaxf(fmaxf(ux * ux + uy * uy + uz * uz, wx * wx + wy * wy + wz * wz), vx * vx + vy * vy + vz * vz));
-      }
+    constexpr float R = 1.7320508f * off + rho;        // the parent's, from its centre
+    // the children's factors of the first `n` triangles from queue[wave][from]
+    const auto near = [&](int from, int n) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (lane < n) {
+        const Seen s(tris, queue[wave][from + lane], hi, lo, inv);
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const float ox = c & 4 ? off : -off, oy = c & 2 ? off : -off, oz = c & 1 ? off : -off;
-        const float Ax = ax - ox, Ay = ay - oy, Az = az - oz, Bx = bx - ox, By = by - oy, Bz = bz - oz, Cx = cx - ox,
-                    Cy = cy - oy, Cz = cz - oz;
-        const float la = __builtin_amdgcn_sqrtf(Ax * Ax + Ay * Ay + Az * Az);
-        const float lb = __builtin_amdgcn_sqrtf(Bx * Bx + By * By + Bz * Bz);
-        const float lc = __builtin_amdgcn_sqrtf(Cx * Cx + Cy * Cy + Cz * Cz);
-        const float det = Ax * (By * Cz - Bz * Cy) - Ay * (Bx * Cz - Bz * Cx) + Az * (Bx * Cy - By * Cx);
-        const float L = la * lb * lc;
-        const float den = L + (Ax * Bx + Ay * By + Az * Bz) * lc + (Bx * Cx + By * Cy + Bz * Cz) * la +
-                          (Cx * Ax + Cy * Ay + Cz * Az) * lb;
-        const float lmin = fminf(fminf(la, lb), lc);
-        const float rz = __builtin_amdgcn_rsqf(det * det + den * den);
-        // Rounding.  A corner is off by at most 2^-24 kappa of its length, kappa = 1 +
-        // (reach + eta 2^24) / lmin; det and den then by (15 kappa + 74) 2^-24 L
-        // together, and the angle by that over |den + i det| (1.5 times for the arc).
-        const float kappa = 1.f + (reach + 1.7e7f * gr.eta) * __builtin_amdgcn_rcpf(lmin);
-        const float q = L * rz;  // at least 17^-1/2, unless something under- or overflowed
-        float e = (1.6e-6f * kappa + 7e-6f) * q;
-        // near the branch cut the sign of det, and with it a full turn, is open
-        if (!(q > 0.2f && e < 0.2f) || (den < 0.f && fabsf(det) * rz <= e)) e = 1e30f;
-        e += 1e-6f;  // the product's own rounding
-        if constexpr (S > 1) {
-          const float gap = lmin * 0.999f - edge - rho;
-          const float r = __builtin_amdgcn_rcpf(gap);
-          e += gap > 0.05f ? 0.51f * rho * area2 * (r * r * r) : 1e30f;  // of Omega / 2
+        for (int c = 0; c < 8; ++c) {
+          const float ox = c & 4 ? off : -off, oy = c & 2 ? off : -off, oz = c & 1 ? off : -off;
+          child[c].take(s.ax - ox, s.ay - oy, s.az - oz, s.bx - ox, s.by - oy, s.bz - oz, s.cx - ox, s.cy - oy,
+                        s.cz - oz, reach + 1.7e7f * gr.eta, s.area2, s.edge, rho);
         }
-        err[c] += e;
-        const float ur = den * rz, ui = det * rz;
-        const float nr = zr[c] * ur - zi[c] * ui, ni = zr[c] * ui + zi[c] * ur;
-        // past +-pi: both angles on one side of the real axis, their sum on the other
-        turns[c] += (zi[c] >= 0.f && ui >= 0.f && ni < 0.f ? 1 : 0) - (zi[c] < 0.f && ui < 0.f && ni >= 0.f ? 1 : 0);
-        zr[c] = nr;
-        zi[c] = ni;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
+    int queued = 0;  // uniform in the wave
+    for (int32_t base = 0; base < gr.n_tris; base += 64) {
+      const int32_t t = base + lane;
+      bool close = false;
+      if (t < gr.n_tris) {
+        const Seen s(tris, t, hi, lo, inv);
+        const float far = kFar * R + s.edge;
+        close = !(s.near2 > far * far);  // NaN too
+        if (!close) all8.take(s.ax, s.ay, s.az, s.bx, s.by, s.bz, s.cx, s.cy, s.cz, 1.7e7f * gr.eta, s.area2, s.edge, R);
+      }
+      const uint64_t m = __ballot(close);
+      if (close)
+        queue[wave][queued + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = t;
+      queued += __popcll(m);
+      if (queued >= 64) {
+        queued -= 64;
+        near(queued, 64);
       }
     }
+    if (queued > 0) near(0, queued);
+    const float half8 = all8.angle(), err8 = all8.bound();
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      float half = atan2f(zi[c], zr[c]) + 6.2831853f * (float)turns[c], e = err[c] + 5e-6f * (1.f + fabsf((float)turns[c]));
+      float half = child[c].angle() + half8, e = child[c].bound() + err8 + 1e-6f * (fabsf(half8) + 1.f);
 #pragma unroll
       for (int d = 32; d > 0; d >>= 1) {
         half += __shfl_xor(half, d);
@@ -286,7 +342,7 @@ int lbm3d_voxelize_blocks(void *stream, const float *tris, int32_t n_tris, doubl
   const double far = std::fmax(std::fmax(std::fmax(std::fabs(x0), std::fabs(x0 + dx * nx)),
                                          std::fmax(std::fabs(y0), std::fabs(y0 + dx * ny))),
                                std::fmax(std::fabs(z0), std::fabs(z0 + dx * nz)));
-  gr.eta = (float)(1e-15 * far / dx);
+  gr.eta = (float)(5e-15 * far / dx);
   int32_t *const ws = (int32_t *)workspace;
   int32_t *const list4 = ws + vox_list(nx, ny, nz, 0), *const list2 = ws + vox_list(nx, ny, nz, 1),
                  *const list1 = ws + vox_list(nx, ny, nz, 2);

@@ -69,3 +69,17 @@ def test_any_scale_and_origin(gpu, name, scale, origin):
     tris = meshes()[name] * scale + np.array(origin)
     want, got = both(gpu, tris, origin, scale, (23, 21, 22))
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("radius,level,dx", [(60.0, 3, 1.0), (60.0, 4, 1.0), (4.0, 4, 0.05), (200.0, 2, 7.0)])
+def test_near_and_far_triangles_give_the_same_flags(gpu, radius, level, dx):
+    """A surface of many triangles, most of them far from any block, some blocks with more
+    near ones than a wave has lanes; triangles smaller and larger than a cell."""
+    from taichi_lbm3d_amd.stl import sphere_mesh
+    shape = (26, 19, 33)
+    origin = np.array([radius * 0.8, -9 * dx, 3 * dx])
+    ball = sphere_mesh((0.0, 0.0, 0.0), radius, level)
+    inner = sphere_mesh((radius, 0.0, 8 * dx), 6 * dx, 2)
+    ref, got = both(gpu, np.concatenate([ball, inner]), origin, dx, shape)
+    assert 0 < ref.sum() < ref.size
+    np.testing.assert_array_equal(got, ref)
