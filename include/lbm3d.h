@@ -201,8 +201,8 @@ int lbm3d_build_neighbors(void *stream, const lbm3d_params *p, const int32_t *ce
 
 /* ---- solver ------------------------------------------------------------- */
 
-/* init (SP:160-170): g = feq(rho0, u0) - w on every fluid cell, and the
- * pressure-face state = u0 at the face nodes.  rho0 [n_cells] and u0 (SoA
+/* init (SP:160-170): g = feq(rho0, u0) - w on every fluid cell, 0 in the slots'
+ * padding up to their stride, and the pressure-face state = u0 at the face nodes.  rho0 [n_cells] and u0 (SoA
  * [3][n_cells], FP32) may be NULL for the reference's rest state rho = 1, u = 0. */
 int lbm3d_init(void *stream, const lbm3d_params *p, int dtype, void *g, const int32_t *cells,
                void *face_u, const float *rho0, const float *u0);

@@ -356,7 +356,8 @@ class LB3D_Solver_Single_Phase:
         p = self._params
         tdt = _lib.torch_storage_dtype(self.dtype)
         stride = _lib.lib().size("lbm3d_slot_stride", p.n_cells)
-        self._dev["g"] = torch.zeros(max(19 * stride, 1), dtype=tdt, device=dev)
+        # lbm3d_init writes all of it, padding included
+        self._dev["g"] = torch.empty(19 * stride, dtype=tdt, device=dev) if stride else torch.zeros(1, dtype=tdt, device=dev)
         self._dev["face_u"] = torch.zeros(max(self._face_u_floats, 1), dtype=self._real_dtype(), device=dev)
 
     def _real_dtype(self):
