@@ -415,8 +415,8 @@ __device__ __forceinline__ void brick_origin(const Bricks &bk, uint32_t bi, int 
 // memory; the next chunk's (or brick's) halo is loaded while the MFMAs of the
 // current one run, so a chunk has one barrier and no exposed load.  Weight
 // fragments are streamed kWRing - 1 steps ahead.
-// Bound by the MFMAs and the LDS reads of the voxels (one 1 KB fragment per
-// MFMA): 192 -> 64 channels at 2 x 48^3 take 150 us (980 TFLOP/s) against 305
+// Bound by the MFMAs (half the LDS reads, with two channel tiles a wave, 145 -> 143
+// us for 192 -> 64, but 382 -> 400 for 96 -> 32 at 2 x 96^3): 192 -> 64 channels at 2 x 48^3 take 150 us (980 TFLOP/s) against 305
 // for one 16-channel tile per workgroup with its halo loaded behind a barrier.
 template <int CT, int MODE>
 __global__ void __launch_bounds__(256, 2)
@@ -622,8 +622,10 @@ __global__ void __launch_bounds__(256, 2)
 // bricks of k_conv3 read each plane twice, 32 bytes of a voxel at a time), and
 // the weights stay in registers.
 // Bound by HBM for 16 -> 16 channels (2 x 192^3: 250 us, 3.6 TB/s of
-// activations, against 480 us before and 360 us in bricks) and by the LDS reads
-// of the voxels for 48 -> 16 (624 us, 940 TFLOP/s, against 1,225 and 841).
+// activations, against 480 us before and 360 us in bricks) and by the MFMAs for
+// 48 -> 16 (624 us, 940 TFLOP/s, against 1,225 and 841; a quarter of the LDS reads
+// saved 12 %, by sharing a fragment between three output planes, which changes the
+// order of the sums).
 constexpr int kRing = 4;
 
 // Columns of one launch: n volumes of nby x nbx columns (x fastest), each cut
