@@ -29,8 +29,13 @@
 #include "geo_ascii.h"
 #include "lbm3d.h"
 #include "lbm3d_io.h"
+#include "winding.h"
 
 namespace {
+
+using lbm3d_winding::blocks_of;
+using lbm3d_winding::Product;
+using lbm3d_winding::Seen;
 
 thread_local char io_err[512] = "";
 
@@ -119,76 +124,6 @@ struct VoxGrid {
   int32_t nx, ny, nz;
   int32_t n_tris;
   float eta;  // rounding of a node's coordinates in FP64 and of a centre's in two FP32, in cells
-};
-
-// how many blocks of side s cover n nodes
-__host__ __device__ __forceinline__ int32_t blocks_of(int32_t n, int32_t s) { return (n + s - 1) / s; }
-
-// A triangle from a point, in cells: its corners, twice its area, a bound on how far it
-// reaches from its nearest corner, that corner's squared distance.
-struct Seen {
-  float ax, ay, az, bx, by, bz, cx, cy, cz, area2, edge, near2;
-  // from the point hi + lo: v - hi is exact where it is not much larger than lo, so
-  // a coordinate is off by 3 roundings of its own size and by the point's 2^-48 (and
-  // by inv's, which scales all alike)
-  __device__ __forceinline__ Seen(const float *tris, int32_t t, const float3 hi, const float3 lo, float inv) {
-    const float *v = tris + (int64_t)t * 9;
-    ax = ((v[0] - hi.x) - lo.x) * inv, ay = ((v[1] - hi.y) - lo.y) * inv, az = ((v[2] - hi.z) - lo.z) * inv;
-    bx = ((v[3] - hi.x) - lo.x) * inv, by = ((v[4] - hi.y) - lo.y) * inv, bz = ((v[5] - hi.z) - lo.z) * inv;
-    cx = ((v[6] - hi.x) - lo.x) * inv, cy = ((v[7] - hi.y) - lo.y) * inv, cz = ((v[8] - hi.z) - lo.z) * inv;
-    const float ux = bx - ax, uy = by - ay, uz = bz - az, wx = cx - ax, wy = cy - ay, wz = cz - az;
-    const float vx = cx - bx, vy = cy - by, vz = cz - bz;
-    const float nx = uy * wz - uz * wy, ny = uz * wx - ux * wz, nz = ux * wy - uy * wx;
-    const float u2 = ux * ux + uy * uy + uz * uz, w2 = wx * wx + wy * wy + wz * wz, v2 = vx * vx + vy * vy + vz * vz;
-    area2 = 1.02f * __builtin_amdgcn_sqrtf(nx * nx + ny * ny + nz * nz) + 1e-5f * (u2 + w2);
-    edge = 0.58f * __builtin_amdgcn_sqrtf(fmaxf(fmaxf(u2, w2), v2));
-    near2 = fminf(fminf(ax * ax + ay * ay + az * az, bx * bx + by * by + bz * bz), cx * cx + cy * cy + cz * cz);
-  }
-};
-
-// a running product of den + i det with its turns, and the bound on its argument's error
-struct Product {
-  float zr = 1.f, zi = 0.f, err = 0.f;
-  int turns = 0;
-
-  // The factor of a triangle seen from the origin.  slack: how far its corners may be
-  // off, in units of 2^-24, besides their own rounding; rho > 0: it stands for all
-  // points within rho.
-  __device__ __forceinline__ void take(float Ax, float Ay, float Az, float Bx, float By, float Bz, float Cx, float Cy,
-                                       float Cz, float slack, float area2, float edge, float rho) {
-    const float la = __builtin_amdgcn_sqrtf(Ax * Ax + Ay * Ay + Az * Az);
-    const float lb = __builtin_amdgcn_sqrtf(Bx * Bx + By * By + Bz * Bz);
-    const float lc = __builtin_amdgcn_sqrtf(Cx * Cx + Cy * Cy + Cz * Cz);
-    const float det = Ax * (By * Cz - Bz * Cy) - Ay * (Bx * Cz - Bz * Cx) + Az * (Bx * Cy - By * Cx);
-    const float L = la * lb * lc;
-    const float den = L + (Ax * Bx + Ay * By + Az * Bz) * lc + (Bx * Cx + By * Cy + Bz * Cz) * la +
-                      (Cx * Ax + Cy * Ay + Cz * Az) * lb;
-    const float lmin = fminf(fminf(la, lb), lc);
-    const float rz = __builtin_amdgcn_rsqf(det * det + den * den);
-    // Rounding.  A corner is off by at most 2^-24 kappa of its length, kappa = 3 +
-    // slack / lmin; det and den then by (15 kappa + 74) 2^-24 L together, and the
-    // angle by that over |den + i det| (1.5 times for the arc).
-    const float kappa = 3.f + slack * __builtin_amdgcn_rcpf(lmin);
-    const float q = L * rz;  // at least 17^-1/2, unless something under- or overflowed
-    float e = (1.6e-6f * kappa + 7e-6f) * q;
-    // near the branch cut the sign of det, and with it a full turn, is open
-    if (!(q > 0.2f && e < 0.2f) || (den < 0.f && fabsf(det) * rz <= e)) e = 1e30f;
-    e += 1e-6f;  // the product's own rounding
-    if (rho > 0.f) {
-      const float gap = lmin * 0.999f - edge - rho;
-      const float r = __builtin_amdgcn_rcpf(gap);
-      e += gap > 0.05f ? 0.51f * rho * area2 * (r * r * r) : 1e30f;  // of Omega / 2
-    }
-    err += e;
-    const float ur = den * rz, ui = det * rz;
-    const float nr = zr * ur - zi * ui, ni = zr * ui + zi * ur;
-    // past +-pi: both angles on one side of the real axis, their sum on the other
-    turns += (zi >= 0.f && ui >= 0.f && ni < 0.f ? 1 : 0) - (zi < 0.f && ui < 0.f && ni >= 0.f ? 1 : 0);
-    zr = nr;
-    zi = ni;
-  }
-  __device__ __forceinline__ float angle() const { return atan2f(zi, zr) + 6.2831853f * (float)turns; }
-  __device__ __forceinline__ float bound() const { return err + 5e-6f * (1.f + fabsf((float)turns)); }
 };
 
 // The children of side S of the parents (side 2S) in `list` (all parents if it is
