@@ -34,6 +34,9 @@
 namespace {
 
 using lbm3d_winding::blocks_of;
+using lbm3d_winding::child_slack;
+using lbm3d_winding::point_error;
+using lbm3d_winding::point_slack;
 using lbm3d_winding::Product;
 using lbm3d_winding::Seen;
 
@@ -123,7 +126,7 @@ struct VoxGrid {
   double x0, y0, z0, dx;
   int32_t nx, ny, nz;
   int32_t n_tris;
-  float eta;  // rounding of a node's coordinates in FP64 and of a centre's in two FP32, in cells
+  float eta;  // point_error
 };
 
 // The children of side S of the parents (side 2S) in `list` (all parents if it is
@@ -152,18 +155,18 @@ __global__ void __launch_bounds__(256)
     Product child[8], all8;
     constexpr float off = 0.5f * S;                    // a child's centre, per axis
     constexpr float rho = 0.866026f * (S - 1);         // its half diagonal
-    constexpr float reach = 2.f * 1.7320508f * off;    // twice the offset's length
-    constexpr float R = 1.7320508f * off + rho;        // the parent's, from its centre
+    constexpr float R = 1.7320509f * off + rho;        // the parent's, from its centre
+    const float slack = point_slack(gr.eta), near_slack = child_slack(1.7320509f * off, gr.eta);
     // the children's factors of the first `n` triangles from queue[wave][from]
     const auto near = [&](int from, int n) {
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       if (lane < n) {
-        const Seen s(tris, queue[wave][from + lane], hi, lo, inv);
+        const Seen s(tris, queue[wave][from + lane], hi, lo, inv, slack);
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
           const float ox = c & 4 ? off : -off, oy = c & 2 ? off : -off, oz = c & 1 ? off : -off;
           child[c].take(s.ax - ox, s.ay - oy, s.az - oz, s.bx - ox, s.by - oy, s.bz - oz, s.cx - ox, s.cy - oy,
-                        s.cz - oz, reach + 1.7e7f * gr.eta, s.area2, s.edge, rho);
+                        s.cz - oz, near_slack, s.area2, s.edge, rho);
         }
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -173,10 +176,10 @@ __global__ void __launch_bounds__(256)
       const int32_t t = base + lane;
       bool close = false;
       if (t < gr.n_tris) {
-        const Seen s(tris, t, hi, lo, inv);
+        const Seen s(tris, t, hi, lo, inv, slack);
         const float far = kFar * R + s.edge;
         close = !(s.near2 > far * far);  // NaN too
-        if (!close) all8.take(s.ax, s.ay, s.az, s.bx, s.by, s.bz, s.cx, s.cy, s.cz, 1.7e7f * gr.eta, s.area2, s.edge, R);
+        if (!close) all8.take(s.ax, s.ay, s.az, s.bx, s.by, s.bz, s.cx, s.cy, s.cz, slack, s.area2, s.edge, R);
       }
       const uint64_t m = __ballot(close);
       if (close)
@@ -274,10 +277,11 @@ int lbm3d_voxelize_blocks(void *stream, const float *tris, int32_t n_tris, doubl
   // it would leave most nodes open
   if (n_tris > 400000) return lbm3d_voxelize(stream, tris, n_tris, x0, y0, z0, dx, nx, ny, nz, solid);
   VoxGrid gr{x0, y0, z0, dx, nx, ny, nz, n_tris, 0.f};
-  const double far = std::fmax(std::fmax(std::fmax(std::fabs(x0), std::fabs(x0 + dx * nx)),
-                                         std::fmax(std::fabs(y0), std::fabs(y0 + dx * ny))),
-                               std::fmax(std::fabs(z0), std::fabs(z0 + dx * nz)));
-  gr.eta = (float)(5e-15 * far / dx);
+  // a block's centre may lie up to 8 cells past the last node
+  const double far = std::fmax(std::fmax(std::fmax(std::fabs(x0), std::fabs(x0 + dx * (nx + 8.0))),
+                                         std::fmax(std::fabs(y0), std::fabs(y0 + dx * (ny + 8.0)))),
+                               std::fmax(std::fabs(z0), std::fabs(z0 + dx * (nz + 8.0))));
+  gr.eta = point_error(far, dx);
   int32_t *const ws = (int32_t *)workspace;
   int32_t *const list4 = ws + vox_list(nx, ny, nz, 0), *const list2 = ws + vox_list(nx, ny, nz, 1),
                  *const list1 = ws + vox_list(nx, ny, nz, 2);

@@ -10,14 +10,27 @@ namespace lbm3d_winding {
 // how many blocks of side s cover n nodes
 __host__ __device__ __forceinline__ int32_t blocks_of(int32_t n, int32_t s) { return (n + s - 1) / s; }
 
-// A triangle from a point, in cells: its corners, twice its area, a bound on how far it
-// reaches from its nearest corner, that corner's squared distance.
+// Corners.  With u = 2^-24: a triangle's corner c seen from a parent's centre is off by
+// at most u (4 |c| + s0): v - hi, - lo, * inv and inv itself round once each (v - hi is
+// exact where it is not much larger than lo), and s0 = 2^24 eta is the centre's own error.
+// Seen from a child's centre at the offset o it rounds once more, and |c| <= |c - o| + |o|:
+// u (5 |c - o| + 4 |o| + s0).
+constexpr float kCornerRoundings = 5.f;
+__host__ __device__ __forceinline__ float point_slack(float eta) { return 1.7e7f * eta; }  // s0
+__host__ __device__ __forceinline__ float child_slack(float offset, float eta) { return 4.01f * offset + point_slack(eta); }
+
+// Error in cells of a block's centre as two FP32 and of its nodes in FP64, for grid
+// coordinates up to far: 2^-49 of an axis for the second FP32, 4 roundings of 2^-53, and
+// the square root of 3 axes.
+__host__ __device__ __forceinline__ float point_error(double far, double dx) { return (float)(5e-15 * far / dx); }
+
+// A triangle from a point, in cells: its corners; bounds on twice its area and on how far
+// it reaches from its nearest corner (the corners' distances over the square root of 3);
+// that corner's squared distance.  Of an edge of length m seen from the distance D the
+// corners' errors leave u (8 D + 8 m + 2 s0) open, of twice the area u (16 D m + 21 m^2 + 4 s0 m).
 struct Seen {
   float ax, ay, az, bx, by, bz, cx, cy, cz, area2, edge, near2;
-  // from the point hi + lo: v - hi is exact where it is not much larger than lo, so
-  // a coordinate is off by 3 roundings of its own size and by the point's 2^-48 (and
-  // by inv's, which scales all alike)
-  __device__ __forceinline__ Seen(const float *tris, int32_t t, const float3 hi, const float3 lo, float inv) {
+  __device__ __forceinline__ Seen(const float *tris, int32_t t, const float3 hi, const float3 lo, float inv, float s0) {
     const float *v = tris + (int64_t)t * 9;
     ax = ((v[0] - hi.x) - lo.x) * inv, ay = ((v[1] - hi.y) - lo.y) * inv, az = ((v[2] - hi.z) - lo.z) * inv;
     bx = ((v[3] - hi.x) - lo.x) * inv, by = ((v[4] - hi.y) - lo.y) * inv, bz = ((v[5] - hi.z) - lo.z) * inv;
@@ -26,11 +39,19 @@ struct Seen {
     const float vx = cx - bx, vy = cy - by, vz = cz - bz;
     const float nx = uy * wz - uz * wy, ny = uz * wx - ux * wz, nz = ux * wy - uy * wx;
     const float u2 = ux * ux + uy * uy + uz * uz, w2 = wx * wx + wy * wy + wz * wz, v2 = vx * vx + vy * vy + vz * vz;
-    area2 = 1.02f * __builtin_amdgcn_sqrtf(nx * nx + ny * ny + nz * nz) + 1e-5f * (u2 + w2);
-    edge = 0.58f * __builtin_amdgcn_sqrtf(fmaxf(fmaxf(u2, w2), v2));
     near2 = fminf(fminf(ax * ax + ay * ay + az * az, bx * bx + by * by + bz * bz), cx * cx + cy * cy + cz * cz);
+    const float near = __builtin_amdgcn_sqrtf(near2);
+    edge = 0.58f * __builtin_amdgcn_sqrtf(fmaxf(fmaxf(u2, w2), v2)) + (3e-7f * near + 7.5e-8f * s0);
+    area2 = 1.02f * __builtin_amdgcn_sqrtf(nx * nx + ny * ny + nz * nz) + 1e-5f * (u2 + w2) +
+            (1.7e-6f * near + 4.2e-7f * s0) * edge;
   }
 };
+
+// A bound from below on how far points within rho of the origin stay from a triangle:
+// its nearest corner at lmin, off as above with `slack`.
+__device__ __forceinline__ float clear_of(float lmin, float slack, float edge, float rho) {
+  return lmin * 0.999f - 6e-8f * slack - edge - rho;
+}
 
 // a running product of den + i det with its turns, and the bound on its argument's error
 struct Product {
@@ -38,8 +59,8 @@ struct Product {
   int turns = 0;
 
   // The factor of a triangle seen from the origin.  slack: how far its corners may be
-  // off, in units of 2^-24, besides their own rounding; rho > 0: it stands for all
-  // points within rho.
+  // off, in units of 2^-24, besides kCornerRoundings of their lengths; rho > 0: it
+  // stands for all points within rho.
   __device__ __forceinline__ void take(float Ax, float Ay, float Az, float Bx, float By, float Bz, float Cx, float Cy,
                                        float Cz, float slack, float area2, float edge, float rho) {
     const float la = __builtin_amdgcn_sqrtf(Ax * Ax + Ay * Ay + Az * Az);
@@ -51,17 +72,18 @@ struct Product {
                       (Cx * Ax + Cy * Ay + Cz * Az) * lb;
     const float lmin = fminf(fminf(la, lb), lc);
     const float rz = __builtin_amdgcn_rsqf(det * det + den * den);
-    // Rounding.  A corner is off by at most 2^-24 kappa of its length, kappa = 3 +
-    // slack / lmin; det and den then by (15 kappa + 74) 2^-24 L together, and the
-    // angle by that over |den + i det| (1.5 times for the arc).
-    const float kappa = 3.f + slack * __builtin_amdgcn_rcpf(lmin);
+    // Rounding.  A corner is off by at most 2^-24 kappa of its length, kappa =
+    // kCornerRoundings + slack / lmin; det then by 3 kappa and den by 12 kappa of 2^-24 L,
+    // their own roundings add less than 74, and the angle is off by the sum over
+    // |den + i det| (1.5 times for the arc).
+    const float kappa = kCornerRoundings + slack * __builtin_amdgcn_rcpf(lmin);
     const float q = L * rz;  // at least 17^-1/2, unless something under- or overflowed
     float e = (1.6e-6f * kappa + 7e-6f) * q;
     // near the branch cut the sign of det, and with it a full turn, is open
     if (!(q > 0.2f && e < 0.2f) || (den < 0.f && fabsf(det) * rz <= e)) e = 1e30f;
     e += 1e-6f;  // the product's own rounding
     if (rho > 0.f) {
-      const float gap = lmin * 0.999f - edge - rho;
+      const float gap = clear_of(lmin, slack, edge, rho);
       const float r = __builtin_amdgcn_rcpf(gap);
       e += gap > 0.05f ? 0.51f * rho * area2 * (r * r * r) : 1e30f;  // of Omega / 2
     }

@@ -41,6 +41,20 @@ void product(const float *t, int n, float slack, float *out) {
   out[0] = p.angle();
   out[1] = p.bound();
 }
+// a triangle seen from the point hi + lo of p: 9 corners, area2, edge, near2; then its
+// corners from the offset o, the bound on a corner's error at length 0 and per length
+void seen(const float *t, const double *p, double dx, float eta, float o, float *out) {
+  const float3 hi{(float)p[0], (float)p[1], (float)p[2]};
+  const float3 lo{(float)(p[0] - (double)hi.x), (float)(p[1] - (double)hi.y), (float)(p[2] - (double)hi.z)};
+  const Seen s(t, 0, hi, lo, (float)(1.0 / dx), point_slack(eta));
+  const float f[12] = {s.ax, s.ay, s.az, s.bx, s.by, s.bz, s.cx, s.cy, s.cz, s.area2, s.edge, s.near2};
+  for (int k = 0; k < 12; ++k) out[k] = f[k];
+  for (int k = 0; k < 9; ++k) out[12 + k] = f[k] - o;
+  out[21] = child_slack(1.7320509f * o, eta);
+  out[22] = kCornerRoundings;
+}
+float error_of_point(double far, double dx) { return point_error(far, dx); }
+float clear(float lmin, float slack, float edge, float rho) { return clear_of(lmin, slack, edge, rho); }
 }
 """
 
@@ -52,7 +66,9 @@ def winding(tmp_path_factory):
     src.write_text(DRIVER)
     subprocess.run(["g++", "-O1", "-std=c++17", "-ffp-contract=off", "-shared", "-fPIC", "-I", CSRC, "-o", str(so),
                     str(src)], check=True, capture_output=True, text=True)
-    return ctypes.CDLL(str(so))
+    lib = ctypes.CDLL(str(so))
+    lib.error_of_point.restype = lib.clear.restype = ctypes.c_float
+    return lib
 
 
 def product(lib, corners, slack=0.0):
@@ -114,3 +130,54 @@ def test_products_stay_within_their_bound(winding, ulps):
                 assert abs(float(half_angles(tris).sum()) - got) <= bound
     winding.set_ulps(0)
     assert settled > 500
+
+
+def triangles(rng, n, dx, p):
+    """Triangles of many shapes around p: general, small and far, slivers."""
+    size = np.exp(rng.uniform(-7, 4, (n, 1, 1))) * dx
+    t = rng.normal(size=(n, 3, 3)) * size
+    thin = rng.random(n) < 0.4
+    t[thin, 2] = t[thin, 0] + rng.random((thin.sum(), 1)) * (t[thin, 1] - t[thin, 0]) + 1e-2 * (t[thin, 2] - t[thin, 0])
+    return (t + rng.normal(size=(n, 1, 3)) * np.exp(rng.uniform(-2, 6, (n, 1, 1))) * dx + p).astype(np.float32)
+
+
+@pytest.mark.parametrize("dx", [1.0, 0.3, 7e-4])
+@pytest.mark.parametrize("offset", [0.5, 2.0])
+@pytest.mark.parametrize("origin", [0.0, 20.0, 1e6])
+def test_corners_areas_and_reaches_within_their_bounds(winding, dx, offset, origin):
+    rng = np.random.default_rng(5)
+    wide = lambda a: np.asarray(a, np.longdouble)
+    length = lambda v: np.sqrt((v * v).sum(-1))
+    out = np.zeros(23, np.float32)
+    for t in triangles(rng, 3000, dx, origin * dx):
+        p = (origin + rng.uniform(-1, 1, 3) * rng.choice([1.0, 30.0])) * dx  # a block's centre
+        far = np.abs(p).max()
+        eta = winding.error_of_point(ctypes.c_double(far), ctypes.c_double(dx))
+        winding.seen(t.ctypes.data_as(ctypes.c_void_p), p.ctypes.data_as(ctypes.c_void_p), ctypes.c_double(dx),
+                     ctypes.c_float(eta), ctypes.c_float(offset), out.ctypes.data_as(ctypes.c_void_p))
+        exact = (wide(t) - wide(p)) / wide(dx)
+        child = exact - offset
+        err = length(wide(out[12:21].reshape(3, 3)) - child)
+        assert (err <= 2.0 ** -24 * (out[22] * length(child) + out[21]) * (1 + 1e-5)).all()
+        u, w = exact[1] - exact[0], exact[2] - exact[0]
+        assert out[9] >= length(np.cross(u, w))
+        longest = max(length(u), length(w), length(u - w))
+        assert out[10] >= longest / math.sqrt(3)
+        lmin = np.float32(length(out[12:21].reshape(3, 3)).min())
+        assert winding.clear(ctypes.c_float(lmin), ctypes.c_float(out[21]), ctypes.c_float(out[10]), ctypes.c_float(0.0)) \
+            <= length(child).min() - longest / math.sqrt(3) + 1e-6
+
+
+def test_a_point_far_from_the_origin_is_off_by_no_more_than_stated(winding):
+    """Coordinates whose second FP32 rounds as much as it can, on all three axes."""
+    rng = np.random.default_rng(2)
+    for far in (1e3, 2.0 ** 20, 3e7):
+        worst = 0.0
+        for _ in range(20000):
+            p = far * (1 + rng.random(3) * 2.0 ** -10)
+            hi = p.astype(np.float32)
+            lo = (p - hi.astype(np.float64)).astype(np.float32)
+            off = p.astype(np.longdouble) - hi.astype(np.longdouble) - lo.astype(np.longdouble)
+            worst = max(worst, float(np.sqrt((off * off).sum())))
+        roundings = 4 * 2.0 ** -53 * math.sqrt(3) * far
+        assert worst + roundings <= winding.error_of_point(ctypes.c_double(far * (1 + 2.0 ** -10)), ctypes.c_double(1.0))
