@@ -144,8 +144,8 @@ __global__ void __launch_bounds__(256)
   const int32_t pny = blocks_of(gr.ny, 2 * S), pnz = blocks_of(gr.nz, 2 * S);
   const int32_t cnx = blocks_of(gr.nx, S), cny = blocks_of(gr.ny, S), cnz = blocks_of(gr.nz, S);
   const float inv = (float)(1.0 / gr.dx);
-  for (int32_t it = (int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6)); it < n; it += waves) {
-    const int32_t id = __builtin_amdgcn_readfirstlane(list ? list[it] : it);
+  for (int64_t it = blockIdx.x * 4 + (threadIdx.x >> 6); it < n; it += waves) {  // n may be near 2^31
+    const int32_t id = __builtin_amdgcn_readfirstlane(list ? list[it] : (int32_t)it);
     const int32_t bk = id % pnz, bt = id / pnz, bj = bt % pny, bi = bt / pny;
     // the parent's reference point, and its children's centres relative to it, in cells
     const double pi = 2 * S * bi + S - 0.5, pj = 2 * S * bj + S - 0.5, pk = 2 * S * bk + S - 0.5;
@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(256)
                     const int32_t *__restrict__ count, int8_t *__restrict__ solid) {
   const int lane = threadIdx.x & 63;
   const int32_t n = *count, waves = (int32_t)(gridDim.x * 4);
-  for (int32_t it = (int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6)); it < n; it += waves) {
+  for (int64_t it = blockIdx.x * 4 + (threadIdx.x >> 6); it < n; it += waves) {  // n may be near 2^31
     const int32_t id = __builtin_amdgcn_readfirstlane(list[it]);
     const int32_t k = id % gr.nz, t0 = id / gr.nz, j = t0 % gr.ny, i = t0 / gr.ny;
     const double px = gr.x0 + gr.dx * (double)i, py = gr.y0 + gr.dx * (double)j, pz = gr.z0 + gr.dx * (double)k;

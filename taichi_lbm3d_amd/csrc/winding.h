@@ -7,8 +7,8 @@
 
 namespace lbm3d_winding {
 
-// how many blocks of side s cover n nodes
-__host__ __device__ __forceinline__ int32_t blocks_of(int32_t n, int32_t s) { return (n + s - 1) / s; }
+// how many blocks of side s cover n nodes (n >= 1; n + s may pass 2^31)
+__host__ __device__ __forceinline__ int32_t blocks_of(int32_t n, int32_t s) { return (n - 1) / s + 1; }
 
 // Corners.  With u = 2^-24: a triangle's corner c seen from a parent's centre is off by
 // at most u (4 |c| + s0): v - hi, - lo, * inv and inv itself round once each (v - hi is

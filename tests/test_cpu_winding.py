@@ -53,6 +53,7 @@ void seen(const float *t, const double *p, double dx, float eta, float o, float 
   out[21] = child_slack(1.7320509f * o, eta);
   out[22] = kCornerRoundings;
 }
+int blocks(int n, int s) { return blocks_of(n, s); }
 float error_of_point(double far, double dx) { return point_error(far, dx); }
 float clear(float lmin, float slack, float edge, float rho) { return clear_of(lmin, slack, edge, rho); }
 }
@@ -181,3 +182,9 @@ def test_a_point_far_from_the_origin_is_off_by_no_more_than_stated(winding):
             worst = max(worst, float(np.sqrt((off * off).sum())))
         roundings = 4 * 2.0 ** -53 * math.sqrt(3) * far
         assert worst + roundings <= winding.error_of_point(ctypes.c_double(far * (1 + 2.0 ** -10)), ctypes.c_double(1.0))
+
+
+def test_blocks_cover_every_extent_up_to_the_largest(winding):
+    for n in (1, 2, 7, 8, 9, 1000, 2 ** 31 - 8, 2 ** 31 - 1):
+        for s in (2, 4, 8):
+            assert winding.blocks(n, s) == -(-n // s)
