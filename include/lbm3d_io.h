@@ -35,7 +35,8 @@ int lbm3d_voxelize(void *stream, const float *tris, int32_t n_tris, double x0, d
 
 /* The same flags, faster: blocks of nodes away from the surface are decided by
  * one bounded sum at their centre, and only nodes that a bounded FP32 sum leaves
- * open take lbm3d_voxelize's FP64 sum.  `workspace`: DEVICE,
+ * open take lbm3d_voxelize's FP64 sum.  Small meshes and those that blocks decide
+ * little of go to lbm3d_voxelize's kernel.  `workspace`: DEVICE,
  * lbm3d_voxelize_workspace_bytes(nx, ny, nz) bytes. */
 size_t lbm3d_voxelize_workspace_bytes(int32_t nx, int32_t ny, int32_t nz);
 int lbm3d_voxelize_blocks(void *stream, const float *tris, int32_t n_tris, double x0, double y0, double z0, double dx,

@@ -17,30 +17,42 @@ __host__ __device__ __forceinline__ int32_t blocks_of(int32_t n, int32_t s) { re
 // u (5 |c - o| + 4 |o| + s0).
 constexpr float kCornerRoundings = 5.f;
 __host__ __device__ __forceinline__ float point_slack(float eta) { return 1.7e7f * eta; }  // s0
-__host__ __device__ __forceinline__ float child_slack(float offset, float eta) { return 4.01f * offset + point_slack(eta); }
+__host__ __device__ __forceinline__ float child_slack(float offset, float eta) {
+  return 4.01f * offset + point_slack(eta);
+}
 
 // Error in cells of a block's centre as two FP32 and of its nodes in FP64, for grid
 // coordinates up to far: 2^-49 of an axis for the second FP32, 4 roundings of 2^-53, and
 // the square root of 3 axes.
 __host__ __device__ __forceinline__ float point_error(double far, double dx) { return (float)(5e-15 * far / dx); }
 
-// A triangle from a point, in cells: its corners; bounds on twice its area and on how far
-// it reaches from its nearest corner (the corners' distances over the square root of 3);
-// that corner's squared distance.  Of an edge of length m seen from the distance D the
-// corners' errors leave u (8 D + 8 m + 2 s0) open, of twice the area u (16 D m + 21 m^2 + 4 s0 m).
-struct Seen {
-  float ax, ay, az, bx, by, bz, cx, cy, cz, area2, edge, near2;
-  __device__ __forceinline__ Seen(const float *tris, int32_t t, const float3 hi, const float3 lo, float inv, float s0) {
+// A triangle's corners from a point, in cells.
+struct Corners {
+  float ax, ay, az, bx, by, bz, cx, cy, cz;
+  __device__ __forceinline__ Corners(const float *tris, int32_t t, const float3 hi, const float3 lo, float inv) {
     const float *v = tris + (int64_t)t * 9;
     ax = ((v[0] - hi.x) - lo.x) * inv, ay = ((v[1] - hi.y) - lo.y) * inv, az = ((v[2] - hi.z) - lo.z) * inv;
     bx = ((v[3] - hi.x) - lo.x) * inv, by = ((v[4] - hi.y) - lo.y) * inv, bz = ((v[5] - hi.z) - lo.z) * inv;
     cx = ((v[6] - hi.x) - lo.x) * inv, cy = ((v[7] - hi.y) - lo.y) * inv, cz = ((v[8] - hi.z) - lo.z) * inv;
+  }
+};
+
+// The same with bounds on twice its area and on how far it reaches from its nearest corner
+// (the longest edge over the square root of 3), and that corner's distance.  Of an edge of
+// length m seen from the distance D the corners' errors leave u (8 D + 8 m + 2 s0) open, of
+// twice the area u (16 D m + 21 m^2 + 4 s0 m).
+struct Seen : Corners {
+  float area2, edge, near;
+  __device__ __forceinline__ Seen(const float *tris, int32_t t, const float3 hi, const float3 lo, float inv, float s0)
+      : Corners(tris, t, hi, lo, inv) {
     const float ux = bx - ax, uy = by - ay, uz = bz - az, wx = cx - ax, wy = cy - ay, wz = cz - az;
     const float vx = cx - bx, vy = cy - by, vz = cz - bz;
     const float nx = uy * wz - uz * wy, ny = uz * wx - ux * wz, nz = ux * wy - uy * wx;
     const float u2 = ux * ux + uy * uy + uz * uz, w2 = wx * wx + wy * wy + wz * wz, v2 = vx * vx + vy * vy + vz * vz;
-    near2 = fminf(fminf(ax * ax + ay * ay + az * az, bx * bx + by * by + bz * bz), cx * cx + cy * cy + cz * cz);
-    const float near = __builtin_amdgcn_sqrtf(near2);
+    // the lengths that Product::take forms too
+    near = fminf(fminf(__builtin_amdgcn_sqrtf(ax * ax + ay * ay + az * az),
+                       __builtin_amdgcn_sqrtf(bx * bx + by * by + bz * bz)),
+                 __builtin_amdgcn_sqrtf(cx * cx + cy * cy + cz * cz));
     edge = 0.58f * __builtin_amdgcn_sqrtf(fmaxf(fmaxf(u2, w2), v2)) + (3e-7f * near + 7.5e-8f * s0);
     area2 = 1.02f * __builtin_amdgcn_sqrtf(nx * nx + ny * ny + nz * nz) + 1e-5f * (u2 + w2) +
             (1.7e-6f * near + 4.2e-7f * s0) * edge;

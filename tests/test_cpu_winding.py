@@ -37,17 +37,18 @@ void set_ulps(int n) { ulps = n; }
 // the product of n triangles (corners from the point, in cells): argument and its bound
 void product(const float *t, int n, float slack, float *out) {
   Product p;
-  for (int i = 0; i < n; ++i, t += 9) p.take(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], slack, 0.f, 0.f, 0.f);
+  for (int i = 0; i < n; ++i, t += 9)
+    p.take(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], slack, 0.f, 0.f, 0.f);
   out[0] = p.angle();
   out[1] = p.bound();
 }
-// a triangle seen from the point hi + lo of p: 9 corners, area2, edge, near2; then its
+// a triangle seen from the point hi + lo of p: 9 corners, area2, edge, near; then its
 // corners from the offset o, the bound on a corner's error at length 0 and per length
 void seen(const float *t, const double *p, double dx, float eta, float o, float *out) {
   const float3 hi{(float)p[0], (float)p[1], (float)p[2]};
   const float3 lo{(float)(p[0] - (double)hi.x), (float)(p[1] - (double)hi.y), (float)(p[2] - (double)hi.z)};
   const Seen s(t, 0, hi, lo, (float)(1.0 / dx), point_slack(eta));
-  const float f[12] = {s.ax, s.ay, s.az, s.bx, s.by, s.bz, s.cx, s.cy, s.cz, s.area2, s.edge, s.near2};
+  const float f[12] = {s.ax, s.ay, s.az, s.bx, s.by, s.bz, s.cx, s.cy, s.cz, s.area2, s.edge, s.near};
   for (int k = 0; k < 12; ++k) out[k] = f[k];
   for (int k = 0; k < 9; ++k) out[12 + k] = f[k] - o;
   out[21] = child_slack(1.7320509f * o, eta);
@@ -164,9 +165,9 @@ def test_corners_areas_and_reaches_within_their_bounds(winding, dx, offset, orig
         assert out[9] >= length(np.cross(u, w))
         longest = max(length(u), length(w), length(u - w))
         assert out[10] >= longest / math.sqrt(3)
-        lmin = np.float32(length(out[12:21].reshape(3, 3)).min())
-        assert winding.clear(ctypes.c_float(lmin), ctypes.c_float(out[21]), ctypes.c_float(out[10]), ctypes.c_float(0.0)) \
-            <= length(child).min() - longest / math.sqrt(3) + 1e-6
+        lmin = length(out[12:21].reshape(3, 3)).min()
+        gap = winding.clear(*(ctypes.c_float(float(v)) for v in (lmin, out[21], out[10], 0.0)))
+        assert gap <= length(child).min() - longest / math.sqrt(3) + 1e-6
 
 
 def test_a_point_far_from_the_origin_is_off_by_no_more_than_stated(winding):
@@ -181,7 +182,8 @@ def test_a_point_far_from_the_origin_is_off_by_no_more_than_stated(winding):
             off = p.astype(np.longdouble) - hi.astype(np.longdouble) - lo.astype(np.longdouble)
             worst = max(worst, float(np.sqrt((off * off).sum())))
         roundings = 4 * 2.0 ** -53 * math.sqrt(3) * far
-        assert worst + roundings <= winding.error_of_point(ctypes.c_double(far * (1 + 2.0 ** -10)), ctypes.c_double(1.0))
+        bound = winding.error_of_point(ctypes.c_double(far * (1 + 2.0 ** -10)), ctypes.c_double(1.0))
+        assert worst + roundings <= bound
 
 
 def test_blocks_cover_every_extent_up_to_the_largest(winding):
