@@ -206,7 +206,7 @@ def _make_conv_functions():
     torch = _torch()
 
     def packed(w, flip, given):  # given: the layer's fragments from pack_layers, or None
-        if given is not None:
+        if given is not None and (not flip or given[1] is not None):
             return given[0], given[1] if flip else None
         w = w if w.dtype == torch.float32 else w.to(torch.bfloat16).float()
         return pack_weights(w.contiguous(), flip)
