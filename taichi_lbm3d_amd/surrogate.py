@@ -202,6 +202,25 @@ def _bf16(t):
     return t.contiguous().to(_torch().bfloat16)
 
 
+def _check_layer(x, cin, w, b, ks, given=None):
+    """The kernels take a layer's shapes from x: its weights have to be of them, or they are read past their end."""
+    k = ks ** 3 * cin
+    kpad = (k + 31) // 32 * 32  # lbm3d_conv_kpad
+    if w.dim() != 2 or w.shape[1] != kpad:
+        raise ValueError(f"a layer of {cin} input channels takes weights (cout, {kpad}), got {tuple(w.shape)}")
+    if b is not None and b.numel() < w.shape[0]:
+        raise ValueError(f"{w.shape[0]} output channels take as many biases, got {b.numel()}")
+    if w.device != x.device or (b is not None and b.device != x.device):
+        raise ValueError(f"weights and biases have to be on the input's device {x.device}")
+    if given is not None and given[0].numel() != 28 * cin * w.shape[0]:
+        raise ValueError(f"the packed weights are not those of a layer {cin} -> {w.shape[0]}")
+
+
+def _check_volume(x, what):
+    if x.dim() != 5 or x.dtype != _torch().bfloat16:
+        raise ValueError(f"{what} has to be (N, X, Y, Z, C) bfloat16, got {tuple(x.shape)} {x.dtype}")
+
+
 def _make_conv_functions():
     torch = _torch()
 
@@ -217,6 +236,7 @@ def _make_conv_functions():
         @staticmethod
         def forward(ctx, x, w, b, ks, relu, need_dx, periodic, given):
             x = x.contiguous()
+            _check_layer(x, x.shape[-1], w, b, ks, given if ks == 3 else None)
             if ks == 3:
                 wp, wb = packed(w, need_dx and ctx.needs_input_grad[0], given)
                 y = conv_fwd_packed(x, wp, b, w.shape[0], relu, periodic)
@@ -245,6 +265,8 @@ def _make_conv_functions():
 
         @staticmethod
         def forward(ctx, x, w, b, periodic, given):
+            _check_volume(x, "the input")
+            _check_layer(x, x.shape[-1], w, b, 3, given)
             x = x.contiguous()
             n, d, h, wd, cin = x.shape
             cout = w.shape[0]
@@ -272,6 +294,14 @@ def _make_conv_functions():
 
         @staticmethod
         def forward(ctx, low, skip, w, b, periodic, given):
+            _check_volume(low, "the low part")
+            _check_volume(skip, "the skip part")
+            if low.shape[0] != skip.shape[0] or any(a != e // 2 for a, e in zip(low.shape[1:4], skip.shape[1:4])):
+                raise ValueError(f"the low part {tuple(low.shape)} does not fit the skip part {tuple(skip.shape)}: "
+                                 "as many volumes of half the extents")
+            if low.device != skip.device:
+                raise ValueError(f"the parts are on {low.device} and {skip.device}")
+            _check_layer(skip, low.shape[-1] + skip.shape[-1], w, b, 3, given)
             low, skip = low.contiguous(), skip.contiguous()
             n, d, h, wd, c_skip = skip.shape
             cout = w.shape[0]
@@ -310,6 +340,10 @@ def _make_conv_functions():
 
         @staticmethod
         def forward(ctx, x, w, b):
+            if x.dtype != torch.bfloat16 or w.shape[0] != HEAD_PAD:
+                raise ValueError(f"the head takes bfloat16 and {HEAD_PAD} rows of weights, got {x.dtype}, "
+                                 f"{tuple(w.shape)}")
+            _check_layer(x, x.shape[-1], w, b, 1)
             x = x.contiguous()
             wb = w.to(torch.bfloat16).contiguous()
             ctx.save_for_backward(x, wb)
