@@ -175,8 +175,10 @@ def head_fwd(x, w_bf16, bias):
 
 def head_fields(x, w_bf16, bias, solid, origin, scale_v, scale_rho, rho_one):
     """(rho, v) of the box at `origin`, of `solid`'s shape, from one volume x
-    (X, Y, Z, C) of the last layer's output (lbm3d_conv_head_fields)."""
+    (X, Y, Z, C) of the last layer's output (lbm3d_conv_head_fields).  solid is any
+    mask, nonzero = solid."""
     torch = _torch()
+    x, solid = x.contiguous(), _solid_bytes(solid, x.device, "head_fields")
     rho = torch.empty(solid.shape, dtype=torch.float32, device=x.device)
     v = torch.empty(tuple(solid.shape) + (3,), dtype=torch.float32, device=x.device)
     box = [(_lib.ctypes.c_int32 * 3)(*t) for t in (x.shape[:3], origin, solid.shape)]
