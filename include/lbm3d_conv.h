@@ -19,6 +19,7 @@
  * Convolutions are "same" (stride 1, zero padding ks/2, or periodic wrap for
  * the forward convolution with LBM3D_CONV_PERIODIC).  cin and cout must
  * be multiples of 16, at most 256; a batch holds fewer than 2^31 voxels.
+ * Activations and BF16 weights start on 16 bytes.
  * Return 0 or a negative LBM3D_E* code (lbm3d.h); lbm3d_conv_last_error()
  * gives the message.
  */

@@ -1218,6 +1218,13 @@ int check_conv(int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin, int32_t
   return LBM3D_OK;
 }
 
+// Kernels that load 16-byte pieces straight to LDS, or through buffer resources, take
+// tensors that start on 16 bytes.
+int check_start(const void *a, const void *b = nullptr, const void *c = nullptr) {
+  if (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) return cfail(LBM3D_EINVAL, "tensors must start on 16 bytes");
+  return LBM3D_OK;
+}
+
 constexpr int kWgTargetBlocks = 2048;
 
 // Weight gradient: bricks per set of partial sums and sets, about kWgTargetBlocks
@@ -1734,7 +1741,10 @@ int lbm3d_conv3d_fwd(void *stream, const uint16_t *x, const uint16_t *w, const f
   const Vol vol = make_vol(n, d, h, wd, (flags & LBM3D_CONV_PERIODIC) ? 1 : 0);
   const int kpad = lbm3d_conv_kpad(cin, ks);
   hipStream_t s = (hipStream_t)stream;
-  if (ks == 3) return launch_conv3<kPlain>(s, ConvCall{x, w, 0, bias, y, vol, cin, cout, kpad, relu, ConvExtra{}});
+  if (ks == 3) {
+    if ((rc = check_start(x, w))) return rc;
+    return launch_conv3<kPlain>(s, ConvCall{x, w, 0, bias, y, vol, cin, cout, kpad, relu, ConvExtra{}});
+  }
   const unsigned gx = (vol.vox + 255u) / 256u;
   if (cout % 64 == 0)
     k_conv1<4><<<dim3(gx, cout / 64), 256, 0, s>>>(x, w, bias, y, vol.vox, cin, cout, kpad, relu);
@@ -1780,6 +1790,7 @@ static int packed_call(const uint16_t *x, const uint16_t *wp, const float *bias,
   int rc = check_conv(n, d, h, wd, cin, cout, 3);
   if (rc) return rc;
   if (!x || !wp || !y) return cfail(LBM3D_EINVAL, "NULL tensor");
+  if ((rc = check_start(x))) return rc;
   if (flags & ~(LBM3D_CONV_RELU | LBM3D_CONV_PERIODIC)) return cfail(LBM3D_EINVAL, "unknown flag bits");
   a = ConvCall{x,   wp,   1, bias, y, make_vol(n, d, h, wd, (flags & LBM3D_CONV_PERIODIC) ? 1 : 0), cin, cout,
                lbm3d_conv_kpad(cin, 3), (flags & LBM3D_CONV_RELU) ? 1 : 0, ConvExtra{}};
@@ -1813,6 +1824,7 @@ int lbm3d_conv3d_fwd_up(void *stream, const uint16_t *low, const uint16_t *skip,
   ConvCall a;
   if (int rc = packed_call(skip, wp, bias, y, n, d, h, wd, c_low + c_skip, cout, flags, a)) return rc;
   if (!low) return cfail(LBM3D_EINVAL, "NULL tensor");
+  if (int rc = check_start(low)) return rc;
   if ((d | h | wd) & 1) return cfail(LBM3D_EINVAL, "upsampling needs even extents");
   a.ex.low = low;
   a.ex.c_low = c_low;
@@ -1865,6 +1877,7 @@ static int wgrad_run(void *stream, const uint16_t *x, const uint16_t *dy, float 
   int rc = check_conv(n, d, h, wd, cin, cout, ks);
   if (rc) return rc;
   if (!x || !dy || !dw || !workspace || (c_low > 0 && !low)) return cfail(LBM3D_EINVAL, "NULL tensor or workspace");
+  if ((rc = check_start(x, dy, low))) return rc;
   if (workspace_bytes < lbm3d_conv3d_wgrad_workspace_bytes(n, d, h, wd, cin, cout, ks))
     return cfail(LBM3D_EINVAL, "wgrad workspace too small");
   const Vol vol = make_vol(n, d, h, wd);

@@ -45,6 +45,12 @@ def _stream(dev):
     return _lib.raw_stream(_torch().cuda.current_device() if dev.index is None else dev.index)
 
 
+def _operand(t):
+    """t contiguous and starting on 16 bytes, as the kernels that load straight to LDS read it."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 # ---- the convolution as an autograd function ----------------------------------------------
 
 CONV_RELU, CONV_PERIODIC = 1, 2  # lbm3d_conv3d_fwd flags
@@ -56,6 +62,7 @@ def conv_fwd(x, w_bf16, bias, cout, ks, relu, periodic=False):
     reading zero padding)."""
     torch = _torch()
     n, d, h, wd, cin = x.shape
+    x, w_bf16 = _operand(x), _operand(w_bf16)
     y = torch.empty((n, d, h, wd, cout), dtype=torch.bfloat16, device=x.device)
     flags = (CONV_RELU if relu else 0) | (CONV_PERIODIC if periodic else 0)
     _lib.lib().call("lbm3d_conv3d_fwd", _stream(x.device), _vp(x), _vp(w_bf16),
@@ -65,6 +72,7 @@ def conv_fwd(x, w_bf16, bias, cout, ks, relu, periodic=False):
 
 def conv_dgrad(dy, w_bf16, cin, ks):
     torch = _torch()
+    dy = _operand(dy)
     n, d, h, wd, cout = dy.shape
     lib = _lib.lib()
     kpad_t = lib.cdll.lbm3d_conv_kpad(cout, ks)
@@ -107,6 +115,7 @@ def conv_fwd_packed(x, wp, bias, cout, relu, periodic=False):
     """conv_fwd with ks = 3 and the fragments of pack_weights."""
     torch = _torch()
     n, d, h, wd, cin = x.shape
+    x = _operand(x)
     y = torch.empty((n, d, h, wd, cout), dtype=torch.bfloat16, device=x.device)
     flags = (CONV_RELU if relu else 0) | (CONV_PERIODIC if periodic else 0)
     _lib.lib().call("lbm3d_conv3d_fwd_packed", _stream(x.device), _vp(x), _vp(wp),
@@ -116,6 +125,7 @@ def conv_fwd_packed(x, wp, bias, cout, relu, periodic=False):
 
 def conv_wgrad(x, dy, ks):
     torch = _torch()
+    x, dy = _operand(x), _operand(dy)
     n, d, h, wd, cin = x.shape
     cout = dy.shape[-1]
     lib = _lib.lib()
@@ -237,8 +247,8 @@ def _make_conv_functions():
 
         @staticmethod
         def forward(ctx, x, w, b, ks, relu, need_dx, periodic, given):
-            x = x.contiguous()
             _check_layer(x, x.shape[-1], w, b, ks, given if ks == 3 else None)
+            x = _operand(x)
             if ks == 3:
                 wp, wb = packed(w, need_dx and ctx.needs_input_grad[0], given)
                 y = conv_fwd_packed(x, wp, b, w.shape[0], relu, periodic)
@@ -269,7 +279,7 @@ def _make_conv_functions():
         def forward(ctx, x, w, b, periodic, given):
             _check_volume(x, "the input")
             _check_layer(x, x.shape[-1], w, b, 3, given)
-            x = x.contiguous()
+            x = _operand(x)
             n, d, h, wd, cin = x.shape
             cout = w.shape[0]
             wp, wt = packed(w, ctx.needs_input_grad[0], given)
@@ -304,7 +314,7 @@ def _make_conv_functions():
             if low.device != skip.device:
                 raise ValueError(f"the parts are on {low.device} and {skip.device}")
             _check_layer(skip, low.shape[-1] + skip.shape[-1], w, b, 3, given)
-            low, skip = low.contiguous(), skip.contiguous()
+            low, skip = _operand(low), _operand(skip)
             n, d, h, wd, c_skip = skip.shape
             cout = w.shape[0]
             wp, wt = packed(w, ctx.needs_input_grad[0] or ctx.needs_input_grad[1], given)
@@ -346,7 +356,7 @@ def _make_conv_functions():
                 raise ValueError(f"the head takes bfloat16 and {HEAD_PAD} rows of weights, got {x.dtype}, "
                                  f"{tuple(w.shape)}")
             _check_layer(x, x.shape[-1], w, b, 1)
-            x = x.contiguous()
+            x = _operand(x)
             wb = w.to(torch.bfloat16).contiguous()
             ctx.save_for_backward(x, wb)
             return head_fwd(x, wb, b)
