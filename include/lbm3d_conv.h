@@ -56,6 +56,8 @@ int lbm3d_conv3d_fwd(void *stream, const uint16_t *x, const uint16_t *w, const f
  * from cout to cin channels). */
 int64_t lbm3d_conv3d_packed_elements(int32_t cin, int32_t cout);
 int lbm3d_conv3d_wpack(void *stream, const float *w, uint16_t *wp, uint16_t *wt, int32_t cin, int32_t cout);
+/* The same from BF16 weights. */
+int lbm3d_conv3d_wpack_bf16(void *stream, const uint16_t *w, uint16_t *wp, uint16_t *wt, int32_t cin, int32_t cout);
 /* Several layers' weights in one go (`layers` is host memory, read during the call). */
 typedef struct lbm3d_conv_pack {
   const float *w;

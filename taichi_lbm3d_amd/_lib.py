@@ -148,6 +148,7 @@ SIGNATURES = {
     "lbm3d_conv3d_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_conv3d_packed_elements": (_i64, [_i32, _i32]),
     "lbm3d_conv3d_wpack": (_int, [_vp, _vp, _vp, _vp, _i32, _i32]),
+    "lbm3d_conv3d_wpack_bf16": (_int, [_vp, _vp, _vp, _vp, _i32, _i32]),
     "lbm3d_conv3d_wpack_many": (_int, [_vp, _i32, ctypes.POINTER(ConvPack)]),
     "lbm3d_conv3d_fwd_packed": (_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "lbm3d_conv3d_fwd_pool": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),

@@ -840,11 +840,11 @@ __global__ void k_wflip(const uint16_t *__restrict__ w, uint16_t *__restrict__ w
 // flipped weights of the data gradient (k_wflip's) in the same order.  One
 // thread per lane of a fragment; the 28th tap slot is zero.  A launch takes up to
 // kPackItems layers: one is 4 to 6 us of latency, so the network's 14 layers take
-// 9 us together and 66 one by one.
+// 9 us together and 66 one by one.  W: float, or the bits of BF16 weights.
 constexpr int kPackItems = 16;
 
 struct PackItem {
-  const float *w;
+  const void *w;
   uint16_t *wp, *wt;
   int32_t cin, cout, kpad;
   uint32_t first;  // block
@@ -854,11 +854,15 @@ struct PackList {
   PackItem item[kPackItems];
 };
 
+__device__ __forceinline__ uint32_t bf16_bits(float f) { return to_bf16(f); }
+__device__ __forceinline__ uint32_t bf16_bits(uint16_t h) { return h; }
+
+template <typename W>
 __global__ void __launch_bounds__(256) k_wpack(const PackList list) {
   int k = 0;
   while (k + 1 < list.n && blockIdx.x >= list.item[k + 1].first) ++k;  // uniform
   const PackItem &it = list.item[k];
-  const float *const w = it.w;
+  const W *const w = static_cast<const W *>(it.w);
   const int cin = it.cin, cout = it.cout, kpad = it.kpad;
   const int frags = kSteps * (cin / 16) * (cout / 16);  // the same for both
   int i = (int)((blockIdx.x - it.first) * 256 + threadIdx.x);
@@ -873,12 +877,12 @@ __global__ void __launch_bounds__(256) k_wpack(const PackList list) {
   const int tap = 2 * s + (g >> 1), ci = 16 * c + 8 * (g & 1);
   u32x4 v = u32x4{0u, 0u, 0u, 0u};
   if (tap < 27) {
-    float f[8];
+    W f[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e)
       f[e] = flip ? w[(size_t)(ci + e) * kpad + (26 - tap) * cin + co] : w[(size_t)co * kpad + tap * cin + ci + e];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = (uint32_t)to_bf16(f[2 * e]) | ((uint32_t)to_bf16(f[2 * e + 1]) << 16);
+    for (int e = 0; e < 4; ++e) v[e] = bf16_bits(f[2 * e]) | (bf16_bits(f[2 * e + 1]) << 16);
   }
   *reinterpret_cast<u32x4 *>((flip ? it.wt : it.wp) + (size_t)i * 8) = v;
 }
@@ -1719,6 +1723,27 @@ int relu_bias_plan(int64_t voxels, int C, int64_t &chunks, int64_t &per_block) {
   return (int)((chunks + per_block - 1) / per_block);
 }
 
+template <typename W>
+int wpack(void *stream, int32_t count, const lbm3d_conv_pack *layers) {
+  if (count < 0 || (count > 0 && !layers)) return cfail(LBM3D_EINVAL, "no layers");
+  for (int32_t k = 0; k < count; ++k) {
+    if (int rc = check_conv(1, 1, 1, 1, layers[k].cin, layers[k].cout, 3)) return rc;
+    if (!layers[k].w || !layers[k].wp) return cfail(LBM3D_EINVAL, "NULL tensor");
+  }
+  for (int32_t k0 = 0; k0 < count; k0 += kPackItems) {
+    PackList list{};
+    uint32_t blocks = 0;
+    for (int32_t k = k0; k < count && k < k0 + kPackItems; ++k) {
+      const lbm3d_conv_pack &l = layers[k];
+      list.item[list.n++] = PackItem{l.w, l.wp, l.wt, l.cin, l.cout, lbm3d_conv_kpad(l.cin, 3), blocks};
+      blocks += (uint32_t)(kSteps * (l.cin / 16) * (l.cout / 16) * 64 * (l.wt ? 2 : 1) + 255) / 256;
+    }
+    k_wpack<W><<<blocks, 256, 0, (hipStream_t)stream>>>(list);
+    if (int rc = ccheck("lbm3d_conv3d_wpack")) return rc;
+  }
+  return LBM3D_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1761,28 +1786,17 @@ int64_t lbm3d_conv3d_packed_elements(int32_t cin, int32_t cout) {
 }
 
 int lbm3d_conv3d_wpack_many(void *stream, int32_t count, const lbm3d_conv_pack *layers) {
-  if (count < 0 || (count > 0 && !layers)) return cfail(LBM3D_EINVAL, "no layers");
-  for (int32_t k = 0; k < count; ++k) {
-    if (int rc = check_conv(1, 1, 1, 1, layers[k].cin, layers[k].cout, 3)) return rc;
-    if (!layers[k].w || !layers[k].wp) return cfail(LBM3D_EINVAL, "NULL tensor");
-  }
-  for (int32_t k0 = 0; k0 < count; k0 += kPackItems) {
-    PackList list{};
-    uint32_t blocks = 0;
-    for (int32_t k = k0; k < count && k < k0 + kPackItems; ++k) {
-      const lbm3d_conv_pack &l = layers[k];
-      list.item[list.n++] = PackItem{l.w, l.wp, l.wt, l.cin, l.cout, lbm3d_conv_kpad(l.cin, 3), blocks};
-      blocks += (uint32_t)(kSteps * (l.cin / 16) * (l.cout / 16) * 64 * (l.wt ? 2 : 1) + 255) / 256;
-    }
-    k_wpack<<<blocks, 256, 0, (hipStream_t)stream>>>(list);
-    if (int rc = ccheck("lbm3d_conv3d_wpack")) return rc;
-  }
-  return LBM3D_OK;
+  return wpack<float>(stream, count, layers);
 }
 
 int lbm3d_conv3d_wpack(void *stream, const float *w, uint16_t *wp, uint16_t *wt, int32_t cin, int32_t cout) {
   const lbm3d_conv_pack one{w, wp, wt, cin, cout};
-  return lbm3d_conv3d_wpack_many(stream, 1, &one);
+  return wpack<float>(stream, 1, &one);
+}
+
+int lbm3d_conv3d_wpack_bf16(void *stream, const uint16_t *w, uint16_t *wp, uint16_t *wt, int32_t cin, int32_t cout) {
+  const lbm3d_conv_pack one{reinterpret_cast<const float *>(w), wp, wt, cin, cout};  // read as the BF16 it is
+  return wpack<uint16_t>(stream, 1, &one);
 }
 
 static int packed_call(const uint16_t *x, const uint16_t *wp, const float *bias, uint16_t *y, int32_t n, int32_t d,

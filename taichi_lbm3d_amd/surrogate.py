@@ -47,8 +47,9 @@ def _stream(dev):
 
 def _operand(t):
     """t contiguous and starting on 16 bytes, as the kernels that load straight to LDS read it."""
-    t = t.contiguous()
-    return t if t.data_ptr() % 16 == 0 else t.clone()
+    if t.is_contiguous() and not t.data_ptr() & 15:
+        return t
+    return t.clone(memory_format=_torch().contiguous_format)
 
 
 # ---- the convolution as an autograd function ----------------------------------------------
@@ -85,21 +86,30 @@ def conv_dgrad(dy, w_bf16, cin, ks):
 
 
 def pack_weights(w, flip: bool):
-    """FP32 3x3x3 weights (cout, kpad) as BF16 MFMA fragments: (forward, data
+    """FP32 or BF16 3x3x3 weights (cout, kpad) as BF16 MFMA fragments: (forward, data
     gradient or None)."""
-    return pack_layers([(w, flip)])[0]
+    torch = _torch()
+    cout, kpad = w.shape
+    cin = kpad // 27 // 16 * 16
+    n = 28 * cin * cout  # lbm3d_conv3d_packed_elements
+    buf = torch.empty(n * (2 if flip else 1), dtype=torch.bfloat16, device=w.device)
+    at = buf.data_ptr()
+    _lib.lib().call("lbm3d_conv3d_wpack_bf16" if w.dtype == torch.bfloat16 else "lbm3d_conv3d_wpack", _stream(w.device),
+                    w.data_ptr(), at, at + 2 * n if flip else None, cin, cout)
+    return (buf[:n], buf[n:]) if flip else (buf, None)
 
 
 def pack_layers(layers):
-    """pack_weights of several (w, flip), in one launch."""
+    """pack_weights of several (w, flip), all FP32, in one launch."""
     torch = _torch()
     lib = _lib.lib()
     if not layers:
         return []
     items, spans, total = (_lib.ConvPack * len(layers))(), [], 0
     for it, (w, flip) in zip(items, layers):
-        it.cout, it.cin = w.shape[0], w.shape[1] // 27 // 16 * 16
-        n = lib.size("lbm3d_conv3d_packed_elements", it.cin, it.cout)
+        cout, kpad = w.shape
+        it.cout, it.cin = cout, kpad // 27 // 16 * 16
+        n = 28 * it.cin * cout  # lbm3d_conv3d_packed_elements
         spans.append((total, n, flip))
         total += n * (2 if flip else 1)
     dev = layers[0][0].device
@@ -216,16 +226,17 @@ def _bf16(t):
 
 def _check_layer(x, cin, w, b, ks, given=None):
     """The kernels take a layer's shapes from x: its weights have to be of them, or they are read past their end."""
-    k = ks ** 3 * cin
+    k, shape = ks ** 3 * cin, w.shape
     kpad = (k + 31) // 32 * 32  # lbm3d_conv_kpad
-    if w.dim() != 2 or w.shape[1] != kpad:
-        raise ValueError(f"a layer of {cin} input channels takes weights (cout, {kpad}), got {tuple(w.shape)}")
-    if b is not None and b.numel() < w.shape[0]:
-        raise ValueError(f"{w.shape[0]} output channels take as many biases, got {b.numel()}")
-    if w.device != x.device or (b is not None and b.device != x.device):
-        raise ValueError(f"weights and biases have to be on the input's device {x.device}")
-    if given is not None and given[0].numel() != 28 * cin * w.shape[0]:
-        raise ValueError(f"the packed weights are not those of a layer {cin} -> {w.shape[0]}")
+    if len(shape) != 2 or shape[1] != kpad:
+        raise ValueError(f"a layer of {cin} input channels takes weights (cout, {kpad}), got {tuple(shape)}")
+    device = x.get_device()
+    if b is not None and (b.numel() < shape[0] or b.get_device() != device):
+        raise ValueError(f"{shape[0]} output channels take as many biases on {x.device}, got {b.numel()} on {b.device}")
+    if w.get_device() != device:
+        raise ValueError(f"the weights have to be on the input's device {x.device}")
+    if given is not None and given[0].numel() != 28 * cin * shape[0]:
+        raise ValueError(f"the packed weights are not those of a layer {cin} -> {shape[0]}")
 
 
 def _check_volume(x, what):
@@ -239,18 +250,23 @@ def _make_conv_functions():
     def packed(w, flip, given):  # given: the layer's fragments from pack_layers, or None
         if given is not None and (not flip or given[1] is not None):
             return given[0], given[1] if flip else None
-        w = w if w.dtype == torch.float32 else w.to(torch.bfloat16).float()
-        return pack_weights(w.contiguous(), flip)
+        return pack_weights((w if w.dtype == torch.float32 else w.to(torch.bfloat16)).contiguous(), flip)
 
     class Conv3dMFMA(torch.autograd.Function):
         """y = act(conv3d(x, w) + b) with the MFMA kernels in both directions."""
 
         @staticmethod
         def forward(ctx, x, w, b, ks, relu, need_dx, periodic, given):
+            x = x.contiguous()
             _check_layer(x, x.shape[-1], w, b, ks, given if ks == 3 else None)
-            x = _operand(x)
-            if ks == 3:
-                wp, wb = packed(w, need_dx and ctx.needs_input_grad[0], given)
+            # Weights that are not FP32 are read as rows where the kernels keep them in registers (few channels):
+            # BF16 ones 16 -> 16 channels at 6^3 voxels 13.5 us without the pass that packs them, 20 with it; but
+            # 128 -> 128 at 24^3 48 us against 30.
+            flip = need_dx and ctx.needs_input_grad[0]
+            ctx.packed = ks == 3 and (given is not None or w.dtype == torch.float32
+                                      or max(x.shape[-1], w.shape[0] if flip else 0) > 48)
+            if ctx.packed:
+                wp, wb = packed(w, flip, given)
                 y = conv_fwd_packed(x, wp, b, w.shape[0], relu, periodic)
             else:
                 wb = w.to(torch.bfloat16).contiguous()
@@ -268,7 +284,7 @@ def _make_conv_functions():
             dw = conv_wgrad(x, g, ctx.ks)
             dx = None
             if ctx.need_dx and ctx.needs_input_grad[0]:
-                dx = (conv_fwd_packed(g, wb, None, x.shape[-1], False) if ctx.ks == 3
+                dx = (conv_fwd_packed(g, wb, None, x.shape[-1], False) if ctx.packed
                       else conv_dgrad(g, wb, x.shape[-1], ctx.ks))
             return dx, dw, db, None, None, None, None, None
 
