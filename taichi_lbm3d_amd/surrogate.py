@@ -89,6 +89,9 @@ def pack_weights(w, flip: bool):
     """FP32 or BF16 3x3x3 weights (cout, kpad) as BF16 MFMA fragments: (forward, data
     gradient or None)."""
     torch = _torch()
+    if w.dim() != 2 or w.dtype not in (torch.float32, torch.bfloat16) or not w.is_contiguous():
+        raise ValueError("weights to pack have to be contiguous FP32 or BF16 (cout, kpad), got "
+                         f"{tuple(w.shape)} {w.dtype}")
     cout, kpad = w.shape
     cin = kpad // 27 // 16 * 16
     n = 28 * cin * cout  # lbm3d_conv3d_packed_elements
@@ -105,14 +108,16 @@ def pack_layers(layers):
     lib = _lib.lib()
     if not layers:
         return []
-    items, spans, total = (_lib.ConvPack * len(layers))(), [], 0
+    items, spans, total, dev = (_lib.ConvPack * len(layers))(), [], 0, layers[0][0].device
     for it, (w, flip) in zip(items, layers):
+        if w.dim() != 2 or w.dtype != torch.float32 or not w.is_contiguous() or w.device != dev:
+            raise ValueError("weights to pack have to be contiguous FP32 (cout, kpad) on one device, got "
+                             f"{tuple(w.shape)} {w.dtype}")
         cout, kpad = w.shape
         it.cout, it.cin = cout, kpad // 27 // 16 * 16
         n = 28 * it.cin * cout  # lbm3d_conv3d_packed_elements
         spans.append((total, n, flip))
         total += n * (2 if flip else 1)
-    dev = layers[0][0].device
     buf = torch.empty(total, dtype=torch.bfloat16, device=dev)
     for it, (w, _), (at, n, flip) in zip(items, layers, spans):
         it.w, it.wp = w.data_ptr(), buf.data_ptr() + 2 * at
@@ -125,6 +130,8 @@ def conv_fwd_packed(x, wp, bias, cout, relu, periodic=False):
     """conv_fwd with ks = 3 and the fragments of pack_weights."""
     torch = _torch()
     n, d, h, wd, cin = x.shape
+    if wp.numel() != 28 * cin * cout:
+        raise ValueError(f"the packed weights are not those of a layer {cin} -> {cout}")
     x = _operand(x)
     y = torch.empty((n, d, h, wd, cout), dtype=torch.bfloat16, device=x.device)
     flags = (CONV_RELU if relu else 0) | (CONV_PERIODIC if periodic else 0)

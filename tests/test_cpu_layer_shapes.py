@@ -57,3 +57,22 @@ def test_volumes_have_to_be_bfloat16(dtype):
         sg.conv3d_pool(vol(1, 4, 4, 4, 32, dtype), w, b)
     with pytest.raises(ValueError, match="bfloat16"):
         sg.conv_head(vol(1, 4, 4, 4, 32, dtype), torch.zeros(16, 32), b)
+
+
+@pytest.mark.parametrize("w", [weights(16, 32).half(), weights(16, 32).double(), weights(16, 32).t(),
+                               weights(16, 32)[:, ::2], weights(16, 32).view(-1)])
+def test_weights_that_cannot_be_packed_are_refused(w):
+    with pytest.raises(ValueError, match="pack"):
+        sg.pack_weights(w, True)
+    with pytest.raises(ValueError, match="pack"):
+        sg.pack_layers([(weights(16, 16), False), (w, True)])
+
+
+def test_a_convolution_takes_its_own_fragments():
+    with pytest.raises(ValueError, match="packed"):
+        sg.conv_fwd_packed(vol(1, 4, 4, 4, 32), torch.zeros(28 * 16 * 16, dtype=torch.bfloat16), None, 16, False)
+
+
+def test_layers_packed_together_are_fp32():
+    with pytest.raises(ValueError, match="pack"):
+        sg.pack_layers([(weights(16, 32).to(torch.bfloat16), True)])

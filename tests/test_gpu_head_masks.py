@@ -28,6 +28,7 @@ def test_any_mask_gives_the_same_fields(gpu, form):
     solid = (torch.rand((4, 5, 7), generator=torch.Generator().manual_seed(92)) < 0.4).to(gpu)
     want = sg.head_fields(x, wt, b, solid, (1, 0, 2), 2.0, 3.0, False)
     got = sg.head_fields(x, wt, b, forms(solid)[form], (1, 0, 2), 2.0, 3.0, False)
-    view = sg.head_fields(x.permute(1, 0, 2, 3).contiguous().permute(1, 0, 2, 3), wt, b, solid, (1, 0, 2), 2.0, 3.0, False)
+    turned = x.permute(1, 0, 2, 3).contiguous().permute(1, 0, 2, 3)
+    view = sg.head_fields(turned, wt, b, solid, (1, 0, 2), 2.0, 3.0, False)
     for g, v, e in zip(got, view, want):
         assert torch.equal(g, e) and torch.equal(v, e)
