@@ -216,17 +216,22 @@ __device__ __forceinline__ uint2 pack4(const f32x4 v) {
 
 // 1x1x1 convolutions: a matrix product of the voxels' channels, bound by its
 // bytes.  A wave computes 4 fragments of 16 voxels x NT of 16 output channels with
-// the weights as the A operand, so a lane has 4 channels of a voxel (8-byte
-// stores, whole lines per fragment) and all of a chunk's loads are in flight
-// together.  16 -> 16 channels at 2 x 128^3 (268 MB): 75 us with 2-byte stores and
-// an address from coordinates per load -> 48 us (5.6 TB/s).
+// the weights as the A operand, so a lane has 4 channels of a voxel, and all of a
+// chunk's loads are in flight together.  Two tiles' rows are interleaved by fours, so
+// that a lane has 8 consecutive channels of both and a store takes 16 bytes, 64 of a
+// voxel.  16 -> 16 channels at 2 x 128^3 (268 MB): 75 us with 2-byte stores and an
+// address from coordinates per load -> 48 us (5.6 TB/s).  16 -> 128 at 2 x 96^3: 253 us
+// with 2-byte stores, 337 with 8-byte ones of 32 bytes a voxel, 168 with 16-byte ones.
 template <int NT>
 __global__ void __launch_bounds__(256)
     k_conv1(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const float *__restrict__ bias,
             uint16_t *__restrict__ y, uint32_t vox, int cin, int cout, int kpad, int relu) {
+  constexpr int H = NT > 1 ? 2 : 1;  // tiles whose rows are interleaved
   const int lane = threadIdx.x & 63, g = lane >> 4, r16 = lane & 15;
   const uint32_t m0 = blockIdx.x * 256u + (threadIdx.x & ~63u) + (uint32_t)r16;
   const int co0 = blockIdx.y * 16 * NT;
+  // first of the 4 channels that rows 4 q .. 4 q + 3 of tile t stand for
+  const auto channel = [&](int t, int q) { return co0 + 16 * H * (t / H) + 4 * H * q + 4 * (t % H); };
   f32x4 acc[4][NT];
 #pragma unroll
   for (int f = 0; f < 4; ++f)
@@ -241,7 +246,8 @@ __global__ void __launch_bounds__(256)
       b[f] = m < vox && k < cin ? ld16(x + (size_t)m * cin + k) : u32x4{0u, 0u, 0u, 0u};
     }
 #pragma unroll
-    for (int t = 0; t < NT; ++t) a[t] = ld16(w + (size_t)(co0 + 16 * t + r16) * kpad + k);  // kpad: 32-multiple
+    for (int t = 0; t < NT; ++t)  // kpad: 32-multiple
+      a[t] = ld16(w + (size_t)(channel(t, r16 >> 2) + (r16 & 3)) * kpad + k);
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -250,14 +256,25 @@ __global__ void __launch_bounds__(256)
                                                             __builtin_bit_cast(bf16x8, b[f]), acc[f][t], 0, 0, 0);
   }
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int co = co0 + 16 * t + 4 * g;
-    f32x4 b4 = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (bias) b4 = f32x4{bias[co], bias[co + 1], bias[co + 2], bias[co + 3]};
+  for (int t = 0; t < NT; t += H) {
+    f32x4 b4[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int co = channel(t + h, g);
+      b4[h] = bias ? f32x4{bias[co], bias[co + 1], bias[co + 2], bias[co + 3]} : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
       const uint32_t m = m0 + 16u * f;
-      if (m < vox) *reinterpret_cast<uint2 *>(y + (size_t)m * cout + co) = pack4(finish4(acc[f][t], b4, relu));
+      if (m >= vox) continue;
+      uint16_t *const to = y + (size_t)m * cout + channel(t, g);
+      const uint2 lo = pack4(finish4(acc[f][t], b4[0], relu));
+      if constexpr (H == 2) {
+        const uint2 hi = pack4(finish4(acc[f][t + 1], b4[1], relu));
+        *reinterpret_cast<u32x4 *>(to) = u32x4{lo.x, lo.y, hi.x, hi.y};
+      } else {
+        *reinterpret_cast<uint2 *>(to) = lo;
+      }
     }
   }
 }
@@ -1033,15 +1050,18 @@ __global__ void __launch_bounds__(192 * WCO)
 // 1x1x1: workgroup (p, channel tiles): a run of bricks, staged one at a time in
 // 16 KB, so that eight workgroups' loads are in flight on a CU; wave w takes K
 // chunks 2w and 2w + 1 of each.  Partial sets: one per wave, part[4 p +
-// wave][co][kpad].  Bound by HBM.
+// wave][co][kpad].  Bound by HBM.  Jobs in the order of k_wgrad3's: 32 -> 32 at 2 x 128^3
+// 338 us with the tiles slowest, 139 with them fastest.
 __global__ void __launch_bounds__(256)
     k_wgrad1(const uint16_t *__restrict__ x, const uint16_t *__restrict__ dy, float *__restrict__ part, const Vol vol,
-             int cin, int cout, int kpad, const Bricks bk, uint32_t per_block) {
+             int cin, int cout, int kpad, const Bricks bk, uint32_t per_block, uint32_t n, Div tiles) {
   __shared__ u32x4 tile[1024];  // 256 voxels x 16 channels of x, then of dy
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r16 = lane & 15;
-  const int nci = cin / 16;
-  const int co0 = (int)(blockIdx.y / (unsigned)nci) * 16, c0 = (int)(blockIdx.y % (unsigned)nci) * 16;
+  const uint32_t job = xcd_block(LBM3D_CONV_WGRAD_XCD_CHUNK, blockIdx.x & 7u, blockIdx.x >> 3, n);
+  if (job >= n) return;  // padding block of the grid
+  const uint32_t set = qdiv(job, tiles), ct = job - set * tiles.d, nci = (uint32_t)cin / 16u;
+  const int co0 = (int)(ct / nci) * 16, c0 = (int)(ct % nci) * 16;
   auto load = [&](uint32_t brick) {
     const uint16_t *const zero = reinterpret_cast<const uint16_t *>(conv_zero);
     int bb, z0, y0, x0;
@@ -1059,7 +1079,7 @@ __global__ void __launch_bounds__(256)
   };
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
   const int off = (64 * wave + 8 * g + (r16 >> 2)) * 32 + 8 * (r16 & 3);
-  const uint32_t b0 = blockIdx.x * per_block, b1 = b0 + per_block < bk.n ? b0 + per_block : bk.n;
+  const uint32_t b0 = set * per_block, b1 = b0 + per_block < bk.n ? b0 + per_block : bk.n;
   const char *const p = reinterpret_cast<const char *>(tile) + off;
   for (uint32_t br = b0; br < b1; ++br) {
     if (br != b0) __syncthreads();  // the previous brick's reads are done
@@ -1071,7 +1091,7 @@ __global__ void __launch_bounds__(256)
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(read_tr(p + 8192 + 1024 * c, 128), read_tr(p + 1024 * c, 128), acc,
                                                     0, 0, 0);
   }
-  float *dst = part + ((size_t)blockIdx.x * 4 + wave) * cout * kpad + (size_t)(co0 + 4 * g) * kpad + c0 + r16;
+  float *dst = part + ((size_t)set * 4 + wave) * cout * kpad + (size_t)(co0 + 4 * g) * kpad + c0 + r16;
 #pragma unroll
   for (int e = 0; e < 4; ++e) dst[(size_t)e * kpad] = acc[e];
 }
@@ -1901,8 +1921,9 @@ static int wgrad_run(void *stream, const uint16_t *x, const uint16_t *dy, float 
   const int sets = wgrad_plan(bk, cin, cout, per), kpad = lbm3d_conv_kpad(cin, ks);
   float *part = (float *)workspace;
   if (ks == 1) {
-    k_wgrad1<<<dim3((unsigned)sets, (unsigned)((cout / 16) * (cin / 16))), 256, 0, s>>>(x, dy, part, vol, cin, cout,
-                                                                                      kpad, bk, per);
+    const uint32_t tiles = (uint32_t)((cout / 16) * (cin / 16)), jobs = (uint32_t)sets * tiles;
+    k_wgrad1<<<(unsigned)xcd_grid(jobs, LBM3D_CONV_WGRAD_XCD_CHUNK), 256, 0, s>>>(x, dy, part, vol, cin, cout, kpad, bk,
+                                                                              per, jobs, make_div(tiles));
   } else {
     // two output channel tiles a workgroup where there are, which share the staged x
     const int wco = cout % 32 == 0 ? 2 : 1;
