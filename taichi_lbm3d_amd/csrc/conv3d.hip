@@ -431,11 +431,14 @@ __device__ __forceinline__ void brick_origin(const Bricks &bk, uint32_t bi, int 
 // (4 x 10 x 18 voxels) is staged in one of two LDS buffers, straight from
 // memory; the next chunk's (or brick's) halo is loaded while the MFMAs of the
 // current one run, so a chunk has one barrier and no exposed load.  Weight
-// fragments are streamed kWRing - 1 steps ahead.
+// fragments are streamed kWRing - 1 steps ahead.  STAGE (weights as rows, one tile a
+// workgroup): a fragment comes from 32 places, too many for each of four waves to
+// fetch; they are staged with the halo, once for the workgroup (80 -> 80 channels at
+// 2 x 64^3 467 -> 296 us, 64 -> 64 at 2 x 24^3 28 -> 25).
 // Bound by the MFMAs (half the LDS reads, with two channel tiles a wave, 145 -> 143
 // us for 192 -> 64, but 382 -> 400 for 96 -> 32 at 2 x 96^3): 192 -> 64 channels at 2 x 48^3 take 150 us (980 TFLOP/s) against 305
 // for one 16-channel tile per workgroup with its halo loaded behind a barrier.
-template <int CT, int MODE>
+template <int CT, int MODE, bool STAGE>
 __global__ void __launch_bounds__(256, 2)
     k_conv3(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, int packed,
             const float *__restrict__ bias, uint16_t *__restrict__ y, const Vol vol, int cin, int cout, int kpad,
@@ -444,6 +447,7 @@ __global__ void __launch_bounds__(256, 2)
   // [voxel][16 channels as two 16-byte halves]; two arrays, so that a read of
   // one never waits for the loads into the other
   __shared__ u32x4 haloA[kHaloBuf], haloB[kHaloBuf];
+  __shared__ u32x4 fragA[STAGE ? kSteps * 64 : 1], fragB[STAGE ? kSteps * 64 : 1];  // [step][lane]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r16 = lane & 15;
   const int half = g & 1, second = g >> 1;  // channel half and tap parity of this lane's K values
@@ -454,8 +458,18 @@ __global__ void __launch_bounds__(256, 2)
 
   const Weights weight(w, packed, cin, cout, kpad, tile, lane);
   u32x4 wr[kWRing];
+  if constexpr (!STAGE) {
 #pragma unroll
-  for (int s = 0; s < kWRing - 1; ++s) wr[s] = weight(0, s);
+    for (int s = 0; s < kWRing - 1; ++s) wr[s] = weight(0, s);
+  }
+  auto load_weights = [&](int c, u32x4 *frag) {
+    const uint16_t *const row = w + ((size_t)(16 * tile + r16) * kpad + second * cin + 8 * half + 16 * c);
+    for (int s = wave; s < kSteps; s += 4) {
+      const uint16_t *const src = s == kSteps - 1 && second ? reinterpret_cast<const uint16_t *>(conv_zero)
+                                                            : row + 2 * s * cin;
+      __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)(frag + 64 * s), 16, 0, 0);
+    }
+  };
 
   // halo loads of one brick: entry e = 256 q + thread is half e & 1 of halo
   // voxel e / 2; its voxel index in the volume, or -1 outside it
@@ -487,6 +501,7 @@ __global__ void __launch_bounds__(256, 2)
     }
   };
   auto load_halo = [&](int c, u32x4 *buf) {
+    if constexpr (STAGE) load_weights(c, buf == haloA ? fragA : fragB);
 #pragma unroll
     for (int q = 0; q < kHaloLoads; ++q) {
       const uint16_t *src = xv + ((int64_t)hvox[q] * c_skip + 16 * (c - nlow) + 8 * ((int)threadIdx.x & 1));
@@ -523,11 +538,14 @@ __global__ void __launch_bounds__(256, 2)
       }
     };
     read_group(0);
+    if constexpr (STAGE) wr[0] = (buf == haloA ? fragA : fragB)[lane];
 #pragma unroll
     for (int k = 0; k < NG; ++k) {
       if (k + 1 < NG) read_group(k + 1);
       const int s = k / GS;
-      if (k % GS == 0) {  // the fragment kWRing - 1 steps on, of this, the next or the next brick's first chunk
+      if constexpr (STAGE) {
+        if (k % GS == 0 && s + 1 < kSteps) wr[(s + 1) % kWRing] = (buf == haloA ? fragA : fragB)[64 * (s + 1) + lane];
+      } else if (k % GS == 0) {  // the fragment kWRing - 1 steps on, of this, the next or the next brick's first chunk
         const int sn = s + kWRing - 1;
         const int cn = sn < kSteps ? c : (c + 1 < nch ? c + 1 : 0);
         wr[sn % kWRing] = weight(cn, sn % kSteps);
@@ -1647,16 +1665,16 @@ struct ConvCall {
   ConvExtra ex;
 };
 
-template <int CT, int MODE>
+template <int CT, int MODE, bool STAGE = false>
 void launch_conv3_bricks(hipStream_t s, const ConvCall &a, const Bricks &bk) {
   const unsigned gy = (unsigned)(a.cout / (16 * CT));
-  // persistent workgroups: as many as are resident (3 per CU by LDS, 2 where the
-  // kernel takes more than 168 VGPRs), in whole groups of 8 XCDs
-  const int64_t resident = (CT == 1 || (CT == 2 && MODE != kUp) ? 768 : 512) / gy;
+  // persistent workgroups: as many as are resident (3 per CU by LDS, 2 with staged
+  // weights or where the kernel takes more than 168 VGPRs), in whole groups of 8 XCDs
+  const int64_t resident = ((CT == 1 && !STAGE) || (CT == 2 && MODE != kUp) ? 768 : 512) / gy;
   int64_t gx = xcd_grid(bk.n, LBM3D_CONV_XCD_CHUNK);
   if (gx > resident) gx = resident & ~int64_t(7);
   if (gx < 8) gx = 8;
-  k_conv3<CT, MODE><<<dim3((unsigned)gx, gy), 256, 0, s>>>(a.x, a.w, a.packed, a.bias, a.y, a.vol, a.cin, a.cout,
+  k_conv3<CT, MODE, STAGE><<<dim3((unsigned)gx, gy), 256, 0, s>>>(a.x, a.w, a.packed, a.bias, a.y, a.vol, a.cin, a.cout,
                                                            a.kpad, a.relu, bk, a.ex);
 }
 
@@ -1728,6 +1746,7 @@ int launch_conv3(hipStream_t s, const ConvCall &a) {
   while (ct > 1 && (int64_t)bk.n * (tiles / ct) < 512) ct >>= 1;
   if (ct == 4) launch_conv3_bricks<4, MODE>(s, a, bk);
   else if (ct == 2) launch_conv3_bricks<2, MODE>(s, a, bk);
+  else if (MODE == kPlain && !a.packed) launch_conv3_bricks<1, MODE, MODE == kPlain>(s, a, bk);
   else launch_conv3_bricks<1, MODE>(s, a, bk);
   return ccheck("lbm3d_conv3d_fwd");
 }
