@@ -119,8 +119,7 @@ __device__ __forceinline__ uint16_t to_bf16(float f) {
 // Forward: y[v][co] = act(sum_{tap, ci} x[v + off(tap)][ci] * w[co][tap*cin + ci] + bias[co])
 // MFMA 16x16x32 lane layout: A (16 x 32): lane l holds row l%16, k = 8*(l/16) .. +7;
 // B (32 x 16): column l%16, the same k; C (16 x 16): column l%16, rows 4*(l/16) .. +3.
-// ---------------------------------------------------------------------------
-// ---------------------------------------------------------------------------
+//
 // Forward 3x3x3 convolutions.  Both kernels below compute, per wave, fragments
 // of 16 voxels (one x row) x 16 output channels.  K runs over chunks of 16
 // input channels x 27 taps, 14 MFMA steps of two taps each (the 28th slot is
@@ -364,14 +363,15 @@ __device__ __forceinline__ f32x4 max4(const f32x4 a, const f32x4 b) {
   return f32x4{fmaxf(a[0], b[0]), fmaxf(a[1], b[1]), fmaxf(a[2], b[2]), fmaxf(a[3], b[3])};
 }
 
-// the maximum over an x pair of voxels (lanes r16 and r16 ^ 1)
-__device__ __forceinline__ f32x4 other_x(f32x4 v) {  // the value of the other voxel of the x pair
+// the value of the other voxel of an x pair (lanes r16 and r16 ^ 1)
+__device__ __forceinline__ f32x4 other_x(f32x4 v) {
   f32x4 o;
 #pragma unroll
   for (int e = 0; e < 4; ++e)  // quad_perm [1, 0, 3, 2]
     o[e] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v[e]), 0xB1, 0xF, 0xF, true));
   return o;
 }
+// the maximum over the pair
 __device__ __forceinline__ f32x4 max_xpair(f32x4 v) { return max4(v, other_x(v)); }
 
 // The sum over a 2 x 2 x 2 block of voxels rounded to BF16, at its even x, in the
@@ -436,8 +436,9 @@ __device__ __forceinline__ void brick_origin(const Bricks &bk, uint32_t bi, int 
 // fetch; they are staged with the halo, once for the workgroup (80 -> 80 channels at
 // 2 x 64^3 467 -> 296 us, 64 -> 64 at 2 x 24^3 28 -> 25).
 // Bound by the MFMAs (half the LDS reads, with two channel tiles a wave, 145 -> 143
-// us for 192 -> 64, but 382 -> 400 for 96 -> 32 at 2 x 96^3): 192 -> 64 channels at 2 x 48^3 take 150 us (980 TFLOP/s) against 305
-// for one 16-channel tile per workgroup with its halo loaded behind a barrier.
+// us for 192 -> 64, but 382 -> 400 for 96 -> 32 at 2 x 96^3): 192 -> 64 channels at
+// 2 x 48^3 take 150 us (980 TFLOP/s) against 305 for one 16-channel tile per workgroup
+// with its halo loaded behind a barrier.
 template <int CT, int MODE, bool STAGE>
 __global__ void __launch_bounds__(256, 2)
     k_conv3(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, int packed,
@@ -1544,7 +1545,6 @@ struct PoolGrad {
   Div pieces;  // by C / 8
 };
 
-//
 // kGradHead: g is the FP32 gradient of k_head's 4 channels; dz is it in BF16 as the
 // first 4 of 16 channels (the others zero), and there is no ReLU.
 enum GradMode { kGradPlain = 0, kGradPool = 1, kGradHead = 2 };

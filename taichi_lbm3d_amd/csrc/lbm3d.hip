@@ -1017,9 +1017,10 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
 // cell or later mark it, and a cell counts the marks up to its own.  Two LDS round
 // trips in place of 12 dependent lane permutes (a suffix minimum and a binary
 // search); with the divisions gone from here and tile_stage and the neighbour lookup
-// below 600 vector instructions a wave from 759 (FP16, stochastic rounding).  Odd
-// steps: 256^3 pack in FP32 197 -> 190 us, 211 x 187 x 203 in FP16 61 -> 57, the
-// 131 x 67 x 93 channel in FP64 40.0 -> 38.2, the 50^3 cavity 10.6 -> 9.9.
+// below 600 vector instructions a wave from 759 (FP16, stochastic rounding).  All of
+// it together, odd steps traced in turn on one card: 256^3 pack in FP32 192.0 -> 188.5
+// us (steps of both parities 163.6 -> 162.1), 211 x 187 x 203 in FP16 63 -> 59, the
+// 131 x 67 x 93 channel in FP64 40.8 -> 39.5, the 50^3 cavity 10.7 -> 9.9.
 // Every lane of the wave must call it.
 __device__ __forceinline__ void tile_place(const Geo &gm, const uint4 *win, const TileSegs &t, uint32_t x,
                                            RowView &rv) {
