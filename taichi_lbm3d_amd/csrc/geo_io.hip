@@ -126,13 +126,12 @@ __global__ void __launch_bounds__(256)
 // side of a closed surface; a smaller kFar leaves more nodes open where surfaces meet.
 // Lengths are in cells, relative to the parent's centre.
 // Bound by FP32 arithmetic.  7,680 triangles on 96 x 104 x 88 nodes: every node in FP64
-// 33.2 ms, this 1.4 ms.
-// Measured before the children's sums were taken together: every triangle for every child
-// 3.2 ms; kFar 10.5 to 12 1.65 ms, 9 1.87 ms and 16 1.74 ms.  With corners from FP64
-// differences and near triangles as they come kFar 12 took 2.02 ms, 6 8.3 ms.  Loading the
-// next triangle ahead changed nothing.
+// 33.2 ms, every triangle for every child 3.2 ms, kFar 8 / 9 / 10 / 11 / 12 1.37 / 1.35 /
+// 1.36 / 1.40 / 1.45 ms; 1,000 triangles of 6 cells on 48^3 560 / 522 / 462 / 425 / 393 us.
+// With corners from FP64 differences and near triangles as they come (kFar 12) 2.02 ms
+// instead of 1.65; loading the next triangle ahead changed nothing.
 // ---------------------------------------------------------------------------
-constexpr float kFar = 11.f;
+constexpr float kFar = 10.f;
 
 struct VoxGrid {
   double x0, y0, z0, dx;
