@@ -105,14 +105,17 @@ def pack_weights(w, flip: bool):
 def pack_layers(layers):
     """pack_weights of several (w, flip), all FP32, in one launch."""
     torch = _torch()
-    lib = _lib.lib()
-    if not layers:
-        return []
-    items, spans, total, dev = (_lib.ConvPack * len(layers))(), [], 0, layers[0][0].device
-    for it, (w, flip) in zip(items, layers):
-        if w.dim() != 2 or w.dtype != torch.float32 or not w.is_contiguous() or w.device != dev:
+    for w, _ in layers:
+        if w.dim() != 2 or w.dtype != torch.float32 or not w.is_contiguous() or w.device != layers[0][0].device:
             raise ValueError("weights to pack have to be contiguous FP32 (cout, kpad) on one device, got "
                              f"{tuple(w.shape)} {w.dtype}")
+    return _pack_layers(layers) if layers else []
+
+
+def _pack_layers(layers):
+    torch = _torch()
+    items, spans, total, dev = (_lib.ConvPack * len(layers))(), [], 0, layers[0][0].device
+    for it, (w, flip) in zip(items, layers):
         cout, kpad = w.shape
         it.cout, it.cin = cout, kpad // 27 // 16 * 16
         n = 28 * it.cin * cout  # lbm3d_conv3d_packed_elements
@@ -122,17 +125,20 @@ def pack_layers(layers):
     for it, (w, _), (at, n, flip) in zip(items, layers, spans):
         it.w, it.wp = w.data_ptr(), buf.data_ptr() + 2 * at
         it.wt = it.wp + 2 * n if flip else None
-    lib.call("lbm3d_conv3d_wpack_many", _stream(dev), len(layers), items)
+    _lib.lib().call("lbm3d_conv3d_wpack_many", _stream(dev), len(layers), items)
     return [(buf[at:at + n], buf[at + n:at + 2 * n] if flip else None) for at, n, flip in spans]
 
 
 def conv_fwd_packed(x, wp, bias, cout, relu, periodic=False):
     """conv_fwd with ks = 3 and the fragments of pack_weights."""
+    if wp.numel() != 28 * x.shape[-1] * cout:
+        raise ValueError(f"the packed weights are not those of a layer {x.shape[-1]} -> {cout}")
+    return _conv_fwd_packed(_operand(x), wp, bias, cout, relu, periodic)
+
+
+def _conv_fwd_packed(x, wp, bias, cout, relu, periodic=False):
     torch = _torch()
     n, d, h, wd, cin = x.shape
-    if wp.numel() != 28 * cin * cout:
-        raise ValueError(f"the packed weights are not those of a layer {cin} -> {cout}")
-    x = _operand(x)
     y = torch.empty((n, d, h, wd, cout), dtype=torch.bfloat16, device=x.device)
     flags = (CONV_RELU if relu else 0) | (CONV_PERIODIC if periodic else 0)
     _lib.lib().call("lbm3d_conv3d_fwd_packed", _stream(x.device), _vp(x), _vp(wp),
@@ -141,8 +147,11 @@ def conv_fwd_packed(x, wp, bias, cout, relu, periodic=False):
 
 
 def conv_wgrad(x, dy, ks):
+    return _conv_wgrad(_operand(x), _operand(dy), ks)
+
+
+def _conv_wgrad(x, dy, ks):
     torch = _torch()
-    x, dy = _operand(x), _operand(dy)
     n, d, h, wd, cin = x.shape
     cout = dy.shape[-1]
     lib = _lib.lib()
@@ -264,8 +273,7 @@ def _make_conv_functions():
 
         @staticmethod
         def forward(ctx, x, w, b, ks, relu, need_dx, periodic, given):
-            x = x.contiguous()
-            _check_layer(x, x.shape[-1], w, b, ks, given if ks == 3 else None)
+            x = _operand(x)
             # Weights that are not FP32 are read as rows where the kernels keep them in registers (few channels):
             # BF16 ones 16 -> 16 channels at 6^3 voxels 13.5 us without the pass that packs them, 20 with it; but
             # 128 -> 128 at 24^3 48 us against 30.
@@ -274,7 +282,7 @@ def _make_conv_functions():
                                       or max(x.shape[-1], w.shape[0] if flip else 0) > 48)
             if ctx.packed:
                 wp, wb = packed(w, flip, given)
-                y = conv_fwd_packed(x, wp, b, w.shape[0], relu, periodic)
+                y = _conv_fwd_packed(x, wp, b, w.shape[0], relu, periodic)
             else:
                 wb = w.to(torch.bfloat16).contiguous()
                 y = conv_fwd(x, wb, b, w.shape[0], ks, relu, periodic)
@@ -288,10 +296,10 @@ def _make_conv_functions():
                 raise NotImplementedError("periodic convolutions are forward-only (inference)")
             x, wb, y = ctx.saved_tensors
             g, db = relu_bias_grad(_bf16(gy), y if ctx.relu else None)
-            dw = conv_wgrad(x, g, ctx.ks)
+            dw = _conv_wgrad(x, g, ctx.ks)
             dx = None
             if ctx.need_dx and ctx.needs_input_grad[0]:
-                dx = (conv_fwd_packed(g, wb, None, x.shape[-1], False) if ctx.packed
+                dx = (_conv_fwd_packed(g, wb, None, x.shape[-1], False) if ctx.packed
                       else conv_dgrad(g, wb, x.shape[-1], ctx.ks))
             return dx, dw, db, None, None, None, None, None
 
@@ -300,8 +308,6 @@ def _make_conv_functions():
 
         @staticmethod
         def forward(ctx, x, w, b, periodic, given):
-            _check_volume(x, "the input")
-            _check_layer(x, x.shape[-1], w, b, 3, given)
             x = _operand(x)
             n, d, h, wd, cin = x.shape
             cout = w.shape[0]
@@ -320,8 +326,8 @@ def _make_conv_functions():
                 raise NotImplementedError("periodic convolutions are forward-only (inference)")
             x, wt, y, pooled = ctx.saved_tensors
             g, db = relu_pool_grad(_bf16(gy), _bf16(g_pool), y, pooled)
-            dw = conv_wgrad(x, g, 3)
-            dx = conv_fwd_packed(g, wt, None, x.shape[-1], False) if ctx.needs_input_grad[0] else None
+            dw = _conv_wgrad(x, g, 3)
+            dx = _conv_fwd_packed(g, wt, None, x.shape[-1], False) if ctx.needs_input_grad[0] else None
             return dx, dw, db, None, None
 
     class ConvUp(torch.autograd.Function):
@@ -329,14 +335,6 @@ def _make_conv_functions():
 
         @staticmethod
         def forward(ctx, low, skip, w, b, periodic, given):
-            _check_volume(low, "the low part")
-            _check_volume(skip, "the skip part")
-            if low.shape[0] != skip.shape[0] or any(a != e // 2 for a, e in zip(low.shape[1:4], skip.shape[1:4])):
-                raise ValueError(f"the low part {tuple(low.shape)} does not fit the skip part {tuple(skip.shape)}: "
-                                 "as many volumes of half the extents")
-            if low.device != skip.device:
-                raise ValueError(f"the parts are on {low.device} and {skip.device}")
-            _check_layer(skip, low.shape[-1] + skip.shape[-1], w, b, 3, given)
             low, skip = _operand(low), _operand(skip)
             n, d, h, wd, c_skip = skip.shape
             cout = w.shape[0]
@@ -375,10 +373,6 @@ def _make_conv_functions():
 
         @staticmethod
         def forward(ctx, x, w, b):
-            if x.dtype != torch.bfloat16 or w.shape[0] != HEAD_PAD:
-                raise ValueError(f"the head takes bfloat16 and {HEAD_PAD} rows of weights, got {x.dtype}, "
-                                 f"{tuple(w.shape)}")
-            _check_layer(x, x.shape[-1], w, b, 1)
             x = _operand(x)
             wb = w.to(torch.bfloat16).contiguous()
             ctx.save_for_backward(x, wb)
@@ -388,7 +382,7 @@ def _make_conv_functions():
         def backward(ctx, gy):
             x, wb = ctx.saved_tensors
             g, db = head_grad(gy.contiguous())
-            dw = conv_wgrad(x, g, 1)
+            dw = _conv_wgrad(x, g, 1)
             dx = conv_dgrad(g, wb, x.shape[-1], 1) if ctx.needs_input_grad[0] else None
             return dx, dw, db
 
@@ -407,21 +401,35 @@ def _conv_functions():
 
 def conv3d(x, w, b, ks: int = 3, relu: bool = True, need_dx: bool = True, periodic: bool = False, packed=None):
     """act(conv(x, w) + b); packed: the weights' pack_layers entry, if there is one."""
+    _check_layer(x, x.shape[-1], w, b, ks, packed if ks == 3 else None)
     return _conv_functions()[0].apply(x, w, b, ks, relu, need_dx, periodic, packed)
 
 
 def conv3d_pool(x, w, b, periodic: bool = False, packed=None):
     """(y, its 2x2x2 maximum) of a 3x3x3 layer with ReLU; even extents."""
+    _check_volume(x, "the input")
+    _check_layer(x, x.shape[-1], w, b, 3, packed)
     return _conv_functions()[1].apply(x, w, b, periodic, packed)
 
 
 def conv3d_up(low, skip, w, b, periodic: bool = False, packed=None):
     """A 3x3x3 layer with ReLU on the concatenation of `low`, upsampled by 2 (nearest), and `skip`."""
+    _check_volume(low, "the low part")
+    _check_volume(skip, "the skip part")
+    if low.shape[0] != skip.shape[0] or any(a != e // 2 for a, e in zip(low.shape[1:4], skip.shape[1:4])):
+        raise ValueError(f"the low part {tuple(low.shape)} does not fit the skip part {tuple(skip.shape)}: "
+                         "as many volumes of half the extents")
+    if low.device != skip.device:
+        raise ValueError(f"the parts are on {low.device} and {skip.device}")
+    _check_layer(skip, low.shape[-1] + skip.shape[-1], w, b, 3, packed)
     return _conv_functions()[2].apply(low, skip, w, b, periodic, packed)
 
 
 def conv_head(x, w, b):
     """The network's head: (..., C) bf16 -> (..., 4) float32."""
+    if x.dtype != _torch().bfloat16 or w.shape[0] != HEAD_PAD:
+        raise ValueError(f"the head takes bfloat16 and {HEAD_PAD} rows of weights, got {x.dtype}, {tuple(w.shape)}")
+    _check_layer(x, x.shape[-1], w, b, 1)
     return _conv_functions()[3].apply(x, w, b)
 
 
@@ -475,10 +483,14 @@ class UNet3D:
         """Every 3x3x3 layer's weight fragments by name: the data gradient's too where one will be taken."""
         torch = _torch()
         ws = {n: self.params[n + ".w"] for n, (_, _, ks) in self.specs.items() if ks == 3}
-        if not all(w.dtype == torch.float32 and w.is_contiguous() for w in ws.values()):
-            return {}  # a layer at a time
+        index = next(iter(ws.values())).get_device()
+        for n, w in ws.items():
+            cin, cout, _ = self.specs[n]
+            if w.dtype != torch.float32 or not w.is_contiguous() or w.get_device() != index \
+                    or w.shape != (cout, (27 * cin + 31) // 32 * 32):
+                return {}  # a layer at a time, each checked by itself
         grad = torch.is_grad_enabled()
-        return dict(zip(ws, pack_layers([(w.detach(), grad and n != "e1a") for n, w in ws.items()])))
+        return dict(zip(ws, _pack_layers([(w.detach(), grad and n != "e1a") for n, w in ws.items()])))
 
     def forward(self, x, periodic: bool = False):
         """x (N,X,Y,Z,16) bf16 with channels 0-1 the inputs -> (N,X,Y,Z,4) float32.
@@ -490,18 +502,23 @@ class UNet3D:
     def _features(self, x, p):
         """The last layer's output before the head, (N,X,Y,Z,C) bf16; p: periodic."""
         packs = self._packed()
+        _check_volume(x, "the network's input")
+        _check_layer(x, x.shape[-1], self.params["e1a.w"], self.params["e1a.b"], 3)
+        # layers that packed fit each other: without the checks of the public calls, 2 us each (a step on 2 x 72^3
+        # is bound by the host)
+        plain, pooled, joined = (f.apply for f in _conv_functions()[:3]) if packs else (conv3d, conv3d_pool, conv3d_up)
 
         def conv(name, x, need_dx=True):
-            return conv3d(x, *layer(name), 3, True, need_dx, p, packs.get(name))
+            return plain(x, *layer(name), 3, True, need_dx, p, packs.get(name))
 
         def layer(name):
             return self.params[name + ".w"], self.params[name + ".b"]
 
         def level(a, b, x, need_dx=True):  # of the encoder: its output, and pooled
-            return conv3d_pool(conv(a, x, need_dx), *layer(b), p, packs.get(b))
+            return pooled(conv(a, x, need_dx), *layer(b), p, packs.get(b))
 
         def up(a, b, low, skip):  # of the decoder
-            return conv(b, conv3d_up(low, skip, *layer(a), p, packs.get(a)))
+            return conv(b, joined(low, skip, *layer(a), p, packs.get(a)))
 
         e1, low = level("e1a", "e1b", x, False)
         e2, low = level("e2a", "e2b", low)
